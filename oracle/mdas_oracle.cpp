@@ -716,6 +716,40 @@ void orc_eval_scene_grouped(const void* params, const void* coords, int dim, lon
     }
 }
 
+// The same through the sets of spheres by cell; returns the number of cells
+// (0: the scene has none).
+int orc_eval_scene_cells(const void* params, const void* coords, int dim, long long count, int fp64,
+                         void* values) {
+    const mscene::Params& P = *(const mscene::Params*)params;
+    mscene::Accel A;
+    mscene::build_accel(P, &A);
+    mscene::Cells C;
+    mscene::describe_cells(P, &C);
+    std::vector<uint64_t> tab((size_t)C.n_cells * C.words);
+#pragma omp parallel for schedule(dynamic, 1024) num_threads(nthreads())
+    for (long long i = 0; i < (long long)tab.size(); ++i)
+        tab[i] = mscene::cell_word(P, C, (int)(i / C.words), (int)(i % C.words));
+#pragma omp parallel for schedule(dynamic, 1024) num_threads(nthreads())
+    for (long long k = 0; k < count; ++k) {
+        if (fp64) {
+            const mscene::V3<double> v =
+                mscene::eval<double>(P, P.obj, (const double*)coords + k * dim, &A, &C, tab.data());
+            double* o = (double*)values + 3 * k;
+            o[0] = v.x;
+            o[1] = v.y;
+            o[2] = v.z;
+        } else {
+            const mscene::V3<float> v =
+                mscene::eval<float>(P, P.obj, (const float*)coords + k * dim, &A, &C, tab.data());
+            float* o = (float*)values + 3 * k;
+            o[0] = v.x;
+            o[1] = v.y;
+            o[2] = v.z;
+        }
+    }
+    return C.words > 0 ? C.n_cells : 0;
+}
+
 float orc_halton(int dim, int i) { return halton<float>(dim, i); }
 
 void orc_qmc_image(const void* params, int w, int h, int spp, int first, uint32_t frame, int fp64,

@@ -61,6 +61,8 @@ void orc_eval_scene_f64(const void* scene_params, const double* coords, int dim,
  * restatement of the reference. */
 void orc_eval_scene_grouped(const void* scene_params, const void* coords, int dim,
                             long long count, int fp64, void* values);
+int orc_eval_scene_cells(const void* scene_params, const void* coords, int dim, long long count,
+                         int fp64, void* values);
 /* The plain QMC sampler's image (cuda/sampler.h:4-28, random.h:74-89,
  * whitted.cu:59-69): float4 pixels (fp64 = 0) or double4 (fp64 = 1). */
 void orc_qmc_image(const void* scene_params, int w, int h, int spp, int first_sample,

@@ -36,6 +36,7 @@ _SIGS = {
     "orc_eval_scene": (None, [_P, _P, _I, _LL, _LL, _P]),
     "orc_eval_scene_f64": (None, [_P, _P, _I, _LL, _P]),
     "orc_eval_scene_grouped": (None, [_P, _P, _I, _LL, _I, _P]),
+    "orc_eval_scene_cells": (_I, [_P, _P, _I, _LL, _I, _P]),
     "orc_qmc_image": (None, [_P, _I, _I, _I, _I, _U, _I, _P]),
     "orc_halton": (_F, [_I, _I]),
     "orc_eval_range": (None, [_P, _P, _LL, _LL]),
@@ -232,6 +233,16 @@ def eval_scene_grouped(params, coords, dim, fp64=False):
     out = np.empty((len(c), 3), t)
     load().orc_eval_scene_grouped(params, vp(c), dim, len(c), 1 if fp64 else 0, vp(out))
     return out
+
+
+def eval_scene_cells(params, coords, dim, fp64=False):
+    """(values, cells): the integrand through the product's sphere sets by
+    cell (CPU build), to be held against eval_scene / eval_scene_f64."""
+    t = np.float64 if fp64 else np.float32
+    c = np.ascontiguousarray(coords, t).reshape(-1, dim)
+    out = np.empty((len(c), 3), t)
+    n = load().orc_eval_scene_cells(params, vp(c), dim, len(c), 1 if fp64 else 0, vp(out))
+    return out, n
 
 
 def qmc_image(params, w, h, spp, first_sample=0, frame=0, fp64=False):

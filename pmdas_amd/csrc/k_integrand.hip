@@ -1,8 +1,13 @@
 // Analytic integrand launch: the replacement of optixLaunch over the new
 // sample slice (optixMotionBlur.cpp:458-467 with sample_offset/sample_count,
-// SDK/cuda/whitted.cu:164-293).  The scene's object table (<= 12 KB) and its
-// sphere groups (2.5 KB) are staged in LDS once per workgroup; every thread
-// then evaluates samples grid-stride.
+// SDK/cuda/whitted.cu:164-293).  The scene's object table (<= 12 KB) is staged
+// in LDS once per workgroup that has a sample; every thread then evaluates
+// samples grid-stride.  A ray looks its spheres up by cell (scenes.hpp): what
+// bounds the kernel is the serial chain of a ray's sphere tests and its lanes'
+// divergence, so fewer tests per ray beat any arrangement of them.  Against
+// group tests over all spheres: the 5D 1080p run's 41 launches 7.53 -> 2.79 ms,
+// a launch for the ~500 samples of a thumbnail's pass 38 -> 10 us, the FP64
+// ground truth at 240x135, 64 samples per pixel 2.28 -> 0.49 ms.
 #include "mdas_device.hpp"
 #include "mdas_internal.hpp"
 #include "scenes.hpp"
@@ -11,16 +16,17 @@
 
 namespace mdas {
 
-// The scene's object table and groups into LDS (every thread of the
-// workgroup takes part).
-__device__ __forceinline__ void stage_scene(const mscene::SceneBlock* __restrict__ B, float* obj,
-                                            mscene::Accel* acc) {
+// The scene's object table into LDS (every thread of the workgroup takes
+// part).
+__device__ __forceinline__ void stage_scene(const mscene::SceneBlock* __restrict__ B, float* obj) {
     const int nobj = B->p.n_obj;
     for (int k = threadIdx.x; k < nobj * mscene::OBJ_STRIDE; k += blockDim.x) obj[k] = B->p.obj[k];
-    const int* src = reinterpret_cast<const int*>(&B->accel);
-    int* dst = reinterpret_cast<int*>(acc);
-    for (int k = threadIdx.x; k < (int)(sizeof(mscene::Accel) / 4); k += blockDim.x) dst[k] = src[k];
     __syncthreads();
+}
+
+// The cells' words follow the scene block.
+__device__ __forceinline__ const uint64_t* cell_words(const mscene::SceneBlock* B) {
+    return reinterpret_cast<const uint64_t*>(B + 1);
 }
 
 __device__ __forceinline__ void eval_body(const float* __restrict__ coords,
@@ -29,21 +35,20 @@ __device__ __forceinline__ void eval_body(const float* __restrict__ coords,
                                           int count, const DevCounters* cnt, int dev_range, int blk,
                                           int nblk) {
     __shared__ float obj[mscene::MAX_OBJ * mscene::OBJ_STRIDE];
-    __shared__ mscene::Accel acc;
     int beg = first, end = first + count;
     if (dev_range) {
         if (cnt->done) return;
         beg = cnt->n_samples_old;
         end = cnt->n_samples;
     }
-    if (beg >= end) return;
-    stage_scene(B, obj, &acc);
+    if (blk * 256 >= end - beg) return;  // uniform: no sample for this workgroup
+    stage_scene(B, obj);
     const mscene::Params* P = &B->p;
     for (int i = beg + blk * 256 + threadIdx.x; i < end; i += nblk * 256) {
         float x[6];
         const float* c = coords + (size_t)i * dim;
         for (int d = 0; d < dim; ++d) x[d] = c[d];
-        mscene::V3<float> v = mscene::eval<float>(*P, obj, x, &acc);
+        mscene::V3<float> v = mscene::eval<float>(*P, obj, x, &B->accel, &B->cells, cell_words(B));
         float* o = values + (size_t)i * 3;
         o[0] = v.x;
         o[1] = v.y;
@@ -63,6 +68,28 @@ __global__ __launch_bounds__(256) void k_eval_b(const DevGrid* grids, const void
     const DevGrid& a = grids[blockIdx.y];
     eval_body(a.coords, a.values, a.D, (const mscene::SceneBlock*)params[blockIdx.y], 0, 0, a.cnt,
               1, blockIdx.x, gridDim.x);
+}
+
+// The words of a scene's cells (scenes.hpp), once per scene: a wave per word,
+// a lane per sphere (a thread per word, its 64 spheres one after another, took
+// 40 us on the 64-sphere scenes).
+__global__ __launch_bounds__(256) void k_scene_cells(mscene::SceneBlock* B) {
+    const mscene::Cells& C = B->cells;
+    uint64_t* tab = reinterpret_cast<uint64_t*>(B + 1);
+    const int n = C.n_cells * C.words, lane = threadIdx.x & 63;
+    for (int i = blockIdx.x * 4 + (threadIdx.x >> 6); i < n; i += gridDim.x * 4) {
+        const int c = i / C.words, k = 64 * (i % C.words) + lane;
+        const uint64_t word = __ballot(k < B->p.n_obj && mscene::cell_holds(B->p, C, c, k));
+        if (lane == 0) tab[i] = word;
+    }
+}
+
+hipError_t launch_scene_cells(void* dparams, int words, hipStream_t st) {
+    if (words <= 0) return hipSuccess;
+    const int blocks = (words + 3) / 4;
+    hipLaunchKernelGGL(k_scene_cells, dim3(blocks < 2048 ? blocks : 2048), dim3(256), 0, st,
+                       (mscene::SceneBlock*)dparams);
+    return hipGetLastError();
 }
 
 // ------------------------------------------------- QMC and ground truth --
@@ -92,8 +119,7 @@ __global__ __launch_bounds__(256) void k_qmc_image(const mscene::SceneBlock* __r
                                                    int W, int H, int spp, int first_sample,
                                                    unsigned frame, real* out) {
     __shared__ float obj[mscene::MAX_OBJ * mscene::OBJ_STRIDE];
-    __shared__ mscene::Accel acc;
-    stage_scene(B, obj, &acc);
+    stage_scene(B, obj);
     const mscene::Params* P = &B->p;
     const int dim = P->dim;
     for (int pix = blockIdx.x * 256 + threadIdx.x; pix < W * H; pix += gridDim.x * 256) {
@@ -111,7 +137,7 @@ __global__ __launch_bounds__(256) void k_qmc_image(const mscene::SceneBlock* __r
             }
             x[0] = ((real)px + x[0]) * (real)P->scale_x / (real)W;
             x[1] = ((real)py + x[1]) * (real)P->scale_y / (real)H;
-            const mscene::V3<real> v = mscene::eval<real>(*P, obj, x, &acc);
+            const mscene::V3<real> v = mscene::eval<real>(*P, obj, x, &B->accel, &B->cells, cell_words(B));
             ax += v.x;
             ay += v.y;
             az += v.z;

@@ -671,13 +671,18 @@ int mdas_scene_create(int kind, uint32_t seed, int dim, float sx, float sy, mdas
     if (dim < need[kind] || dim > 6) return fail(MDAS_ERR_INVALID, "scene needs more dimensions");
     mdas_scene* s = new mdas_scene;
     mscene::make_scene(&s->host, kind, seed, dim, sx, sy);
-    // the device copy: the parameters followed by the sphere groups
+    // the device copy: the parameters, the sphere groups and the cells, whose
+    // words a kernel fills (other streams read them: complete on return)
     std::vector<mscene::SceneBlock> blk(1);
     blk[0].p = s->host;
     mscene::build_accel(s->host, &blk[0].accel);
-    hipError_t e = hipMalloc(&s->dev, sizeof(mscene::SceneBlock));
+    mscene::describe_cells(s->host, &blk[0].cells);
+    const int words = blk[0].cells.n_cells * blk[0].cells.words;
+    hipError_t e = hipMalloc(&s->dev, sizeof(mscene::SceneBlock) + sizeof(uint64_t) * (size_t)words);
     if (e == hipSuccess)
         e = hipMemcpy(s->dev, blk.data(), sizeof(mscene::SceneBlock), hipMemcpyHostToDevice);
+    if (e == hipSuccess) e = mdas::launch_scene_cells(s->dev, words, nullptr);
+    if (e == hipSuccess && words > 0) e = hipStreamSynchronize(nullptr);
     if (e != hipSuccess) {
         if (s->dev) hipFree(s->dev);
         delete s;

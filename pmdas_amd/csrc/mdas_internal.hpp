@@ -253,6 +253,8 @@ hipError_t launch_pass_b(int D, const DevGrid* grids, int n, int blocks, hipStre
                          const LearnDev* learns = nullptr);
 
 // Integrand (k_integrand.hip)
+// Fills the `words` words of the cells that follow a scene block.
+hipError_t launch_scene_cells(void* dparams, int words, hipStream_t st);
 hipError_t launch_eval(Grid& g, const void* dparams, int first, int count, bool dev_range,
                        hipStream_t st);
 // Batched integrand over the new slice of every grid; params[i] is image i's

@@ -18,6 +18,7 @@
 // The `real` template parameter also gives an FP64 evaluation of the same
 // scene, used for high-sample-count ground-truth images.
 #pragma once
+#include <stddef.h>
 #include <stdint.h>
 
 #if defined(__HIPCC__)
@@ -205,11 +206,143 @@ struct Accel {
     int32_t member[MAX_OBJ];     // sphere indices, group by group
 };
 
-// A scene as the integrand kernels read it: the parameters, then the groups.
+// --------------------------------------------------- sphere sets by cell --
+// Tables that name, for the rays a sample can send, the spheres they can
+// meet, one bit per sphere.  The groups above still cost a ray 8 to 32 group
+// tests and the members of every group that it passes; with a set looked up
+// by where the ray starts it tests 2 to 3 spheres on average.
+//
+//  * Camera cells: CAM_T x CAM_T cells of the image times the shutter bins.
+//    A ray of image position (dx, dy) passes its focus point and a lens
+//    point, so at depth z it lies within h z + a |1 - z / f| of its cell's
+//    centre ray (h the cell's half diagonal at depth 1, a the lens radius, f
+//    the focus distance).
+//  * Light cells (directional light): LGT_T x LGT_T cells of the plane
+//    across the light, times the shutter bins, by the projection of the
+//    shadow ray's start.
+//  * Ambient-occlusion cells: AO_T^3 cells over the ray's start, the spheres
+//    within the ray's length of the cell.
+//
+// A sphere is left out only where its own test (hit_sphere, in the ray's own
+// arithmetic) reports no hit, by the bound of the groups above: it can report
+// a root only for |X_perp| <= r + sqrt(G), G = (2e-6 + |e|) |X|^2; the lookups
+// require |e| <= kCellE for the camera rays and the light, kCellAoE for the
+// occlusion rays (their root t <= tmax puts a point within
+// r + sqrt(|e| t^2 + 4e-6 |X|^2) of the centre), and the tables widen every
+// sphere by that and kCellSlack.  Spheres are tested in index order, so ties
+// fall as in the plain loop.  Rays outside these conditions (coordinates out
+// of their ranges, far starts) take the groups.
+static const int CAM_T = 64, LGT_T = 64, AO_T = 24;
+static const int MAX_TBINS = 4;
+constexpr double kCellE = 1e-6, kCellAoE = 2.5e-3, kCellSlack = 0.005;
+
+struct Cells {
+    int32_t words;      // 64-bit words of a cell's set; 0: no tables
+    int32_t tbins;      // shutter bins (1: the spheres rest)
+    int32_t sec;        // first cell of the light / occlusion cells
+    int32_t n_cells;    // cells in all
+    float bound[4];     // sphere around every sphere's sweep
+    float reach;        // light cells hold for starts within reach of its centre
+    float lo[3];        // corner of the light / occlusion cells
+    float inv[3];       // cells per unit
+    float e1[3], e2[3]; // axes of the plane across the light
+    float pad[2];
+};
+
+// A scene as the integrand kernels read it: the parameters, the groups, and
+// the cells' description; the cells' words follow the block.
 struct SceneBlock {
     Params p;
     Accel accel;
+    Cells cells;
 };
+
+MDAS_HD int imin(int a, int b) { return a < b ? a : b; }
+
+// Sphere k over shutter bin tb: centre of its sweep and radius around it.
+MDAS_HD double cell_sphere(const Params& P, const Cells& C, int k, int tb, double* m) {
+    const float* s = P.obj + k * OBJ_STRIDE;
+    // only the motion-blurred scene moves its spheres (the others trace at t = 0)
+    const double t0 = P.kind == SCENE_SPHERES_MBDOF ? (double)tb / C.tbins - 1e-6 : 0.0;
+    const double t1 = P.kind == SCENE_SPHERES_MBDOF ? (double)(tb + 1) / C.tbins + 1e-6 : 0.0;
+    double vv = 0.0;
+    for (int a = 0; a < 3; ++a) {
+        m[a] = (double)s[a] + (double)s[4 + a] * 0.5 * (t0 + t1);
+        vv += (double)s[4 + a] * (double)s[4 + a];
+    }
+    return (double)s[3] + 0.5 * (t1 - t0) * __builtin_sqrt(vv);
+}
+
+// Whether the rays of cell c can meet sphere k.
+MDAS_HD bool cell_holds(const Params& P, const Cells& C, int c, int k) {
+    const bool cam = c < C.sec;
+    const int q = cam ? c : c - C.sec;
+    double m[3];
+    if (cam) {
+        const int ix = q % CAM_T, iy = q / CAM_T % CAM_T;
+        const double R0 = cell_sphere(P, C, k, q / (CAM_T * CAM_T), m);
+        for (int a = 0; a < 3; ++a) m[a] -= (double)P.eye[a];
+        const double a = P.lens_radius > 0.0f ? (double)P.lens_radius : 0.0, f = (double)P.focal_distance;
+        const double mm = m[0] * m[0] + m[1] * m[1] + m[2] * m[2], l = __builtin_sqrt(mm);
+        const double R = R0 + __builtin_sqrt(2e-6 + kCellE) * (l + R0 + a + 1.0) + kCellSlack;
+        const double hx = (double)P.tan_x / CAM_T + 1e-5, hy = (double)P.tan_y / CAM_T + 1e-5;
+        const double h = __builtin_sqrt(hx * hx + hy * hy);
+        const double cx = ((2.0 * ix + 1.0) / CAM_T - 1.0) * (double)P.tan_x;
+        const double cy = ((2.0 * iy + 1.0) / CAM_T - 1.0) * (double)P.tan_y;
+        const double z0 = m[2] - R, z1 = m[2] + R;
+        const double l0 = 1.0 - z0 / f, l1 = 1.0 - z1 / f;
+        const double d0 = h * z0 + a * (l0 < 0.0 ? -l0 : l0), d1 = h * z1 + a * (l1 < 0.0 ? -l1 : l1);
+        const double reach = R + (d0 > d1 ? d0 : d1);  // the deviation is convex in z
+        const double p = (m[0] * cx + m[1] * cy + m[2]);
+        // squared distance of the centre from the cell's centre ray
+        const double perp = mm - p * p / (cx * cx + cy * cy + 1.0);
+        return z0 < 0.1 || !(perp > reach * reach);
+    } else if (P.kind == SCENE_AO) {
+        const int i[3] = {q % AO_T, q / AO_T % AO_T, q / (AO_T * AO_T)};
+        const double R0 = cell_sphere(P, C, k, 0, m), D = (double)P.ao_radius;
+        const double R = R0 + D * (1.0 + kCellAoE) + __builtin_sqrt(kCellAoE * D * D + 4e-6 * 4.0 * (D + R0) * (D + R0)) + kCellSlack;
+        double d2 = 0.0;
+        for (int a = 0; a < 3; ++a) {
+            const double b0 = (double)C.lo[a] + i[a] / (double)C.inv[a], b1 = (double)C.lo[a] + (i[a] + 1) / (double)C.inv[a];
+            const double d = m[a] < b0 ? b0 - m[a] : (m[a] > b1 ? m[a] - b1 : 0.0);
+            d2 += d * d;
+        }
+        return d2 <= R * R;
+    } else {
+        const int ix = q % LGT_T, iy = q / LGT_T % LGT_T;
+        const double R0 = cell_sphere(P, C, k, q / (LGT_T * LGT_T), m);
+        const double R = R0 + __builtin_sqrt(2e-6 + kCellE) * ((double)C.reach + (double)C.bound[3]) + kCellSlack;
+        const double x = m[0] * C.e1[0] + m[1] * C.e1[1] + m[2] * C.e1[2];
+        const double y = m[0] * C.e2[0] + m[1] * C.e2[1] + m[2] * C.e2[2];
+        const double x0 = C.lo[0] + ix / (double)C.inv[0], x1 = C.lo[0] + (ix + 1) / (double)C.inv[0];
+        const double y0 = C.lo[1] + iy / (double)C.inv[1], y1 = C.lo[1] + (iy + 1) / (double)C.inv[1];
+        const double dx = x < x0 ? x0 - x : (x > x1 ? x - x1 : 0.0);
+        const double dy = y < y0 ? y0 - y : (y > y1 ? y - y1 : 0.0);
+        return dx * dx + dy * dy <= R * R;
+    }
+}
+
+// Word w of cell c: bit k - 64 w for sphere k of [64 w, 64 w + 64).
+MDAS_HD uint64_t cell_word(const Params& P, const Cells& C, int c, int w) {
+    uint64_t bits = 0;
+    for (int k = 64 * w; k < imin(P.n_obj, 64 * w + 64); ++k)
+        if (cell_holds(P, C, c, k)) bits |= (uint64_t)1 << (k - 64 * w);
+    return bits;
+}
+
+// The set of a camera ray's cell, from the image position (u, v) in [0, 1],
+// the lens sample and the time; null without tables or out of their ranges.
+template <typename real>
+MDAS_HD const uint64_t* camera_cell(const Cells* C, const uint64_t* tab, real u, real v, real lu,
+                                    real lv, real t) {
+    if (C == nullptr || C->words == 0) return nullptr;
+    const real z = (real)0, o = (real)1;
+    if (!(u >= z && u <= o && v >= z && v <= o && lu >= z && lu <= o && lv >= z && lv <= o && t >= z && t <= o))
+        return nullptr;
+    const int ix = imin((int)(u * (real)CAM_T), CAM_T - 1), iy = imin((int)(v * (real)CAM_T), CAM_T - 1);
+    const int tb = imin((int)(t * (real)C->tbins), C->tbins - 1);
+    return tab + (size_t)((tb * CAM_T + iy) * CAM_T + ix) * C->words;
+}
 
 // Whether a member of group g may report a hit in (tmin, tmax) for the ray
 // (o, d); e = |d.d - 1|.
@@ -228,15 +361,31 @@ MDAS_HD bool group_may_hit(const float* g, V3<real> o, V3<real> d, real e, real 
 
 // Closest hit among spheres (centres moved to time t) and the ground plane.
 // Returns the hit distance (tmax on a miss); *id = sphere index, -1 plane, -2 miss.
-// With groups (A != null, A->n_grp > 0) the spheres of the groups the ray can
-// meet are tested group by group; the result is the same.
+// With a cell's set (of `words` words) only its spheres are tested; else with
+// groups (A != null, A->n_grp > 0) the spheres of the groups the ray can meet,
+// group by group; the result is the same.
 template <typename real>
 MDAS_HD real trace(const Params& P, const float* obj, V3<real> o, V3<real> d, real t,
-                   real tmin, real tmax, int* id, const Accel* A = nullptr) {
+                   real tmin, real tmax, int* id, const Accel* A = nullptr,
+                   const uint64_t* cell = nullptr, int words = 0) {
     real best = tmax;
     *id = -2;
-    if (A != nullptr && A->n_grp > 0) {
-        const real e = r_abs(dot3(d, d) - (real)1);
+    const real e = r_abs(dot3(d, d) - (real)1);
+    if (cell != nullptr && e <= (real)kCellE) {
+        for (int w = 0; w < words; ++w) {
+            uint64_t m = cell[w];
+            while (m != 0) {
+                const int k = 64 * w + __builtin_ctzll(m);
+                m &= m - 1;
+                const float* s = obj + k * OBJ_STRIDE;
+                real cx = (real)s[0] + (real)s[4] * t;
+                real cy = (real)s[1] + (real)s[5] * t;
+                real cz = (real)s[2] + (real)s[6] * t;
+                real th = hit_sphere(o, d, cx, cy, cz, (real)s[3], tmin, best);
+                if (th < best) { best = th; *id = k; }
+            }
+        }
+    } else if (A != nullptr && A->n_grp > 0) {
         for (int g = 0; g < A->n_grp; ++g) {
             if (!group_may_hit(A->grp + 4 * g, o, d, e, tmin, best)) continue;
             const int j0 = A->range[2 * g], j1 = j0 + A->range[2 * g + 1];
@@ -301,13 +450,70 @@ MDAS_HD bool occluded(const Params& P, const float* obj, V3<real> o, V3<real> d,
     return false;
 }
 
+// Any hit in (tmin, tmax) among the spheres of a cell's set.
+template <typename real>
+MDAS_HD bool occluded_by_set(const float* obj, V3<real> o, V3<real> d, real t, real tmin, real tmax,
+                             const uint64_t* cell, int words) {
+    for (int w = 0; w < words; ++w) {
+        uint64_t m = cell[w];
+        while (m != 0) {
+            const float* s = obj + (64 * w + __builtin_ctzll(m)) * OBJ_STRIDE;
+            m &= m - 1;
+            real cx = (real)s[0] + (real)s[4] * t;
+            real cy = (real)s[1] + (real)s[5] * t;
+            real cz = (real)s[2] + (real)s[6] * t;
+            if (hit_sphere(o, d, cx, cy, cz, (real)s[3], tmin, tmax) < tmax) return true;
+        }
+    }
+    return false;
+}
+
+// occluded() of a shadow ray towards the directional light (no plane) by the
+// light cells: no hit where the ray passes all the spheres by or where its
+// start projects outside the cells, the groups where the start is far away.
+template <typename real>
+MDAS_HD bool occluded_light(const Params& P, const float* obj, V3<real> o, V3<real> d, real t,
+                            real tmax, const Accel* A, const Cells* C, const uint64_t* tab) {
+    if (C == nullptr || C->words == 0 || !(t >= (real)0 && t <= (real)1))
+        return occluded(P, obj, o, d, t, (real)0, tmax, false, A);
+    if (!group_may_hit(C->bound, o, d, r_abs(dot3(d, d) - (real)1), (real)0, tmax)) return false;
+    const real x = o.x - (real)C->bound[0], y = o.y - (real)C->bound[1], z = o.z - (real)C->bound[2];
+    if (!(x * x + y * y + z * z <= (real)C->reach * (real)C->reach))
+        return occluded(P, obj, o, d, t, (real)0, tmax, false, A);
+    const real a = (dot3(o, v3((real)C->e1[0], (real)C->e1[1], (real)C->e1[2])) - (real)C->lo[0]) * (real)C->inv[0];
+    const real b = (dot3(o, v3((real)C->e2[0], (real)C->e2[1], (real)C->e2[2])) - (real)C->lo[1]) * (real)C->inv[1];
+    if (!(a >= (real)0 && a < (real)LGT_T && b >= (real)0 && b < (real)LGT_T)) return false;
+    const int tb = imin((int)(t * (real)C->tbins), C->tbins - 1);
+    const int c = C->sec + (tb * LGT_T + (int)b) * LGT_T + (int)a;
+    return occluded_by_set(obj, o, d, t, (real)0, tmax, tab + (size_t)c * C->words, C->words);
+}
+
+// The spheres' part of occluded() for an occlusion ray of length P.ao_radius
+// (at t = 0) by the occlusion cells: no hit for a start outside them.
+template <typename real>
+MDAS_HD bool occluded_near(const Params& P, const float* obj, V3<real> o, V3<real> d, const Accel* A,
+                           const Cells* C, const uint64_t* tab) {
+    const real tmax = (real)P.ao_radius;
+    const real e = r_abs(dot3(d, d) - (real)1);
+    if (C == nullptr || C->words == 0 || !(e <= (real)kCellAoE))
+        return occluded(P, obj, o, d, (real)0, (real)0, tmax, false, A);
+    const real a = (o.x - (real)C->lo[0]) * (real)C->inv[0];
+    const real b = (o.y - (real)C->lo[1]) * (real)C->inv[1];
+    const real c = (o.z - (real)C->lo[2]) * (real)C->inv[2];
+    const real n = (real)AO_T;
+    if (!(a >= (real)0 && a < n && b >= (real)0 && b < n && c >= (real)0 && c < n)) return false;
+    const int q = C->sec + ((int)c * AO_T + (int)b) * AO_T + (int)a;
+    return occluded_by_set(obj, o, d, (real)0, (real)0, tmax, tab + (size_t)q * C->words, C->words);
+}
+
 // Lambertian shading of a directional-light scene (DOF and MB+DOF scenes).
 template <typename real>
 MDAS_HD V3<real> shade_spheres(const Params& P, const float* obj, V3<real> o, V3<real> d,
-                               real t, const Accel* A) {
+                               real t, const Accel* A, const uint64_t* cell, const Cells* C,
+                               const uint64_t* tab) {
     int id;
     const real big = (real)1e30;
-    real th = trace(P, obj, o, d, t, (real)1e-3, big, &id, A);
+    real th = trace(P, obj, o, d, t, (real)1e-3, big, &id, A, cell, C != nullptr ? C->words : 0);
     if (id == -2) {
         real a = (real)0.5 * (d.y + (real)1);
         return v3((real)1 - a * (real)0.5, (real)1 - a * (real)0.3, (real)1);
@@ -333,7 +539,7 @@ MDAS_HD V3<real> shade_spheres(const Params& P, const float* obj, V3<real> o, V3
     if (ndl > (real)0) {
         real eps = (real)1e-3;
         V3<real> so = v3(p.x + eps * n.x, p.y + eps * n.y, p.z + eps * n.z);
-        if (!occluded(P, obj, so, l, t, (real)0, big, false, A)) direct = ndl;
+        if (!occluded_light(P, obj, so, l, t, big, A, C, tab)) direct = ndl;
     }
     real amb = (real)P.ambient;
     return v3(ar * (amb + direct * (real)P.light_color[0]),
@@ -342,23 +548,23 @@ MDAS_HD V3<real> shade_spheres(const Params& P, const float* obj, V3<real> o, V3
 }
 
 // Evaluate one sample.  `x` holds P.dim coordinates; A: the scene's sphere
-// groups, or null to test every sphere.
+// groups, or null to test every sphere; C, tab: its cells and their words, or
+// null.
 template <typename real>
 MDAS_HD V3<real> eval(const Params& P, const float* obj, const real* x,
-                      const Accel* A = nullptr) {
-    real dx = (real)2 * (x[0] / (real)P.scale_x) - (real)1;
-    real dy = (real)2 * (x[1] / (real)P.scale_y) - (real)1;
+                      const Accel* A = nullptr, const Cells* C = nullptr,
+                      const uint64_t* tab = nullptr) {
+    const real u = x[0] / (real)P.scale_x, v = x[1] / (real)P.scale_y;
+    real dx = (real)2 * u - (real)1;
+    real dy = (real)2 * v - (real)1;
     switch (P.kind) {
     case SCENE_CONSTANT:
         return v3((real)P.constant[0], (real)P.constant[1], (real)P.constant[2]);
     case SCENE_RAMP:
-        return v3(x[0] / (real)P.scale_x, x[1] / (real)P.scale_y,
-                  P.dim > 2 ? x[2] : (real)0);
+        return v3(u, v, P.dim > 2 ? x[2] : (real)0);
     case SCENE_DISKS_MB: {
         // screen space [0,1)^2, disks moving linearly over the shutter t in [0,1);
         // the highest index on top.
-        real u = x[0] / (real)P.scale_x;
-        real v = x[1] / (real)P.scale_y;
         real t = x[2];
         for (int k = P.n_obj - 1; k >= 0; --k) {
             const float* s = obj + k * OBJ_STRIDE;
@@ -373,19 +579,20 @@ MDAS_HD V3<real> eval(const Params& P, const float* obj, const real* x,
     case SCENE_SPHERES_DOF: {
         V3<real> o, d;
         camera_ray(P, dx, dy, x[2], x[3], true, &o, &d);
-        return shade_spheres(P, obj, o, d, (real)0, A);
+        return shade_spheres(P, obj, o, d, (real)0, A, camera_cell(C, tab, u, v, x[2], x[3], (real)0), C, tab);
     }
     case SCENE_SPHERES_MBDOF: {
         V3<real> o, d;
         camera_ray(P, dx, dy, x[3], x[4], true, &o, &d);
-        return shade_spheres(P, obj, o, d, x[2], A);
+        return shade_spheres(P, obj, o, d, x[2], A, camera_cell(C, tab, u, v, x[3], x[4], x[2]), C, tab);
     }
     case SCENE_AO: {
         V3<real> o, d;
         camera_ray(P, dx, dy, x[2], x[3], true, &o, &d);
         int id;
         const real big = (real)1e30;
-        real th = trace(P, obj, o, d, (real)0, (real)1e-3, big, &id, A);
+        real th = trace(P, obj, o, d, (real)0, (real)1e-3, big, &id, A,
+                        camera_cell(C, tab, u, v, x[2], x[3], (real)0), C != nullptr ? C->words : 0);
         if (id == -2) return v3((real)1, (real)1, (real)1);
         V3<real> p = v3(o.x + th * d.x, o.y + th * d.y, o.z + th * d.z);
         V3<real> n;
@@ -412,7 +619,11 @@ MDAS_HD V3<real> eval(const Params& P, const float* obj, const real* x,
                         hx * t1.z + hy * t2.z + hz * n.z);
         real eps = (real)1e-3;
         V3<real> so = v3(p.x + eps * n.x, p.y + eps * n.y, p.z + eps * n.z);
-        bool occ = occluded(P, obj, so, w, (real)0, (real)0, (real)P.ao_radius, true, A);
+        bool occ = occluded_near(P, obj, so, w, A, C, tab);
+        if (!occ && w.y != (real)0) {  // the plane
+            real tp = ((real)P.plane_y - so.y) / w.y;
+            occ = tp > (real)0 && tp < (real)P.ao_radius;
+        }
         real vis = occ ? (real)0 : (real)1;
         return v3(vis, vis, vis);
     }
@@ -608,6 +819,85 @@ inline void build_accel(const Params& P, Accel* A) {
         for (int j = gb[g]; j < ge[g]; ++j) A->member[pos++] = idx[j];
     }
     A->n_grp = ng;
+}
+
+// Describes the cells of a sphere scene (cell_word then gives their words);
+// words = 0 where the tables do not apply.
+inline void describe_cells(const Params& P, Cells* C) {
+    char* raw = (char*)C;
+    for (unsigned i = 0; i < sizeof(Cells); ++i) raw[i] = 0;
+    if (P.kind != SCENE_SPHERES_DOF && P.kind != SCENE_SPHERES_MBDOF && P.kind != SCENE_AO) return;
+    if (P.n_obj <= 0 || P.n_obj > MAX_OBJ || !(P.focal_distance > 0.0f)) return;
+    C->tbins = P.kind == SCENE_SPHERES_MBDOF ? MAX_TBINS : 1;
+    // box around the sweeps, then the sphere around its centre
+    double lo[3], hi[3];
+    for (int pass = 0; pass < 2; ++pass) {
+        double R = 0.0;
+        for (int k = 0; k < P.n_obj; ++k) {
+            const float* s = P.obj + k * OBJ_STRIDE;
+            double d2 = 0.0, vv = 0.0;
+            for (int a = 0; a < 3; ++a) vv += (double)s[4 + a] * (double)s[4 + a];
+            const double ext = (double)s[3] + 0.5 * __builtin_sqrt(vv);
+            for (int a = 0; a < 3; ++a) {
+                const double m = (double)s[a] + 0.5 * (double)s[4 + a];
+                if (pass == 0) {
+                    lo[a] = k == 0 || m - ext < lo[a] ? m - ext : lo[a];
+                    hi[a] = k == 0 || m + ext > hi[a] ? m + ext : hi[a];
+                } else {
+                    d2 += (m - (double)C->bound[a]) * (m - (double)C->bound[a]);
+                }
+            }
+            const double r = __builtin_sqrt(d2) + ext;
+            R = r > R ? r : R;
+        }
+        if (pass == 0)
+            for (int a = 0; a < 3; ++a) C->bound[a] = (float)(0.5 * (lo[a] + hi[a]));
+        else
+            C->bound[3] = (float)(R * (1.0 + 1e-6) + 1e-6);
+    }
+    const double R = (double)C->bound[3];
+    C->reach = (float)(2.0 * R + 8.0);
+    if (!(R < 1e3)) return;  // not a scene the tables resolve
+    C->sec = C->tbins * CAM_T * CAM_T;
+    if (P.kind == SCENE_AO) {
+        // starts farther from every sphere than a ray's length see none
+        const double D = (double)P.ao_radius;
+        const double w = D * (1.0 + kCellAoE) + __builtin_sqrt(kCellAoE) * D + 0.004 * (D + R) + 2.0 * kCellSlack;
+        for (int a = 0; a < 3; ++a) {
+            const double b0 = lo[a] - w, b1 = hi[a] + w;
+            C->lo[a] = (float)(b0 - 1e-3);
+            C->inv[a] = (float)(AO_T / (b1 - b0 + 2e-3));
+        }
+        C->n_cells = C->sec + AO_T * AO_T * AO_T;
+    } else {
+        const double l[3] = {P.light_dir[0], P.light_dir[1], P.light_dir[2]};
+        const double ll = l[0] * l[0] + l[1] * l[1] + l[2] * l[2];
+        if (!(ll > 1.0 - kCellE && ll < 1.0 + kCellE)) return;
+        // the two axes: across the light and across the coordinate it is least along
+        int j = 0;
+        for (int a = 1; a < 3; ++a)
+            if (l[a] * l[a] < l[j] * l[j]) j = a;
+        double e1[3] = {0.0, 0.0, 0.0}, n = 0.0;
+        e1[(j + 1) % 3] = -l[(j + 2) % 3];
+        e1[(j + 2) % 3] = l[(j + 1) % 3];
+        for (int a = 0; a < 3; ++a) n += e1[a] * e1[a];
+        for (int a = 0; a < 3; ++a) e1[a] /= __builtin_sqrt(n);
+        const double e2[3] = {l[1] * e1[2] - l[2] * e1[1], l[2] * e1[0] - l[0] * e1[2], l[0] * e1[1] - l[1] * e1[0]};
+        double c[2] = {0.0, 0.0};
+        for (int a = 0; a < 3; ++a) {
+            C->e1[a] = (float)e1[a];
+            C->e2[a] = (float)e2[a];
+            c[0] += (double)C->bound[a] * e1[a];
+            c[1] += (double)C->bound[a] * e2[a];
+        }
+        const double w = R + __builtin_sqrt(2e-6 + kCellE) * ((double)C->reach + R) + 2.0 * kCellSlack;
+        for (int a = 0; a < 2; ++a) {
+            C->lo[a] = (float)(c[a] - w);
+            C->inv[a] = (float)(LGT_T / (2.0 * w));
+        }
+        C->n_cells = C->sec + C->tbins * LGT_T * LGT_T;
+    }
+    C->words = (P.n_obj + 63) / 64;
 }
 
 }  // namespace mscene
