@@ -431,7 +431,7 @@ __global__ __launch_bounds__(256) void k_mlp_forward(MlpDev M, const float* __re
             mlp_stage_row(M, f, &xs[w][lane * kMlpIn]);
         }
         float y[4];
-        mlp16(M, xs[w], acts[w], y, nullptr);
+        mlp16(M, xs[w], acts[w], y);
         if ((lane & 15) == 0) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
@@ -451,118 +451,260 @@ hipError_t launch_mlp_forward(const MlpDev& M, const float* X, long long n, floa
     return hipGetLastError();
 }
 
-// Gradient of mean((y - t)^2) over a batch.  Each wave runs the MFMA forward
-// of its 16-row tiles (keeping Z1, A1, Z2, A2 in LDS), then the backward in
-// FP32: lane k owns hidden unit k of both layers, i.e. column k of dW2,
-// row k of dW1, and entry k of db1, db2, dw3; W2's column k stays in
-// registers for dA1 = W2^T dZ2.  Each wave writes its partial gradient and
-// squared-error sum; the sums over waves run in a fixed order afterwards.
-__global__ __launch_bounds__(256) void k_mlp_grad(MlpDev M, const float* __restrict__ X,
-                                                  const float* __restrict__ T, long long n_rows,
-                                                  long long start, int count,
-                                                  unsigned long long pa, unsigned long long pc,
-                                                  float* __restrict__ gpart,
-                                                  float* __restrict__ lpart) {
-    __shared__ float xs[4][16 * kMlpIn];
-    __shared__ float sv[4][16 * 256];
-    __shared__ float dz[4][16 * kMlpH];
-    __shared__ float dys[4][16];
+// Gradient of mean((y - t)^2) over a batch.  A wave takes 16 rows at a time:
+// the bf16 MFMA forward, then the backward in FP32 on
+// v_mfma_f32_16x16x4_f32.  All of a tile stays in registers in the layout the
+// products leave (lane l: rows 4 (l/16) + i, column l%16): a K step that
+// takes row 4 (l/16) + i from lane group l/16 is step i's register of both
+// operands, so dW2 = dZ2^T A1 and dW1 = dZ1^T X need no data movement; only
+// dA1 = dZ2 W2 turns dZ2 over through LDS (rows padded to 68 floats, X's to
+// 20: conflict-free).  The sums of dW1, dW2 and a tile's activations leave
+// 2 waves per SIMD, which is what bounds the kernel: a tile is one dependent
+// chain from its rows to its sums.  The same sums on the vector units, one lane per hidden unit,
+// read every dZ2 element through LDS broadcasts at 1 wave per SIMD: 116 us for
+// 60013 rows, now 40 (18 of it a
+// single tile's chain).  The four waves' sums are added in LDS, pairwise, and
+// written as one partial per workgroup.
+static const int kGradTr = 68, kGradX = 20;  // padded LDS rows of dZ2 / activations and X
+
+// One wave's sums: row 16 t + 4 kg + i, column 16 u + col of dW2 and so on.
+struct MlpSums {
+    f32x4 w2[4][4], w1[4];
+    float b1[4], b2[4], w3[4], b3, loss;
+};
+
+// f(parameter index, sum) over the sums this lane holds (those replicated
+// over lane groups once); the loss goes last, at index kMlpParams.
+template <typename F>
+__device__ __forceinline__ void for_each_sum(MlpSums& g, int lane, F f) {
+    const int col = lane & 15, kg = lane >> 4;
+#pragma unroll
+    for (int t = 0; t < 4; ++t) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int n = 16 * t + 4 * kg + i;
+            float v = g.w1[t][i];
+            f(kOffW1 + n * kMlpIn + col, v);
+            g.w1[t][i] = v;
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+                v = g.w2[t][u][i];
+                f(kOffW2 + n * kMlpH + 16 * u + col, v);
+                g.w2[t][u][i] = v;
+            }
+        }
+        if (kg == 0) {
+            f(kOffB1 + 16 * t + col, g.b1[t]);
+            f(kOffB2 + 16 * t + col, g.b2[t]);
+            f(kOffW3 + 16 * t + col, g.w3[t]);
+        }
+    }
+    if (lane == 0) {
+        f(kOffB3, g.b3);
+        f(kMlpParams, g.loss);
+    }
+}
+
+__global__ __launch_bounds__(256, 2) void k_mlp_grad(MlpDev M, const float* __restrict__ X,
+                                                     const float* __restrict__ T, long long n_rows,
+                                                     long long start, int count,
+                                                     unsigned long long pa, unsigned long long pc,
+                                                     float* __restrict__ gpart,
+                                                     float* __restrict__ lpart) {
+    constexpr int kTile = 16 * (kGradTr + kGradX);         // a wave's scratch, floats
+    constexpr int kWeights = (64 * 32 + 64 * 64) / 2;      // the bf16 weights, floats
+    constexpr int kSumsPad = (kMlpParams + 1 + 3) & ~3;
+    constexpr int kLds = 4 * kTile + kWeights + kMlpH * kGradTr;
+    static_assert(kLds >= 2 * kSumsPad, "two waves' sums");
+    __shared__ __align__(16) float lds[kLds];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int k = lane;
-    float w2c[kMlpH];
+    const int col = lane & 15, kg = lane >> 4;
+    float* tr = lds + w * kTile;
+    float* xs = tr + 16 * kGradTr;
+    unsigned short* w1s = (unsigned short*)(lds + 4 * kTile);
+    unsigned short* w2s = w1s + 64 * 32;
+    for (int k = threadIdx.x; k < 64 * 32 / 8; k += 256) ((u16x8*)w1s)[k] = ((const u16x8*)M.w1p)[k];
+    for (int k = threadIdx.x; k < 64 * 64 / 8; k += 256) ((u16x8*)w2s)[k] = ((const u16x8*)M.w2p)[k];
+    // dA1's operand, W2 turned over: K step s takes unit n = 16 kg + s from
+    // lane group kg
+    float* w2t = lds + 4 * kTile + kWeights;
+    for (int k = threadIdx.x; k < kMlpH * kMlpH; k += 256)
+        w2t[(k % kMlpH) * kGradTr + k / kMlpH] = M.w2r[k];
+    float b1[4], b2[4], w3[4];
 #pragma unroll
-    for (int n = 0; n < kMlpH; ++n) w2c[n] = M.w2r[n * kMlpH + k];
-    const float w3k = M.w3r[k];
-    float g2[kMlpH], g1[kMlpIn];
+    for (int t = 0; t < 4; ++t) {
+        b1[t] = M.p[kOffB1 + 16 * t + col];
+        b2[t] = M.p[kOffB2 + 16 * t + col];
+        w3[t] = M.w3r[16 * t + col];
+    }
+    const float b3 = M.p[kOffB3];
+    MlpSums g;
+    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
-    for (int n = 0; n < kMlpH; ++n) g2[n] = 0.0f;
+    for (int t = 0; t < 4; ++t) {
 #pragma unroll
-    for (int j = 0; j < kMlpIn; ++j) g1[j] = 0.0f;
-    float gb1 = 0.0f, gb2 = 0.0f, gw3 = 0.0f, gb3 = 0.0f, loss = 0.0f;
+        for (int u = 0; u < 4; ++u) g.w2[t][u] = zero;
+        g.w1[t] = zero;
+        g.b1[t] = g.b2[t] = g.w3[t] = 0.0f;
+    }
+    g.b3 = g.loss = 0.0f;
     const float scale = 2.0f / (float)count;
     const int tiles = (count + 15) / 16;
-    for (int tile = blockIdx.x * 4 + w; tile < tiles; tile += gridDim.x * 4) {
-        const int q0 = tile * 16;
-        if (lane < 16) {
-            float f[kMlpIn];
-            const int q = q0 + lane;
-            if (q < count) {
-                const long long r = (long long)((pa * (unsigned long long)(start + q) + pc) %
-                                                (unsigned long long)n_rows);
-#pragma unroll
-                for (int j = 0; j < kMlpIn; ++j) f[j] = X[r * kMlpIn + j];
-            } else {
-#pragma unroll
-                for (int j = 0; j < kMlpIn; ++j) f[j] = 0.0f;
-            }
-            mlp_stage_row(M, f, &xs[w][lane * kMlpIn]);
+    __syncthreads();
+    // lane l fetches quarter l%4 of the tile's row l/4 and that row's target,
+    // one tile ahead
+    const int fr = lane >> 2, fq = lane & 3;
+    f32x4 xv = zero;
+    float tv = 0.0f;
+    auto fetch = [&](int tile) {
+        const int q = tile * 16 + fr;
+        if (tile < tiles && q < count) {
+            const long long r = (long long)((pa * (unsigned long long)(start + q) + pc) %
+                                            (unsigned long long)n_rows);
+            xv = *(const f32x4u*)(X + r * kMlpIn + 4 * fq);
+            tv = T[r];
+        } else {
+            xv = zero;
+            tv = 0.0f;
         }
-        float y[4];
-        mlp16(M, xs[w], dz[w], y, sv[w]);
-        if ((lane & 15) == 0) {
+    };
+    fetch(blockIdx.x * 4 + w);
+    const float* mp = M.p + kOffMu + 4 * fq;
+    const float* ip = M.p + kOffIsd + 4 * fq;
+    const float4 mu = make_float4(mp[0], mp[1], mp[2], mp[3]), isd = make_float4(ip[0], ip[1], ip[2], ip[3]);
+    for (int tile = blockIdx.x * 4 + w; tile < tiles; tile += gridDim.x * 4) {
+        *(float4*)(xs + fr * kGradX + 4 * fq) =
+            make_float4(bfround((xv.x - mu.x) * isd.x), bfround((xv.y - mu.y) * isd.y),
+                        bfround((xv.z - mu.z) * isd.z), bfround((xv.w - mu.w) * isd.w));
+        float tgt[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) tgt[i] = __shfl(tv, (4 * kg + i) * 4, 64);
+        fetch(tile + gridDim.x * 4);
+        wave_sync_lds();
+        // forward, as mlp16
+        float av[8];
+#pragma unroll
+        for (int k = 0; k < 8; ++k) av[k] = kg < 2 ? xs[col * kGradX + 8 * kg + k] : 0.0f;
+        const bf16x8 ax = pack_b8(av);
+        float a1[4][4], g1[4][4], d2[4][4], a2[4][4];
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            const f32x4 z = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                ax, load_b8(w1s + (16 * t + col) * 32 + 8 * kg), zero, 0, 0, 0);
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const int q = q0 + 4 * (lane >> 4) + i;
-                float dy = 0.0f;
-                if (q < count) {
-                    const long long r = (long long)((pa * (unsigned long long)(start + q) + pc) %
-                                                    (unsigned long long)n_rows);
-                    const float diff = y[i] - T[r];
-                    loss += diff * diff;
-                    dy = scale * diff;
-                }
-                dys[w][4 * (lane >> 4) + i] = dy;
+                float v;
+                gelu_both(z[i] + b1[t], v, g1[t][i]);
+                a1[t][i] = bfround(v);
+                tr[(4 * kg + i) * kGradTr + 16 * t + col] = a1[t][i];
             }
         }
         wave_sync_lds();
-        // layer 3 and dZ2 (lane k = hidden unit k of layer 2)
-#pragma unroll 4
-        for (int r = 0; r < 16; ++r) {
-            const float dy = dys[w][r];
-            const float* s = &sv[w][r * 256];
-            gb3 += dy;
-            gw3 += dy * s[192 + k];
-            const float d2 = dy * w3k * gelu_grad(s[128 + k]);
-            dz[w][r * kMlpH + k] = d2;
-            gb2 += d2;
-        }
-        wave_sync_lds();
-        // dW2 column k, dA1 / dZ1 of unit k, dW1 row k
-        for (int r = 0; r < 16; ++r) {
-            const float* d2 = &dz[w][r * kMlpH];
-            const float* s = &sv[w][r * 256];
-            const float a1 = s[64 + k];
-            float da = 0.0f;
+        bf16x8 aa[2];
 #pragma unroll
-            for (int n = 0; n < kMlpH; ++n) {
-                const float dn = d2[n];
-                g2[n] += dn * a1;
-                da += w2c[n] * dn;
+        for (int c = 0; c < 2; ++c) {
+            float v[8];
+#pragma unroll
+            for (int k = 0; k < 8; ++k) v[k] = tr[col * kGradTr + 32 * c + 8 * kg + k];
+            aa[c] = pack_b8(v);
+        }
+        wave_sync_lds();  // tr is written again below
+        float y[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+        for (int t = 0; t < 4; ++t) {
+            f32x4 z = zero;
+#pragma unroll
+            for (int c = 0; c < 2; ++c)
+                z = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                    aa[c], load_b8(w2s + (16 * t + col) * 64 + 32 * c + 8 * kg), z, 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                float v;
+                gelu_both(z[i] + b2[t], v, d2[t][i]);
+                a2[t][i] = bfround(v);
+                y[i] += a2[t][i] * w3[t];
             }
-            const float d1 = da * gelu_grad(s[k]);
-            gb1 += d1;
-            const float* xr = &xs[w][r * kMlpIn];
+        }
+        // output, loss, and layer 3
 #pragma unroll
-            for (int j = 0; j < kMlpIn; ++j) g1[j] += d1 * xr[j];
+        for (int i = 0; i < 4; ++i) {
+            float sum = y[i];
+#pragma unroll
+            for (int o = 1; o < 16; o <<= 1) sum += __shfl_xor(sum, o, 64);
+            const float diff = sum + b3 - tgt[i];
+            const bool in = tile * 16 + 4 * kg + i < count;
+            const float dy = in ? scale * diff : 0.0f;
+            g.loss += in ? diff * diff : 0.0f;
+            g.b3 += dy;
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                g.w3[t] += dy * a2[t][i];
+                d2[t][i] = dy * w3[t] * d2[t][i];
+                g.b2[t] += d2[t][i];
+                tr[(4 * kg + i) * kGradTr + 16 * t + col] = d2[t][i];
+            }
         }
         wave_sync_lds();
+        // dA1 = dZ2 W2: row l%16 of dZ2, units 16 kg + s
+        f32x4 da[4] = {zero, zero, zero, zero};
+#pragma unroll
+        for (int q4 = 0; q4 < 4; ++q4) {
+            const f32x4 v = *(const f32x4*)(tr + col * kGradTr + 16 * kg + 4 * q4);
+            f32x4 wv[4];
+#pragma unroll
+            for (int u = 0; u < 4; ++u) wv[u] = *(const f32x4*)(w2t + (16 * u + col) * kGradTr + 16 * kg + 4 * q4);
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    da[u] = __builtin_amdgcn_mfma_f32_16x16x4f32(v[q], wv[u][q], da[u], 0, 0, 0);
+        }
+        // dW2 = dZ2^T A1
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int t = 0; t < 4; ++t)
+#pragma unroll
+                for (int u = 0; u < 4; ++u)
+                    g.w2[t][u] = __builtin_amdgcn_mfma_f32_16x16x4f32(d2[t][i], a1[u][i], g.w2[t][u], 0, 0, 0);
+        // dZ1 and dW1 = dZ1^T X
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float xr = xs[(4 * kg + i) * kGradX + col];
+#pragma unroll
+            for (int t = 0; t < 4; ++t) {
+                const float d1 = da[t][i] * g1[t][i];
+                g.b1[t] += d1;
+                g.w1[t] = __builtin_amdgcn_mfma_f32_16x16x4f32(d1, xr, g.w1[t], 0, 0, 0);
+            }
+        }
+        wave_sync_lds();  // xs and tr are written by the next tile
     }
-    // partial of this wave, parameter layout of the blob
-    const int wid = blockIdx.x * 4 + w;
-    float* o = gpart + (size_t)wid * kMlpParams;
+    // sums that every lane group holds a part of
 #pragma unroll
-    for (int j = 0; j < kMlpIn; ++j) o[kOffW1 + k * kMlpIn + j] = g1[j];
-    o[kOffB1 + k] = gb1;
+    for (int o = 16; o < 64; o <<= 1) {
 #pragma unroll
-    for (int n = 0; n < kMlpH; ++n) o[kOffW2 + n * kMlpH + k] = g2[n];
-    o[kOffB2 + k] = gb2;
-    o[kOffW3 + k] = gw3;
-    // gb3 and the loss are the same in every lane / in lanes 0, 16, 32, 48
-    loss += __shfl_xor(loss, 16, 64);
-    loss += __shfl_xor(loss, 32, 64);
-    if (lane == 0) {
-        o[kOffB3] = gb3;
-        lpart[wid] = loss;
+        for (int t = 0; t < 4; ++t) {
+            g.b1[t] += __shfl_xor(g.b1[t], o, 64);
+            g.b2[t] += __shfl_xor(g.b2[t], o, 64);
+            g.w3[t] += __shfl_xor(g.w3[t], o, 64);
+        }
+        g.b3 += __shfl_xor(g.b3, o, 64);
+        g.loss += __shfl_xor(g.loss, o, 64);
+    }
+    // the workgroup's partial: (wave 0 + wave 2) + (wave 1 + wave 3)
+    __syncthreads();
+    float* buf = lds + (w & 1) * kSumsPad;
+    if (w >= 2) for_each_sum(g, lane, [&](int k, float& v) { buf[k] = v; });
+    __syncthreads();
+    if (w < 2) for_each_sum(g, lane, [&](int k, float& v) { v += buf[k]; });
+    __syncthreads();
+    if (w == 1) for_each_sum(g, lane, [&](int k, float& v) { lds[k] = v; });
+    __syncthreads();
+    if (w == 0) {
+        float* o = gpart + (size_t)blockIdx.x * kMlpParams;
+        float* lo = lpart + blockIdx.x;
+        for_each_sum(g, lane, [&](int k, float& v) { *(k < kMlpParams ? o + k : lo) = v + lds[k]; });
     }
 }
 
@@ -575,29 +717,47 @@ int launch_mlp_grad(const MlpDev& M, const float* X, const float* T, long long n
     hipLaunchKernelGGL(k_mlp_grad, dim3(blocks), dim3(256), 0, st, M, X, T, n_rows, start, count,
                        pa, pc, gpart, lpart);
     *err = hipGetLastError();
-    return blocks * 4;
+    return blocks;
 }
 
-// Sum of the wave partials in wave order (deterministic).
-__global__ __launch_bounds__(256) void k_mlp_sum(const float* __restrict__ gpart,
-                                                 const float* __restrict__ lpart, int nparts,
-                                                 float* gsum, float* loss) {
-    const int t = blockIdx.x * 256 + threadIdx.x;
-    if (t < kMlpParams) {
-        float s = 0.0f;
-        for (int w = 0; w < nparts; ++w) s += gpart[(size_t)w * kMlpParams + t];
-        gsum[t] = s;
-    }
-    if (t == 0) {
-        float s = 0.0f;
-        for (int w = 0; w < nparts; ++w) s += lpart[w];
-        *loss = s;
+// Sum of the partials of the workgroup's 32 parameters, in a fixed order: 32
+// slices of every 32nd partial, then the slices.  Returns parameter t's sum
+// in the threads of slice 0.  One thread per parameter walking all the
+// partials was a chain of 1024 dependent loads and adds (271 us a step, now 6.4
+// with the update).
+__device__ __forceinline__ float sum_partials(const float* __restrict__ part, int nparts, int stride,
+                                              int t, int limit) {
+    __shared__ float red[32][33];
+    const int j = threadIdx.x & 31, slice = threadIdx.x >> 5;
+    float s = 0.0f;
+    if (t < limit)
+#pragma unroll 8
+        for (int q = slice; q < nparts; q += 32) s += part[(size_t)q * stride + t];
+    __syncthreads();  // the previous sum's readers are done
+    red[slice][j] = s;
+    __syncthreads();
+    s = 0.0f;
+    if (slice == 0)
+#pragma unroll
+        for (int q = 0; q < 32; ++q) s += red[q][j];
+    return s;
+}
+
+__global__ __launch_bounds__(1024) void k_mlp_sum(const float* __restrict__ gpart,
+                                                  const float* __restrict__ lpart, int nparts,
+                                                  float* gsum, float* loss) {
+    const int t = blockIdx.x * 32 + (threadIdx.x & 31);
+    const float s = sum_partials(gpart, nparts, kMlpParams, t, kMlpParams);
+    if (threadIdx.x < 32 && t < kMlpParams) gsum[t] = s;
+    if (blockIdx.x == 0) {
+        const float l = sum_partials(lpart, nparts, 1, threadIdx.x & 31, 1);
+        if (threadIdx.x == 0) *loss = l;
     }
 }
 
 hipError_t launch_mlp_sum(const float* gpart, const float* lpart, int nparts, float* gsum,
                           float* loss, hipStream_t st) {
-    hipLaunchKernelGGL(k_mlp_sum, dim3((kMlpParams + 255) / 256), dim3(256), 0, st, gpart, lpart,
+    hipLaunchKernelGGL(k_mlp_sum, dim3((kMlpParams + 31) / 32), dim3(1024), 0, st, gpart, lpart,
                        nparts, gsum, loss);
     return hipGetLastError();
 }
@@ -606,16 +766,15 @@ hipError_t launch_mlp_sum(const float* gpart, const float* lpart, int nparts, fl
 // master weights, then the bf16 forms of the updated weight.  bc1 / bc2 are
 // the bias corrections 1 - beta^t.  loss_acc (if non-null) accumulates the
 // batch's squared-error sum.
-__global__ __launch_bounds__(256) void k_mlp_adam(float* p, float* m, float* v,
-                                                  const float* __restrict__ gpart,
-                                                  const float* __restrict__ lpart, int nparts,
-                                                  float lr, float bc1, float bc2, float* loss_acc,
-                                                  unsigned short* w1p, unsigned short* w2p,
-                                                  float* w2r, float* w3r) {
-    const int t = blockIdx.x * 256 + threadIdx.x;
-    if (t < kMlpParams) {
-        float g = 0.0f;
-        for (int w = 0; w < nparts; ++w) g += gpart[(size_t)w * kMlpParams + t];
+__global__ __launch_bounds__(1024) void k_mlp_adam(float* p, float* m, float* v,
+                                                   const float* __restrict__ gpart,
+                                                   const float* __restrict__ lpart, int nparts,
+                                                   float lr, float bc1, float bc2, float* loss_acc,
+                                                   unsigned short* w1p, unsigned short* w2p,
+                                                   float* w2r, float* w3r) {
+    const int t = blockIdx.x * 32 + (threadIdx.x & 31);
+    const float g = sum_partials(gpart, nparts, kMlpParams, t, kMlpParams);
+    if (threadIdx.x < 32 && t < kMlpParams) {
         const float mt = 0.9f * m[t] + 0.1f * g;
         const float vt = 0.999f * v[t] + 0.001f * g * g;
         m[t] = mt;
@@ -634,10 +793,9 @@ __global__ __launch_bounds__(256) void k_mlp_adam(float* p, float* m, float* v,
             w3r[t - kOffW3] = bfround(nw);
         }
     }
-    if (t == 0 && loss_acc != nullptr) {
-        float s = 0.0f;
-        for (int w = 0; w < nparts; ++w) s += lpart[w];
-        *loss_acc += s;
+    if (blockIdx.x == 0 && loss_acc != nullptr) {
+        const float l = sum_partials(lpart, nparts, 1, threadIdx.x & 31, 1);
+        if (threadIdx.x == 0) *loss_acc += l;
     }
 }
 
@@ -645,7 +803,7 @@ hipError_t launch_mlp_adam(float* p, float* m, float* v, const float* gpart, con
                            int nparts, float lr, float bc1, float bc2, float* loss_acc,
                            unsigned short* w1p, unsigned short* w2p, float* w2r, float* w3r,
                            hipStream_t st) {
-    hipLaunchKernelGGL(k_mlp_adam, dim3((kMlpParams + 255) / 256), dim3(256), 0, st, p, m, v, gpart,
+    hipLaunchKernelGGL(k_mlp_adam, dim3((kMlpParams + 31) / 32), dim3(1024), 0, st, p, m, v, gpart,
                        lpart, nparts, lr, bc1, bc2, loss_acc, w1p, w2p, w2r, w3r);
     return hipGetLastError();
 }

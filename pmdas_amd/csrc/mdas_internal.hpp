@@ -288,9 +288,9 @@ hipError_t launch_mlp_pack(float* p, unsigned short* w1p, unsigned short* w2p, f
                            float* w3r, hipStream_t st);
 hipError_t launch_mlp_forward(const MlpDev& M, const float* X, long long n, float* Y,
                               hipStream_t st);
-// Per-wave partial gradients of mean((y - t)^2) over rows perm(q),
+// Per-workgroup partial gradients of mean((y - t)^2) over rows perm(q),
 // q in [start, start + count), perm(q) = (pa * q + pc) mod n_rows.  Returns
-// the number of wave partials written to gpart / lpart.
+// the number of partials written to gpart / lpart.
 int launch_mlp_grad(const MlpDev& M, const float* X, const float* T, long long n_rows,
                     long long start, int count, unsigned long long pa, unsigned long long pc,
                     float* gpart, float* lpart, hipStream_t st, hipError_t* err);
@@ -302,7 +302,7 @@ hipError_t launch_mlp_adam(float* p, float* m, float* v, const float* gpart, con
                            hipStream_t st);
 hipError_t launch_feat_stats(const float* X, long long n, double* part, int nblocks,
                              hipStream_t st);
-static const int kMlpGradBlocks = 256;  // workgroups of the gradient kernel (4 waves each)
+static const int kMlpGradBlocks = 512;  // most workgroups of the gradient kernel (4 waves each, 2 per CU)
 hipError_t recon_reserve(Grid& g, int W, int H);
 hipError_t recon_prepare(Grid& g, int W, int H, hipStream_t st);
 

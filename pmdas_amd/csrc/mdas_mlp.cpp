@@ -21,8 +21,8 @@ struct mdas_mlp {
     float* w3r = nullptr;           // [64]
     float* m = nullptr;             // Adam moments [kMlpParams]
     float* v = nullptr;
-    float* gpart = nullptr;         // [kMlpGradBlocks*4][kMlpParams] wave partials
-    float* lpart = nullptr;         // [kMlpGradBlocks*4]
+    float* gpart = nullptr;         // [kMlpGradBlocks][kMlpParams] workgroup partials
+    float* lpart = nullptr;         // [kMlpGradBlocks]
     float* gsum = nullptr;          // [kMlpParams + 1] summed gradient and loss
     double* spart = nullptr;        // feature statistics partials
     long long t = 0;                // Adam steps taken
@@ -94,7 +94,7 @@ int mdas_mlp_create(uint32_t seed, mdas_mlp_handle* out) {
     if (!out) return set_error(MDAS_ERR_INVALID, "null output handle");
     *out = nullptr;
     mdas_mlp* m = new mdas_mlp;
-    const size_t waves = (size_t)mdas::kMlpGradBlocks * 4;
+    const size_t parts = (size_t)mdas::kMlpGradBlocks;
     hipError_t e = hipMalloc((void**)&m->p, sizeof(float) * mdas::kMlpFloats);
     if (e == hipSuccess) e = hipMalloc((void**)&m->w1p, sizeof(unsigned short) * 64 * 32);
     if (e == hipSuccess) e = hipMalloc((void**)&m->w2p, sizeof(unsigned short) * 64 * 64);
@@ -102,8 +102,8 @@ int mdas_mlp_create(uint32_t seed, mdas_mlp_handle* out) {
     if (e == hipSuccess) e = hipMalloc((void**)&m->w3r, sizeof(float) * 64);
     if (e == hipSuccess) e = hipMalloc((void**)&m->m, sizeof(float) * mdas::kMlpParams);
     if (e == hipSuccess) e = hipMalloc((void**)&m->v, sizeof(float) * mdas::kMlpParams);
-    if (e == hipSuccess) e = hipMalloc((void**)&m->gpart, sizeof(float) * waves * mdas::kMlpParams);
-    if (e == hipSuccess) e = hipMalloc((void**)&m->lpart, sizeof(float) * waves);
+    if (e == hipSuccess) e = hipMalloc((void**)&m->gpart, sizeof(float) * parts * mdas::kMlpParams);
+    if (e == hipSuccess) e = hipMalloc((void**)&m->lpart, sizeof(float) * parts);
     if (e == hipSuccess) e = hipMalloc((void**)&m->gsum, sizeof(float) * (mdas::kMlpParams + 1));
     if (e == hipSuccess) e = hipMalloc((void**)&m->spart, sizeof(double) * kStatBlocks * 32);
     if (e != hipSuccess) {

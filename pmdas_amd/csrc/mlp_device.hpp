@@ -19,6 +19,7 @@ namespace mdas {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned short u16x8 __attribute__((ext_vector_type(8)));
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));  // rows of any float alignment
 
 static const int kMlpIn = 16, kMlpH = 64;
 // Parameter blob (floats): W1 [64][16], b1 [64], W2 [64][64], b2 [64],
@@ -54,9 +55,11 @@ __device__ __forceinline__ float gelu_tanh(float x) {
     return 1.0f - 2.0f * __builtin_amdgcn_rcpf(__expf(2.0f * z) + 1.0f);
 }
 __device__ __forceinline__ float gelu(float x) { return 0.5f * x * (1.0f + gelu_tanh(x)); }
-__device__ __forceinline__ float gelu_grad(float x) {
+// GELU and its derivative.
+__device__ __forceinline__ void gelu_both(float x, float& v, float& grad) {
     const float t = gelu_tanh(x);
-    return 0.5f * (1.0f + t) +
+    v = 0.5f * x * (1.0f + t);
+    grad = 0.5f * (1.0f + t) +
            0.5f * x * (1.0f - t * t) * 0.7978845608f * (1.0f + 3.0f * 0.044715f * x * x);
 }
 
@@ -88,11 +91,8 @@ __device__ __forceinline__ void mlp_stage_row(const MlpDev& M, const float* f, f
 
 // Forward pass of 16 rows by one wave (every lane calls it).  x (LDS,
 // [16][16]) holds the staged rows, act (LDS, [16][64]) is scratch.  Returns
-// in y[i] the output of row 4*(lane/16)+i.  When save is non-null (LDS,
-// [16][256]) it receives per row the pre-activations Z1 (0..63), the bf16
-// layer-2 inputs A1 (64..127), Z2 (128..191) and the bf16 A2 (192..255).
-__device__ __forceinline__ void mlp16(const MlpDev& M, const float* x, float* act, float y[4],
-                                      float* save) {
+// in y[i] the output of row 4*(lane/16)+i.
+__device__ __forceinline__ void mlp16(const MlpDev& M, const float* x, float* act, float y[4]) {
     const int lane = threadIdx.x & 63;
     const int col = lane & 15, kg = lane >> 4;
     wave_sync_lds();
@@ -117,13 +117,7 @@ __device__ __forceinline__ void mlp16(const MlpDev& M, const float* x, float* ac
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             const int r = 4 * kg + i;
-            const float zz = z[t][i] + bias;
-            const float a = bfround(gelu(zz));
-            act[r * kMlpH + n] = a;
-            if (save) {
-                save[r * 256 + n] = zz;
-                save[r * 256 + 64 + n] = a;
-            }
+            act[r * kMlpH + n] = bfround(gelu(z[t][i] + bias));
         }
     }
     wave_sync_lds();
@@ -148,14 +142,7 @@ __device__ __forceinline__ void mlp16(const MlpDev& M, const float* x, float* ac
         const float bias = M.p[kOffB2 + n], w3 = M.w3r[n];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const float zz = c[i] + bias;
-            const float a = bfround(gelu(zz));
-            part[i] += a * w3;
-            if (save) {
-                const int r = 4 * kg + i;
-                save[r * 256 + 128 + n] = zz;
-                save[r * 256 + 192 + n] = a;
-            }
+            part[i] += bfround(gelu(c[i] + bias)) * w3;
         }
     }
 #pragma unroll

@@ -112,6 +112,28 @@ def test_mlp_gradient_matches_oracle(mdas):
     m.close()
 
 
+# one row, the edges of a 16-row tile and of a workgroup's four, and a second
+# tile for some waves of the largest grid (512 workgroups of 64 rows)
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 63, 65, 1025, 32768 + 17])
+def test_mlp_gradient_row_counts(mdas, n):
+    _say(f"mlp gradient n={n}")
+    p = _params(6)
+    r = np.random.default_rng(n)
+    X = r.standard_normal((n, 16)).astype(np.float32)
+    T = r.standard_normal(n).astype(np.float32)
+    m = mdas.Mlp(0)
+    m.set_params(p)
+    g, loss = m.grad(X, T)
+    gw, lw = mo.grad(p, X, T)
+    # a row whose activation lies at a bf16 tie moves by an ulp (2^-8) of one
+    # of 64 terms, its residual by as much: below 1 % of the row's gradient
+    assert abs(loss - lw) < 1e-2 * max(lw, 1e-2)
+    assert np.linalg.norm(g - gw) < 1e-2 * np.linalg.norm(gw)
+    g2, _ = m.grad(X, T)
+    assert np.array_equal(g, g2)
+    m.close()
+
+
 def test_adam_step_matches_oracle(mdas):
     _say("adam step")
     from pmdas_amd import hip
