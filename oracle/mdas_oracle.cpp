@@ -716,6 +716,25 @@ void orc_eval_scene_grouped(const void* params, const void* coords, int dim, lon
     }
 }
 
+// How many times the product's fused division of the count doubles by the
+// series' constants and the Halton bases rounds otherwise than a division.
+long long orc_div_by_mismatches(const double* x, long long count) {
+    long long bad = 0;
+    for (long long k = 0; k < count; ++k) {
+#define MDAS_DIV(N) bad += mscene::div_by_fma<N>(x[k]) != x[k] / (double)(N);
+        MDAS_DIV(342) MDAS_DIV(272) MDAS_DIV(210) MDAS_DIV(156) MDAS_DIV(110) MDAS_DIV(72)
+        MDAS_DIV(42) MDAS_DIV(20) MDAS_DIV(6) MDAS_DIV(306) MDAS_DIV(240) MDAS_DIV(182)
+        MDAS_DIV(132) MDAS_DIV(90) MDAS_DIV(56) MDAS_DIV(30) MDAS_DIV(12) MDAS_DIV(2)
+#undef MDAS_DIV
+        const float f = (float)x[k];  // the Halton bases, in both precisions
+#define MDAS_DIV(N) bad += mscene::div_by_fma<N>(x[k]) != x[k] / (double)(N); \
+        if (f > 1e-30f) bad += mscene::div_by_fma<N>(f) != f / (float)(N);
+        MDAS_DIV(2) MDAS_DIV(3) MDAS_DIV(5) MDAS_DIV(7) MDAS_DIV(11) MDAS_DIV(13)
+#undef MDAS_DIV
+    }
+    return bad;
+}
+
 // The same through the sets of spheres by cell; returns the number of cells
 // (0: the scene has none).
 int orc_eval_scene_cells(const void* params, const void* coords, int dim, long long count, int fp64,

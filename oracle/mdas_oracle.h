@@ -61,6 +61,7 @@ void orc_eval_scene_f64(const void* scene_params, const double* coords, int dim,
  * restatement of the reference. */
 void orc_eval_scene_grouped(const void* scene_params, const void* coords, int dim,
                             long long count, int fp64, void* values);
+long long orc_div_by_mismatches(const double* x, long long count);
 int orc_eval_scene_cells(const void* scene_params, const void* coords, int dim, long long count,
                          int fp64, void* values);
 /* The plain QMC sampler's image (cuda/sampler.h:4-28, random.h:74-89,

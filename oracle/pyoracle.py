@@ -36,6 +36,7 @@ _SIGS = {
     "orc_eval_scene": (None, [_P, _P, _I, _LL, _LL, _P]),
     "orc_eval_scene_f64": (None, [_P, _P, _I, _LL, _P]),
     "orc_eval_scene_grouped": (None, [_P, _P, _I, _LL, _I, _P]),
+    "orc_div_by_mismatches": (_LL, [_P, _LL]),
     "orc_eval_scene_cells": (_I, [_P, _P, _I, _LL, _I, _P]),
     "orc_qmc_image": (None, [_P, _I, _I, _I, _I, _U, _I, _P]),
     "orc_halton": (_F, [_I, _I]),
@@ -243,6 +244,11 @@ def eval_scene_cells(params, coords, dim, fp64=False):
     out = np.empty((len(c), 3), t)
     n = load().orc_eval_scene_cells(params, vp(c), dim, len(c), 1 if fp64 else 0, vp(out))
     return out, n
+
+
+def div_by_mismatches(x):
+    x = np.ascontiguousarray(x, np.float64)
+    return load().orc_div_by_mismatches(vp(x), len(x))
 
 
 def qmc_image(params, w, h, spp, first_sample=0, frame=0, fp64=False):

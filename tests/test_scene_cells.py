@@ -72,3 +72,17 @@ def test_cells_hand_built_scenes(orc):
     s = Scene(orc, 4, 6)
     s.objects([[0.0, 1e4, 0.0, 1e4, 0, 0, 0, 1, 1, 1]])
     _hold(orc, bytes(s.buf), _coords(rng, 20000, 6, 1.0, 1.0), 6, cells=False)
+
+
+def test_division_by_the_series_constants(orc):
+    """The lens map's series and the Halton points divide by whole numbers
+    with two fused operations on the GPU: the value of a division for squares of
+    32-bit and 64-bit angles, mantissas next to powers of two and to
+    multiples of the constants."""
+    rng = np.random.default_rng(8)
+    f = rng.uniform(0, np.pi / 4, 400000)
+    x = [f ** 2, f.astype(np.float32).astype(np.float64) ** 2, np.exp(rng.uniform(-300, 0, 400000)), [0.0]]
+    near = np.concatenate([np.ldexp(1.0, -np.arange(0, 900)), rng.integers(1, 1 << 50, 20000) * 342.0 / 2.0 ** 70,
+                           rng.integers(1, 1 << 50, 20000) * 171.5 / 2.0 ** 70])
+    x += [near, np.nextafter(near, 0), np.nextafter(near, 1e9)]
+    assert orc.div_by_mismatches(np.concatenate(x)) == 0
