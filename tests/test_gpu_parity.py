@@ -386,6 +386,20 @@ def _random_runs():
     return _configs(16, 31)
 
 
+# lanes per pixel 64, 32 and 1 .. 8 (2^19 lanes where the samples allow it) and
+# chunks of 64 samples with remainders
+@pytest.mark.parametrize("W,H,spp,first", [(37, 29, 1, 0), (37, 29, 2, 5), (37, 29, 63, 0), (37, 29, 64, 1), (37, 29, 65, 0),
+                                           (1, 1, 200, 7), (131, 97, 130, 0), (400, 301, 9, 2), (1031, 517, 3, 0)])
+@pytest.mark.parametrize("fp64", [False, True])
+def test_render_qmc_lanes_and_chunks(mdas, W, H, spp, first, fp64):
+    _say(f"render_qmc {W}x{H} {spp} spp fp64={fp64}")
+    sc = mdas.Scene(3, 4, 5, float(W), float(H))
+    got = sc.render_qmc(W, H, spp, first_sample=first, frame=1, fp64=fp64)
+    want = pyoracle.qmc_image(sc.params_bytes(), W, H, spp, first, 1, fp64=fp64)
+    u = np.uint64 if fp64 else np.uint32
+    assert np.array_equal(got.view(u), want.view(u))
+
+
 @pytest.mark.parametrize("c", _random_runs(), ids=lambda c: f"rnd{c['id']}-d{c['dim']}")
 def test_pass_by_pass_random_configs(mdas, c):
     """The one-call-at-a-time sequence (ComputeErrors, AdaptiveSampling, the
