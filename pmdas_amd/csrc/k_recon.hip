@@ -773,11 +773,11 @@ hipError_t recon_prepare(Grid& g, int W, int H, hipStream_t st) {
     ReconGeo G = make_geo(g, W, H);
     g.recon_pixels = (long long)W * H;
     kbeg(g, st, "k_recon_prep");
-    MDAS_DISPATCH_D(g.D, hipLaunchKernelGGL(k_recon_prep<DD>, dim3(g.chunk_blocks), dim3(256), 0, st,
+    MDAS_DISPATCH_D(g.D, hipLaunchKernelGGL(k_recon_prep<DD>, dim3(g.chunks()), dim3(256), 0, st,
                                             g.dev, G, g.rb.rrec));
     kend(g, st);
     kbeg(g, st, "k_scan_keys");
-    hipLaunchKernelGGL(k_scan_keys, dim3(1), dim3(1024), 0, st, g.dev, g.chunk_blocks,
+    hipLaunchKernelGGL(k_scan_keys, dim3(1), dim3(1024), 0, st, g.dev, g.chunks(),
                        g.recon_bounded ? g.rb.keys_cap : (long long)0x7fffffff);
     kend(g, st);
     if (!g.recon_bounded) {
@@ -799,7 +799,7 @@ static hipError_t recon_finish(Grid& g, ReconBufs& rb, float* pixels, int W, int
                                hipEvent_t ev_sort0, hipEvent_t ev_sort1) {
     ReconGeo G = make_geo(g, W, H);
     kbeg(g, st, "k_recon_emit");
-    hipLaunchKernelGGL(k_recon_emit, dim3(g.chunk_blocks), dim3(256), 0, st, g.dev, G, rb.rrec, rb.keys);
+    hipLaunchKernelGGL(k_recon_emit, dim3(g.chunks()), dim3(256), 0, st, g.dev, G, rb.rrec, rb.keys);
     kend(g, st);
     if (ev_sort0) (void)hipEventRecord(ev_sort0, st);
     // the sorted keys end in keys or keys_alt by the parity of the pass
@@ -840,9 +840,9 @@ hipError_t launch_integrate_gather(Grid& g, float* pixels, int W, int H, hipStre
 hipError_t recon_on_buffers(Grid& g, ReconBufs& rb, float* pixels, int W, int H, hipStream_t st) {
     ReconGeo G = make_geo(g, W, H);
     g.recon_pixels = (long long)W * H;
-    MDAS_DISPATCH_D(g.D, hipLaunchKernelGGL(k_recon_prep<DD>, dim3(g.chunk_blocks), dim3(256), 0, st,
+    MDAS_DISPATCH_D(g.D, hipLaunchKernelGGL(k_recon_prep<DD>, dim3(g.chunks()), dim3(256), 0, st,
                                             g.dev, G, rb.rrec));
-    hipLaunchKernelGGL(k_scan_keys, dim3(1), dim3(1024), 0, st, g.dev, g.chunk_blocks, rb.keys_cap);
+    hipLaunchKernelGGL(k_scan_keys, dim3(1), dim3(1024), 0, st, g.dev, g.chunks(), rb.keys_cap);
     return recon_finish(g, rb, pixels, W, H, st, nullptr, nullptr);
 }
 

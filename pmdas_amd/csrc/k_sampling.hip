@@ -10,6 +10,7 @@
 // sweep over all leaves.  Cross-workgroup reductions go through per-workgroup
 // partials (no same-address atomics).
 #include "mdas_leaf.hpp"
+#include "scenes.hpp"
 
 #pragma clang fp contract(off)
 
@@ -89,12 +90,20 @@ __global__ __launch_bounds__(256) void k_initial(DevGrid a, int L0) {
 // configuration.
 template <int D>
 __global__ __launch_bounds__(256) void k_initial_b(const DevGrid* grids) {
-    const DevGrid& a = grids[blockIdx.y];
+    const DevGrid a = grids[blockIdx.y];
     initial_body<D>(a, 1 << (a.b * D + 2 * a.e), blockIdx.x, gridDim.x);
 }
 
 // Counter set-up of InitialSampling (kdgrid.cu:639-642).
-__device__ __forceinline__ void initial_counters_body(DevCounters* c, int L0) {
+__device__ __forceinline__ void initial_counters_body(const DevGrid& a, int L0) {
+    DevCounters* c = a.cnt;
+    if (threadIdx.x < 2 * kSuper) {
+        a.ssum[threadIdx.x].sel = a.ssum[threadIdx.x].split = a.ssum[threadIdx.x].held = 0;
+        a.smax[threadIdx.x].err = 0u;
+    }
+    if (threadIdx.x != 0) return;
+    c->cur = 0;
+    c->slot[0] = c->slot[1] = LoopSlot{4 * L0, L0, 0, 0, 4 * L0, 0};
     c->n_leaves = L0;
     c->n_samples = 4 * L0;
     c->n_leaves_old = 0;
@@ -112,7 +121,9 @@ __device__ __forceinline__ void initial_counters_body(DevCounters* c, int L0) {
     c->carry_bits = 0;
     c->guard_cap = 0;
 }
-__global__ void k_initial_counters(DevCounters* c, int L0) { initial_counters_body(c, L0); }
+__global__ __launch_bounds__(2 * kSuper) void k_initial_counters(DevGrid a, int L0) {
+    initial_counters_body(a, L0);
+}
 
 // ComputeErrors prologue (kdgrid.cu:684-685): g_error = 0.  A standalone call
 // also re-arms the pass kernels and lifts the sampling loop's limit.
@@ -130,15 +141,14 @@ __global__ void k_set_limit(DevCounters* c, int limit, int guard_cap) {
     c->guard_cap = guard_cap;
 }
 
-// Batched counter kernels: one thread per image.
-__global__ void k_initial_counters_b(const DevGrid* grids, int n, const int* limits) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t >= n) return;
-    const DevGrid& a = grids[t];
+// Batched form: one workgroup per image.
+__global__ __launch_bounds__(2 * kSuper) void k_initial_counters_b(const DevGrid* grids, const int* limits) {
+    const DevGrid& a = grids[blockIdx.x];
     DevCounters* c = a.cnt;
-    initial_counters_body(c, 1 << (a.b * a.D + 2 * a.e));
-    c->limit = limits[t];
-    c->guard_cap = limits[t] >= a.cap_s ? a.cap_s : 0;
+    initial_counters_body(a, 1 << (a.b * a.D + 2 * a.e));
+    if (threadIdx.x != 0) return;
+    c->limit = limits[blockIdx.x];
+    c->guard_cap = limits[blockIdx.x] >= a.cap_s ? a.cap_s : 0;
 }
 
 // Re-arms the pass kernels for a standalone AdaptiveSampling call.
@@ -250,7 +260,39 @@ __global__ __launch_bounds__(256) void k_errors_stale(DevGrid a) {
 }
 template <int D>
 __global__ __launch_bounds__(256) void k_errors_stale_b(const DevGrid* grids) {
-    errors_stale_body<D>(grids[blockIdx.y], blockIdx.x, gridDim.x);
+    const DevGrid a = grids[blockIdx.y];  // by value: scalar registers
+    errors_stale_body<D>(a, blockIdx.x, gridDim.x);
+}
+
+// Errors of the initial leaves for the fused loop: every leaf holds four
+// samples; the largest goes to the super group of the workgroup.
+template <int D>
+__device__ __forceinline__ void first_errors_body(const DevGrid& a, int blk, int nblk) {
+    __shared__ float wmax[4];
+    const int L = a.cnt->slot[0].L;
+    if (loop_limit_reached(a.cnt, a.cnt->slot[0].N, L)) return;  // no pass: the errors stay stale
+    float m = 0.0f;
+    for (int i = blk * 256 + threadIdx.x; i < L; i += nblk * 256) {
+        int n;
+        const float e = leaf_error<D>(a, i, &n);
+        a.err[i] = e;
+        m = fmaxf(m, e);
+    }
+    m = wave_max(m);
+    if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0)
+        atomicMax(&a.smax[blk % kSuper].err,
+                  __float_as_uint(fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]))));
+}
+template <int D>
+__global__ __launch_bounds__(256) void k_first_errors(DevGrid a) {
+    first_errors_body<D>(a, blockIdx.x, gridDim.x);
+}
+template <int D>
+__global__ __launch_bounds__(256) void k_first_errors_b(const DevGrid* grids) {
+    const DevGrid a = grids[blockIdx.y];  // by value: scalar registers
+    first_errors_body<D>(a, blockIdx.x, gridDim.x);
 }
 
 // Folds the error partials into gmax and the per-pass statistics.  A full
@@ -307,6 +349,9 @@ __global__ __launch_bounds__(1024) void k_err_reduce_b(const DevGrid* grids, int
 }
 
 // --------------------------------------------------------------- selection --
+// Chunks per super group of the fused loop, for `chunks` in all.
+__device__ __forceinline__ int super_size(int chunks) { return (chunks + kSuper - 1) / kSuper; }
+
 // kdgrid.cu:316-326.  Per leaf: the seed (tea4(i,0) when unset), one draw u,
 // selected iff pow(err / g_error, alpha) >= u.  A selected full leaf splits.
 // Writes the flags, and per workgroup the (selected, split) counts for the
@@ -314,12 +359,12 @@ __global__ __launch_bounds__(1024) void k_err_reduce_b(const DevGrid* grids, int
 // of the leaves that do not split.  The LCG states are not written here: the
 // compaction stores them once the scan has accepted the pass, so that a pass
 // refused for capacity leaves every state as it was.
-// Chunk blk of nblk (the compaction's partition of the leaves).
-__device__ __forceinline__ void select_chunk(const DevGrid& a, int blk, int nblk) {
+// Chunk blk of nblk (the compaction's partition of the leaves).  ssum, smax:
+// the super groups of the fused loop, which take the chunk's totals too; else null.
+__device__ __forceinline__ void select_chunk(const DevGrid& a, int L, float gmax, int blk, int nblk,
+                                             SuperSum* ssum, SuperMax* smax) {
     __shared__ int red[12];
     __shared__ float rmax[4];
-    const int L = a.cnt->n_leaves;
-    const float gmax = __uint_as_float(a.cnt->gmax_bits);
     const float alpha = a.alpha;
     int beg, end;
     chunk_range(L, nblk, blk, beg, end);
@@ -370,8 +415,16 @@ __device__ __forceinline__ void select_chunk(const DevGrid& a, int blk, int nblk
     __syncthreads();
     if (threadIdx.x == 0) {
         const float cm = fmaxf(fmaxf(rmax[0], rmax[1]), fmaxf(rmax[2], rmax[3]));
-        a.part[blk] = make_int4(red[0] + red[1] + red[2] + red[3], red[4] + red[5] + red[6] + red[7],
-                                red[8] + red[9] + red[10] + red[11], (int)__float_as_uint(cm));
+        const int4 p = make_int4(red[0] + red[1] + red[2] + red[3], red[4] + red[5] + red[6] + red[7],
+                                 red[8] + red[9] + red[10] + red[11], (int)__float_as_uint(cm));
+        a.part[blk] = p;
+        if (ssum != nullptr) {
+            const int g = blk / super_size(nblk);
+            if (p.x != 0) atomicAdd(&ssum[g].sel, p.x);
+            if (p.y != 0) atomicAdd(&ssum[g].split, p.y);
+            if (p.z != 0) atomicAdd(&ssum[g].held, p.z);
+            if (p.w != 0) atomicMax(&smax[g].err, (unsigned)p.w);
+        }
     }
     __syncthreads();  // red / rmax are reused by the workgroup's next chunk
 }
@@ -380,13 +433,42 @@ __device__ __forceinline__ void select_chunk(const DevGrid& a, int blk, int nblk
 // selection's streaming sweep runs best with fewer, longer ones.
 __device__ __forceinline__ void select_body(const DevGrid& a, int blk, int nblk, int cpw) {
     if (a.cnt->done) return;
-    for (int c = blk * cpw; c < (blk + 1) * cpw; ++c) select_chunk(a, c, nblk * cpw);
+    const int L = a.cnt->n_leaves;
+    const float gmax = __uint_as_float(a.cnt->gmax_bits);
+    for (int c = blk * cpw; c < (blk + 1) * cpw; ++c) select_chunk(a, L, gmax, c, nblk * cpw, nullptr, nullptr);
 }
 __global__ __launch_bounds__(256) void k_select(DevGrid a, int cpw) {
     select_body(a, blockIdx.x, gridDim.x, cpw);
 }
 __global__ __launch_bounds__(256) void k_select_b(const DevGrid* grids, int cpw) {
-    select_body(grids[blockIdx.y], blockIdx.x, gridDim.x, cpw);
+    const DevGrid a = grids[blockIdx.y];  // by value: scalar registers
+    select_body(a, blockIdx.x, gridDim.x, cpw);
+}
+
+// The same in the fused loop: the stopping test and the largest error come
+// first, from the pass's slot and super groups, in place of the reduction
+// kernel; the largest error among the leaves that do not split goes on to the
+// next pass.  A single thread keeps the counters that are read after the loop.
+__device__ __forceinline__ void select_fused_body(const DevGrid& a, int blk, int nblk, int cpw, int par) {
+    DevCounters* cn = a.cnt;
+    if (cn->done) return;
+    const int N = cn->slot[par].N, L = cn->slot[par].L;
+    if (loop_limit_reached(cn, N, L)) {  // every workgroup finds the same
+        if (blk == 0 && threadIdx.x == 0) cn->done = 1;
+        return;
+    }
+    const unsigned e = a.smax[par * kSuper + (threadIdx.x & 63)].err;
+    const float gmax = wave_max(__uint_as_float(e));  // no NaN among them: each is a maximum from 0
+    if (blk == 0 && threadIdx.x == 0) cn->gmax_bits = __float_as_uint(gmax);
+    for (int c = blk * cpw; c < (blk + 1) * cpw; ++c)
+        select_chunk(a, L, gmax, c, nblk * cpw, a.ssum + par * kSuper, a.smax + (par ^ 1) * kSuper);
+}
+__global__ __launch_bounds__(256) void k_select_fused(DevGrid a, int cpw, int par) {
+    select_fused_body(a, blockIdx.x, gridDim.x, cpw, par);
+}
+__global__ __launch_bounds__(256) void k_select_fused_b(const DevGrid* grids, int cpw, int par) {
+    const DevGrid a = grids[blockIdx.y];  // by value: scalar registers
+    select_fused_body(a, blockIdx.x, gridDim.x, cpw, par);
 }
 
 // Chunks per selection workgroup for `chunks` compaction chunks: as many as
@@ -524,9 +606,14 @@ __global__ __launch_bounds__(1024) void k_scan_counts_b(const DevGrid* grids, in
 // sample index k, the draws starting from LCG state s; a full leaf is split
 // at the median of its 5 samples along the largest box axis, keeping the left
 // half in place and the right half at leaf index m.
-template <int D>
+// With a scene B (FUSED; its objects in LDS at obj) the new sample is evaluated
+// here and a split's children get their errors here, from the leaf's values
+// and the new one, in place of the next pass's error kernel; emax takes the
+// larger.
+template <int D, bool FUSED>
 __device__ __forceinline__ void place_leaf(const DevGrid& a, int i, int k, int m, unsigned cnt,
-                                           int L, unsigned s) {
+                                           int L, unsigned s, const mscene::SceneBlock* B,
+                                           const float* obj, float& emax) {
     constexpr int P = line_pts(D);
     // the leaf's line: slots, box and its first points, one 128-byte read
     float f[kLineFloats];
@@ -609,7 +696,8 @@ __device__ __forceinline__ void place_leaf(const DevGrid& a, int i, int k, int m
     float* out = a.coords + (size_t)k * D;
 #pragma unroll
     for (int d = 0; d < D; ++d) out[d] = best[d];
-
+    int kid[5] = {k, k, k, k, k};     // FUSED: a split's samples in sorted order,
+    float vol_l = 0.0f, vol_r = 0.0f;  // its children's volumes
     if (cnt < 4u) {
         // kdgrid.cu:393-396: insert into the first free slot; the error is kept
         store_point_slot<D>(a, i, (int)cnt, best, k);
@@ -687,27 +775,34 @@ __device__ __forceinline__ void place_leaf(const DevGrid& a, int i, int k, int m
         store_line_head2<D>(a, i, make_int4(v[0], v[1], E, E), mn, cmx, sp[0], sp[1]);
         store_line<D>(a, m, make_int4(v[2], v[3], v[4], E), cmn, mx, &sp[2], 3);
         if constexpr (P < 3) store_point_slot<D>(a, m, 2, sp[4], v[4]);  // D = 6: overflow row
-        // what the next error pass needs of both children, coalesced by
-        // split rank: their sample indices and box volumes
-        a.sdat[2 * (m - L)] = make_int4(v[0], v[1], v[2], v[3]);
-        a.sdat[2 * (m - L) + 1] = make_int4(v[4], __float_as_int(box_volume<D>(mn, cmx)),
-                                            __float_as_int(box_volume<D>(cmn, mx)), 0);
-        if (a.sext) {  // learned mode: the children's extents for their features
-            float ex[6];
+        if constexpr (FUSED) {
 #pragma unroll
-            for (int d = 0; d < 6; ++d) ex[d] = d < D ? (d == axis ? cmx[d] - mn[d] : diag[d]) : 0.0f;
-            a.sext[2 * (m - L)] = make_int4(__float_as_int(ex[0]), __float_as_int(ex[1]),
-                                            __float_as_int(ex[2]), __float_as_int(ex[3]));
-            float right = 0.0f;
+            for (int j = 0; j < 5; ++j) kid[j] = v[j];
+            vol_l = box_volume<D>(mn, cmx);
+            vol_r = box_volume<D>(cmn, mx);
+        } else {
+            // what the next error pass needs of both children, coalesced by
+            // split rank: their sample indices and box volumes
+            a.sdat[2 * (m - L)] = make_int4(v[0], v[1], v[2], v[3]);
+            a.sdat[2 * (m - L) + 1] = make_int4(v[4], __float_as_int(box_volume<D>(mn, cmx)),
+                                                __float_as_int(box_volume<D>(cmn, mx)), 0);
+            if (a.sext) {  // learned mode: the children's extents for their features
+                float ex[6];
 #pragma unroll
-            for (int d = 0; d < D; ++d)
-                if (d == axis) right = mx[d] - cmn[d];
-            a.sext[2 * (m - L) + 1] = make_int4(__float_as_int(ex[4]), __float_as_int(ex[5]),
-                                                __float_as_int(right), axis);
-        }
-        if (!a.in_loop) {  // in the loop the next error pass overwrites both
-            a.err[i] = -1.0f;
-            a.err[m] = -1.0f;
+                for (int d = 0; d < 6; ++d) ex[d] = d < D ? (d == axis ? cmx[d] - mn[d] : diag[d]) : 0.0f;
+                a.sext[2 * (m - L)] = make_int4(__float_as_int(ex[0]), __float_as_int(ex[1]),
+                                                __float_as_int(ex[2]), __float_as_int(ex[3]));
+                float right = 0.0f;
+#pragma unroll
+                for (int d = 0; d < D; ++d)
+                    if (d == axis) right = mx[d] - cmn[d];
+                a.sext[2 * (m - L) + 1] = make_int4(__float_as_int(ex[4]), __float_as_int(ex[5]),
+                                                    __float_as_int(right), axis);
+            }
+            if (!a.in_loop) {  // in the loop the next error pass overwrites both
+                a.err[i] = -1.0f;
+                a.err[m] = -1.0f;
+            }
         }
         a.seed[m] = 0u;
         a.flags[m] = 3;
@@ -715,6 +810,100 @@ __device__ __forceinline__ void place_leaf(const DevGrid& a, int i, int k, int m
     }
     // the leaf's own state (already jumped) and count were written by the
     // selection and compaction kernels
+    if constexpr (FUSED) {
+        // the line's stores are out and its registers free; the values of a
+        // split's other samples load while the new one is evaluated
+        const bool split = cnt == 4u;
+        LeafSamples ch[2];
+        if (split) {
+#pragma unroll
+            for (int j = 0; j < 5; ++j) {
+                const float* o = a.values + (size_t)(kid[j] == k ? kid[j == 0 ? 1 : 0] : kid[j]) * 3;
+                LeafSamples& c = ch[j < 2 ? 0 : 1];
+                const int q = j < 2 ? j : j - 2;
+                c.vx[q] = o[0];
+                c.vy[q] = o[1];
+                c.vz[q] = o[2];
+            }
+        }
+        float xe[6];
+#pragma unroll
+        for (int d = 0; d < 6; ++d) xe[d] = d < D ? best[d] : 0.0f;
+        const mscene::V3<float> val =
+            mscene::eval<float>(B->p, obj, xe, &B->accel, &B->cells, reinterpret_cast<const uint64_t*>(B + 1));
+        float* vo = a.values + (size_t)k * 3;
+        vo[0] = val.x;
+        vo[1] = val.y;
+        vo[2] = val.z;
+        if (split) {
+#pragma unroll
+            for (int j = 0; j < 5; ++j) {
+                LeafSamples& c = ch[j < 2 ? 0 : 1];
+                const int q = j < 2 ? j : j - 2;
+                c.vx[q] = kid[j] == k ? val.x : c.vx[q];
+                c.vy[q] = kid[j] == k ? val.y : c.vy[q];
+                c.vz[q] = kid[j] == k ? val.z : c.vz[q];
+            }
+            const int two[4] = {0, 0, -1, -1}, three[4] = {0, 0, 0, -1};
+            const float el = error_of_values(two, vol_l, ch[0]);
+            const float er = error_of_values(three, vol_r, ch[1]);
+            a.err[i] = el;
+            a.err[m] = er;
+            emax = fmaxf(emax, fmaxf(el, er));
+        }
+    }
+}
+
+// Where chunk blk's new samples and right children start (base: ranks among
+// all selected and split leaves), from the super groups and the partials of
+// its own group; every wave computes it for itself.  False if the pass would
+// exceed the capacity.  One thread writes the next slot, the pass's
+// statistics and the totals' zeros for the pass after (no kernel of this pass
+// reads those).
+__device__ __forceinline__ bool fused_offsets(const DevGrid& a, int blk, int nblk, int par, int& L,
+                                              int& N, int2& base) {
+    DevCounters* cn = a.cnt;
+    const LoopSlot s = cn->slot[par];
+    L = s.L;
+    N = s.N;
+    const int lane = threadIdx.x & 63;
+    const int per = super_size(nblk), g = blk / per;
+    const SuperSum t = a.ssum[par * kSuper + lane];
+    const int sel = wave_sum(t.sel), split = wave_sum(t.split);
+    const bool fits = (long long)N + sel <= a.cap_s && (long long)L + split <= a.cap_l;
+    if (blk == 0 && threadIdx.x < kSuper) {
+        const int held = wave_sum(t.held);
+        if (fits) {
+            SuperSum& z = a.ssum[(par ^ 1) * kSuper + lane];
+            z.sel = z.split = z.held = 0;
+            a.smax[par * kSuper + lane].err = 0u;  // the selection has read it
+        }
+        if (lane == 0) {
+            if (!fits) {
+                cn->status = MDAS_ERR_CAPACITY_DEV;
+                cn->done = 1;
+            } else {
+                const int P = cn->passes;
+                // leaves whose errors were estimated since the last pass, and
+                // the values that took: the initial leaves, then the children
+                const int stale = P == 0 ? L : 2 * s.new_n, vals = P == 0 ? 4 * L : 5 * s.new_n;
+                a.pstats[P & (kMaxPassStats - 1)] = PassStat{L, N, sel, split, held, stale, vals, 0};
+                cn->passes = P + 1;
+                cn->slot[par ^ 1] = LoopSlot{N + sel, L + split, N, L, sel, split};
+                cn->cur = par ^ 1;
+            }
+        }
+    }
+    if (!fits) return false;
+    int2 own = make_int2(0, 0);
+    for (int c = g * per + lane; c < blk; c += 64) {
+        const int4 p = a.part[c];
+        own.x += p.x;
+        own.y += p.y;
+    }
+    base.x = wave_sum(own.x + (lane < g ? t.sel : 0));
+    base.y = wave_sum(own.y + (lane < g ? t.split : 0));
+    return true;
 }
 
 // Compaction and placement in one kernel.  Each workgroup ranks the selected
@@ -726,19 +915,40 @@ __device__ __forceinline__ void place_leaf(const DevGrid& a, int i, int k, int m
 // they start from queue up in LDS and are placed a round of 256 at a time,
 // one per thread.  Every leaf's count and LCG state are rewritten in the
 // same sweep, as they stand after the placement, in full coalesced lines.
-template <int D>
-__device__ __forceinline__ void compact_place_body(const DevGrid& a, int blk, int nblk) {
+// What bounds it at 1080p is the traffic of its scattered leaf lines; a small
+// tree's pass is the chain of its launches and of one leaf's work.  FUSED (the
+// new sample's integrand and the children's errors taken here) leaves the
+// traffic of a large pass as it was less the split entries, and two launches
+// of six: 5D 1080p (1.5 M leaves a pass) 15.6 -> 14.7 ms a run, 64x48 (12
+// passes of 2000) 617 -> 458 us, 3D 256x256 1240 -> 850 us.  One chunk per wave
+// in place of one per workgroup (fewer barriers, 4x the chunks) was slower at
+// 1080p (12.0 -> 12.9 ms a run at its best count) and no faster below.
+// FUSED: see place_leaf; the offsets come from the super groups' totals and
+// the partials of the chunk's own group, in place of the scan kernel; every
+// workgroup finds the same totals, so a pass beyond the capacity writes nothing.
+template <int D, bool FUSED>
+__device__ __forceinline__ void compact_place_body(const DevGrid& a, int blk, int nblk, int par,
+                                                   const mscene::SceneBlock* B, float* obj) {
     constexpr int U = 4;                   // tiles whose flags and states are loaded together
     constexpr int QCAP = U * 256 + 256;    // one step's entries plus an unplaced remainder
     __shared__ int lds[8];
     __shared__ int2 qe[QCAP];
     __shared__ unsigned qs[QCAP];
     if (a.cnt->done) return;
-    const int L = a.cnt->n_leaves_old;
-    const int N0 = a.cnt->n_samples_old;
+    int L, N0;
+    int2 base;
+    if constexpr (FUSED) {
+        if (!fused_offsets(a, blk, nblk, par, L, N0, base)) return;
+        for (int q = threadIdx.x; q < B->p.n_obj * mscene::OBJ_STRIDE; q += 256) obj[q] = B->p.obj[q];
+        __syncthreads();
+    } else {
+        L = a.cnt->n_leaves_old;
+        N0 = a.cnt->n_samples_old;
+        base = a.part_off[blk];
+    }
+    float emax = 0.0f;
     int beg, end;
     chunk_range(L, nblk, blk, beg, end);
-    int2 base = a.part_off[blk];
     int jq = base.x;  // global rank of the entry at the front of the queue
     int qn = 0;       // queued entries
     auto place_round = [&](int p0, int count) {
@@ -746,7 +956,7 @@ __device__ __forceinline__ void compact_place_body(const DevGrid& a, int blk, in
         if ((int)threadIdx.x < count) {
             const int2 q = qe[p];
             const unsigned cnt = q.y >= 0 ? 4u : ((unsigned)q.x >> 30);
-            place_leaf<D>(a, q.x & 0x3fffffff, N0 + jq + p, q.y, cnt, L, qs[p]);
+            place_leaf<D, FUSED>(a, q.x & 0x3fffffff, N0 + jq + p, q.y, cnt, L, qs[p], B, obj, emax);
         }
     };
     for (int t00 = beg; t00 < end; t00 += U * 256) {
@@ -807,15 +1017,64 @@ __device__ __forceinline__ void compact_place_body(const DevGrid& a, int blk, in
         __syncthreads();
     }
     place_round(0, qn);
+    if constexpr (FUSED) {
+        emax = wave_max(emax);
+        __syncthreads();
+        if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = (int)__float_as_uint(emax);
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            const unsigned m = max(max((unsigned)lds[0], (unsigned)lds[1]), max((unsigned)lds[2], (unsigned)lds[3]));
+            if (m != 0u) atomicMax(&a.smax[(par ^ 1) * kSuper + blk / super_size(nblk)].err, m);
+        }
+    }
 }
 
 template <int D>
 __global__ __launch_bounds__(256) void k_compact_place(DevGrid a) {
-    compact_place_body<D>(a, blockIdx.x, gridDim.x);
+    compact_place_body<D, false>(a, blockIdx.x, gridDim.x, 0, nullptr, nullptr);
 }
 template <int D>
 __global__ __launch_bounds__(256) void k_compact_place_b(const DevGrid* grids) {
-    compact_place_body<D>(grids[blockIdx.y], blockIdx.x, gridDim.x);
+    const DevGrid a = grids[blockIdx.y];  // by value: scalar registers
+    compact_place_body<D, false>(a, blockIdx.x, gridDim.x, 0, nullptr, nullptr);
+}
+// The scene's objects in dynamic LDS (48 bytes each).
+template <int D>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_place_fused(DevGrid a, const mscene::SceneBlock* B, int par) {
+    extern __shared__ float obj[];
+    compact_place_body<D, true>(a, blockIdx.x, gridDim.x, par, B, obj);
+}
+template <int D>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_place_fused_b(const DevGrid* grids, const void* const* params, int par) {
+    extern __shared__ float obj[];
+    const DevGrid a = grids[blockIdx.y];  // by value: scalar registers
+    compact_place_body<D, true>(a, blockIdx.x, gridDim.x, par,
+                                (const mscene::SceneBlock*)params[blockIdx.y], obj);
+}
+
+// The counters that are read outside the fused loop, from the current slot;
+// `done` once the loop has reached its limit, so that the host need not
+// launch another pass to learn it.
+__device__ __forceinline__ void loop_end_body(DevCounters* c) {
+    const LoopSlot s = c->slot[c->cur];
+    c->n_samples = s.N;
+    c->n_leaves = s.L;
+    c->n_samples_old = s.N_old;
+    c->n_leaves_old = s.L_old;
+    c->new_samples = s.new_s;
+    c->new_nodes = s.new_n;
+    if (loop_limit_reached(c)) c->done = 1;
+}
+__global__ void k_loop_end(DevCounters* c) { loop_end_body(c); }
+__global__ void k_loop_status_b(const DevGrid* grids, int n, int fused, int* out) {
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= n) return;
+    DevCounters* c = grids[t].cnt;
+    if (fused) loop_end_body(c);
+    out[4 * t] = c->done;
+    out[4 * t + 1] = c->status;
+    out[4 * t + 2] = c->n_samples;
+    out[4 * t + 3] = c->passes;
 }
 
 // After the device-side loop: when it stopped at its limit, no error pass
@@ -883,7 +1142,7 @@ static int grid_for(long long n, int cap_blocks = 8192) {
 hipError_t launch_initial(Grid& g, int L0, hipStream_t st) {
     const int blocks = grid_for(L0, 4096);
     MDAS_DISPATCH_D(g.D, hipLaunchKernelGGL(k_initial<DD>, dim3(blocks), dim3(256), 0, st, g.dev, L0));
-    hipLaunchKernelGGL(k_initial_counters, dim3(1), dim3(1), 0, st, g.dev.cnt, L0);
+    hipLaunchKernelGGL(k_initial_counters, dim3(1), dim3(2 * kSuper), 0, st, g.dev, L0);
     return hipGetLastError();
 }
 
@@ -918,18 +1177,18 @@ hipError_t launch_errors_stale(Grid& g, hipStream_t st) {
 }
 
 hipError_t launch_select(Grid& g, hipStream_t st) {
-    const int cpw = select_cpw(g.chunk_blocks);
-    hipLaunchKernelGGL(k_select, dim3(g.chunk_blocks / cpw), dim3(256), 0, st, g.dev, cpw);
+    const int cpw = select_cpw(g.chunks());
+    hipLaunchKernelGGL(k_select, dim3(g.chunks() / cpw), dim3(256), 0, st, g.dev, cpw);
     return hipGetLastError();
 }
 
 hipError_t launch_scan(Grid& g, hipStream_t st) {
-    hipLaunchKernelGGL(k_scan_counts, dim3(1), dim3(1024), 0, st, g.dev, g.chunk_blocks);
+    hipLaunchKernelGGL(k_scan_counts, dim3(1), dim3(1024), 0, st, g.dev, g.chunks());
     return hipGetLastError();
 }
 
 hipError_t launch_place(Grid& g, hipStream_t st) {
-    MDAS_DISPATCH_D(g.D, hipLaunchKernelGGL(k_compact_place<DD>, dim3(g.chunk_blocks), dim3(256), 0, st,
+    MDAS_DISPATCH_D(g.D, hipLaunchKernelGGL(k_compact_place<DD>, dim3(g.chunks()), dim3(256), 0, st,
                                             g.dev));
     return hipGetLastError();
 }
@@ -939,6 +1198,46 @@ hipError_t launch_adaptive(Grid& g, hipStream_t st) {
     if (e == hipSuccess) e = launch_scan(g, st);
     if (e == hipSuccess) e = launch_place(g, st);
     return e;
+}
+
+hipError_t launch_first_errors(Grid& g, hipStream_t st) {
+    const int blocks = grid_for(1ll << (g.b * g.D + 2 * g.e), g.err_blocks);
+    MDAS_DISPATCH_D(g.D, hipLaunchKernelGGL(k_first_errors<DD>, dim3(blocks), dim3(256), 0, st, g.dev));
+    return hipGetLastError();
+}
+
+hipError_t launch_fused_pass(Grid& g, const void* dparams, int n_obj, int parity, hipStream_t st) {
+    const int chunks = g.chunks(), cpw = select_cpw(chunks);
+    hipLaunchKernelGGL(k_select_fused, dim3(chunks / cpw), dim3(256), 0, st, g.dev, cpw, parity);
+    MDAS_DISPATCH_D(g.D, hipLaunchKernelGGL(k_place_fused<DD>, dim3(chunks), dim3(256),
+                                            n_obj * mscene::OBJ_STRIDE * sizeof(float), st, g.dev,
+                                            (const mscene::SceneBlock*)dparams, parity));
+    return hipGetLastError();
+}
+
+hipError_t launch_loop_end(Grid& g, hipStream_t st) {
+    hipLaunchKernelGGL(k_loop_end, dim3(1), dim3(1), 0, st, g.dev.cnt);
+    return hipGetLastError();
+}
+
+hipError_t launch_first_errors_b(int D, const DevGrid* grids, int n, int blocks, hipStream_t st) {
+    MDAS_DISPATCH_D(D, hipLaunchKernelGGL(k_first_errors_b<DD>, dim3(blocks < 1024 ? blocks : 1024, n), dim3(256), 0,
+                                          st, grids));
+    return hipGetLastError();
+}
+
+hipError_t launch_fused_pass_b(int D, const DevGrid* grids, const void* const* params, int n_obj,
+                               int n, int blocks, int parity, hipStream_t st) {
+    const int cpw = select_cpw(blocks);
+    hipLaunchKernelGGL(k_select_fused_b, dim3(blocks / cpw, n), dim3(256), 0, st, grids, cpw, parity);
+    MDAS_DISPATCH_D(D, hipLaunchKernelGGL(k_place_fused_b<DD>, dim3(blocks, n), dim3(256),
+                                          n_obj * mscene::OBJ_STRIDE * sizeof(float), st, grids, params, parity));
+    return hipGetLastError();
+}
+
+hipError_t launch_loop_status_b(const DevGrid* grids, int n, int fused, int* out, hipStream_t st) {
+    hipLaunchKernelGGL(k_loop_status_b, dim3((n + 63) / 64), dim3(64), 0, st, grids, n, fused, out);
+    return hipGetLastError();
 }
 
 hipError_t launch_mark_last_children(Grid& g, hipStream_t st) {
@@ -974,7 +1273,7 @@ hipError_t launch_fill_f32(float* p, float v, long long n, hipStream_t st) {
 hipError_t launch_initial_b(int D, const DevGrid* grids, int n, int blocks, const int* limits,
                             hipStream_t st) {
     MDAS_DISPATCH_D(D, hipLaunchKernelGGL(k_initial_b<DD>, dim3(blocks, n), dim3(256), 0, st, grids));
-    hipLaunchKernelGGL(k_initial_counters_b, dim3((n + 63) / 64), dim3(64), 0, st, grids, n, limits);
+    hipLaunchKernelGGL(k_initial_counters_b, dim3(n), dim3(2 * kSuper), 0, st, grids, limits);
     return hipGetLastError();
 }
 

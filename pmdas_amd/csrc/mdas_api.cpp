@@ -57,7 +57,7 @@ void free_grid(Grid& g) {
     mdas::ReconBufs& rb = g.rb;
     void* ptrs[] = {d.coords,   d.values,  d.leaf,        d.err,        d.seed,     d.flags,
                     d.xpts,     d.split_list, d.sdat,     d.sext,       d.part,     d.part_off,
-                    d.epart,    d.cnt,     d.pstats,      rb.rrec,      rb.keys,    rb.keys_alt,
+                    d.epart,    d.cnt,     d.ssum, d.smax, d.pstats,      rb.rrec,      rb.keys,    rb.keys_alt,
                     rb.tile_start, rb.tile_end, rb.rs_hist, g.d_scalar, g.learn.feat, g.learn.perr,
                     g.learn.rows};
     for (void* p : ptrs)
@@ -238,6 +238,8 @@ int mdas_create(const mdas_config* cfg, mdas_handle* out) {
     if (e == hipSuccess) e = dalloc(&d.part_off, (size_t)mdas::kChunkBlocks);
     if (e == hipSuccess) e = dalloc(&d.epart, (size_t)mdas::kErrBlocks);
     if (e == hipSuccess) e = dalloc(&d.cnt, 1);
+    if (e == hipSuccess) e = dalloc(&d.ssum, (size_t)(2 * mdas::kSuper));
+    if (e == hipSuccess) e = dalloc(&d.smax, (size_t)(2 * mdas::kSuper));
     if (e == hipSuccess) e = dalloc(&d.pstats, (size_t)mdas::kMaxPassStats);
     if (e == hipSuccess) e = dalloc(&g.d_scalar, 64);
     if (e != hipSuccess) {
@@ -757,7 +759,7 @@ int mdas_run(mdas_handle h, mdas_scene_handle s, long long target, void* stream)
     hipStream_t st = S(stream);
     const int L0 = 1 << (g.b * g.D + 2 * g.e);
     const long long limit = std::min<long long>(target, g.max_samples);
-    const int B = std::max(1, g.passes_per_sync);
+    const int B = std::max(2, g.passes_per_sync & ~1);  // even: the fused passes alternate
     // the log needs per-pass times: logging times the run like mdas_set_timing
     const bool logging = g.logging();
     const bool timing_was = g.timing;
@@ -790,8 +792,16 @@ int mdas_run(mdas_handle h, mdas_scene_handle s, long long target, void* stream)
         explicit LoopMode(mdas::DevGrid& x) : d(x) { d.in_loop = 1; }
         ~LoopMode() { d.in_loop = 0; }
     } loop_mode{g.dev};
+    // The plain method's pass is two kernels, the new samples evaluated and
+    // the children's errors taken where they are placed.  Timing and logs want
+    // the phases apart and the learned error pass is a kernel of its own:
+    // those run the separate kernels, with the same results.
+    const bool fused = !g.timing && g.learn_mode == 0;
+    if (fused) HIP_TRY(mdas::launch_first_errors(g, st));
     for (;;) {
-        for (int b = 0; b < B; ++b) {
+        for (int b = 0; b < B && fused; ++b) HIP_TRY(mdas::launch_fused_pass(g, s->dev, s->host.n_obj, b & 1, st));
+        if (fused) HIP_TRY(mdas::launch_loop_end(g, st));
+        for (int b = 0; b < B && !fused; ++b) {
             mdas::kbeg(g, st, "k_errors");
             HIP_TRY(g.learn_mode ? mdas::launch_errors_learned(g, st)
                                  : mdas::launch_errors_stale(g, st));
@@ -895,7 +905,7 @@ static double kernel_bytes(const Grid& g, const std::string& k) {
         else if (k == "k_select")  // error, state, flags read; flags written
             b += 10.0 * p.L;
         else if (k == "k_scan_counts")
-            b += (16.0 + 8.0) * g.chunk_blocks;
+            b += (16.0 + 8.0) * g.chunks();
         else if (k == "k_place")  // compaction and placement
             b += 10.0 * p.L +                                    // flags, states read and written
                  (double)p.sel * (SB + 4.0 * D) +                // slots + box, the new sample
@@ -907,7 +917,7 @@ static double kernel_bytes(const Grid& g, const std::string& k) {
     const double L = (double)g.host.n_leaves, N = (double)g.host.n_samples;
     const double K = (double)g.host.n_keys;
     if (k == "k_recon_prep") return L * (SB + 32.0) + 12.0 * N;
-    if (k == "k_scan_keys") return (16.0 + 8.0) * g.chunk_blocks;
+    if (k == "k_scan_keys") return (16.0 + 8.0) * g.chunks();
     if (k == "k_recon_emit") return L * 16.0 + K * 8.0;
     if (k == "k_rs_hist") return K * 8.0 * g.recon_sort_passes;
     if (k == "k_rs_scan") return 3.0 * 4.0 * (1 << g.recon_sort_bits) * 1024 * g.recon_sort_passes;

@@ -27,6 +27,22 @@ struct Group {
     int* d_status = nullptr;             // (done, status, samples, passes) per member
     mdas::LearnDev* d_learn = nullptr;   // per member, when any member is in learned mode
     int blocks = 0;
+    int max_chunks = 1;                  // chunks the largest member's capacity fills
+    int n_obj = 0;                       // most objects of a member's scene
+    bool fused() const { return d_learn == nullptr; }  // plain members only: two kernels per pass
+    hipError_t first_errors(hipStream_t st) const {
+        return fused() ? mdas::launch_first_errors_b(D, d_grids, (int)members.size(), blocks, st) : hipSuccess;
+    }
+    hipError_t pass(int p, hipStream_t st) const {
+        const int m = (int)members.size();
+        if (fused()) return mdas::launch_fused_pass_b(D, d_grids, d_params, n_obj, m, blocks, p & 1, st);
+        const hipError_t e = mdas::launch_pass_b(D, d_grids, m, blocks, st, d_learn);
+        return e != hipSuccess ? e : mdas::launch_eval_b(d_grids, d_params, m, blocks, st);
+    }
+    void set_blocks(int total) {
+        blocks = std::max(64, std::min(mdas::kChunkBlocks, total / (int)members.size()));
+        blocks = std::min(blocks, max_chunks);
+    }
     hipGraph_t graph = nullptr;
     hipGraphExec_t exec = nullptr;
 };
@@ -37,16 +53,6 @@ struct Group {
         if (e_ != hipSuccess)                                                                  \
             return mdas::set_error(MDAS_ERR_HIP, std::string(#expr) + ": " + hipGetErrorString(e_)); \
     } while (0)
-
-__global__ void k_batch_status(const mdas::DevGrid* grids, int n, int* out) {
-    const int t = blockIdx.x * blockDim.x + threadIdx.x;
-    if (t < n) {
-        out[4 * t] = grids[t].cnt->done;
-        out[4 * t + 1] = grids[t].cnt->status;
-        out[4 * t + 2] = grids[t].cnt->n_samples;
-        out[4 * t + 3] = grids[t].cnt->passes;
-    }
-}
 
 }  // namespace
 
@@ -127,8 +133,13 @@ int mdas_batch_create(mdas_handle* grids, mdas_scene_handle* scenes, int n, mdas
             if (grids[i]->g.D == D) gr.members.push_back(i);
         if (gr.members.empty()) continue;
         const int m = (int)gr.members.size();
+        for (int i : gr.members) {
+            gr.max_chunks = std::max(gr.max_chunks, grids[i]->g.cap_l / 256 + 1);
+            gr.n_obj = std::max(gr.n_obj, (int)scenes[i]->host.n_obj);
+        }
         // workgroups per image: about 8192 per launch in all, at least 64
-        gr.blocks = std::max(64, std::min(mdas::kChunkBlocks, 8192 / m));
+        // where the leaves fill them
+        gr.set_blocks(8192);
         std::vector<mdas::DevGrid> dg(m);
         std::vector<const void*> dp(m);
         std::vector<mdas::LearnDev> dl(m);
@@ -191,7 +202,7 @@ int mdas_batch_run(mdas_batch_handle b, const long long* targets, void* stream, 
     hipStream_t st = nullptr;
     B_TRY(enter_stream(b, stream, use_graph != 0, &st));
     const auto t0 = std::chrono::steady_clock::now();
-    const int B = std::max(1, b->passes_per_block);
+    const int B = std::max(2, b->passes_per_block & ~1);  // even: the fused passes alternate
     // initial grids and their integrand, one launch per kernel per group
     std::vector<std::vector<int>> limits(b->groups.size());
     for (size_t gi = 0; gi < b->groups.size(); ++gi) {
@@ -205,6 +216,7 @@ int mdas_batch_run(mdas_batch_handle b, const long long* targets, void* stream, 
         B_TRY(hipMemcpyAsync(g.d_limits, limits[gi].data(), sizeof(int) * m, hipMemcpyHostToDevice, st));
         B_TRY(mdas::launch_initial_b(g.D, g.d_grids, m, g.blocks, g.d_limits, st));
         B_TRY(mdas::launch_eval_b(g.d_grids, g.d_params, m, g.blocks, st));
+        B_TRY(g.first_errors(st));
         for (int k = 0; k < m; ++k) {
             b->grids[g.members[k]]->g.initialized = true;
             mdas::initial_extents(b->grids[g.members[k]]->g);
@@ -223,22 +235,16 @@ int mdas_batch_run(mdas_batch_handle b, const long long* targets, void* stream, 
                 if (!g.exec) {
                     B_TRY(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
                     hipError_t ce = hipSuccess;
-                    for (int p = 0; p < B && ce == hipSuccess; ++p) {
-                        ce = mdas::launch_pass_b(g.D, g.d_grids, m, g.blocks, st, g.d_learn);
-                        if (ce == hipSuccess) ce = mdas::launch_eval_b(g.d_grids, g.d_params, m, g.blocks, st);
-                    }
+                    for (int p = 0; p < B && ce == hipSuccess; ++p) ce = g.pass(p, st);
                     B_TRY(hipStreamEndCapture(st, &g.graph));
                     B_TRY(ce);
                     B_TRY(hipGraphInstantiate(&g.exec, g.graph, nullptr, nullptr, 0));
                 }
                 B_TRY(hipGraphLaunch(g.exec, st));
             } else {
-                for (int p = 0; p < B; ++p) {
-                    B_TRY(mdas::launch_pass_b(g.D, g.d_grids, m, g.blocks, st, g.d_learn));
-                    B_TRY(mdas::launch_eval_b(g.d_grids, g.d_params, m, g.blocks, st));
-                }
+                for (int p = 0; p < B; ++p) B_TRY(g.pass(p, st));
             }
-            hipLaunchKernelGGL(k_batch_status, dim3((m + 63) / 64), dim3(64), 0, st, g.d_grids, m, g.d_status);
+            B_TRY(mdas::launch_loop_status_b(g.d_grids, m, g.fused() ? 1 : 0, g.d_status, st));
         }
         ++blocks_run;
         B_TRY(hipStreamSynchronize(st));
@@ -370,8 +376,7 @@ int mdas_batch_integrate(mdas_batch_handle b, float* const* pixels, const int* w
 // (per launch about `total` in all, clamped to [64, kChunkBlocks] per image).
 static void set_batch_shape(mdas_batch* b, int total) {
     for (Group& g : b->groups) {
-        const int m = (int)g.members.size();
-        g.blocks = std::max(64, std::min(mdas::kChunkBlocks, total / m));
+        g.set_blocks(total);
         if (g.exec) (void)hipGraphExecDestroy(g.exec);
         if (g.graph) (void)hipGraphDestroy(g.graph);
         g.exec = nullptr;

@@ -3,10 +3,18 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <string>
 #include <vector>
 
 namespace mdas {
+
+// What a pass of the device-side loop starts from: sample and leaf counts,
+// those before the pass that led here and that pass's new ones.  Two slots by
+// pass parity: a pass's kernels read one while a single thread writes the other.
+struct LoopSlot {
+    int N, L, N_old, L_old, new_s, new_n;
+};
 
 // Device-resident counters of one grid.  Every kernel reads N / L from here,
 // so a whole sampling loop can be enqueued without host round trips.
@@ -32,6 +40,20 @@ struct DevCounters {
     int guard_cap;       // device-side loop: no pass starts once N + L > guard_cap (the
                          //   sample capacity when the target is at or beyond it; 0 = no
                          //   guard: a smaller target, standalone calls)
+    int cur;             // fused loop: the slot that holds the tree's state
+    LoopSlot slot[2];
+};
+
+// Per-pass totals of the fused loop in kSuper groups of chunks, two of each by
+// pass parity: integer sums and maxima taken with atomics, each group in a
+// 128-byte line of its own (a single address would serialise thousands of
+// them), so that any wave gets a total or a prefix with one load per lane.
+static const int kSuper = 64;
+struct SuperSum {  // selected and split leaves, samples the selected hold
+    int sel, split, held, pad[29];
+};
+struct SuperMax {  // float bits of the largest error the next pass starts from
+    unsigned err, pad[31];
 };
 
 // Per-pass statistics, one row per adaptive pass (for algorithmic byte counts):
@@ -102,6 +124,8 @@ struct DevGrid {
     uint4* epart;          // [kErrBlocks] per-workgroup (max error bits, stale, values)
     unsigned char* rcnt;   // [cap_l]      reconstruction tiles per leaf
     DevCounters* cnt;
+    SuperSum* ssum;        // [2][kSuper]
+    SuperMax* smax;        // [2][kSuper]
     PassStat* pstats;
     int D;
     int cap_s, cap_l;
@@ -203,6 +227,10 @@ struct Grid {
     // launch shape of the per-pass kernels (mdas_set_launch_shape)
     int chunk_blocks = 4096;   // leaf chunks of selection / compaction / reconstruction
     int err_blocks = 1024;     // workgroups of the error pass
+    // chunks in use: none for less than 256 leaves of the capacity (for a
+    // thumbnail's 20 thousand leaves, 4096 nearly all empty workgroups cost
+    // the selection 7.9 us a launch, 90 cost 5.0)
+    int chunks() const { return std::min(chunk_blocks, cap_l / 256 + 1); }
     // learned proposal (mode bits: 1 collect rows, 2 score with the MLP)
     int learn_mode = 0;
     LearnDev learn{};
@@ -238,6 +266,13 @@ hipError_t launch_select(Grid& g, hipStream_t st);
 hipError_t launch_scan(Grid& g, hipStream_t st);
 hipError_t launch_place(Grid& g, hipStream_t st);
 hipError_t launch_set_limit(Grid& g, int limit, hipStream_t st);
+// The fused loop: errors of the initial leaves, then per pass one selection
+// and one placement kernel (which evaluates the new samples and the errors of
+// the children); parity alternates from 0.  launch_loop_end brings the
+// counters up to date and raises `done` at the limit.
+hipError_t launch_first_errors(Grid& g, hipStream_t st);
+hipError_t launch_fused_pass(Grid& g, const void* dparams, int n_obj, int parity, hipStream_t st);
+hipError_t launch_loop_end(Grid& g, hipStream_t st);
 hipError_t launch_arm(Grid& g, hipStream_t st);
 hipError_t launch_build_pts(Grid& g, int n_leaves, hipStream_t st);
 hipError_t launch_mark_last_children(Grid& g, hipStream_t st);
@@ -248,6 +283,12 @@ hipError_t launch_fill_f32(float* p, float v, long long n, hipStream_t st);
 // Batched forms over a device array of n grids of dimension D (k_sampling.hip)
 hipError_t launch_initial_b(int D, const DevGrid* grids, int n, int blocks, const int* limits,
                             hipStream_t st);
+hipError_t launch_first_errors_b(int D, const DevGrid* grids, int n, int blocks, hipStream_t st);
+hipError_t launch_fused_pass_b(int D, const DevGrid* grids, const void* const* params, int n_obj,
+                               int n, int blocks, int parity, hipStream_t st);
+// out[4 i ..]: done, status, samples, passes of image i, after the end of a
+// block of fused passes (fused != 0) or of the separate kernels.
+hipError_t launch_loop_status_b(const DevGrid* grids, int n, int fused, int* out, hipStream_t st);
 // learns: device array of n LearnDev (the learned error pass) or null (plain)
 hipError_t launch_pass_b(int D, const DevGrid* grids, int n, int blocks, hipStream_t st,
                          const LearnDev* learns = nullptr);

@@ -185,9 +185,11 @@ __device__ __forceinline__ void store_line_head2(const DevGrid& a, int i, int4 i
 // The error kernels of a pass test it (every workgroup reads the same
 // counters) and the reduction after them raises `done` for the rest of the
 // pass.
+__device__ __forceinline__ bool loop_limit_reached(const DevCounters* c, int N, int L) {
+    return N >= c->limit || (c->guard_cap != 0 && (long long)N + L > (long long)c->guard_cap);
+}
 __device__ __forceinline__ bool loop_limit_reached(const DevCounters* c) {
-    return c->n_samples >= c->limit ||
-           (c->guard_cap != 0 && (long long)c->n_samples + c->n_leaves > (long long)c->guard_cap);
+    return loop_limit_reached(c, c->n_samples, c->n_leaves);
 }
 __device__ __forceinline__ bool pass_stopped(const DevCounters* c) {
     return c->done || loop_limit_reached(c);
