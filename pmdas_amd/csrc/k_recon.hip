@@ -19,7 +19,6 @@
 //     index order.
 #include <algorithm>
 #include <cmath>
-#include <type_traits>
 
 #include "mdas_leaf.hpp"
 
@@ -417,22 +416,63 @@ __global__ __launch_bounds__(256) void k_tile_ranges(const unsigned long long* k
 }
 
 // ---------------------------------------------------------------- gather --
-// GS = pixels per tile (16 or 64); a wave holds 64/GS tiles.
+// GS = pixels per tile (16 or 64); a wave holds 64/GS tiles and takes GS
+// records of each at a time, a record per lane, then a pixel per lane.  What
+// bounds it is arithmetic (a record covers 2 to 5 pixels of a tile), so all
+// that depends on the record and a column or a row only is done once, by the
+// record's lane: the walk of the accumulated pixel bounds (kdgrid.cu:532-576)
+// and the overlap with each of its columns and rows, kept in LDS (a pixel's
+// lane did both for itself, per record: 920 us at 1080p for 26 M records, now
+// 525; 640x360 48 -> 25 us), and the lanes of the
+// pixels it overlaps get its bit with LDS atomics (one ballot per pixel where
+// a record overlaps more than kOrPixels).  A pixel then adds its records'
+// contributions in index order: two overlaps, a product and a quotient each.
+static const int kOrPixels = 20;
+// Dynamic LDS of one wave: means and volumes, coverage words, xy areas, and
+// the overlaps, TW + TH per record (an odd stride spreads them over the banks).
+__host__ __device__ constexpr int gather_stride(int TW, int TH) { return (TW + TH) | 1; }
+__host__ __device__ constexpr int gather_lds(int TW, int TH) { return 64 * (16 + 8 + 4 + 4 * gather_stride(TW, TH)); }
+
+// Overlap of [mn, mx] with the pixels [p0, p1) of an axis, of which the span
+// starts at s0 (at coordinate lo), into ov[p - base]; a bit per positive one.
+__device__ __forceinline__ unsigned long long axis_overlaps(float mn, float mx, int s0, float lo, float step,
+                                                            int p0, int p1, int base, float* ov) {
+    float pMin = lo, pMax = lo + step;
+    for (int q = s0; q < p0; ++q) {  // exactly as kdgrid.cu:536-576 walks them
+        pMin = pMax;
+        pMax += step;
+    }
+    unsigned long long bits = 0ull;
+    for (int q = p0; q < p1; ++q) {
+        const float d = fminf(pMax, mx) - fmaxf(pMin, mn);
+        ov[q - base] = d;
+        if (d > 0.0f) bits |= 1ull << (q - base);
+        pMin = pMax;
+        pMax += step;
+    }
+    return bits;
+}
+
 template <int GS>
 __global__ __launch_bounds__(256) void k_gather(ReconGeo G, const float4* __restrict__ rrec,
                                                 const unsigned long long* __restrict__ keys,
                                                 const int* __restrict__ tstart,
                                                 const int* __restrict__ tend, float4* pixels) {
-    __shared__ float4 r0[4][64], r1[4][64], r2[4][64];
-    __shared__ float2 r3[4][64];
+    extern __shared__ float4 gather_mem[];
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+    const int stride = gather_stride(G.TW, G.TH);
+    char* mem = reinterpret_cast<char*>(gather_mem) + w * gather_lds(G.TW, G.TH);
+    float4* mean = reinterpret_cast<float4*>(mem);
+    unsigned long long* covers = reinterpret_cast<unsigned long long*>(mem + 64 * 16);
+    float* area = reinterpret_cast<float*>(mem + 64 * 24);
+    float* ov = area + 64;
     const int grp = lane / GS, gl = lane % GS;      // tile within the wave, lane within the tile
-    const int tile = (blockIdx.x * 4 + w) * (64 / GS) + grp;
+    const int tile = (blockIdx.x * (blockDim.x >> 6) + w) * (64 / GS) + grp;
     const int ntiles = G.tilesX * G.tilesY;
     const bool live = tile < ntiles;
     const int tx = live ? tile % G.tilesX : 0, ty = live ? tile / G.tilesX : 0;
-    const int px = tx * G.TW + gl % G.TW;
-    const int py = ty * G.TH + gl / G.TW;
+    const int pc = gl % G.TW, pr = gl / G.TW;       // this lane's pixel in the tile
+    const int ox = tx * G.TW, oy = ty * G.TH;
     int s0 = 0, s1 = 0;
     if (live) {
         const unsigned code = morton2(tx, ty);
@@ -456,106 +496,63 @@ __global__ __launch_bounds__(256) void k_gather(ReconGeo G, const float4* __rest
     }
     unsigned long long knext = gl < nrec_of(1) ? keys[s0 + GS + gl] : 0ull;
     for (int rd = 0; rd < rounds; ++rd) {
-        const int nrec = nrec_of(rd);
-        unsigned long long own = 0ull;  // 64-pixel tiles: the pixels this lane's record covers
-        if (gl < nrec) {
-            // per record, once: span, xy area, the span's first pixel bounds
-            // (kdgrid.cu:532-536, the same operations every lane would do)
-            // and the mask of the tile's pixels inside the span
+        covers[lane] = 0ull;
+        unsigned long long own = 0ull;  // the tile's pixels this lane's record overlaps
+        if (gl < nrec_of(rd)) {
             int x0, x1, y0, y1;
             record_span(c0, G, x0, x1, y0, y1);
-            unsigned mask = 0u;  // tiles of up to 32 pixels; larger tiles test the span
-            if (GS <= 32) {
-                for (int k = 0; k < GS; ++k) {
-                    const int qx = tx * G.TW + k % G.TW, qy = ty * G.TH + k / G.TW;
-                    if (qx >= x0 && qx < x1 && qy >= y0 && qy < y1) mask |= 1u << k;
-                }
-            } else {
-                // the span clipped to the tile is a rectangle of bits: columns
-                // [cx0, cx1) of every row in [cy0, cy1), row r at bits TW r..
-                const int cx0 = min(max(x0 - tx * G.TW, 0), G.TW), cx1 = min(max(x1 - tx * G.TW, 0), G.TW);
-                const int cy0 = min(max(y0 - ty * G.TH, 0), G.TH), cy1 = min(max(y1 - ty * G.TH, 0), G.TH);
-                auto low = [](int n) { return n >= 64 ? ~0ull : (1ull << n) - 1ull; };
-                const unsigned long long rep = G.TW >= 64 ? 1ull : ~0ull / low(G.TW);
-                const unsigned long long cols = low(cx1) & ~low(cx0);
-                const unsigned long long rows = rep & low(G.TW * cy1) & ~low(G.TW * cy0);
-                own = cols * rows;  // no carries: the column field is TW bits wide
+            float* o = ov + lane * stride;
+            const unsigned long long cols = axis_overlaps(c0.x, c0.y, x0, (float)x0 * G.sX / G.fW, G.stepX,
+                                                          max(x0, ox), min(x1, ox + G.TW), ox, o);
+            unsigned long long rows = axis_overlaps(c0.z, c0.w, y0, (float)y0 * G.sY / G.fH, G.stepY,
+                                                    max(y0, oy), min(y1, oy + G.TH), oy, o + G.TW);
+            mean[lane] = c1;
+            area[lane] = (c0.y - c0.x) * (c0.w - c0.z);
+            while (rows != 0ull) {
+                own |= cols << (G.TW * __builtin_ctzll(rows));
+                rows &= rows - 1ull;
             }
-            r0[w][gbase + gl] = c0;
-            r1[w][gbase + gl] = c1;
-            r2[w][gbase + gl] = make_float4((c0.y - c0.x) * (c0.w - c0.z),
-                                            __uint_as_float((unsigned)x0 | ((unsigned)x1 << 16)),
-                                            __uint_as_float((unsigned)y0 | ((unsigned)y1 << 16)),
-                                            __uint_as_float(mask));
-            r3[w][gbase + gl] = make_float2((float)x0 * G.sX / G.fW, (float)y0 * G.sY / G.fH);
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_sync_lds();
         if (gl < nrec_of(rd + 1)) {
             const int i = (int)(unsigned)(knext & 0xffffffffull);
             c0 = rrec[(size_t)i * 2];
             c1 = rrec[(size_t)i * 2 + 1];
         }
         knext = gl < nrec_of(rd + 2) ? keys[s0 + (rd + 2) * GS + gl] : 0ull;
-        // the round's records that cover this lane's pixel, then only those,
-        // in index order (the others add nothing): the loop runs as often as
-        // the most-covered pixel of the wave needs, not once per record
-        using CovT = typename std::conditional<(GS > 32), unsigned long long, unsigned>::type;
-        CovT cov = 0;
-        if constexpr (GS > 32) {
+        // the round's records that overlap this lane's pixel, bit j for the
+        // tile's record j
+        unsigned long long cov = 0ull;
+        if (GS > 32 && __any(__popcll(own) > kOrPixels)) {
             // one tile per wave, record j in lane j: the wave's coverage
             // matrix transposed by ballots, column p delivered to lane p
-#pragma unroll
             for (int p = 0; p < 64; ++p) {
                 const unsigned long long b = __ballot(((own >> p) & 1ull) != 0ull);
-                cov = lane == p ? (CovT)b : cov;
+                cov = lane == p ? b : cov;
             }
         } else {
-            for (int j = 0; j < nrec; ++j) {
-                const float4 q2 = r2[w][gbase + j];
-                cov |= (CovT)((__float_as_uint(q2.w) >> gl) & 1u) << j;
+            while (own != 0ull) {
+                atomicOr(&covers[gbase + __builtin_ctzll(own)], 1ull << gl);
+                own &= own - 1ull;
             }
+            wave_sync_lds();
+            cov = covers[lane];
         }
-        while (cov != 0) {
-            const int j = GS > 32 ? __builtin_ctzll((unsigned long long)cov) : __builtin_ctz((unsigned)cov);
-            cov &= cov - 1;
-            {
-                const float4 q2 = r2[w][gbase + j];
-                const unsigned spx = __float_as_uint(q2.y), spy = __float_as_uint(q2.z);
-                const int x0 = (int)(spx & 0xffffu), y0 = (int)(spy & 0xffffu);
-                const float4 q0 = r0[w][gbase + j];
-                const float4 q1 = r1[w][gbase + j];
-                const float2 q3 = r3[w][gbase + j];
-                // accumulated pixel bounds exactly as kdgrid.cu:536-576 walks them
-                float pMinX = q3.x;
-                float pMaxX = pMinX + G.stepX;
-                for (int q = x0; q < px; ++q) {
-                    pMinX = pMaxX;
-                    pMaxX += G.stepX;
-                }
-                float pMinY = q3.y;
-                float pMaxY = pMinY + G.stepY;
-                for (int q = y0; q < py; ++q) {
-                    pMinY = pMaxY;
-                    pMaxY += G.stepY;
-                }
-                const float clox = fmaxf(pMinX, q0.x);
-                const float chix = fminf(pMaxX, q0.y);
-                const float cloy = fmaxf(pMinY, q0.z);
-                const float chiy = fminf(pMaxY, q0.w);
-                if (clox < chix && cloy < chiy) {
-                    const float v = (chix - clox) * (chiy - cloy) * q1.w / q2.x;
-                    accx += (q1.x * v) * G.invPixArea;
-                    accy += (q1.y * v) * G.invPixArea;
-                    accz += (q1.z * v) * G.invPixArea;
-                }
-            }
+        // in index order (the other records add nothing): the loop runs as
+        // often as the most-covered pixel of the wave needs
+        while (cov != 0ull) {
+            const int j = gbase + __builtin_ctzll(cov);
+            cov &= cov - 1ull;
+            const float dx = ov[j * stride + pc], dy = ov[j * stride + G.TW + pr];
+            const float4 m = mean[j];
+            const float v = dx * dy * m.w / area[j];
+            accx += (m.x * v) * G.invPixArea;
+            accy += (m.y * v) * G.invPixArea;
+            accz += (m.z * v) * G.invPixArea;
         }
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        wave_sync_lds();
     }
+    const int px = ox + pc, py = oy + pr;
     if (live && px < G.W && py < G.H) pixels[(size_t)py * G.W + px] = make_float4(accx, accy, accz, 0.0f);
 }
 
@@ -818,15 +815,17 @@ static hipError_t recon_finish(Grid& g, ReconBufs& rb, float* pixels, int W, int
     kend(g, st);
     const int ntiles = G.tilesX * G.tilesY;
     const int gs = G.TW * G.TH;
-    const int tiles_per_block = 4 * (64 / gs);
+    // four waves a workgroup; one where their LDS would exceed 64 KB (tiles
+    // of more than 48 pixels along an axis)
+    const int lds = gather_lds(G.TW, G.TH), waves = 4 * lds <= 65536 ? 4 : 1;
+    const int per = waves * (64 / gs);  // tiles of a workgroup
+    const dim3 grid((ntiles + per - 1) / per), block(64 * waves);
     kbeg(g, st, "k_gather");
     if (gs == 64)
-        hipLaunchKernelGGL(k_gather<64>, dim3((ntiles + tiles_per_block - 1) / tiles_per_block),
-                           dim3(256), 0, st, G, rb.rrec, sorted, rb.tile_start, rb.tile_end,
+        hipLaunchKernelGGL(k_gather<64>, grid, block, waves * lds, st, G, rb.rrec, sorted, rb.tile_start, rb.tile_end,
                            (float4*)pixels);
     else
-        hipLaunchKernelGGL(k_gather<16>, dim3((ntiles + tiles_per_block - 1) / tiles_per_block),
-                           dim3(256), 0, st, G, rb.rrec, sorted, rb.tile_start, rb.tile_end,
+        hipLaunchKernelGGL(k_gather<16>, grid, block, waves * lds, st, G, rb.rrec, sorted, rb.tile_start, rb.tile_end,
                            (float4*)pixels);
     kend(g, st);
     return hipGetLastError();

@@ -222,6 +222,13 @@ __device__ __forceinline__ int block_exscan(int v, int* lds, int& total) {
     return pre + x - v;
 }
 
+// Orders the LDS accesses of one wave (all lanes of the wave take part).
+__device__ __forceinline__ void wave_sync_lds() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Chunk of leaves handled by workgroup `g` of `G` (multiple of 256 leaves).
 __device__ __forceinline__ void chunk_range(int n, int G, int g, int& beg, int& end) {
     int c = (n + G - 1) / G;

@@ -12,6 +12,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include "mdas_device.hpp"
 #include "mdas_internal.hpp"
 
 namespace mdas {
@@ -73,13 +74,6 @@ __device__ __forceinline__ bf16x8 pack_b8(const float* f) {
 #pragma unroll
     for (int k = 0; k < 8; ++k) v[k] = f2bf(f[k]);
     return __builtin_bit_cast(bf16x8, v);
-}
-
-// Orders the LDS accesses of one wave (all lanes of the wave take part).
-__device__ __forceinline__ void wave_sync_lds() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
 
 // Normalised, bf16-rounded feature row r of the tile into x (LDS [16][16]).

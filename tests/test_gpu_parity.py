@@ -164,6 +164,22 @@ def test_integrate_bit_exact(mdas, kind, dim, b, e, W, H, spp, alpha, cand, tile
     assert np.allclose(sc_px, want, rtol=1e-5, atol=1e-7)
 
 
+# tiles of one pixel's height and width, of more than 48 pixels along an axis
+# (one wave a workgroup), and cells of 1, 8 x 6 and 32 x 24 pixels (more than
+# 20 pixels of a tile per record, and all of them)
+@pytest.mark.parametrize("tile", [(64, 1), (1, 64), (32, 2), (4, 16), (1, 16), (16, 1), (2, 8)])
+@pytest.mark.parametrize("b,e", [(0, 0), (0, 2), (1, 4)])
+def test_integrate_long_tiles(mdas, tile, b, e):
+    W, H = 75, 50
+    _say(f"integrate tile={tile} b={b} e={e}")
+    g, o, sc, target = _make(mdas, 3, 5, b, e, W, H, 9, 0.25, 4)
+    g.Run(sc, target)
+    o.run(sc.params_bytes(), target)
+    g.set_recon_tile(*tile)
+    for w, h in ((W, H), (201, 33)):
+        assert np.array_equal(g.integrate_image(w, h).view(np.uint32), o.integrate(w, h).view(np.uint32))
+
+
 def test_integrate_other_resolution(mdas):
     """Pixel grid finer and coarser than the sample space (scaleFactor != 1)."""
     g, o, sc, target = _make(mdas, 2, 4, 1, 2, 40, 30, 8, 0.25, 4)
