@@ -38,8 +38,9 @@ __device__ __forceinline__ void eval_body(const float* __restrict__ coords,
     int beg = first, end = first + count;
     if (dev_range) {
         if (cnt->done) return;
-        beg = cnt->n_samples_old;
-        end = cnt->n_samples;
+        const TreeCounts t = cnt->slot[cnt->cur];
+        beg = t.N_old;
+        end = t.N;
     }
     if (blk * 256 >= end - beg) return;  // uniform: no sample for this workgroup
     stage_scene(B, obj);

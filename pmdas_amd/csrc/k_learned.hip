@@ -111,18 +111,18 @@ __device__ __forceinline__ float image_label(float mp, const float* mc, const fl
 // workgroup max of the scores feeds the selection's global max.
 template <int D>
 __device__ __forceinline__ void errors_learned_body(const DevGrid& a, const LearnDev& l, int blk,
-                                                    int nblk) {
-    __shared__ float wmax[4];
-    __shared__ int wst[8];
+                                                    int nblk, int par) {
     __shared__ unsigned short xsb[4][128 * kMlpIn];  // a wave's staged rows (bf16)
     __shared__ unsigned short actb[4][16 * kMlpH];   // layer-1 activations (bf16)
     __shared__ float ys[4][16];
     __shared__ __align__(16) unsigned short w1s[64 * 32], w2s[64 * 64];  // the bf16 weights
     __shared__ float bl[3 * 64 + 1];  // b1, b2, bf16-rounded w3, b3
-    if (pass_stopped(a.cnt)) return;
+    const TreeCounts counts = a.cnt->slot[par];
+    if (a.cnt->done || loop_limit_reached(a.cnt, counts.N, counts.L)) return;
     const bool first = a.cnt->passes == 0;
-    const int n_items = first ? a.cnt->n_leaves : a.cnt->new_nodes;
-    const int L_old = a.cnt->n_leaves_old;
+    const int n_items = first ? counts.L : counts.new_n;
+    if (blk * 256 >= n_items) return;
+    const int L_old = counts.L_old;
     const long long rows_base = (first || l.X == nullptr) ? 0 : *l.rows;
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     const bool feats = l.feat != nullptr;  // false: a plain member of a batch
@@ -141,7 +141,6 @@ __device__ __forceinline__ void errors_learned_body(const DevGrid& a, const Lear
         __syncthreads();
     }
     float m = 0.0f;
-    int n_stale = 0, n_vals = 0;
     for (int t0 = blk * 256; t0 < n_items; t0 += nblk * 256) {
         const int t = t0 + threadIdx.x;
         const bool act = t < n_items;
@@ -215,8 +214,6 @@ __device__ __forceinline__ void errors_learned_body(const DevGrid& a, const Lear
                 e[h] = error_of_values(ids[h], vol[h], ls[h]);
                 leaf_features_ext<D>(ls[h], ex, e[h], depth, a.sX, a.sY, f);
                 axy[h] = ex[0] * ex[1];
-                n_stale += 1;
-                n_vals += ls[h].n;
                 finish(h, f);
             }
         } else {
@@ -230,8 +227,6 @@ __device__ __forceinline__ void errors_learned_body(const DevGrid& a, const Lear
                     leaf_features<D>(ls, mn, mx, e[h], depth, a.sX, a.sY, f);
                     vol[h] = ls.vol;
                     axy[h] = (mx[0] - mn[0]) * (mx[1] - mn[1]);
-                    n_stale += 1;
-                    n_vals += ls.n;
                 } else {
 #pragma unroll
                     for (int k = 0; k < kFeat; ++k) f[k] = 0.0f;
@@ -283,111 +278,44 @@ __device__ __forceinline__ void errors_learned_body(const DevGrid& a, const Lear
             }
         }
     }
-    // (max, stale count, values read) per workgroup, as the plain pass
-    m = wave_max(m);
-    n_stale = wave_sum(n_stale);
-    n_vals = wave_sum(n_vals);
-    if (lane == 0) {
-        wmax[w] = m;
-        wst[w] = n_stale;
-        wst[4 + w] = n_vals;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const float b = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
-        a.epart[blk] = make_uint4(__float_as_uint(b), (unsigned)(wst[0] + wst[1] + wst[2] + wst[3]),
-                                  (unsigned)(wst[4] + wst[5] + wst[6] + wst[7]), 0u);
-    }
+    super_max(a.smax + par * kSuper, m, blk);
 }
 
 // 4 waves per SIMD: the feature phase and the network fit the register file
 // at that occupancy without spilling (the default allocation gave 3).
 template <int D>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_errors_learned(
-    DevGrid a, LearnDev l) {
-    errors_learned_body<D>(a, l, blockIdx.x, gridDim.x);
+    DevGrid a, LearnDev l, int par) {
+    errors_learned_body<D>(a, l, blockIdx.x, gridDim.x, par);
 }
 template <int D>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_errors_learned_b(
-    const DevGrid* grids, const LearnDev* ls) {
-    errors_learned_body<D>(grids[blockIdx.y], ls[blockIdx.y], blockIdx.x, gridDim.x);
+    const DevGrid* grids, const LearnDev* ls, int par) {
+    errors_learned_body<D>(grids[blockIdx.y], ls[blockIdx.y], blockIdx.x, gridDim.x, par);
 }
 
-// Folds the partials like the plain pass, then advances the row counter by
-// the splits whose rows this pass offered.
-__device__ __forceinline__ void err_reduce_learned_body(const DevGrid& a, const LearnDev& l, int G) {
-    __shared__ unsigned sm[16];
-    __shared__ int ss[16], sv[16];
-    if (a.cnt->done) return;
-    if (loop_limit_reached(a.cnt)) {  // the loop stops before this pass
-        if (threadIdx.x == 0) a.cnt->done = 1;
-        return;
-    }
-    unsigned mx = 0;
-    int st = 0, va = 0;
-    for (int k = threadIdx.x; k < G; k += 1024) {
-        const uint4 p = a.epart[k];
-        mx = max(mx, p.x);
-        st += (int)p.y;
-        va += (int)p.z;
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        mx = max(mx, (unsigned)__shfl_xor((int)mx, o, 64));
-        st += __shfl_xor(st, o, 64);
-        va += __shfl_xor(va, o, 64);
-    }
-    if ((threadIdx.x & 63) == 0) {
-        sm[threadIdx.x >> 6] = mx;
-        ss[threadIdx.x >> 6] = st;
-        sv[threadIdx.x >> 6] = va;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        unsigned mm = a.cnt->carry_bits;  // the loop's pass: from the scan's carried max
-        int s1 = 0, s2 = 0;
-        for (int k = 0; k < 16; ++k) {
-            mm = max(mm, sm[k]);
-            s1 += ss[k];
-            s2 += sv[k];
-        }
-        a.cnt->gmax_bits = mm;
-        a.cnt->stale += s1;
-        a.cnt->stale_vals += s2;
-        if (l.X != nullptr && l.feat != nullptr && a.cnt->passes > 0) *l.rows += a.cnt->new_nodes;
-    }
-}
-__global__ __launch_bounds__(1024) void k_err_reduce_learned(DevGrid a, LearnDev l, int G) {
-    err_reduce_learned_body(a, l, G);
-}
-__global__ __launch_bounds__(1024) void k_err_reduce_learned_b(const DevGrid* grids,
-                                                                const LearnDev* ls, int G) {
-    err_reduce_learned_body(grids[blockIdx.x], ls[blockIdx.x], G);
-}
-
-hipError_t launch_errors_learned(Grid& g, hipStream_t st) {
+hipError_t launch_errors_learned(Grid& g, int parity, hipStream_t st) {
+    const dim3 grid(g.error_blocks()), block(256);
     switch (g.D) {
-    case 3: hipLaunchKernelGGL(k_errors_learned<3>, dim3(g.err_blocks), dim3(256), 0, st, g.dev, g.learn); break;
-    case 4: hipLaunchKernelGGL(k_errors_learned<4>, dim3(g.err_blocks), dim3(256), 0, st, g.dev, g.learn); break;
-    case 5: hipLaunchKernelGGL(k_errors_learned<5>, dim3(g.err_blocks), dim3(256), 0, st, g.dev, g.learn); break;
-    case 6: hipLaunchKernelGGL(k_errors_learned<6>, dim3(g.err_blocks), dim3(256), 0, st, g.dev, g.learn); break;
+    case 3: hipLaunchKernelGGL(k_errors_learned<3>, grid, block, 0, st, g.dev, g.learn, parity); break;
+    case 4: hipLaunchKernelGGL(k_errors_learned<4>, grid, block, 0, st, g.dev, g.learn, parity); break;
+    case 5: hipLaunchKernelGGL(k_errors_learned<5>, grid, block, 0, st, g.dev, g.learn, parity); break;
+    case 6: hipLaunchKernelGGL(k_errors_learned<6>, grid, block, 0, st, g.dev, g.learn, parity); break;
     default: return hipErrorInvalidValue;
     }
-    hipLaunchKernelGGL(k_err_reduce_learned, dim3(1), dim3(1024), 0, st, g.dev, g.learn, g.err_blocks);
     return hipGetLastError();
 }
 
 hipError_t launch_errors_learned_b(int D, const DevGrid* grids, const LearnDev* ls, int n, int blocks,
-                                   hipStream_t st) {
-    const int eb = blocks < 1024 ? blocks : 1024;
+                                   int parity, hipStream_t st) {
+    const dim3 grid(blocks < 1024 ? blocks : 1024, n), block(256);
     switch (D) {
-    case 3: hipLaunchKernelGGL(k_errors_learned_b<3>, dim3(eb, n), dim3(256), 0, st, grids, ls); break;
-    case 4: hipLaunchKernelGGL(k_errors_learned_b<4>, dim3(eb, n), dim3(256), 0, st, grids, ls); break;
-    case 5: hipLaunchKernelGGL(k_errors_learned_b<5>, dim3(eb, n), dim3(256), 0, st, grids, ls); break;
-    case 6: hipLaunchKernelGGL(k_errors_learned_b<6>, dim3(eb, n), dim3(256), 0, st, grids, ls); break;
+    case 3: hipLaunchKernelGGL(k_errors_learned_b<3>, grid, block, 0, st, grids, ls, parity); break;
+    case 4: hipLaunchKernelGGL(k_errors_learned_b<4>, grid, block, 0, st, grids, ls, parity); break;
+    case 5: hipLaunchKernelGGL(k_errors_learned_b<5>, grid, block, 0, st, grids, ls, parity); break;
+    case 6: hipLaunchKernelGGL(k_errors_learned_b<6>, grid, block, 0, st, grids, ls, parity); break;
     default: return hipErrorInvalidValue;
     }
-    hipLaunchKernelGGL(k_err_reduce_learned_b, dim3(n), dim3(1024), 0, st, grids, ls, eb);
     return hipGetLastError();
 }
 

@@ -73,7 +73,7 @@ __device__ __forceinline__ int tiles_of(int x0, int x1, int y0, int y1, const Re
 template <int D>
 __global__ __launch_bounds__(256) void k_recon_prep(DevGrid a, ReconGeo G, float4* rrec) {
     __shared__ int red[4];
-    const int L = a.cnt->n_leaves;
+    const int L = leaf_total(a);
     int beg, end;
     chunk_range(L, gridDim.x, blockIdx.x, beg, end);
     int c = 0;
@@ -160,7 +160,7 @@ __global__ __launch_bounds__(1024) void k_scan_keys(DevGrid a, int G, long long 
 __global__ __launch_bounds__(256) void k_recon_emit(DevGrid a, ReconGeo G, const float4* rrec,
                                                     unsigned long long* keys) {
     __shared__ int lds[4];
-    const int L = a.cnt->n_leaves;
+    const int L = leaf_total(a);
     if (a.cnt->recon_overflow != 0) return;  // the keys do not fit the buffer
     int beg, end;
     chunk_range(L, gridDim.x, blockIdx.x, beg, end);
@@ -560,7 +560,7 @@ __global__ __launch_bounds__(256) void k_gather(ReconGeo G, const float4* __rest
 // kdgrid.cu:483-582 as written: one thread per leaf, float atomics per pixel.
 template <int D>
 __global__ __launch_bounds__(256) void k_scatter(DevGrid a, ReconGeo G, float4* pixels) {
-    const int L = a.cnt->n_leaves;
+    const int L = leaf_total(a);
     for (int i = blockIdx.x * 256 + threadIdx.x; i < L; i += gridDim.x * 256) {
         int4 id4;
         float mn[D], mx[D];

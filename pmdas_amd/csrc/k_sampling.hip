@@ -7,8 +7,9 @@
 // points) plus an overflow row for the other points (D >= 5), so a leaf
 // touched at a random index costs one line; errors, LCG states and a one-byte
 // flag word (the sample count) per leaf as separate streams for the per-pass
-// sweep over all leaves.  Cross-workgroup reductions go through per-workgroup
-// partials (no same-address atomics).
+// sweep over all leaves.  Cross-workgroup totals go through 64 groups of
+// atomics, a line each, and per-workgroup partials (no address takes more than
+// a few dozen atomics).
 #include "mdas_leaf.hpp"
 #include "scenes.hpp"
 
@@ -94,113 +95,68 @@ __global__ __launch_bounds__(256) void k_initial_b(const DevGrid* grids) {
     initial_body<D>(a, 1 << (a.b * D + 2 * a.e), blockIdx.x, gridDim.x);
 }
 
-// Counter set-up of InitialSampling (kdgrid.cu:639-642).
-__device__ __forceinline__ void initial_counters_body(const DevGrid& a, int L0) {
-    DevCounters* c = a.cnt;
-    if (threadIdx.x < 2 * kSuper) {
-        a.ssum[threadIdx.x].sel = a.ssum[threadIdx.x].split = a.ssum[threadIdx.x].held = 0;
-        a.smax[threadIdx.x].err = 0u;
-    }
+// Counter set-up of InitialSampling (kdgrid.cu:639-642): g_error = 0, every
+// total zero, the loop's limit (and the capacity as its guard when the limit
+// is the capacity; below it a pass that would overflow is an error).
+__device__ __forceinline__ void initial_counters_body(const DevGrid& a, int L0, int limit) {
+    if (threadIdx.x < 2 * kSuper) a.ssum[threadIdx.x].sel = a.ssum[threadIdx.x].split = a.ssum[threadIdx.x].held = 0;
+    if (threadIdx.x < kMaxSets * kSuper) a.smax[threadIdx.x].err = 0u;
     if (threadIdx.x != 0) return;
+    DevCounters* c = a.cnt;
     c->cur = 0;
-    c->slot[0] = c->slot[1] = LoopSlot{4 * L0, L0, 0, 0, 4 * L0, 0};
-    c->n_leaves = L0;
-    c->n_samples = 4 * L0;
-    c->n_leaves_old = 0;
-    c->n_samples_old = 0;
-    c->new_samples = 4 * L0;  // the first integrand launch covers all of them
-    c->new_nodes = 0;
-    c->gmax_bits = 0;
+    // the first integrand launch covers all the samples
+    c->slot[0] = c->slot[1] = TreeCounts{4 * L0, L0, 0, 0, 4 * L0, 0};
     c->done = 0;
     c->status = 0;
     c->passes = 0;
-    c->limit = 0x7fffffff;
-    c->sel_cnt = 0;
-    c->stale = 0;
-    c->stale_vals = 0;
-    c->carry_bits = 0;
-    c->guard_cap = 0;
+    c->limit = limit;
+    c->guard_cap = limit >= a.cap_s ? a.cap_s : 0;
 }
-__global__ __launch_bounds__(2 * kSuper) void k_initial_counters(DevGrid a, int L0) {
-    initial_counters_body(a, L0);
+__global__ __launch_bounds__(kMaxSets* kSuper) void k_initial_counters(DevGrid a, int L0, int limit) {
+    initial_counters_body(a, L0, limit);
+}
+// Batched form: one workgroup per image.
+__global__ __launch_bounds__(kMaxSets* kSuper) void k_initial_counters_b(const DevGrid* grids, const int* limits) {
+    const DevGrid& a = grids[blockIdx.x];
+    initial_counters_body(a, 1 << (a.b * a.D + 2 * a.e), limits[blockIdx.x]);
 }
 
-// ComputeErrors prologue (kdgrid.cu:684-685): g_error = 0.  A standalone call
-// also re-arms the pass kernels and lifts the sampling loop's limit.
-__global__ void k_reset_errors(DevCounters* c, int standalone) {
-    if (standalone) {
-        c->done = 0;
+// Before a single call: the pass kernels run again after a loop or a refused
+// pass, without the loop's limit, from zero totals; before ComputeErrors
+// (kdgrid.cu:684-685) g_error = 0.
+__global__ __launch_bounds__(kSuper) void k_arm(DevGrid a, int errors, int adaptive) {
+    DevCounters* c = a.cnt;
+    SuperSum& t = a.ssum[c->cur * kSuper + threadIdx.x];
+    if (adaptive) t.sel = t.split = t.held = 0;
+    if (errors) a.smax[kGError * kSuper + threadIdx.x].err = 0u;
+    if (threadIdx.x != 0) return;
+    c->done = 0;
+    if (adaptive) c->status = 0;
+    if (errors) {
         c->limit = 0x7fffffff;
         c->guard_cap = 0;
     }
-    c->gmax_bits = 0;
-}
-
-__global__ void k_set_limit(DevCounters* c, int limit, int guard_cap) {
-    c->limit = limit;
-    c->guard_cap = guard_cap;
-}
-
-// Batched form: one workgroup per image.
-__global__ __launch_bounds__(2 * kSuper) void k_initial_counters_b(const DevGrid* grids, const int* limits) {
-    const DevGrid& a = grids[blockIdx.x];
-    DevCounters* c = a.cnt;
-    initial_counters_body(a, 1 << (a.b * a.D + 2 * a.e));
-    if (threadIdx.x != 0) return;
-    c->limit = limits[blockIdx.x];
-    c->guard_cap = limits[blockIdx.x] >= a.cap_s ? a.cap_s : 0;
-}
-
-// Re-arms the pass kernels for a standalone AdaptiveSampling call.
-__global__ void k_arm(DevCounters* c) {
-    c->done = 0;
-    c->status = 0;
 }
 
 // ------------------------------------------------------------------ errors --
-// Workgroup reduction of (max, stale count, values read) into epart[block].
-__device__ __forceinline__ void errors_epilogue(const DevGrid& a, float m, int n_stale, int n_vals,
-                                                float* wmax, int* wst, int blk) {
-    m = wave_max(m);
-    n_stale = wave_sum(n_stale);
-    n_vals = wave_sum(n_vals);
-    if ((threadIdx.x & 63) == 0) {
-        wmax[threadIdx.x >> 6] = m;
-        wst[threadIdx.x >> 6] = n_stale;
-        wst[4 + (threadIdx.x >> 6)] = n_vals;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        const float b = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
-        a.epart[blk] = make_uint4(__float_as_uint(b), (unsigned)(wst[0] + wst[1] + wst[2] + wst[3]),
-                                         (unsigned)(wst[4] + wst[5] + wst[6] + wst[7]), 0u);
-    }
-}
-
 // kdgrid.cu:204-288 as the reference runs it: every leaf with error < 0 is
 // re-estimated and every leaf takes part in the global max.  The max of
 // non-negative floats is the max of their bit patterns, so the reduction is
 // exact in any order.
 template <int D>
-__global__ __launch_bounds__(256) void k_errors(DevGrid a) {
-    __shared__ float wmax[4];
-    __shared__ int wst[8];
-    if (a.cnt->done) return;
-    const int L = a.cnt->n_leaves;
+__global__ __launch_bounds__(256) void k_compute_errors(DevGrid a) {
+    const int L = leaf_total(a);
     float m = 0.0f;
-    int n_stale = 0, n_vals = 0;
     for (int i = blockIdx.x * 256 + threadIdx.x; i < L; i += gridDim.x * 256) {
         float e = a.err[i];
         if (e < 0.0f) {
             int n;
             e = leaf_error<D>(a, i, &n);
             a.err[i] = e;
-            n_stale += 1;
-            n_vals += n;
         }
         m = fmaxf(m, e);
     }
-    errors_epilogue(a, m, n_stale, n_vals, wmax, wst, blockIdx.x);
+    super_max(a.smax + kGError * kSuper, m, blockIdx.x);
 }
 
 // The same result inside the sampling loop without the sweep over all
@@ -208,32 +164,24 @@ __global__ __launch_bounds__(256) void k_errors(DevGrid a) {
 // pass split (split_list[t] and L_old + t, whose sample indices and volumes
 // the placement left in the split's entry; inside the loop it does not mark
 // them -1, since they are re-estimated here); the max over the other leaves
-// was carried by the selection kernel into gmax by the allocation scan.  The
-// first pass after the initial grid re-estimates every leaf.
+// was carried into the pass's totals by the selection before.  The first pass
+// after the initial grid re-estimates every leaf.
 template <int D>
-__device__ __forceinline__ void errors_stale_body(const DevGrid& a, int blk, int nblk) {
-    __shared__ float wmax[4];
-    __shared__ int wst[8];
-    if (pass_stopped(a.cnt)) return;
-    const bool first = a.cnt->passes == 0;
+__device__ __forceinline__ void errors_body(const DevGrid& a, int blk, int nblk, int par) {
+    const TreeCounts c = a.cnt->slot[par];
+    if (a.cnt->done || loop_limit_reached(a.cnt, c.N, c.L)) return;
     float m = 0.0f;
-    int n_stale = 0, n_vals = 0;
-    if (first) {
-        const int L = a.cnt->n_leaves;
-        for (int i = blk * 256 + threadIdx.x; i < L; i += nblk * 256) {
+    if (a.cnt->passes == 0) {
+        for (int i = blk * 256 + threadIdx.x; i < c.L; i += nblk * 256) {
             int n;
             const float e = leaf_error<D>(a, i, &n);
             a.err[i] = e;
-            n_stale += 1;
-            n_vals += n;
             m = fmaxf(m, e);
         }
     } else {
         // one thread per split: both children from the split's entry
         // (sample indices and volumes), not from their leaf records
-        const int nn = a.cnt->new_nodes;
-        const int L_old = a.cnt->n_leaves_old;
-        for (int t = blk * 256 + threadIdx.x; t < nn; t += nblk * 256) {
+        for (int t = blk * 256 + threadIdx.x; t < c.new_n; t += nblk * 256) {
             const int4 s0 = a.sdat[2 * t], s1 = a.sdat[2 * t + 1];
             const int il = a.split_list[t];
             LeafSamples lsl, lsr;
@@ -244,125 +192,49 @@ __device__ __forceinline__ void errors_stale_body(const DevGrid& a, int blk, int
             const float el = error_of_values(idl, __int_as_float(s1.y), lsl);
             const float er = error_of_values(idr, __int_as_float(s1.z), lsr);
             a.err[il] = el;
-            a.err[L_old + t] = er;
-            n_stale += 2;
-            n_vals += lsl.n + lsr.n;
+            a.err[c.L_old + t] = er;
             m = fmaxf(m, el);
             m = fmaxf(m, er);
         }
     }
-    errors_epilogue(a, m, n_stale, n_vals, wmax, wst, blk);
+    super_max(a.smax + par * kSuper, m, blk);
 }
 
 template <int D>
-__global__ __launch_bounds__(256) void k_errors_stale(DevGrid a) {
-    errors_stale_body<D>(a, blockIdx.x, gridDim.x);
+__global__ __launch_bounds__(256) void k_errors(DevGrid a, int par) {
+    errors_body<D>(a, blockIdx.x, gridDim.x, par);
 }
 template <int D>
-__global__ __launch_bounds__(256) void k_errors_stale_b(const DevGrid* grids) {
+__global__ __launch_bounds__(256) void k_errors_b(const DevGrid* grids, int par) {
     const DevGrid a = grids[blockIdx.y];  // by value: scalar registers
-    errors_stale_body<D>(a, blockIdx.x, gridDim.x);
-}
-
-// Errors of the initial leaves for the fused loop: every leaf holds four
-// samples; the largest goes to the super group of the workgroup.
-template <int D>
-__device__ __forceinline__ void first_errors_body(const DevGrid& a, int blk, int nblk) {
-    __shared__ float wmax[4];
-    const int L = a.cnt->slot[0].L;
-    if (loop_limit_reached(a.cnt, a.cnt->slot[0].N, L)) return;  // no pass: the errors stay stale
-    float m = 0.0f;
-    for (int i = blk * 256 + threadIdx.x; i < L; i += nblk * 256) {
-        int n;
-        const float e = leaf_error<D>(a, i, &n);
-        a.err[i] = e;
-        m = fmaxf(m, e);
-    }
-    m = wave_max(m);
-    if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = m;
-    __syncthreads();
-    if (threadIdx.x == 0)
-        atomicMax(&a.smax[blk % kSuper].err,
-                  __float_as_uint(fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]))));
-}
-template <int D>
-__global__ __launch_bounds__(256) void k_first_errors(DevGrid a) {
-    first_errors_body<D>(a, blockIdx.x, gridDim.x);
-}
-template <int D>
-__global__ __launch_bounds__(256) void k_first_errors_b(const DevGrid* grids) {
-    const DevGrid a = grids[blockIdx.y];  // by value: scalar registers
-    first_errors_body<D>(a, blockIdx.x, gridDim.x);
-}
-
-// Folds the error partials into gmax and the per-pass statistics.  A full
-// sweep (ComputeErrors, after its reset) starts from gmax = 0; the loop's
-// stale-list pass, which re-estimates only the last pass's children, starts
-// from the max the allocation scan carried over (the leaves that did not
-// split).
-__device__ __forceinline__ void err_reduce_body(const DevGrid& a, int G, int from_carry) {
-    __shared__ unsigned sm[16];
-    __shared__ int ss[16], sv[16];
-    if (a.cnt->done) return;
-    if (loop_limit_reached(a.cnt)) {  // the loop stops before this pass
-        if (threadIdx.x == 0) a.cnt->done = 1;
-        return;
-    }
-    unsigned m = 0;
-    int st = 0, va = 0;
-    for (int k = threadIdx.x; k < G; k += 1024) {
-        const uint4 p = a.epart[k];
-        m = max(m, p.x);
-        st += (int)p.y;
-        va += (int)p.z;
-    }
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        m = max(m, (unsigned)__shfl_xor((int)m, o, 64));
-        st += __shfl_xor(st, o, 64);
-        va += __shfl_xor(va, o, 64);
-    }
-    if ((threadIdx.x & 63) == 0) {
-        sm[threadIdx.x >> 6] = m;
-        ss[threadIdx.x >> 6] = st;
-        sv[threadIdx.x >> 6] = va;
-    }
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        unsigned mm = from_carry ? a.cnt->carry_bits : a.cnt->gmax_bits;
-        int s1 = 0, s2 = 0;
-        for (int k = 0; k < 16; ++k) {
-            mm = max(mm, sm[k]);
-            s1 += ss[k];
-            s2 += sv[k];
-        }
-        a.cnt->gmax_bits = mm;
-        a.cnt->stale += s1;
-        a.cnt->stale_vals += s2;
-    }
-}
-__global__ __launch_bounds__(1024) void k_err_reduce(DevGrid a, int G, int from_carry) {
-    err_reduce_body(a, G, from_carry);
-}
-__global__ __launch_bounds__(1024) void k_err_reduce_b(const DevGrid* grids, int G) {
-    err_reduce_body(grids[blockIdx.x], G, 1);
+    errors_body<D>(a, blockIdx.x, gridDim.x, par);
 }
 
 // --------------------------------------------------------------- selection --
-// Chunks per super group of the fused loop, for `chunks` in all.
+// Chunks a tree of L leaves is cut into, of the n launched (the others
+// return): 256 leaves each until four workgroups per CU have one, then up to
+// 512 before there are more of them, so that the 16 % or so that a pass selects
+// fill their waves.  Runs without reconstruction, against 256 leaves up to 4096
+// chunks: 333x517 884 -> 773 us, 3D 256x256 809 -> 740 us, 1080p the same; at
+// least 1024 leaves (795 us) or 512 chunks (880 us) were slower at 333x517.
+__device__ __forceinline__ int live_chunks(int L, int n) {
+    return min(n, max(min((L + 255) / 256, 1024), L / 512));
+}
+// Chunks per super group, for `chunks` in all.
 __device__ __forceinline__ int super_size(int chunks) { return (chunks + kSuper - 1) / kSuper; }
 
 // kdgrid.cu:316-326.  Per leaf: the seed (tea4(i,0) when unset), one draw u,
 // selected iff pow(err / g_error, alpha) >= u.  A selected full leaf splits.
-// Writes the flags, and per workgroup the (selected, split) counts for the
-// allocation scan, the samples held by the selected leaves, and the max error
-// of the leaves that do not split.  The LCG states are not written here: the
-// compaction stores them once the scan has accepted the pass, so that a pass
-// refused for capacity leaves every state as it was.
-// Chunk blk of nblk (the compaction's partition of the leaves).  ssum, smax:
-// the super groups of the fused loop, which take the chunk's totals too; else null.
+// Writes the flags, and per chunk the (selected, split) counts and the
+// samples held by the selected leaves, also added to the chunk's super group;
+// the max error of the leaves that do not split goes on to the next pass
+// (carried: null for single calls, whose next error pass sees every leaf).
+// The LCG states are not written here: the compaction stores them once it has
+// accepted the pass, so that a pass refused for capacity leaves every state
+// as it was.
+// Chunk blk of nblk (the compaction's partition of the leaves).
 __device__ __forceinline__ void select_chunk(const DevGrid& a, int L, float gmax, int blk, int nblk,
-                                             SuperSum* ssum, SuperMax* smax) {
+                                             SuperSum* ssum, SuperMax* carried) {
     __shared__ int red[12];
     __shared__ float rmax[4];
     const float alpha = a.alpha;
@@ -416,188 +288,52 @@ __device__ __forceinline__ void select_chunk(const DevGrid& a, int L, float gmax
     if (threadIdx.x == 0) {
         const float cm = fmaxf(fmaxf(rmax[0], rmax[1]), fmaxf(rmax[2], rmax[3]));
         const int4 p = make_int4(red[0] + red[1] + red[2] + red[3], red[4] + red[5] + red[6] + red[7],
-                                 red[8] + red[9] + red[10] + red[11], (int)__float_as_uint(cm));
+                                 red[8] + red[9] + red[10] + red[11], 0);
         a.part[blk] = p;
-        if (ssum != nullptr) {
-            const int g = blk / super_size(nblk);
-            if (p.x != 0) atomicAdd(&ssum[g].sel, p.x);
-            if (p.y != 0) atomicAdd(&ssum[g].split, p.y);
-            if (p.z != 0) atomicAdd(&ssum[g].held, p.z);
-            if (p.w != 0) atomicMax(&smax[g].err, (unsigned)p.w);
-        }
+        const int g = blk / super_size(nblk);
+        if (p.x != 0) atomicAdd(&ssum[g].sel, p.x);
+        if (p.y != 0) atomicAdd(&ssum[g].split, p.y);
+        if (p.z != 0) atomicAdd(&ssum[g].held, p.z);
+        if (carried != nullptr && cm != 0.0f) atomicMax(&carried[g].err, __float_as_uint(cm));
     }
     __syncthreads();  // red / rmax are reused by the workgroup's next chunk
 }
 // Workgroup blk takes chunks [blk * cpw, (blk + 1) * cpw) of the compaction's
-// nblk * cpw: the placement balances better over many small chunks, the
-// selection's streaming sweep runs best with fewer, longer ones.
-__device__ __forceinline__ void select_body(const DevGrid& a, int blk, int nblk, int cpw) {
-    if (a.cnt->done) return;
-    const int L = a.cnt->n_leaves;
-    const float gmax = __uint_as_float(a.cnt->gmax_bits);
-    for (int c = blk * cpw; c < (blk + 1) * cpw; ++c) select_chunk(a, L, gmax, c, nblk * cpw, nullptr, nullptr);
-}
-__global__ __launch_bounds__(256) void k_select(DevGrid a, int cpw) {
-    select_body(a, blockIdx.x, gridDim.x, cpw);
-}
-__global__ __launch_bounds__(256) void k_select_b(const DevGrid* grids, int cpw) {
-    const DevGrid a = grids[blockIdx.y];  // by value: scalar registers
-    select_body(a, blockIdx.x, gridDim.x, cpw);
-}
-
-// The same in the fused loop: the stopping test and the largest error come
-// first, from the pass's slot and super groups, in place of the reduction
-// kernel; the largest error among the leaves that do not split goes on to the
-// next pass.  A single thread keeps the counters that are read after the loop.
-__device__ __forceinline__ void select_fused_body(const DevGrid& a, int blk, int nblk, int cpw, int par) {
+// n: the placement balances better over many small chunks, the selection's
+// streaming sweep runs best with fewer, longer ones.  In the loop the stopping
+// test and the largest error of the pass come first, from the pass's slot and
+// totals (a single call selects against g_error as it stands).
+__device__ __forceinline__ void select_body(const DevGrid& a, int blk, int n, int cpw, int par, int loop) {
     DevCounters* cn = a.cnt;
     if (cn->done) return;
-    const int N = cn->slot[par].N, L = cn->slot[par].L;
-    if (loop_limit_reached(cn, N, L)) {  // every workgroup finds the same
+    const TreeCounts c = cn->slot[par];
+    if (loop && loop_limit_reached(cn, c.N, c.L)) {  // every workgroup finds the same
         if (blk == 0 && threadIdx.x == 0) cn->done = 1;
         return;
     }
-    const unsigned e = a.smax[par * kSuper + (threadIdx.x & 63)].err;
+    n = live_chunks(c.L, n);
+    if (blk * cpw >= n) return;
+    const int lane = threadIdx.x & 63;
+    const unsigned e = a.smax[(loop ? par : kGError) * kSuper + lane].err;
     const float gmax = wave_max(__uint_as_float(e));  // no NaN among them: each is a maximum from 0
-    if (blk == 0 && threadIdx.x == 0) cn->gmax_bits = __float_as_uint(gmax);
-    for (int c = blk * cpw; c < (blk + 1) * cpw; ++c)
-        select_chunk(a, L, gmax, c, nblk * cpw, a.ssum + par * kSuper, a.smax + (par ^ 1) * kSuper);
+    if (loop && blk == 0 && threadIdx.x < kSuper) {
+        a.smax[kGError * kSuper + lane].err = e;  // g_error of this pass, for the calls after the loop
+        if (lane == 0 && a.lrows != nullptr && cn->passes > 0) *a.lrows += c.new_n;  // collected by the error pass
+    }
+    for (int k = blk * cpw; k < min(n, (blk + 1) * cpw); ++k)
+        select_chunk(a, c.L, gmax, k, n, a.ssum + par * kSuper, loop ? a.smax + (par ^ 1) * kSuper : nullptr);
 }
-__global__ __launch_bounds__(256) void k_select_fused(DevGrid a, int cpw, int par) {
-    select_fused_body(a, blockIdx.x, gridDim.x, cpw, par);
+__global__ __launch_bounds__(256) void k_select(DevGrid a, int n, int cpw, int par, int loop) {
+    select_body(a, blockIdx.x, n, cpw, par, loop);
 }
-__global__ __launch_bounds__(256) void k_select_fused_b(const DevGrid* grids, int cpw, int par) {
+__global__ __launch_bounds__(256) void k_select_b(const DevGrid* grids, int n, int cpw, int par) {
     const DevGrid a = grids[blockIdx.y];  // by value: scalar registers
-    select_fused_body(a, blockIdx.x, gridDim.x, cpw, par);
+    select_body(a, blockIdx.x, n, cpw, par, 1);
 }
 
 // Chunks per selection workgroup for `chunks` compaction chunks: as many as
 // keep the selection at 4096 workgroups (chunks is then a multiple of it).
 static int select_cpw(int chunks) { return chunks > 4096 && chunks % 4096 == 0 ? chunks / 4096 : 1; }
-
-// Exclusive scan of the per-workgroup counts (one workgroup of 1024 threads),
-// then the capacity check and the counter update (kdgrid.cu:753-759).
-__device__ __forceinline__ void scan_counts_body(const DevGrid& a, int G) {
-    __shared__ int ls[16], ll[16], lc[16];
-    __shared__ unsigned lm[16];
-    DevCounters* cn = a.cnt;
-    if (cn->done) return;
-    // thread 0's counter reads go out together with the partials' loads
-    // (no other kernel runs between the error pass and this one)
-    int N = 0, L = 0, P = 0, st = 0, sv = 0;
-    if (threadIdx.x == 0) {
-        N = cn->n_samples;
-        L = cn->n_leaves;
-        P = cn->passes;
-        st = cn->stale;
-        sv = cn->stale_vals;
-    }
-    const int per = (G + 1023) / 1024;
-    const int g0 = threadIdx.x * per;
-    // up to R partials per thread (G <= 8192 chunks) stay in registers for
-    // the offsets written below; more are read again there
-    constexpr int R = 8;
-    int4 pr[R];
-    int s = 0, l = 0, c = 0;
-    unsigned mx = 0;
-    if (per <= R) {
-#pragma unroll
-        for (int k = 0; k < R; ++k)
-            pr[k] = k < per && g0 + k < G ? a.part[g0 + k] : make_int4(0, 0, 0, 0);
-#pragma unroll
-        for (int k = 0; k < R; ++k) {
-            s += pr[k].x;
-            l += pr[k].y;
-            c += pr[k].z;
-            mx = max(mx, (unsigned)pr[k].w);
-        }
-    } else {
-        for (int k = 0; k < per; ++k)
-            if (g0 + k < G) {
-                int4 p = a.part[g0 + k];
-                s += p.x;
-                l += p.y;
-                c += p.z;
-                mx = max(mx, (unsigned)p.w);
-            }
-    }
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    int xs = s, xl = l, xc = c;
-    unsigned xm = mx;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        int ys = __shfl_up(xs, o, 64), yl = __shfl_up(xl, o, 64), yc = __shfl_up(xc, o, 64);
-        unsigned ym = (unsigned)__shfl_up((int)xm, o, 64);
-        if (lane >= o) {
-            xs += ys;
-            xl += yl;
-            xc += yc;
-            xm = max(xm, ym);
-        }
-    }
-    if (lane == 63) {
-        ls[w] = xs;
-        ll[w] = xl;
-        lc[w] = xc;
-        lm[w] = xm;
-    }
-    __syncthreads();
-    int ps = 0, pl = 0, ts = 0, tl = 0, tc = 0;
-    unsigned tm = 0;
-    for (int k = 0; k < 16; ++k) {
-        if (k < w) {
-            ps += ls[k];
-            pl += ll[k];
-        }
-        ts += ls[k];
-        tl += ll[k];
-        tc += lc[k];
-        tm = max(tm, lm[k]);
-    }
-    int rs = ps + xs - s, rl = pl + xl - l;
-    if (per <= R) {
-#pragma unroll
-        for (int k = 0; k < R; ++k)
-            if (k < per && g0 + k < G) {
-                a.part_off[g0 + k] = make_int2(rs, rl);
-                rs += pr[k].x;
-                rl += pr[k].y;
-            }
-    } else {
-        for (int k = 0; k < per; ++k)
-            if (g0 + k < G) {
-                int4 p = a.part[g0 + k];
-                a.part_off[g0 + k] = make_int2(rs, rl);
-                rs += p.x;
-                rl += p.y;
-            }
-    }
-    if (threadIdx.x == 0) {
-        if ((long long)N + ts > a.cap_s || (long long)L + tl > a.cap_l) {
-            cn->status = MDAS_ERR_CAPACITY_DEV;
-            cn->done = 1;
-        } else {
-            cn->n_samples_old = N;
-            cn->n_leaves_old = L;
-            cn->n_samples = N + ts;
-            cn->n_leaves = L + tl;
-            cn->new_samples = ts;
-            cn->new_nodes = tl;
-            // the next stale-list error pass starts from it; g_error itself
-            // stays until the next error pass (kdgrid.cu:684-716)
-            cn->carry_bits = tm;
-            a.pstats[P & (kMaxPassStats - 1)] = PassStat{L, N, ts, tl, tc, st, sv, 0};
-            cn->passes = P + 1;
-        }
-        cn->sel_cnt = 0;
-        cn->stale = 0;
-        cn->stale_vals = 0;
-    }
-}
-__global__ __launch_bounds__(1024) void k_scan_counts(DevGrid a, int G) { scan_counts_body(a, G); }
-__global__ __launch_bounds__(1024) void k_scan_counts_b(const DevGrid* grids, int G) {
-    scan_counts_body(grids[blockIdx.x], G);
-}
 
 // ----------------------------------------------------- placement and split --
 // kdgrid.cu:328-477 for one selected leaf: best candidate among
@@ -606,11 +342,11 @@ __global__ __launch_bounds__(1024) void k_scan_counts_b(const DevGrid* grids, in
 // sample index k, the draws starting from LCG state s; a full leaf is split
 // at the median of its 5 samples along the largest box axis, keeping the left
 // half in place and the right half at leaf index m.
-// With a scene B (FUSED; its objects in LDS at obj) the new sample is evaluated
-// here and a split's children get their errors here, from the leaf's values
-// and the new one, in place of the next pass's error kernel; emax takes the
-// larger.
-template <int D, bool FUSED>
+// With a scene B (MODE != PLACE_ONLY; its objects in LDS at obj) the new
+// sample is evaluated here, and with PLACE_ERRORS a split's children get their
+// errors here, from the leaf's values and the new one, in place of the next
+// pass's error kernel; emax takes the larger.
+template <int D, int MODE>
 __device__ __forceinline__ void place_leaf(const DevGrid& a, int i, int k, int m, unsigned cnt,
                                            int L, unsigned s, const mscene::SceneBlock* B,
                                            const float* obj, float& emax) {
@@ -696,7 +432,7 @@ __device__ __forceinline__ void place_leaf(const DevGrid& a, int i, int k, int m
     float* out = a.coords + (size_t)k * D;
 #pragma unroll
     for (int d = 0; d < D; ++d) out[d] = best[d];
-    int kid[5] = {k, k, k, k, k};     // FUSED: a split's samples in sorted order,
+    int kid[5] = {k, k, k, k, k};     // PLACE_ERRORS: a split's samples in sorted order,
     float vol_l = 0.0f, vol_r = 0.0f;  // its children's volumes
     if (cnt < 4u) {
         // kdgrid.cu:393-396: insert into the first free slot; the error is kept
@@ -775,7 +511,7 @@ __device__ __forceinline__ void place_leaf(const DevGrid& a, int i, int k, int m
         store_line_head2<D>(a, i, make_int4(v[0], v[1], E, E), mn, cmx, sp[0], sp[1]);
         store_line<D>(a, m, make_int4(v[2], v[3], v[4], E), cmn, mx, &sp[2], 3);
         if constexpr (P < 3) store_point_slot<D>(a, m, 2, sp[4], v[4]);  // D = 6: overflow row
-        if constexpr (FUSED) {
+        if constexpr (MODE == PLACE_ERRORS) {
 #pragma unroll
             for (int j = 0; j < 5; ++j) kid[j] = v[j];
             vol_l = box_volume<D>(mn, cmx);
@@ -810,10 +546,10 @@ __device__ __forceinline__ void place_leaf(const DevGrid& a, int i, int k, int m
     }
     // the leaf's own state (already jumped) and count were written by the
     // selection and compaction kernels
-    if constexpr (FUSED) {
+    if constexpr (MODE != PLACE_ONLY) {
         // the line's stores are out and its registers free; the values of a
         // split's other samples load while the new one is evaluated
-        const bool split = cnt == 4u;
+        const bool split = MODE == PLACE_ERRORS && cnt == 4u;
         LeafSamples ch[2];
         if (split) {
 #pragma unroll
@@ -860,10 +596,10 @@ __device__ __forceinline__ void place_leaf(const DevGrid& a, int i, int k, int m
 // exceed the capacity.  One thread writes the next slot, the pass's
 // statistics and the totals' zeros for the pass after (no kernel of this pass
 // reads those).
-__device__ __forceinline__ bool fused_offsets(const DevGrid& a, int blk, int nblk, int par, int& L,
+__device__ __forceinline__ bool pass_offsets(const DevGrid& a, int blk, int nblk, int par, int& L,
                                               int& N, int2& base) {
     DevCounters* cn = a.cnt;
-    const LoopSlot s = cn->slot[par];
+    const TreeCounts s = cn->slot[par];
     L = s.L;
     N = s.N;
     const int lane = threadIdx.x & 63;
@@ -876,7 +612,7 @@ __device__ __forceinline__ bool fused_offsets(const DevGrid& a, int blk, int nbl
         if (fits) {
             SuperSum& z = a.ssum[(par ^ 1) * kSuper + lane];
             z.sel = z.split = z.held = 0;
-            a.smax[par * kSuper + lane].err = 0u;  // the selection has read it
+            a.smax[par * kSuper + lane].err = 0u;  // the selection has read them
         }
         if (lane == 0) {
             if (!fits) {
@@ -889,7 +625,7 @@ __device__ __forceinline__ bool fused_offsets(const DevGrid& a, int blk, int nbl
                 const int stale = P == 0 ? L : 2 * s.new_n, vals = P == 0 ? 4 * L : 5 * s.new_n;
                 a.pstats[P & (kMaxPassStats - 1)] = PassStat{L, N, sel, split, held, stale, vals, 0};
                 cn->passes = P + 1;
-                cn->slot[par ^ 1] = LoopSlot{N + sel, L + split, N, L, sel, split};
+                cn->slot[par ^ 1] = TreeCounts{N + sel, L + split, N, L, sel, split};
                 cn->cur = par ^ 1;
             }
         }
@@ -923,10 +659,10 @@ __device__ __forceinline__ bool fused_offsets(const DevGrid& a, int blk, int nbl
 // passes of 2000) 617 -> 458 us, 3D 256x256 1240 -> 850 us.  One chunk per wave
 // in place of one per workgroup (fewer barriers, 4x the chunks) was slower at
 // 1080p (12.0 -> 12.9 ms a run at its best count) and no faster below.
-// FUSED: see place_leaf; the offsets come from the super groups' totals and
-// the partials of the chunk's own group, in place of the scan kernel; every
-// workgroup finds the same totals, so a pass beyond the capacity writes nothing.
-template <int D, bool FUSED>
+// MODE: see place_leaf.  The offsets come from the super groups' totals and
+// the partials of the chunk's own group; every workgroup finds the same
+// totals, so a pass beyond the capacity writes nothing.
+template <int D, int MODE>
 __device__ __forceinline__ void compact_place_body(const DevGrid& a, int blk, int nblk, int par,
                                                    const mscene::SceneBlock* B, float* obj) {
     constexpr int U = 4;                   // tiles whose flags and states are loaded together
@@ -935,16 +671,14 @@ __device__ __forceinline__ void compact_place_body(const DevGrid& a, int blk, in
     __shared__ int2 qe[QCAP];
     __shared__ unsigned qs[QCAP];
     if (a.cnt->done) return;
+    nblk = live_chunks(a.cnt->slot[par].L, nblk);
+    if (blk >= nblk) return;
     int L, N0;
     int2 base;
-    if constexpr (FUSED) {
-        if (!fused_offsets(a, blk, nblk, par, L, N0, base)) return;
+    if (!pass_offsets(a, blk, nblk, par, L, N0, base)) return;
+    if constexpr (MODE != PLACE_ONLY) {
         for (int q = threadIdx.x; q < B->p.n_obj * mscene::OBJ_STRIDE; q += 256) obj[q] = B->p.obj[q];
         __syncthreads();
-    } else {
-        L = a.cnt->n_leaves_old;
-        N0 = a.cnt->n_samples_old;
-        base = a.part_off[blk];
     }
     float emax = 0.0f;
     int beg, end;
@@ -956,7 +690,7 @@ __device__ __forceinline__ void compact_place_body(const DevGrid& a, int blk, in
         if ((int)threadIdx.x < count) {
             const int2 q = qe[p];
             const unsigned cnt = q.y >= 0 ? 4u : ((unsigned)q.x >> 30);
-            place_leaf<D, FUSED>(a, q.x & 0x3fffffff, N0 + jq + p, q.y, cnt, L, qs[p], B, obj, emax);
+            place_leaf<D, MODE>(a, q.x & 0x3fffffff, N0 + jq + p, q.y, cnt, L, qs[p], B, obj, emax);
         }
     };
     for (int t00 = beg; t00 < end; t00 += U * 256) {
@@ -1017,7 +751,7 @@ __device__ __forceinline__ void compact_place_body(const DevGrid& a, int blk, in
         __syncthreads();
     }
     place_round(0, qn);
-    if constexpr (FUSED) {
+    if constexpr (MODE == PLACE_ERRORS) {
         emax = wave_max(emax);
         __syncthreads();
         if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = (int)__float_as_uint(emax);
@@ -1029,64 +763,46 @@ __device__ __forceinline__ void compact_place_body(const DevGrid& a, int blk, in
     }
 }
 
-template <int D>
-__global__ __launch_bounds__(256) void k_compact_place(DevGrid a) {
-    compact_place_body<D, false>(a, blockIdx.x, gridDim.x, 0, nullptr, nullptr);
-}
-template <int D>
-__global__ __launch_bounds__(256) void k_compact_place_b(const DevGrid* grids) {
-    const DevGrid a = grids[blockIdx.y];  // by value: scalar registers
-    compact_place_body<D, false>(a, blockIdx.x, gridDim.x, 0, nullptr, nullptr);
-}
-// The scene's objects in dynamic LDS (48 bytes each).
-template <int D>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_place_fused(DevGrid a, const mscene::SceneBlock* B, int par) {
+// The scene's objects in dynamic LDS (48 bytes each).  Four waves per SIMD
+// without spills where the integrand is taken along.
+template <int D, int MODE>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_compact_place(
+    DevGrid a, const mscene::SceneBlock* B, int par) {
     extern __shared__ float obj[];
-    compact_place_body<D, true>(a, blockIdx.x, gridDim.x, par, B, obj);
+    compact_place_body<D, MODE>(a, blockIdx.x, gridDim.x, par, B, obj);
 }
-template <int D>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_place_fused_b(const DevGrid* grids, const void* const* params, int par) {
+template <int D, int MODE>
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_compact_place_b(
+    const DevGrid* grids, const void* const* params, int par) {
     extern __shared__ float obj[];
     const DevGrid a = grids[blockIdx.y];  // by value: scalar registers
-    compact_place_body<D, true>(a, blockIdx.x, gridDim.x, par,
-                                (const mscene::SceneBlock*)params[blockIdx.y], obj);
+    compact_place_body<D, MODE>(a, blockIdx.x, gridDim.x, par, (const mscene::SceneBlock*)params[blockIdx.y], obj);
 }
 
-// The counters that are read outside the fused loop, from the current slot;
-// `done` once the loop has reached its limit, so that the host need not
-// launch another pass to learn it.
-__device__ __forceinline__ void loop_end_body(DevCounters* c) {
-    const LoopSlot s = c->slot[c->cur];
-    c->n_samples = s.N;
-    c->n_leaves = s.L;
-    c->n_samples_old = s.N_old;
-    c->n_leaves_old = s.L_old;
-    c->new_samples = s.new_s;
-    c->new_nodes = s.new_n;
-    if (loop_limit_reached(c)) c->done = 1;
-}
-__global__ void k_loop_end(DevCounters* c) { loop_end_body(c); }
-__global__ void k_loop_status_b(const DevGrid* grids, int n, int fused, int* out) {
+// The loop's state per image: finished once `done` or at the limit, so that the
+// host need not launch another pass to learn it.
+__global__ void k_loop_status_b(const DevGrid* grids, int n, int* out) {
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= n) return;
-    DevCounters* c = grids[t].cnt;
-    if (fused) loop_end_body(c);
-    out[4 * t] = c->done;
+    const DevCounters* c = grids[t].cnt;
+    const TreeCounts s = tree_counts(c);
+    out[4 * t] = c->done || loop_limit_reached(c, s.N, s.L);
     out[4 * t + 1] = c->status;
-    out[4 * t + 2] = c->n_samples;
+    out[4 * t + 2] = s.N;
     out[4 * t + 3] = c->passes;
 }
 
 // After the device-side loop: when it stopped at its limit, no error pass
 // followed the last placement, so its split children get the stale marker
-// (error -1, kdgrid.cu:466-469) the placement left out.
+// (error -1, kdgrid.cu:466-469) the placement left out.  Raises `done`.
 __device__ __forceinline__ void mark_last_children_body(const DevGrid& a, int blk, int nblk) {
-    const DevCounters* c = a.cnt;
-    if (c->status != 0 || !loop_limit_reached(c)) return;
-    const int nn = c->new_nodes, L_old = c->n_leaves_old;
-    for (int t = blk * 256 + threadIdx.x; t < nn; t += nblk * 256) {
+    DevCounters* c = a.cnt;
+    const TreeCounts s = tree_counts(c);
+    if (c->status != 0 || !loop_limit_reached(c, s.N, s.L)) return;
+    if (blk == 0 && threadIdx.x == 0) c->done = 1;
+    for (int t = blk * 256 + threadIdx.x; t < s.new_n; t += nblk * 256) {
         a.err[a.split_list[t]] = -1.0f;
-        a.err[L_old + t] = -1.0f;
+        a.err[s.L_old + t] = -1.0f;
     }
 }
 __global__ __launch_bounds__(256) void k_mark_last_children(DevGrid a) {
@@ -1139,109 +855,58 @@ static int grid_for(long long n, int cap_blocks = 8192) {
     default: return hipErrorInvalidValue;              \
     }
 
-hipError_t launch_initial(Grid& g, int L0, hipStream_t st) {
+hipError_t launch_initial(Grid& g, int L0, int limit, hipStream_t st) {
     const int blocks = grid_for(L0, 4096);
     MDAS_DISPATCH_D(g.D, hipLaunchKernelGGL(k_initial<DD>, dim3(blocks), dim3(256), 0, st, g.dev, L0));
-    hipLaunchKernelGGL(k_initial_counters, dim3(1), dim3(2 * kSuper), 0, st, g.dev, L0);
+    hipLaunchKernelGGL(k_initial_counters, dim3(1), dim3(kMaxSets * kSuper), 0, st, g.dev, L0, limit);
     return hipGetLastError();
 }
 
-hipError_t launch_reset_errors(Grid& g, int standalone, hipStream_t st) {
-    hipLaunchKernelGGL(k_reset_errors, dim3(1), dim3(1), 0, st, g.dev.cnt, standalone);
+hipError_t launch_arm(Grid& g, bool errors, bool adaptive, hipStream_t st) {
+    hipLaunchKernelGGL(k_arm, dim3(1), dim3(kSuper), 0, st, g.dev, errors ? 1 : 0, adaptive ? 1 : 0);
     return hipGetLastError();
 }
 
-hipError_t launch_set_limit(Grid& g, int limit, hipStream_t st) {
-    // the capacity guard applies when the limit is the capacity (a target at
-    // or beyond max_samples); below it a pass that would overflow is an error
-    hipLaunchKernelGGL(k_set_limit, dim3(1), dim3(1), 0, st, g.dev.cnt, limit,
-                       limit >= g.cap_s ? g.cap_s : 0);
+hipError_t launch_compute_errors(Grid& g, hipStream_t st) {
+    MDAS_DISPATCH_D(g.D, hipLaunchKernelGGL(k_compute_errors<DD>, dim3(g.error_blocks()), dim3(256), 0, st, g.dev));
     return hipGetLastError();
 }
 
-hipError_t launch_arm(Grid& g, hipStream_t st) {
-    hipLaunchKernelGGL(k_arm, dim3(1), dim3(1), 0, st, g.dev.cnt);
+hipError_t launch_errors(Grid& g, int parity, hipStream_t st) {
+    MDAS_DISPATCH_D(g.D, hipLaunchKernelGGL(k_errors<DD>, dim3(g.error_blocks()), dim3(256), 0, st, g.dev, parity));
     return hipGetLastError();
 }
 
-hipError_t launch_errors(Grid& g, hipStream_t st) {
-    MDAS_DISPATCH_D(g.D, hipLaunchKernelGGL(k_errors<DD>, dim3(g.err_blocks), dim3(256), 0, st, g.dev));
-    hipLaunchKernelGGL(k_err_reduce, dim3(1), dim3(1024), 0, st, g.dev, g.err_blocks, 0);
+static hipError_t select_chunks(Grid& g, int parity, int loop, hipStream_t st) {
+    const int n = g.chunks(), cpw = select_cpw(n);
+    hipLaunchKernelGGL(k_select, dim3(n / cpw), dim3(256), 0, st, g.dev, n, cpw, parity, loop);
     return hipGetLastError();
 }
+hipError_t launch_select(Grid& g, int parity, hipStream_t st) { return select_chunks(g, parity, 1, st); }
 
-hipError_t launch_errors_stale(Grid& g, hipStream_t st) {
-    MDAS_DISPATCH_D(g.D, hipLaunchKernelGGL(k_errors_stale<DD>, dim3(g.err_blocks), dim3(256), 0, st, g.dev));
-    hipLaunchKernelGGL(k_err_reduce, dim3(1), dim3(1024), 0, st, g.dev, g.err_blocks, 1);
-    return hipGetLastError();
-}
+#define MDAS_DISPATCH_PLACE(D_, MODE_, KERNEL, ...)                                                    \
+    switch (MODE_) {                                                                                   \
+    case PLACE_ONLY: MDAS_DISPATCH_D(D_, hipLaunchKernelGGL((KERNEL<DD, PLACE_ONLY>), __VA_ARGS__)); break;     \
+    case PLACE_EVAL: MDAS_DISPATCH_D(D_, hipLaunchKernelGGL((KERNEL<DD, PLACE_EVAL>), __VA_ARGS__)); break;     \
+    default: MDAS_DISPATCH_D(D_, hipLaunchKernelGGL((KERNEL<DD, PLACE_ERRORS>), __VA_ARGS__)); break;           \
+    }
 
-hipError_t launch_select(Grid& g, hipStream_t st) {
-    const int cpw = select_cpw(g.chunks());
-    hipLaunchKernelGGL(k_select, dim3(g.chunks() / cpw), dim3(256), 0, st, g.dev, cpw);
-    return hipGetLastError();
-}
-
-hipError_t launch_scan(Grid& g, hipStream_t st) {
-    hipLaunchKernelGGL(k_scan_counts, dim3(1), dim3(1024), 0, st, g.dev, g.chunks());
-    return hipGetLastError();
-}
-
-hipError_t launch_place(Grid& g, hipStream_t st) {
-    MDAS_DISPATCH_D(g.D, hipLaunchKernelGGL(k_compact_place<DD>, dim3(g.chunks()), dim3(256), 0, st,
-                                            g.dev));
+hipError_t launch_place(Grid& g, int parity, int mode, const void* dparams, int n_obj, hipStream_t st) {
+    const size_t lds = mode == PLACE_ONLY ? 0 : n_obj * mscene::OBJ_STRIDE * sizeof(float);
+    MDAS_DISPATCH_PLACE(g.D, mode, k_compact_place, dim3(g.chunks()), dim3(256), lds, st, g.dev,
+                        (const mscene::SceneBlock*)dparams, parity);
     return hipGetLastError();
 }
 
 hipError_t launch_adaptive(Grid& g, hipStream_t st) {
-    hipError_t e = launch_select(g, st);
-    if (e == hipSuccess) e = launch_scan(g, st);
-    if (e == hipSuccess) e = launch_place(g, st);
+    const int parity = g.host.cur;  // the host is current after every call that changes the tree
+    hipError_t e = select_chunks(g, parity, 0, st);
+    if (e == hipSuccess) e = launch_place(g, parity, PLACE_ONLY, nullptr, 0, st);
     return e;
 }
 
-hipError_t launch_first_errors(Grid& g, hipStream_t st) {
-    const int blocks = grid_for(1ll << (g.b * g.D + 2 * g.e), g.err_blocks);
-    MDAS_DISPATCH_D(g.D, hipLaunchKernelGGL(k_first_errors<DD>, dim3(blocks), dim3(256), 0, st, g.dev));
-    return hipGetLastError();
-}
-
-hipError_t launch_fused_pass(Grid& g, const void* dparams, int n_obj, int parity, hipStream_t st) {
-    const int chunks = g.chunks(), cpw = select_cpw(chunks);
-    hipLaunchKernelGGL(k_select_fused, dim3(chunks / cpw), dim3(256), 0, st, g.dev, cpw, parity);
-    MDAS_DISPATCH_D(g.D, hipLaunchKernelGGL(k_place_fused<DD>, dim3(chunks), dim3(256),
-                                            n_obj * mscene::OBJ_STRIDE * sizeof(float), st, g.dev,
-                                            (const mscene::SceneBlock*)dparams, parity));
-    return hipGetLastError();
-}
-
-hipError_t launch_loop_end(Grid& g, hipStream_t st) {
-    hipLaunchKernelGGL(k_loop_end, dim3(1), dim3(1), 0, st, g.dev.cnt);
-    return hipGetLastError();
-}
-
-hipError_t launch_first_errors_b(int D, const DevGrid* grids, int n, int blocks, hipStream_t st) {
-    MDAS_DISPATCH_D(D, hipLaunchKernelGGL(k_first_errors_b<DD>, dim3(blocks < 1024 ? blocks : 1024, n), dim3(256), 0,
-                                          st, grids));
-    return hipGetLastError();
-}
-
-hipError_t launch_fused_pass_b(int D, const DevGrid* grids, const void* const* params, int n_obj,
-                               int n, int blocks, int parity, hipStream_t st) {
-    const int cpw = select_cpw(blocks);
-    hipLaunchKernelGGL(k_select_fused_b, dim3(blocks / cpw, n), dim3(256), 0, st, grids, cpw, parity);
-    MDAS_DISPATCH_D(D, hipLaunchKernelGGL(k_place_fused_b<DD>, dim3(blocks, n), dim3(256),
-                                          n_obj * mscene::OBJ_STRIDE * sizeof(float), st, grids, params, parity));
-    return hipGetLastError();
-}
-
-hipError_t launch_loop_status_b(const DevGrid* grids, int n, int fused, int* out, hipStream_t st) {
-    hipLaunchKernelGGL(k_loop_status_b, dim3((n + 63) / 64), dim3(64), 0, st, grids, n, fused, out);
-    return hipGetLastError();
-}
-
 hipError_t launch_mark_last_children(Grid& g, hipStream_t st) {
-    hipLaunchKernelGGL(k_mark_last_children, dim3(1024), dim3(256), 0, st, g.dev);
+    hipLaunchKernelGGL(k_mark_last_children, dim3(g.error_blocks()), dim3(256), 0, st, g.dev);
     return hipGetLastError();
 }
 
@@ -1273,24 +938,31 @@ hipError_t launch_fill_f32(float* p, float v, long long n, hipStream_t st) {
 hipError_t launch_initial_b(int D, const DevGrid* grids, int n, int blocks, const int* limits,
                             hipStream_t st) {
     MDAS_DISPATCH_D(D, hipLaunchKernelGGL(k_initial_b<DD>, dim3(blocks, n), dim3(256), 0, st, grids));
-    hipLaunchKernelGGL(k_initial_counters_b, dim3(n), dim3(2 * kSuper), 0, st, grids, limits);
+    hipLaunchKernelGGL(k_initial_counters_b, dim3(n), dim3(kMaxSets * kSuper), 0, st, grids, limits);
     return hipGetLastError();
 }
 
-hipError_t launch_pass_b(int D, const DevGrid* grids, int n, int blocks, hipStream_t st,
-                         const LearnDev* learns) {
-    const int eb = blocks < 1024 ? blocks : 1024;
-    if (learns) {
-        const hipError_t e = launch_errors_learned_b(D, grids, learns, n, blocks, st);
-        if (e != hipSuccess) return e;
-    } else {
-        MDAS_DISPATCH_D(D, hipLaunchKernelGGL(k_errors_stale_b<DD>, dim3(eb, n), dim3(256), 0, st, grids));
-        hipLaunchKernelGGL(k_err_reduce_b, dim3(n), dim3(1024), 0, st, grids, eb);
-    }
+hipError_t launch_errors_b(int D, const DevGrid* grids, int n, int blocks, int parity, hipStream_t st) {
+    MDAS_DISPATCH_D(D, hipLaunchKernelGGL(k_errors_b<DD>, dim3(blocks < 1024 ? blocks : 1024, n), dim3(256), 0, st,
+                                          grids, parity));
+    return hipGetLastError();
+}
+
+hipError_t launch_select_b(const DevGrid* grids, int n, int blocks, int parity, hipStream_t st) {
     const int cpw = select_cpw(blocks);
-    hipLaunchKernelGGL(k_select_b, dim3(blocks / cpw, n), dim3(256), 0, st, grids, cpw);
-    hipLaunchKernelGGL(k_scan_counts_b, dim3(n), dim3(1024), 0, st, grids, blocks);
-    MDAS_DISPATCH_D(D, hipLaunchKernelGGL(k_compact_place_b<DD>, dim3(blocks, n), dim3(256), 0, st, grids));
+    hipLaunchKernelGGL(k_select_b, dim3(blocks / cpw, n), dim3(256), 0, st, grids, blocks, cpw, parity);
+    return hipGetLastError();
+}
+
+hipError_t launch_place_b(int D, const DevGrid* grids, const void* const* params, int n_obj, int n,
+                          int blocks, int parity, int mode, hipStream_t st) {
+    const size_t lds = mode == PLACE_ONLY ? 0 : n_obj * mscene::OBJ_STRIDE * sizeof(float);
+    MDAS_DISPATCH_PLACE(D, mode, k_compact_place_b, dim3(blocks, n), dim3(256), lds, st, grids, params, parity);
+    return hipGetLastError();
+}
+
+hipError_t launch_loop_status_b(const DevGrid* grids, int n, int* out, hipStream_t st) {
+    hipLaunchKernelGGL(k_loop_status_b, dim3((n + 63) / 64), dim3(64), 0, st, grids, n, out);
     return hipGetLastError();
 }
 

@@ -57,7 +57,7 @@ void free_grid(Grid& g) {
     mdas::ReconBufs& rb = g.rb;
     void* ptrs[] = {d.coords,   d.values,  d.leaf,        d.err,        d.seed,     d.flags,
                     d.xpts,     d.split_list, d.sdat,     d.sext,       d.part,     d.part_off,
-                    d.epart,    d.cnt,     d.ssum, d.smax, d.pstats,      rb.rrec,      rb.keys,    rb.keys_alt,
+                    d.cnt,      d.ssum,    d.smax,        d.pstats,      rb.rrec,      rb.keys,    rb.keys_alt,
                     rb.tile_start, rb.tile_end, rb.rs_hist, g.d_scalar, g.learn.feat, g.learn.perr,
                     g.learn.rows};
     for (void* p : ptrs)
@@ -73,10 +73,10 @@ void free_grid(Grid& g) {
 }
 
 int sync_counters(Grid& g, hipStream_t st) {
-    HIP_TRY(hipMemcpyAsync(&g.host, g.dev.cnt, sizeof(mdas::DevCounters), hipMemcpyDeviceToHost, st));
+    HIP_TRY(hipMemcpyAsync(static_cast<mdas::DevCounters*>(&g.host), g.dev.cnt, sizeof(mdas::DevCounters),
+                           hipMemcpyDeviceToHost, st));
     HIP_TRY(hipStreamSynchronize(st));
-    g.gmax_host = 0.0f;
-    memcpy(&g.gmax_host, &g.host.gmax_bits, 4);
+    g.host.name_counts();
     return MDAS_OK;
 }
 
@@ -149,7 +149,7 @@ void collect_kernel_times(Grid& g, std::vector<std::pair<std::string, double>>* 
     };
     g.t_initial = get("k_initial");
     g.t_errors = get("k_errors");
-    g.t_adaptive = get("k_select") + get("k_scan_counts") + get("k_place") + get("k_mark_last");
+    g.t_adaptive = get("k_select") + get("k_place") + get("k_mark_last");
     g.t_integrand = get("k_eval");
 }
 
@@ -236,10 +236,9 @@ int mdas_create(const mdas_config* cfg, mdas_handle* out) {
     if (e == hipSuccess) e = dalloc(&d.sdat, 2 * (cl / 2 + 1));  // splits per pass <= cap_l / 2
     if (e == hipSuccess) e = dalloc(&d.part, (size_t)mdas::kChunkBlocks);
     if (e == hipSuccess) e = dalloc(&d.part_off, (size_t)mdas::kChunkBlocks);
-    if (e == hipSuccess) e = dalloc(&d.epart, (size_t)mdas::kErrBlocks);
     if (e == hipSuccess) e = dalloc(&d.cnt, 1);
     if (e == hipSuccess) e = dalloc(&d.ssum, (size_t)(2 * mdas::kSuper));
-    if (e == hipSuccess) e = dalloc(&d.smax, (size_t)(2 * mdas::kSuper));
+    if (e == hipSuccess) e = dalloc(&d.smax, (size_t)(mdas::kMaxSets * mdas::kSuper));
     if (e == hipSuccess) e = dalloc(&d.pstats, (size_t)mdas::kMaxPassStats);
     if (e == hipSuccess) e = dalloc(&g.d_scalar, 64);
     if (e != hipSuccess) {
@@ -248,6 +247,7 @@ int mdas_create(const mdas_config* cfg, mdas_handle* out) {
         return fail(MDAS_ERR_HIP, std::string("device allocation failed: ") + hipGetErrorString(e));
     }
     e = hipMemset(d.cnt, 0, sizeof(mdas::DevCounters));
+    if (e == hipSuccess) e = hipMemset(d.smax, 0, sizeof(mdas::SuperMax) * mdas::kMaxSets * mdas::kSuper);
     if (e == hipSuccess) e = hipMemset(d.values, 0, sizeof(float) * cs * 3);
     // overflow rows start as -1 slots (a stale slot is then -1 or an index
     // written before, never garbage)
@@ -295,14 +295,12 @@ int mdas_initial_sampling(mdas_handle h, void* stream) {
     // The reference zeroes every seed here (kdgrid.cu:637) so that a leaf
     // created later starts from tea4(index, 0); a split writes seed 0 into
     // the new leaf's slot, which gives the same result without the fill.
-    HIP_TRY(mdas::launch_initial(g, L0, st));
+    HIP_TRY(mdas::launch_initial(g, L0, 0x7fffffff, st));
     g.initialized = true;
     set_initial_extents(g);
-    g.host.n_leaves = L0;
-    g.host.n_samples = 4 * L0;
-    g.host.new_samples = 4 * L0;
-    g.host.new_nodes = 0;
-    g.host.passes = 0;
+    g.host = mdas::HostCounters{};
+    g.host.slot[0] = mdas::TreeCounts{4 * L0, L0, 0, 0, 4 * L0, 0};
+    g.host.name_counts();
     if (logging) {
         HIP_TRY(hipEventRecord(ev.e[1], st));
         HIP_TRY(hipEventSynchronize(ev.e[1]));
@@ -312,19 +310,17 @@ int mdas_initial_sampling(mdas_handle h, void* stream) {
     return MDAS_OK;
 }
 
-int mdas_compute_errors(mdas_handle h, void* stream) {
-    if (!h) return fail(MDAS_ERR_INVALID, "null handle");
-    Grid& g = h->g;
-    if (!g.initialized) return fail(MDAS_ERR_STATE, "InitialSampling has not been called");
-    hipStream_t st = S(stream);
+// The error pass and the adaptive pass of the single calls; `armed`: the
+// kernels have been re-armed for both by the caller.
+static int compute_errors(Grid& g, bool armed, hipStream_t st) {
     CallEvents ev;
     const bool logging = g.logging();
     if (logging) {
         HIP_TRY(ev.create(2));
         HIP_TRY(hipEventRecord(ev.e[0], st));
     }
-    HIP_TRY(mdas::launch_reset_errors(g, 1, st));
-    HIP_TRY(mdas::launch_errors(g, st));
+    if (!armed) HIP_TRY(mdas::launch_arm(g, true, false, st));
+    HIP_TRY(mdas::launch_compute_errors(g, st));
     if (logging) {
         HIP_TRY(hipEventRecord(ev.e[1], st));
         HIP_TRY(hipEventSynchronize(ev.e[1]));
@@ -333,29 +329,24 @@ int mdas_compute_errors(mdas_handle h, void* stream) {
     return MDAS_OK;
 }
 
-int mdas_adaptive_sampling(mdas_handle h, void* stream) {
-    if (!h) return fail(MDAS_ERR_INVALID, "null handle");
-    Grid& g = h->g;
-    if (!g.initialized) return fail(MDAS_ERR_STATE, "InitialSampling has not been called");
-    hipStream_t st = S(stream);
+static int adaptive_sampling(Grid& g, bool armed, hipStream_t st) {
     CallEvents ev;
     const bool logging = g.logging();
     if (logging) {
         HIP_TRY(ev.create(2));
         HIP_TRY(hipEventRecord(ev.e[0], st));
     }
-    HIP_TRY(mdas::launch_arm(g, st));
+    if (!armed) HIP_TRY(mdas::launch_arm(g, false, true, st));
     HIP_TRY(mdas::launch_adaptive(g, st));
     int rc = sync_counters(g, st);  // kdgrid.cu:753-759 reads the counters back
     if (rc) return rc;
     if (g.host.status != 0) {
         int s = g.host.status;
         // clear the device error so that the grid stays usable
-        mdas::DevCounters c = g.host;
-        c.status = 0;
-        c.done = 0;
-        HIP_TRY(hipMemcpy(g.dev.cnt, &c, sizeof(c), hipMemcpyHostToDevice));
-        g.host = c;
+        g.host.status = 0;
+        g.host.done = 0;
+        HIP_TRY(hipMemcpy(g.dev.cnt, static_cast<mdas::DevCounters*>(&g.host), sizeof(mdas::DevCounters),
+                          hipMemcpyHostToDevice));
         if (s == MDAS_ERR_CAPACITY)
             return fail(MDAS_ERR_CAPACITY, "adaptive pass would exceed max_samples (" +
                                                std::to_string(g.max_samples) + ")");
@@ -370,10 +361,26 @@ int mdas_adaptive_sampling(mdas_handle h, void* stream) {
     return MDAS_OK;
 }
 
+int mdas_compute_errors(mdas_handle h, void* stream) {
+    if (!h) return fail(MDAS_ERR_INVALID, "null handle");
+    if (!h->g.initialized) return fail(MDAS_ERR_STATE, "InitialSampling has not been called");
+    return compute_errors(h->g, false, S(stream));
+}
+
+int mdas_adaptive_sampling(mdas_handle h, void* stream) {
+    if (!h) return fail(MDAS_ERR_INVALID, "null handle");
+    if (!h->g.initialized) return fail(MDAS_ERR_STATE, "InitialSampling has not been called");
+    return adaptive_sampling(h->g, false, S(stream));
+}
+
 int mdas_sampling_pass(mdas_handle h, void* stream) {
-    int rc = mdas_compute_errors(h, stream);
+    if (!h) return fail(MDAS_ERR_INVALID, "null handle");
+    Grid& g = h->g;
+    if (!g.initialized) return fail(MDAS_ERR_STATE, "InitialSampling has not been called");
+    HIP_TRY(mdas::launch_arm(g, true, true, S(stream)));
+    int rc = compute_errors(g, true, S(stream));
     if (rc) return rc;
-    return mdas_adaptive_sampling(h, stream);
+    return adaptive_sampling(g, true, S(stream));
 }
 
 static int check_image(Grid& g, int w, int hgt) {
@@ -560,12 +567,16 @@ int mdas_upload_state(mdas_handle h, int n, int l, const float* coords, const fl
         HIP_TRY(mdas::launch_build_pts(g, l, 0));
         HIP_TRY(hipDeviceSynchronize());
     }
-    mdas::DevCounters c{};
-    c.n_samples = n;
-    c.n_leaves = l;
+    // g_error in one of its groups, the others and the loop's sets zero
+    std::vector<mdas::SuperMax> sm((size_t)(mdas::kMaxSets * mdas::kSuper), mdas::SuperMax{});
+    memcpy(&sm[(size_t)(mdas::kGError * mdas::kSuper)].err, &max_error, 4);
+    HIP_TRY(hipMemcpy(g.dev.smax, sm.data(), sizeof(mdas::SuperMax) * sm.size(), hipMemcpyHostToDevice));
+    HIP_TRY(hipMemset(g.dev.ssum, 0, sizeof(mdas::SuperSum) * 2 * mdas::kSuper));
+    mdas::HostCounters c{};
+    c.slot[0] = mdas::TreeCounts{n, l, 0, 0, 0, 0};
     c.limit = 0x7fffffff;
-    memcpy(&c.gmax_bits, &max_error, 4);
-    HIP_TRY(hipMemcpy(g.dev.cnt, &c, sizeof(c), hipMemcpyHostToDevice));
+    c.name_counts();
+    HIP_TRY(hipMemcpy(g.dev.cnt, static_cast<mdas::DevCounters*>(&c), sizeof(mdas::DevCounters), hipMemcpyHostToDevice));
     g.host = c;
     g.initialized = true;
     return MDAS_OK;
@@ -659,8 +670,15 @@ float mdas_get_scale_x(mdas_handle h) { return h ? h->g.sX : 0.0f; }
 float mdas_get_scale_y(mdas_handle h) { return h ? h->g.sY : 0.0f; }
 float mdas_get_max_error(mdas_handle h) {
     if (!h) return 0.0f;
-    if (sync_counters(h->g, nullptr)) return 0.0f;
-    return h->g.gmax_host;
+    std::vector<mdas::SuperMax> sm((size_t)mdas::kSuper);
+    if (hipMemcpy(sm.data(), h->g.dev.smax + mdas::kGError * mdas::kSuper, sizeof(mdas::SuperMax) * sm.size(),
+                  hipMemcpyDeviceToHost) != hipSuccess)
+        return 0.0f;
+    unsigned bits = 0u;
+    for (const auto& t : sm) bits = std::max(bits, t.err);
+    float e;
+    memcpy(&e, &bits, 4);
+    return e;
 }
 int mdas_get_passes(mdas_handle h) { return h ? h->g.passes : 0; }
 
@@ -775,8 +793,7 @@ int mdas_run(mdas_handle h, mdas_scene_handle s, long long target, void* stream)
     g.t_recon = g.t_sort = 0.0;
     g.pstats_host.clear();
     mdas::kbeg(g, st, "k_initial");
-    HIP_TRY(mdas::launch_initial(g, L0, st));
-    HIP_TRY(mdas::launch_set_limit(g, (int)limit, st));
+    HIP_TRY(mdas::launch_initial(g, L0, (int)limit, st));
     mdas::kend(g, st);
     g.initialized = true;
     set_initial_extents(g);
@@ -792,38 +809,40 @@ int mdas_run(mdas_handle h, mdas_scene_handle s, long long target, void* stream)
         explicit LoopMode(mdas::DevGrid& x) : d(x) { d.in_loop = 1; }
         ~LoopMode() { d.in_loop = 0; }
     } loop_mode{g.dev};
-    // The plain method's pass is two kernels, the new samples evaluated and
-    // the children's errors taken where they are placed.  Timing and logs want
-    // the phases apart and the learned error pass is a kernel of its own:
-    // those run the separate kernels, with the same results.
-    const bool fused = !g.timing && g.learn_mode == 0;
-    if (fused) HIP_TRY(mdas::launch_first_errors(g, st));
+    // The placement takes the integrand along and, for the plain method, the
+    // children's errors (the learned error pass is a kernel of its own);
+    // timing and logs want the phases apart.  The results are the same.
+    const int mode = g.timing ? mdas::PLACE_ONLY : (g.learn_mode ? mdas::PLACE_EVAL : mdas::PLACE_ERRORS);
+    bool errors_taken = false;  // by the placement before
     for (;;) {
-        for (int b = 0; b < B && fused; ++b) HIP_TRY(mdas::launch_fused_pass(g, s->dev, s->host.n_obj, b & 1, st));
-        if (fused) HIP_TRY(mdas::launch_loop_end(g, st));
-        for (int b = 0; b < B && !fused; ++b) {
-            mdas::kbeg(g, st, "k_errors");
-            HIP_TRY(g.learn_mode ? mdas::launch_errors_learned(g, st)
-                                 : mdas::launch_errors_stale(g, st));
-            mdas::kend(g, st);
+        for (int b = 0; b < B; ++b) {
+            const int par = b & 1;
+            if (!errors_taken) {
+                mdas::kbeg(g, st, "k_errors");
+                HIP_TRY(g.learn_mode ? mdas::launch_errors_learned(g, par, st) : mdas::launch_errors(g, par, st));
+                mdas::kend(g, st);
+                errors_taken = mode == mdas::PLACE_ERRORS;
+            }
             mdas::kbeg(g, st, "k_select");
-            HIP_TRY(mdas::launch_select(g, st));
-            mdas::kend(g, st);
-            mdas::kbeg(g, st, "k_scan_counts");
-            HIP_TRY(mdas::launch_scan(g, st));
+            HIP_TRY(mdas::launch_select(g, par, st));
             mdas::kend(g, st);
             mdas::kbeg(g, st, "k_place");
-            HIP_TRY(mdas::launch_place(g, st));
+            HIP_TRY(mdas::launch_place(g, par, mode, s->dev, s->host.n_obj, st));
             mdas::kend(g, st);
-            mdas::kbeg(g, st, "k_eval");
-            HIP_TRY(mdas::launch_eval(g, s->dev, 0, 0, true, st));
-            mdas::kend(g, st);
+            if (mode == mdas::PLACE_ONLY) {
+                mdas::kbeg(g, st, "k_eval");
+                HIP_TRY(mdas::launch_eval(g, s->dev, 0, 0, true, st));
+                mdas::kend(g, st);
+            }
         }
         int rc = sync_counters(g, st);
         if (rc == MDAS_OK) rc = mdas::drain_pass_stats(g, false);
         if (rc) return rc;
         if (g.timing) collect_kernel_times(g, logging ? &seq : nullptr);
-        if (g.host.done || g.host.status) break;
+        // the stopping rule, as the next pass's kernels would find it
+        if (g.host.done || g.host.status || g.host.n_samples >= g.host.limit ||
+            (g.host.guard_cap != 0 && (long long)g.host.n_samples + g.host.n_leaves > (long long)g.host.guard_cap))
+            break;
         // every pass selects the leaf of maximum error (its ratio is 1), so
         // each block adds samples and the loop ends at the limit; a block that
         // adds none means no leaf passed the selection test: the maximum error
@@ -851,11 +870,11 @@ int mdas_run(mdas_handle h, mdas_scene_handle s, long long target, void* stream)
         log_time(g, "INITIAL SAMPLING TIME", seq[0].second);
         log_time(g, "TRACE TIME", seq[1].second);
         size_t k = 2;
-        for (int p = 0; p < g.passes && k + 4 < seq.size(); ++p, k += 5) {
+        for (int p = 0; p < g.passes && k + 3 < seq.size(); ++p, k += 4) {
             log_time(g, "COMPUTE ERRORS TIME", seq[k].second);
             log_count(g, "SAMPLES", p < (int)g.pstats_host.size() ? g.pstats_host[p].sel : 0);
-            log_time(g, "ADAPTIVE SAMPLING TIME", seq[k + 1].second + seq[k + 2].second + seq[k + 3].second);
-            log_time(g, "TRACE TIME", seq[k + 4].second);
+            log_time(g, "ADAPTIVE SAMPLING TIME", seq[k + 1].second + seq[k + 2].second);
+            log_time(g, "TRACE TIME", seq[k + 3].second);
         }
     }
     if (g.host.status) {
@@ -904,8 +923,6 @@ static double kernel_bytes(const Grid& g, const std::string& k) {
         }
         else if (k == "k_select")  // error, state, flags read; flags written
             b += 10.0 * p.L;
-        else if (k == "k_scan_counts")
-            b += (16.0 + 8.0) * g.chunks();
         else if (k == "k_place")  // compaction and placement
             b += 10.0 * p.L +                                    // flags, states read and written
                  (double)p.sel * (SB + 4.0 * D) +                // slots + box, the new sample
@@ -959,8 +976,7 @@ int mdas_get_phase_times(mdas_handle h, mdas_phase_times* o) {
     o->final_leaves = g.host.n_leaves;
     o->bytes_initial = kernel_bytes(g, "k_initial");
     o->bytes_errors = kernel_bytes(g, "k_errors");
-    o->bytes_adaptive = kernel_bytes(g, "k_select") + kernel_bytes(g, "k_scan_counts") +
-                        kernel_bytes(g, "k_place");
+    o->bytes_adaptive = kernel_bytes(g, "k_select") + kernel_bytes(g, "k_place");
     double br = 0.0;
     for (const char* k : {"k_recon_prep", "k_scan_keys", "k_recon_emit", "k_rs_hist", "k_rs_scan",
                           "k_rs_scatter", "k_tile_ranges", "k_gather"})

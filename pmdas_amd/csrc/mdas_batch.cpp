@@ -29,15 +29,17 @@ struct Group {
     int blocks = 0;
     int max_chunks = 1;                  // chunks the largest member's capacity fills
     int n_obj = 0;                       // most objects of a member's scene
-    bool fused() const { return d_learn == nullptr; }  // plain members only: two kernels per pass
-    hipError_t first_errors(hipStream_t st) const {
-        return fused() ? mdas::launch_first_errors_b(D, d_grids, (int)members.size(), blocks, st) : hipSuccess;
-    }
+    // pass p: the placement takes the integrand along, and the children's
+    // errors in a group of plain members (the initial leaves' are taken before)
     hipError_t pass(int p, hipStream_t st) const {
-        const int m = (int)members.size();
-        if (fused()) return mdas::launch_fused_pass_b(D, d_grids, d_params, n_obj, m, blocks, p & 1, st);
-        const hipError_t e = mdas::launch_pass_b(D, d_grids, m, blocks, st, d_learn);
-        return e != hipSuccess ? e : mdas::launch_eval_b(d_grids, d_params, m, blocks, st);
+        const int m = (int)members.size(), par = p & 1;
+        hipError_t e = hipSuccess;
+        if (d_learn) e = mdas::launch_errors_learned_b(D, d_grids, d_learn, m, blocks, par, st);
+        if (e == hipSuccess) e = mdas::launch_select_b(d_grids, m, blocks, par, st);
+        if (e == hipSuccess)
+            e = mdas::launch_place_b(D, d_grids, d_params, n_obj, m, blocks, par,
+                                     d_learn ? mdas::PLACE_EVAL : mdas::PLACE_ERRORS, st);
+        return e;
     }
     void set_blocks(int total) {
         blocks = std::max(64, std::min(mdas::kChunkBlocks, total / (int)members.size()));
@@ -216,7 +218,7 @@ int mdas_batch_run(mdas_batch_handle b, const long long* targets, void* stream, 
         B_TRY(hipMemcpyAsync(g.d_limits, limits[gi].data(), sizeof(int) * m, hipMemcpyHostToDevice, st));
         B_TRY(mdas::launch_initial_b(g.D, g.d_grids, m, g.blocks, g.d_limits, st));
         B_TRY(mdas::launch_eval_b(g.d_grids, g.d_params, m, g.blocks, st));
-        B_TRY(g.first_errors(st));
+        if (!g.d_learn) B_TRY(mdas::launch_errors_b(g.D, g.d_grids, m, g.blocks, 0, st));
         for (int k = 0; k < m; ++k) {
             b->grids[g.members[k]]->g.initialized = true;
             mdas::initial_extents(b->grids[g.members[k]]->g);
@@ -244,7 +246,7 @@ int mdas_batch_run(mdas_batch_handle b, const long long* targets, void* stream, 
             } else {
                 for (int p = 0; p < B; ++p) B_TRY(g.pass(p, st));
             }
-            B_TRY(mdas::launch_loop_status_b(g.d_grids, m, g.fused() ? 1 : 0, g.d_status, st));
+            B_TRY(mdas::launch_loop_status_b(g.d_grids, m, g.d_status, st));
         }
         ++blocks_run;
         B_TRY(hipStreamSynchronize(st));

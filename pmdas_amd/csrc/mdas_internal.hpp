@@ -9,52 +9,54 @@
 
 namespace mdas {
 
-// What a pass of the device-side loop starts from: sample and leaf counts,
-// those before the pass that led here and that pass's new ones.  Two slots by
-// pass parity: a pass's kernels read one while a single thread writes the other.
-struct LoopSlot {
+// Sample and leaf counts of a tree, those before the adaptive pass that led
+// here and that pass's new ones.  Two slots, used in turn: a pass's kernels
+// read one while a single thread writes the other.
+struct TreeCounts {
     int N, L, N_old, L_old, new_s, new_n;
 };
 
 // Device-resident counters of one grid.  Every kernel reads N / L from here,
 // so a whole sampling loop can be enqueued without host round trips.
 struct DevCounters {
-    int n_samples;       // N
-    int n_leaves;        // L
-    int n_samples_old;   // N before the last adaptive pass (new slice = [old, N))
-    int n_leaves_old;    // L before the last adaptive pass
-    unsigned gmax_bits;  // global max leaf error (float bits, errors are >= 0)
-    int new_samples;
-    int new_nodes;
+    TreeCounts slot[2];
+    int cur;             // the slot that holds the tree's counts
     int done;            // stopping rule reached or error: pass kernels return early
     int status;          // 0 or an MDAS_ERR_* code raised on the device
     int passes;          // adaptive passes performed
     int limit;           // stopping limit min(target, max_samples)
-    int n_keys;          // reconstruction keys emitted
-    int sel_cnt;         // samples held by the leaves selected in this pass
-    int stale;           // leaves whose error was recomputed in this pass
-    int stale_vals;      // sample values read for them
-    unsigned carry_bits; // max error of the leaves the last adaptive pass did not split
-    int recon_overflow;  // keys counted by the last reconstruction when they exceeded the
-                         //   key buffer (then nothing was emitted), else 0
     int guard_cap;       // device-side loop: no pass starts once N + L > guard_cap (the
                          //   sample capacity when the target is at or beyond it; 0 = no
                          //   guard: a smaller target, standalone calls)
-    int cur;             // fused loop: the slot that holds the tree's state
-    LoopSlot slot[2];
+    int n_keys;          // reconstruction keys emitted
+    int recon_overflow;  // keys counted by the last reconstruction when they exceeded the
+                         //   key buffer (then nothing was emitted), else 0
+};
+// The host's mirror, with the current slot's counts by name.
+struct HostCounters : DevCounters {
+    int n_samples, n_leaves, new_samples, new_nodes;
+    void name_counts() {
+        const TreeCounts& t = slot[cur];
+        n_samples = t.N;
+        n_leaves = t.L;
+        new_samples = t.new_s;
+        new_nodes = t.new_n;
+    }
 };
 
-// Per-pass totals of the fused loop in kSuper groups of chunks, two of each by
-// pass parity: integer sums and maxima taken with atomics, each group in a
-// 128-byte line of its own (a single address would serialise thousands of
-// them), so that any wave gets a total or a prefix with one load per lane.
+// Totals of a pass in kSuper groups of chunks: integer sums and maxima taken
+// with atomics, each group in a 128-byte line of its own (a single address
+// would serialise thousands of them), so that any wave gets a total or a
+// prefix with one load per lane.
 static const int kSuper = 64;
 struct SuperSum {  // selected and split leaves, samples the selected hold
     int sel, split, held, pad[29];
 };
-struct SuperMax {  // float bits of the largest error the next pass starts from
+struct SuperMax {  // float bits of a largest error (errors are >= 0)
     unsigned err, pad[31];
 };
+static const int kMaxSets = 3;   // of SuperMax: the loop's two, by pass parity, and
+static const int kGError = 2;    //   g_error, as the last error pass left it
 
 // Per-pass statistics, one row per adaptive pass (for algorithmic byte counts):
 // leaves and samples before the pass, selected and split leaves, the samples
@@ -119,13 +121,13 @@ struct DevGrid {
     int4* sext;            // [cap_l/2+1][2] learned mode only (else null): per split the
                            //   parent's box extents with the left child's at the split axis,
                            //   the right child's extent at the axis, the axis
-    int4* part;            // [kChunkBlocks] per-workgroup (selected, split, samples, carry)
-    int2* part_off;        // [kChunkBlocks] exclusive prefix of (selected, split)
-    uint4* epart;          // [kErrBlocks] per-workgroup (max error bits, stale, values)
+    int4* part;            // [kChunkBlocks] per-workgroup (selected, split, samples held)
+    int2* part_off;        // [kChunkBlocks] exclusive prefix of the reconstruction's counts
     unsigned char* rcnt;   // [cap_l]      reconstruction tiles per leaf
     DevCounters* cnt;
     SuperSum* ssum;        // [2][kSuper]
-    SuperMax* smax;        // [2][kSuper]
+    SuperMax* smax;        // [kMaxSets][kSuper]
+    long long* lrows;      // rows offered to the learned collection so far (null: none)
     PassStat* pstats;
     int D;
     int cap_s, cap_l;
@@ -172,7 +174,8 @@ struct LearnDev {
     float* perr;         // [cap_l] plain error of each leaf (err holds the score)
     float* X;            // [cap_rows][16] collected rows: features of split leaves
     float* Y;            // [cap_rows] their labels; X == null: no collection
-    long long* rows;     // rows offered so far (index >= cap_rows: dropped)
+    long long* rows;     // rows offered so far (index >= cap_rows: dropped); the selection
+                         //   after an error pass adds its splits
     long long cap_rows;
     MlpDev mlp;          // mlp.p == null: the score is the plain error
     float ylo, yhi;      // clamp of the network output
@@ -189,8 +192,7 @@ struct Grid {
     long long max_samples = 0;
     bool initialized = false;
     DevGrid dev{};
-    DevCounters host{};  // mirror after the last synchronising call
-    float gmax_host = 0.0f;
+    HostCounters host{};  // mirror after the last synchronising call
     std::string log_path;
     // log sink (mdas_set_log_sink): each "KEY", value pair the reference
     // writes to its std::ofstream; is_count marks integral values
@@ -231,6 +233,7 @@ struct Grid {
     // thumbnail's 20 thousand leaves, 4096 nearly all empty workgroups cost
     // the selection 7.9 us a launch, 90 cost 5.0)
     int chunks() const { return std::min(chunk_blocks, cap_l / 256 + 1); }
+    int error_blocks() const { return std::min(err_blocks, cap_l / 256 + 1); }
     // learned proposal (mode bits: 1 collect rows, 2 score with the MLP)
     int learn_mode = 0;
     LearnDev learn{};
@@ -256,42 +259,41 @@ inline void kend(Grid& g, hipStream_t st) {
     if (g.krecs.back().b) (void)hipEventRecord(g.krecs.back().b, st);
 }
 
-// Launchers (k_sampling.hip)
-hipError_t launch_initial(Grid& g, int L0, hipStream_t st);
-hipError_t launch_reset_errors(Grid& g, int standalone, hipStream_t st);
-hipError_t launch_errors(Grid& g, hipStream_t st);
-hipError_t launch_errors_stale(Grid& g, hipStream_t st);
-hipError_t launch_adaptive(Grid& g, hipStream_t st);
-hipError_t launch_select(Grid& g, hipStream_t st);
-hipError_t launch_scan(Grid& g, hipStream_t st);
-hipError_t launch_place(Grid& g, hipStream_t st);
-hipError_t launch_set_limit(Grid& g, int limit, hipStream_t st);
-// The fused loop: errors of the initial leaves, then per pass one selection
-// and one placement kernel (which evaluates the new samples and the errors of
-// the children); parity alternates from 0.  launch_loop_end brings the
-// counters up to date and raises `done` at the limit.
-hipError_t launch_first_errors(Grid& g, hipStream_t st);
-hipError_t launch_fused_pass(Grid& g, const void* dparams, int n_obj, int parity, hipStream_t st);
-hipError_t launch_loop_end(Grid& g, hipStream_t st);
-hipError_t launch_arm(Grid& g, hipStream_t st);
-hipError_t launch_build_pts(Grid& g, int n_leaves, hipStream_t st);
+// Launchers (k_sampling.hip).  A pass of the device-side loop is an error
+// pass, a selection and a placement of the given parity (0, 1, 0, ..),
+// and the integrand over the new samples; the placement takes the kernels
+// after it along as its mode says.
+enum PlaceMode {
+    PLACE_ONLY = 0,    // the integrand and the children's errors follow
+    PLACE_EVAL = 1,    // evaluates its new samples
+    PLACE_ERRORS = 2,  // and the errors of the children it makes
+};
+hipError_t launch_initial(Grid& g, int L0, int limit, hipStream_t st);
+hipError_t launch_errors(Grid& g, int parity, hipStream_t st);
+hipError_t launch_select(Grid& g, int parity, hipStream_t st);
+hipError_t launch_place(Grid& g, int parity, int mode, const void* dparams, int n_obj, hipStream_t st);
 hipError_t launch_mark_last_children(Grid& g, hipStream_t st);
-hipError_t launch_mark_last_children_b(const DevGrid* grids, int n, hipStream_t st);
+// Single calls: ComputeErrors over every leaf (g_error starts from 0), and
+// AdaptiveSampling against g_error on the host's slot; arm resets what an
+// earlier loop or a refused pass left.
+hipError_t launch_arm(Grid& g, bool errors, bool adaptive, hipStream_t st);
+hipError_t launch_compute_errors(Grid& g, hipStream_t st);
+hipError_t launch_adaptive(Grid& g, hipStream_t st);
+hipError_t launch_build_pts(Grid& g, int n_leaves, hipStream_t st);
 hipError_t launch_fill_i32(int* p, int v, long long n, hipStream_t st);
 hipError_t launch_fill_f32(float* p, float v, long long n, hipStream_t st);
 
-// Batched forms over a device array of n grids of dimension D (k_sampling.hip)
+// Batched forms over a device array of n grids of dimension D, `blocks`
+// chunks per image.
 hipError_t launch_initial_b(int D, const DevGrid* grids, int n, int blocks, const int* limits,
                             hipStream_t st);
-hipError_t launch_first_errors_b(int D, const DevGrid* grids, int n, int blocks, hipStream_t st);
-hipError_t launch_fused_pass_b(int D, const DevGrid* grids, const void* const* params, int n_obj,
-                               int n, int blocks, int parity, hipStream_t st);
-// out[4 i ..]: done, status, samples, passes of image i, after the end of a
-// block of fused passes (fused != 0) or of the separate kernels.
-hipError_t launch_loop_status_b(const DevGrid* grids, int n, int fused, int* out, hipStream_t st);
-// learns: device array of n LearnDev (the learned error pass) or null (plain)
-hipError_t launch_pass_b(int D, const DevGrid* grids, int n, int blocks, hipStream_t st,
-                         const LearnDev* learns = nullptr);
+hipError_t launch_errors_b(int D, const DevGrid* grids, int n, int blocks, int parity, hipStream_t st);
+hipError_t launch_select_b(const DevGrid* grids, int n, int blocks, int parity, hipStream_t st);
+hipError_t launch_place_b(int D, const DevGrid* grids, const void* const* params, int n_obj, int n,
+                          int blocks, int parity, int mode, hipStream_t st);
+hipError_t launch_mark_last_children_b(const DevGrid* grids, int n, hipStream_t st);
+// out[4 i ..]: finished, status, samples, passes of image i.
+hipError_t launch_loop_status_b(const DevGrid* grids, int n, int* out, hipStream_t st);
 
 // Integrand (k_integrand.hip)
 // Fills the `words` words of the cells that follow a scene block.
@@ -322,9 +324,9 @@ hipError_t launch_integrate_scatter(Grid& g, float* pixels, int W, int H, hipStr
 hipError_t launch_bytes(const float* pixels, unsigned char* out, long long n, hipStream_t st);
 
 // learned proposal (k_learned.hip)
-hipError_t launch_errors_learned(Grid& g, hipStream_t st);
+hipError_t launch_errors_learned(Grid& g, int parity, hipStream_t st);
 hipError_t launch_errors_learned_b(int D, const DevGrid* grids, const LearnDev* ls, int n, int blocks,
-                                   hipStream_t st);
+                                   int parity, hipStream_t st);
 hipError_t launch_mlp_pack(float* p, unsigned short* w1p, unsigned short* w2p, float* w2r,
                            float* w3r, hipStream_t st);
 hipError_t launch_mlp_forward(const MlpDev& M, const float* X, long long n, float* Y,

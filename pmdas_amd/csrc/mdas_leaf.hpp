@@ -182,17 +182,24 @@ __device__ __forceinline__ void store_line_head2(const DevGrid& a, int i, int4 i
 // overflow it, N + L > max_samples (every leaf selected adds L samples; the
 // guard of the app's interactive loop, optixMotionBlur.cpp:723-724), so that
 // such a run ends cleanly instead of with a capacity error.
-// The error kernels of a pass test it (every workgroup reads the same
-// counters) and the reduction after them raises `done` for the rest of the
-// pass.
+// The kernels of a pass test it (every workgroup reads the same counters) and
+// the selection raises `done` for the rest of the pass.
 __device__ __forceinline__ bool loop_limit_reached(const DevCounters* c, int N, int L) {
     return N >= c->limit || (c->guard_cap != 0 && (long long)N + L > (long long)c->guard_cap);
 }
-__device__ __forceinline__ bool loop_limit_reached(const DevCounters* c) {
-    return loop_limit_reached(c, c->n_samples, c->n_leaves);
-}
-__device__ __forceinline__ bool pass_stopped(const DevCounters* c) {
-    return c->done || loop_limit_reached(c);
+__device__ __forceinline__ const TreeCounts& tree_counts(const DevCounters* c) { return c->slot[c->cur]; }
+__device__ __forceinline__ int leaf_total(const DevGrid& a) { return tree_counts(a.cnt).L; }
+
+// Workgroup maximum of m (>= 0, float) into the super group of workgroup blk.
+__device__ __forceinline__ void super_max(SuperMax* smax, float m, int blk) {
+    __shared__ float wmax[4];
+    m = wave_max(m);
+    if ((threadIdx.x & 63) == 0) wmax[threadIdx.x >> 6] = m;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        m = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
+        if (m != 0.0f) atomicMax(&smax[blk % kSuper].err, __float_as_uint(m));
+    }
 }
 
 struct LeafSamples {

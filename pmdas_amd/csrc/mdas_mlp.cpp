@@ -275,6 +275,7 @@ int mdas_set_learned(mdas_handle h, int mode, mdas_mlp_handle m, float* rows, fl
     g.learn.X = (mode & MDAS_LEARN_COLLECT) ? rows : nullptr;
     g.learn.Y = (mode & MDAS_LEARN_COLLECT) ? labels : nullptr;
     g.learn.cap_rows = (mode & MDAS_LEARN_COLLECT) ? cap_rows : 0;
+    g.dev.lrows = (mode & MDAS_LEARN_COLLECT) ? g.learn.rows : nullptr;
     g.learn.mlp = (mode & MDAS_LEARN_SCORE) ? m->dev() : mdas::MlpDev{};
     g.learn.label_mode = (mode & MDAS_LEARN_IMAGE_LABEL) ? 1 : 0;
     g.learn.keep = (mode & (MDAS_LEARN_COLLECT | MDAS_LEARN_KEEP_FEATURES)) ? 1 : 0;
