@@ -4,9 +4,9 @@
 //  1. k_recon_prep: one coalesced pass over the leaves writes a 32-byte
 //     record per leaf (xy box, mean value, volume) and counts the pixel tiles
 //     each leaf's span touches.
-//  2. k_scan_keys / k_recon_emit: every leaf emits one 64-bit key per tile,
+//  2. k_recon_emit: every leaf emits one 64-bit key per tile,
 //         key = morton2(tile_x, tile_y) << 32 | leaf index,
-//     in leaf order (a workgroup-chunked exclusive scan gives the offsets).
+//     in leaf order (offsets from the chunks' counts).
 //  3. radix_sort_keys: stable LSD radix sort (digits of up to 10 bits,
 //     LDS-staged scatter) on the Morton bits only; since keys are emitted in leaf order
 //     the result is the total 64-bit order.
@@ -26,6 +26,8 @@
 
 namespace mdas {
 
+static const int kReconChunks = 4096;  // most leaf chunks of the record and key kernels
+static int recon_chunks(const Grid& g) { return std::min(g.chunks(), kReconChunks); }
 static const int kSortBlocks = 1024;
 static const int kSortMaxBits = 10;  // digit width limit (histograms of 1024 bins)
 static const int kSortKeysPerThread = 16;  // scatter tile: 4096 keys staged in LDS (8192: slower)
@@ -65,6 +67,10 @@ __device__ __forceinline__ int tiles_of(int x0, int x1, int y0, int y1, const Re
     if (x0 >= x1 || y0 >= y1) return 0;
     return ((x1 - 1) / G.TW - x0 / G.TW + 1) * ((y1 - 1) / G.TH - y0 / G.TH + 1);
 }
+
+// Keys counted by each of the reconstruction's chunks (the passes' partials are
+// free between passes).
+__device__ __forceinline__ int* key_counts(const DevGrid& a) { return reinterpret_cast<int*>(a.part); }
 
 // Record of leaf i: q0 = (mn0, mx0, mn1, mx1), q1 = (mean value, volume).
 // The mean is the slot-order sum times 1/n (kdgrid.cu:510-518,
@@ -116,55 +122,53 @@ __global__ __launch_bounds__(256) void k_recon_prep(DevGrid a, ReconGeo G, float
     c = wave_sum(c);
     if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = c;
     __syncthreads();
-    if (threadIdx.x == 0) a.part[blockIdx.x] = make_int4(red[0] + red[1] + red[2] + red[3], 0, 0, 0);
+    if (threadIdx.x == 0) key_counts(a)[blockIdx.x] = red[0] + red[1] + red[2] + red[3];
 }
 
-// Exclusive scan of part[].x into part_off[].x; total -> cnt->n_keys.  A
-// total beyond the key buffer (cap_keys) is recorded in recon_overflow and
-// leaves n_keys = 0, so that no later kernel reads or writes past the buffer.
-__global__ __launch_bounds__(1024) void k_scan_keys(DevGrid a, int G, long long cap_keys) {
-    __shared__ int ls[16];
-    const int per = (G + 1023) / 1024;
-    const int g0 = threadIdx.x * per;
-    int s = 0;
-    for (int k = 0; k < per; ++k)
-        if (g0 + k < G) s += a.part[g0 + k].x;
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    int x = s;
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        int y = __shfl_up(x, o, 64);
-        if (lane >= o) x += y;
+// Total of the counted keys -> n_keys.  A total beyond the key buffer
+// (cap_keys) is recorded in recon_overflow and leaves n_keys = 0, so that no
+// later kernel reads or writes past the buffer.
+__device__ __forceinline__ bool keys_fit(const DevGrid& a, int total, long long cap_keys, bool lead) {
+    const bool over = (long long)total > cap_keys;
+    if (lead) {
+        a.cnt->n_keys = over ? 0 : total;
+        a.cnt->recon_overflow = over ? total : 0;
     }
-    if (lane == 63) ls[w] = x;
-    __syncthreads();
-    int p = 0, t = 0;
-    for (int k = 0; k < 16; ++k) {
-        if (k < w) p += ls[k];
-        t += ls[k];
-    }
-    int r = p + x - s;
-    for (int k = 0; k < per; ++k)
-        if (g0 + k < G) {
-            int c = a.part[g0 + k].x;
-            a.part_off[g0 + k] = make_int2(r, 0);
-            r += c;
-        }
-    if (threadIdx.x == 0) {
-        const bool over = (long long)t > cap_keys;
-        a.cnt->n_keys = over ? 0 : t;
-        a.cnt->recon_overflow = over ? t : 0;
-    }
+    return !over;
 }
-
-__global__ __launch_bounds__(256) void k_recon_emit(DevGrid a, ReconGeo G, const float4* rrec,
-                                                    unsigned long long* keys) {
+// For a host that sizes the buffers from the count.
+__global__ __launch_bounds__(256) void k_count_keys(DevGrid a, int chunks) {
     __shared__ int lds[4];
+    int c = 0, total;
+    for (int k = threadIdx.x; k < chunks; k += 256) c += key_counts(a)[k];
+    block_exscan(c, lds, total);
+    keys_fit(a, total, 0x7fffffff, threadIdx.x == 0);
+}
+
+// Every workgroup sums the chunks' counts for itself (at most kReconChunks, 16
+// coalesced loads a thread: about 1 us in place of a scan kernel of 7 and its
+// launch).  Also clears the tiles' ranges (n_tiles entries each) for
+// k_tile_ranges.
+__global__ __launch_bounds__(256) void k_recon_emit(DevGrid a, ReconGeo G, const float4* rrec,
+                                                    unsigned long long* keys, long long cap_keys,
+                                                    int* tstart, int* tend, int n_tiles) {
+    __shared__ int lds[4];
+    for (int t = blockIdx.x * 256 + threadIdx.x; t < n_tiles; t += gridDim.x * 256) tstart[t] = tend[t] = 0;
     const int L = leaf_total(a);
-    if (a.cnt->recon_overflow != 0) return;  // the keys do not fit the buffer
-    int beg, end;
+    int beg, end, base, first_end;
     chunk_range(L, gridDim.x, blockIdx.x, beg, end);
-    int base = a.part_off[blockIdx.x].x;
+    if (beg >= end && blockIdx.x > 0) return;
+    chunk_range(L, gridDim.x, 0, base, first_end);
+    const int chunks = first_end > 0 ? (L + first_end - 1) / first_end : 0;  // those that hold leaves
+    int before = 0, after = 0, total;
+    for (int k = threadIdx.x; k < chunks; k += 256) {
+        const int c = key_counts(a)[k];
+        before += k < (int)blockIdx.x ? c : 0;
+        after += k < (int)blockIdx.x ? 0 : c;
+    }
+    block_exscan(before, lds, base);
+    block_exscan(after, lds, total);
+    if (!keys_fit(a, base + total, cap_keys, blockIdx.x == 0 && threadIdx.x == 0)) return;
     for (int t0 = beg; t0 < end; t0 += 256) {
         const int i = t0 + threadIdx.x;
         int x0 = 0, x1 = 0, y0 = 0, y1 = 0, c = 0;
@@ -172,7 +176,6 @@ __global__ __launch_bounds__(256) void k_recon_emit(DevGrid a, ReconGeo G, const
             record_span(rrec[(size_t)i * 2], G, x0, x1, y0, y1);
             c = tiles_of(x0, x1, y0, y1, G);
         }
-        int total;
         int off = base + block_exscan(c, lds, total);
         if (c > 0) {
             for (int ty = y0 / G.TH; ty <= (y1 - 1) / G.TH; ++ty)
@@ -184,8 +187,8 @@ __global__ __launch_bounds__(256) void k_recon_emit(DevGrid a, ReconGeo G, const
 }
 
 // ---------------------------------------------------------- device scan --
-// Exclusive scan of n <= 1024*1024 unsigned ints in place: block sums, a
-// scan of the block sums, then the block-local scans with their offsets.
+// Exclusive scan of n <= 1024*1024 unsigned ints in place: block sums, then the
+// block-local scans with their offsets.
 __device__ __forceinline__ unsigned block_scan_u32(unsigned v, unsigned* ls, unsigned& total) {
     const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
     unsigned x = v;
@@ -214,20 +217,15 @@ __global__ __launch_bounds__(1024) void k_scan_reduce(const unsigned* data, int 
     if (threadIdx.x == 0) sums[blockIdx.x] = total;
 }
 
-__global__ __launch_bounds__(1024) void k_scan_top(unsigned* sums, int nb) {
-    __shared__ unsigned ls[16];
-    unsigned total;
-    const unsigned v = threadIdx.x < (unsigned)nb ? sums[threadIdx.x] : 0u;
-    const unsigned ex = block_scan_u32(v, ls, total);
-    if (threadIdx.x < (unsigned)nb) sums[threadIdx.x] = ex;
-}
-
+// Every workgroup adds up the block sums before its own (at most 1024, one
+// load a thread).
 __global__ __launch_bounds__(1024) void k_scan_down(unsigned* data, int n, const unsigned* sums) {
     __shared__ unsigned ls[16];
     const int i = blockIdx.x * 1024 + threadIdx.x;
-    unsigned total;
+    unsigned before, total;
+    (void)block_scan_u32(threadIdx.x < blockIdx.x ? sums[threadIdx.x] : 0u, ls, before);
     const unsigned ex = block_scan_u32(i < n ? data[i] : 0u, ls, total);
-    if (i < n) data[i] = ex + sums[blockIdx.x];
+    if (i < n) data[i] = before + ex;
 }
 
 // ------------------------------------------------------------ radix sort --
@@ -235,10 +233,13 @@ __global__ __launch_bounds__(1024) void k_scan_down(unsigned* data, int n, const
 // pass, BITS chosen per sort so the Morton bits take as few passes as
 // possible (at most 10 bits a pass).  Reduce-then-scan: per-workgroup digit
 // histograms, one exclusive scan over (digit, workgroup), then a scatter in
-// which every workgroup ranks a tile of 4096 keys by digit with wave ballots
-// (16 sub-tiles of 256), stages the tile in LDS in digit order and writes each
-// digit run contiguously -- runs of 8 keys on average at 512 digits, where a
-// 256-key tile would leave most keys alone in their line.
+// which every workgroup ranks a tile of up to 4096 keys by digit, stages it in
+// LDS in digit order and writes each digit run contiguously -- runs of 8 keys
+// on average at 512 digits, where a 256-key tile would leave most keys alone
+// in their line.  A wave ranks its quarter of the tile, 64 keys at a time, by
+// ballots against counters of its own; the waves meet once per tile (meeting
+// three times per 256 keys, as before, made the ranking the larger part:
+// 26 M keys in 8-bit passes 139 -> 115 us each, 1 M keys 16.8 -> 9.0).
 template <int BITS>
 __global__ __launch_bounds__(256) void k_rs_hist(const unsigned long long* keys, const int* n_ptr,
                                                  int shift, unsigned* hist) {
@@ -263,60 +264,57 @@ __global__ __launch_bounds__(256) void k_rs_scatter(const unsigned long long* in
     constexpr int R = NB > 256 ? NB / 256 : 1;  // digits per thread in the tile scan
     constexpr int KPT = kSortKeysPerThread;
     constexpr int TILE = 256 * KPT;
-    __shared__ unsigned base[NB];
-    __shared__ int wcnt[4][NB];
-    __shared__ int run[NB];   // keys of each digit in the tile's earlier sub-tiles
-    __shared__ int toff[NB];
+    __shared__ unsigned base[NB];   // where the workgroup's next key of a digit goes
+    __shared__ int wcnt[4][NB];     // keys of a digit per wave, then its offset in the tile
+    __shared__ int toff[NB];        // the digit's offset in the tile
     __shared__ int scr[4];
     __shared__ unsigned long long stage[TILE];
     const int n = *n_ptr;
-    const int w = threadIdx.x >> 6;
-    for (int d = threadIdx.x; d < NB; d += 256) base[d] = hist[d * gridDim.x + blockIdx.x];
+    const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
     int beg, end;
     chunk_range(n, gridDim.x, blockIdx.x, beg, end);
+    if (beg >= end) return;
+    for (int d = threadIdx.x; d < NB; d += 256) base[d] = hist[d * gridDim.x + blockIdx.x];
     for (int t0 = beg; t0 < end; t0 += TILE) {
-        // sub-tile s holds keys t0 + 256 s + thread; their loads go out together
+        const int nvalid = min(TILE, end - t0);
+        const int subs = (nvalid + 255) / 256;      // rounds of 64 keys per wave
+        const int first = w * subs * 64 + lane;     // this lane's key of round s: first + 64 s
         unsigned long long k[KPT];
 #pragma unroll
-        for (int s = 0; s < KPT; ++s) {
-            const int i = t0 + s * 256 + threadIdx.x;
-            k[s] = i < end ? in[i] : 0ull;
-        }
-        for (int d = threadIdx.x; d < NB; d += 256) run[d] = 0;
-        // rank of each key among the tile's keys of its digit, in input
-        // order: earlier sub-tiles, then lower waves, then lower lanes
+        for (int s = 0; s < KPT; ++s)
+            k[s] = s < subs && first + 64 * s < nvalid ? in[t0 + first + 64 * s] : 0ull;
+        for (int q = 0; q < 4; ++q)
+            for (int d = threadIdx.x; d < NB; d += 256) wcnt[q][d] = 0;
+        __syncthreads();
+        // rank of each key among the wave's keys of its digit, in input order
         int rk[KPT];
 #pragma unroll
         for (int s = 0; s < KPT; ++s) {
-            const bool valid = t0 + s * 256 + (int)threadIdx.x < end;
-            const unsigned d = (unsigned)(k[s] >> shift) & (unsigned)(NB - 1);
-            for (int q = 0; q < 4; ++q)
-                for (int dd = threadIdx.x; dd < NB; dd += 256) wcnt[q][dd] = 0;
-            __syncthreads();
-            unsigned long long m = __ballot(valid);
+            if (s < subs) {  // uniform
+                const bool valid = first + 64 * s < nvalid;
+                const unsigned d = (unsigned)(k[s] >> shift) & (unsigned)(NB - 1);
+                unsigned long long m = __ballot(valid);
 #pragma unroll
-            for (int b = 0; b < BITS; ++b) {
-                const bool bit = (d >> b) & 1u;
-                const unsigned long long bal = __ballot(bit);
-                m &= bit ? bal : ~bal;
+                for (int b = 0; b < BITS; ++b) {
+                    const bool bit = (d >> b) & 1u;
+                    const unsigned long long bal = __ballot(bit);
+                    m &= bit ? bal : ~bal;
+                }
+                const int below = lanes_below(m), before = wcnt[w][d];
+                rk[s] = before + below;
+                wave_sync_lds();
+                if (valid && below == 0) wcnt[w][d] = before + __popcll(m);
+                wave_sync_lds();
             }
-            const int rw = lanes_below(m);
-            if (valid && rw == 0) wcnt[w][d] = __popcll(m);
-            __syncthreads();
-            int pre = run[d];
-            for (int q = 0; q < w; ++q) pre += wcnt[q][d];
-            rk[s] = pre + rw;
-            __syncthreads();
-            for (int dd = threadIdx.x; dd < NB; dd += 256)
-                run[dd] += wcnt[0][dd] + wcnt[1][dd] + wcnt[2][dd] + wcnt[3][dd];
         }
         __syncthreads();
+        // offsets of the digits in the tile, then of each wave's keys
         {
             int loc[R], sum = 0;
 #pragma unroll
             for (int r = 0; r < R; ++r) {
                 const int dd = (int)threadIdx.x * R + r;
-                loc[r] = dd < NB ? run[dd] : 0;
+                loc[r] = dd < NB ? wcnt[0][dd] + wcnt[1][dd] + wcnt[2][dd] + wcnt[3][dd] : 0;
                 sum += loc[r];
             }
             int all;
@@ -326,6 +324,12 @@ __global__ __launch_bounds__(256) void k_rs_scatter(const unsigned long long* in
                 const int dd = (int)threadIdx.x * R + r;
                 if (dd < NB) {
                     toff[dd] = ex;
+                    int o = ex;
+                    for (int q = 0; q < 4; ++q) {
+                        const int c = wcnt[q][dd];
+                        wcnt[q][dd] = o;
+                        o += c;
+                    }
                     ex += loc[r];
                 }
             }
@@ -333,52 +337,59 @@ __global__ __launch_bounds__(256) void k_rs_scatter(const unsigned long long* in
         __syncthreads();
 #pragma unroll
         for (int s = 0; s < KPT; ++s) {
-            if (t0 + s * 256 + (int)threadIdx.x < end) {
+            if (s < subs && first + 64 * s < nvalid) {
                 const unsigned d = (unsigned)(k[s] >> shift) & (unsigned)(NB - 1);
-                stage[toff[d] + rk[s]] = k[s];
+                stage[wcnt[w][d] + rk[s]] = k[s];
             }
         }
         __syncthreads();
         // the tile in digit order: each digit's run goes to its own range
-        const int nvalid = min(TILE, end - t0);
         for (int p = threadIdx.x; p < nvalid; p += 256) {
             const unsigned long long kk = stage[p];
             const unsigned dd = (unsigned)(kk >> shift) & (unsigned)(NB - 1);
             out[base[dd] + (p - toff[dd])] = kk;
         }
         __syncthreads();
-        for (int dd = threadIdx.x; dd < NB; dd += 256) base[dd] += run[dd];
+        for (int dd = threadIdx.x; dd < NB; dd += 256)
+            base[dd] += (dd + 1 < NB ? toff[dd + 1] : nvalid) - toff[dd];
         __syncthreads();
     }
+}
+
+// Workgroups of the sort: half a tile of the expected keys each (a leaf is in
+// 1.1 to 1.5 tiles), at most kSortBlocks; the kernels take any number of keys.
+static int sort_blocks(long long leaves, long long bound) {
+    const long long keys = std::min(leaves + leaves / 2, bound);
+    return (int)std::max<long long>(1, std::min<long long>(kSortBlocks, (keys + 2047) / 2048));
 }
 
 static void scan_u32(unsigned* data, int n, unsigned* sums, hipStream_t st) {
     const int nb = (n + 1023) / 1024;
     hipLaunchKernelGGL(k_scan_reduce, dim3(nb), dim3(1024), 0, st, data, n, sums);
-    hipLaunchKernelGGL(k_scan_top, dim3(1), dim3(1024), 0, st, sums, nb);
     hipLaunchKernelGGL(k_scan_down, dim3(nb), dim3(1024), 0, st, data, n, sums);
 }
 
 template <int BITS>
 static void sort_pass(Grid& g, unsigned* rs_hist, const unsigned long long* a, unsigned long long* b,
-                      int sh, hipStream_t st) {
+                      int sh, int blocks, hipStream_t st) {
     const int* n_ptr = &g.dev.cnt->n_keys;
-    const int nh = (1 << BITS) * kSortBlocks;
+    const int nh = (1 << BITS) * blocks;
     kbeg(g, st, "k_rs_hist");
-    hipLaunchKernelGGL(k_rs_hist<BITS>, dim3(kSortBlocks), dim3(256), 0, st, a, n_ptr, sh, rs_hist);
+    hipLaunchKernelGGL(k_rs_hist<BITS>, dim3(blocks), dim3(256), 0, st, a, n_ptr, sh, rs_hist);
     kend(g, st);
     kbeg(g, st, "k_rs_scan");
     scan_u32(rs_hist, nh, rs_hist + nh, st);
     kend(g, st);
     kbeg(g, st, "k_rs_scatter");
-    hipLaunchKernelGGL(k_rs_scatter<BITS>, dim3(kSortBlocks), dim3(256), 0, st, a, b, n_ptr, sh,
+    hipLaunchKernelGGL(k_rs_scatter<BITS>, dim3(blocks), dim3(256), 0, st, a, b, n_ptr, sh,
                        rs_hist);
     kend(g, st);
 }
 
 // Sorts keys[0, n) by bits [lo, hi) in ceil((hi - lo) / 10) passes of equal
 // digit width; returns the buffer holding the result.
-static unsigned long long* radix_sort_keys(Grid& g, ReconBufs& rb, int lo, int hi, hipStream_t st) {
+static unsigned long long* radix_sort_keys(Grid& g, ReconBufs& rb, int lo, int hi, long long bound,
+                                           hipStream_t st) {
     unsigned long long* a = rb.keys;
     unsigned long long* b = rb.keys_alt;
     g.recon_sort_passes = 0;
@@ -386,15 +397,16 @@ static unsigned long long* radix_sort_keys(Grid& g, ReconBufs& rb, int lo, int h
     if (total <= 0) return a;
     const int passes = (total + kSortMaxBits - 1) / kSortMaxBits;
     const int bits = max(4, (total + passes - 1) / passes);
+    const int blocks = sort_blocks(g.host.n_leaves, bound);
     for (int sh = lo; sh < hi; sh += bits) {
         switch (bits) {
-        case 4: sort_pass<4>(g, rb.rs_hist, a, b, sh, st); break;
-        case 5: sort_pass<5>(g, rb.rs_hist, a, b, sh, st); break;
-        case 6: sort_pass<6>(g, rb.rs_hist, a, b, sh, st); break;
-        case 7: sort_pass<7>(g, rb.rs_hist, a, b, sh, st); break;
-        case 8: sort_pass<8>(g, rb.rs_hist, a, b, sh, st); break;
-        case 9: sort_pass<9>(g, rb.rs_hist, a, b, sh, st); break;
-        default: sort_pass<10>(g, rb.rs_hist, a, b, sh, st); break;
+        case 4: sort_pass<4>(g, rb.rs_hist, a, b, sh, blocks, st); break;
+        case 5: sort_pass<5>(g, rb.rs_hist, a, b, sh, blocks, st); break;
+        case 6: sort_pass<6>(g, rb.rs_hist, a, b, sh, blocks, st); break;
+        case 7: sort_pass<7>(g, rb.rs_hist, a, b, sh, blocks, st); break;
+        case 8: sort_pass<8>(g, rb.rs_hist, a, b, sh, blocks, st); break;
+        case 9: sort_pass<9>(g, rb.rs_hist, a, b, sh, blocks, st); break;
+        default: sort_pass<10>(g, rb.rs_hist, a, b, sh, blocks, st); break;
         }
         g.recon_sort_passes++;
         g.recon_sort_bits = bits;
@@ -770,15 +782,12 @@ hipError_t recon_prepare(Grid& g, int W, int H, hipStream_t st) {
     ReconGeo G = make_geo(g, W, H);
     g.recon_pixels = (long long)W * H;
     kbeg(g, st, "k_recon_prep");
-    MDAS_DISPATCH_D(g.D, hipLaunchKernelGGL(k_recon_prep<DD>, dim3(g.chunks()), dim3(256), 0, st,
+    MDAS_DISPATCH_D(g.D, hipLaunchKernelGGL(k_recon_prep<DD>, dim3(recon_chunks(g)), dim3(256), 0, st,
                                             g.dev, G, g.rb.rrec));
-    kend(g, st);
-    kbeg(g, st, "k_scan_keys");
-    hipLaunchKernelGGL(k_scan_keys, dim3(1), dim3(1024), 0, st, g.dev, g.chunks(),
-                       g.recon_bounded ? g.rb.keys_cap : (long long)0x7fffffff);
     kend(g, st);
     if (!g.recon_bounded) {
         int nk = 0;
+        hipLaunchKernelGGL(k_count_keys, dim3(1), dim3(256), 0, st, g.dev, recon_chunks(g));
         e = hipMemcpyAsync(&nk, &g.dev.cnt->n_keys, sizeof(int), hipMemcpyDeviceToHost, st);
         if (e == hipSuccess) e = hipStreamSynchronize(st);
         if (e != hipSuccess) return e;
@@ -795,21 +804,23 @@ hipError_t recon_prepare(Grid& g, int W, int H, hipStream_t st) {
 static hipError_t recon_finish(Grid& g, ReconBufs& rb, float* pixels, int W, int H, hipStream_t st,
                                hipEvent_t ev_sort0, hipEvent_t ev_sort1) {
     ReconGeo G = make_geo(g, W, H);
+    const long long tiles = 1ll << (2 * G.tbits);
     kbeg(g, st, "k_recon_emit");
-    hipLaunchKernelGGL(k_recon_emit, dim3(g.chunks()), dim3(256), 0, st, g.dev, G, rb.rrec, rb.keys);
+    hipLaunchKernelGGL(k_recon_emit, dim3(recon_chunks(g)), dim3(256), 0, st, g.dev, G, rb.rrec, rb.keys, rb.keys_cap,
+                       rb.tile_start, rb.tile_end, (int)tiles);
     kend(g, st);
+    // keys there can be: the bound, or the buffers where they were sized from
+    // the count
+    const long long bound = std::min(key_bound(g, G), rb.keys_cap);
     if (ev_sort0) (void)hipEventRecord(ev_sort0, st);
     // the sorted keys end in keys or keys_alt by the parity of the pass
     // count; the buffers keep their roles, so a captured graph stays valid
-    unsigned long long* sorted = radix_sort_keys(g, rb, 32, 32 + 2 * G.tbits, st);
+    unsigned long long* sorted = radix_sort_keys(g, rb, 32, 32 + 2 * G.tbits, bound, st);
     g.keys_sorted = sorted;
     if (ev_sort1) (void)hipEventRecord(ev_sort1, st);
-    const long long tiles = 1ll << (2 * G.tbits);
     kbeg(g, st, "k_tile_ranges");
-    launch_fill_i32(rb.tile_start, 0, tiles, st);
-    launch_fill_i32(rb.tile_end, 0, tiles, st);
-    int blocks = (int)std::min<long long>((rb.keys_cap + 255) / 256, 8192);  // grid-stride over
-    if (blocks < 1) blocks = 1;                                              // the device count
+    int blocks = (int)std::min<long long>((bound + 255) / 256, 8192);  // grid-stride over
+    if (blocks < 1) blocks = 1;                                        // the device count
     hipLaunchKernelGGL(k_tile_ranges, dim3(blocks), dim3(256), 0, st, sorted, &g.dev.cnt->n_keys,
                        rb.tile_start, rb.tile_end);
     kend(g, st);
@@ -839,9 +850,8 @@ hipError_t launch_integrate_gather(Grid& g, float* pixels, int W, int H, hipStre
 hipError_t recon_on_buffers(Grid& g, ReconBufs& rb, float* pixels, int W, int H, hipStream_t st) {
     ReconGeo G = make_geo(g, W, H);
     g.recon_pixels = (long long)W * H;
-    MDAS_DISPATCH_D(g.D, hipLaunchKernelGGL(k_recon_prep<DD>, dim3(g.chunks()), dim3(256), 0, st,
+    MDAS_DISPATCH_D(g.D, hipLaunchKernelGGL(k_recon_prep<DD>, dim3(recon_chunks(g)), dim3(256), 0, st,
                                             g.dev, G, rb.rrec));
-    hipLaunchKernelGGL(k_scan_keys, dim3(1), dim3(1024), 0, st, g.dev, g.chunks(), rb.keys_cap);
     return recon_finish(g, rb, pixels, W, H, st, nullptr, nullptr);
 }
 

@@ -99,8 +99,9 @@ __global__ __launch_bounds__(256) void k_initial_b(const DevGrid* grids) {
 // total zero, the loop's limit (and the capacity as its guard when the limit
 // is the capacity; below it a pass that would overflow is an error).
 __device__ __forceinline__ void initial_counters_body(const DevGrid& a, int L0, int limit) {
-    if (threadIdx.x < 2 * kSuper) a.ssum[threadIdx.x].sel = a.ssum[threadIdx.x].split = a.ssum[threadIdx.x].held = 0;
-    if (threadIdx.x < kMaxSets * kSuper) a.smax[threadIdx.x].err = 0u;
+    if (threadIdx.x < kSumSets * kSuper)
+        a.ssum[threadIdx.x].sel = a.ssum[threadIdx.x].split = a.ssum[threadIdx.x].held = 0;
+    a.smax[threadIdx.x].err = 0u;
     if (threadIdx.x != 0) return;
     DevCounters* c = a.cnt;
     c->cur = 0;
@@ -220,8 +221,6 @@ __global__ __launch_bounds__(256) void k_errors_b(const DevGrid* grids, int par)
 __device__ __forceinline__ int live_chunks(int L, int n) {
     return min(n, max(min((L + 255) / 256, 1024), L / 512));
 }
-// Chunks per super group, for `chunks` in all.
-__device__ __forceinline__ int super_size(int chunks) { return (chunks + kSuper - 1) / kSuper; }
 
 // kdgrid.cu:316-326.  Per leaf: the seed (tea4(i,0) when unset), one draw u,
 // selected iff pow(err / g_error, alpha) >= u.  A selected full leaf splits.
@@ -831,9 +830,6 @@ __global__ __launch_bounds__(256) void k_build_pts(DevGrid a, int L) {
 }
 
 // --------------------------------------------------------------- fills --
-__global__ void k_fill_i32(int* p, int v, long long n) {
-    for (long long i = blockIdx.x * 256ll + threadIdx.x; i < n; i += (long long)gridDim.x * 256) p[i] = v;
-}
 __global__ void k_fill_f32(float* p, float v, long long n) {
     for (long long i = blockIdx.x * 256ll + threadIdx.x; i < n; i += (long long)gridDim.x * 256) p[i] = v;
 }
@@ -919,11 +915,6 @@ hipError_t launch_build_pts(Grid& g, int n_leaves, hipStream_t st) {
     if (n_leaves <= 0) return hipSuccess;
     const int blocks = grid_for(n_leaves, 4096);
     MDAS_DISPATCH_D(g.D, hipLaunchKernelGGL(k_build_pts<DD>, dim3(blocks), dim3(256), 0, st, g.dev, n_leaves));
-    return hipGetLastError();
-}
-
-hipError_t launch_fill_i32(int* p, int v, long long n, hipStream_t st) {
-    hipLaunchKernelGGL(k_fill_i32, dim3(grid_for(n)), dim3(256), 0, st, p, v, n);
     return hipGetLastError();
 }
 

@@ -56,7 +56,7 @@ void free_grid(Grid& g) {
     mdas::DevGrid& d = g.dev;
     mdas::ReconBufs& rb = g.rb;
     void* ptrs[] = {d.coords,   d.values,  d.leaf,        d.err,        d.seed,     d.flags,
-                    d.xpts,     d.split_list, d.sdat,     d.sext,       d.part,     d.part_off,
+                    d.xpts,     d.split_list, d.sdat,     d.sext,       d.part,
                     d.cnt,      d.ssum,    d.smax,        d.pstats,      rb.rrec,      rb.keys,    rb.keys_alt,
                     rb.tile_start, rb.tile_end, rb.rs_hist, g.d_scalar, g.learn.feat, g.learn.perr,
                     g.learn.rows};
@@ -235,9 +235,8 @@ int mdas_create(const mdas_config* cfg, mdas_handle* out) {
     if (e == hipSuccess) e = dalloc(&d.split_list, cl);
     if (e == hipSuccess) e = dalloc(&d.sdat, 2 * (cl / 2 + 1));  // splits per pass <= cap_l / 2
     if (e == hipSuccess) e = dalloc(&d.part, (size_t)mdas::kChunkBlocks);
-    if (e == hipSuccess) e = dalloc(&d.part_off, (size_t)mdas::kChunkBlocks);
     if (e == hipSuccess) e = dalloc(&d.cnt, 1);
-    if (e == hipSuccess) e = dalloc(&d.ssum, (size_t)(2 * mdas::kSuper));
+    if (e == hipSuccess) e = dalloc(&d.ssum, (size_t)(mdas::kSumSets * mdas::kSuper));
     if (e == hipSuccess) e = dalloc(&d.smax, (size_t)(mdas::kMaxSets * mdas::kSuper));
     if (e == hipSuccess) e = dalloc(&d.pstats, (size_t)mdas::kMaxPassStats);
     if (e == hipSuccess) e = dalloc(&g.d_scalar, 64);
@@ -247,6 +246,7 @@ int mdas_create(const mdas_config* cfg, mdas_handle* out) {
         return fail(MDAS_ERR_HIP, std::string("device allocation failed: ") + hipGetErrorString(e));
     }
     e = hipMemset(d.cnt, 0, sizeof(mdas::DevCounters));
+    if (e == hipSuccess) e = hipMemset(d.ssum, 0, sizeof(mdas::SuperSum) * mdas::kSumSets * mdas::kSuper);
     if (e == hipSuccess) e = hipMemset(d.smax, 0, sizeof(mdas::SuperMax) * mdas::kMaxSets * mdas::kSuper);
     if (e == hipSuccess) e = hipMemset(d.values, 0, sizeof(float) * cs * 3);
     // overflow rows start as -1 slots (a stale slot is then -1 or an index
@@ -571,7 +571,7 @@ int mdas_upload_state(mdas_handle h, int n, int l, const float* coords, const fl
     std::vector<mdas::SuperMax> sm((size_t)(mdas::kMaxSets * mdas::kSuper), mdas::SuperMax{});
     memcpy(&sm[(size_t)(mdas::kGError * mdas::kSuper)].err, &max_error, 4);
     HIP_TRY(hipMemcpy(g.dev.smax, sm.data(), sizeof(mdas::SuperMax) * sm.size(), hipMemcpyHostToDevice));
-    HIP_TRY(hipMemset(g.dev.ssum, 0, sizeof(mdas::SuperSum) * 2 * mdas::kSuper));
+    HIP_TRY(hipMemset(g.dev.ssum, 0, sizeof(mdas::SuperSum) * mdas::kSumSets * mdas::kSuper));
     mdas::HostCounters c{};
     c.slot[0] = mdas::TreeCounts{n, l, 0, 0, 0, 0};
     c.limit = 0x7fffffff;
@@ -934,7 +934,6 @@ static double kernel_bytes(const Grid& g, const std::string& k) {
     const double L = (double)g.host.n_leaves, N = (double)g.host.n_samples;
     const double K = (double)g.host.n_keys;
     if (k == "k_recon_prep") return L * (SB + 32.0) + 12.0 * N;
-    if (k == "k_scan_keys") return (16.0 + 8.0) * g.chunks();
     if (k == "k_recon_emit") return L * 16.0 + K * 8.0;
     if (k == "k_rs_hist") return K * 8.0 * g.recon_sort_passes;
     if (k == "k_rs_scan") return 3.0 * 4.0 * (1 << g.recon_sort_bits) * 1024 * g.recon_sort_passes;
@@ -978,7 +977,7 @@ int mdas_get_phase_times(mdas_handle h, mdas_phase_times* o) {
     o->bytes_errors = kernel_bytes(g, "k_errors");
     o->bytes_adaptive = kernel_bytes(g, "k_select") + kernel_bytes(g, "k_place");
     double br = 0.0;
-    for (const char* k : {"k_recon_prep", "k_scan_keys", "k_recon_emit", "k_rs_hist", "k_rs_scan",
+    for (const char* k : {"k_recon_prep", "k_recon_emit", "k_rs_hist", "k_rs_scan",
                           "k_rs_scatter", "k_tile_ranges", "k_gather"})
         br += kernel_bytes(g, k);
     o->bytes_recon = br;

@@ -55,6 +55,7 @@ struct SuperSum {  // selected and split leaves, samples the selected hold
 struct SuperMax {  // float bits of a largest error (errors are >= 0)
     unsigned err, pad[31];
 };
+static const int kSumSets = 2;   // of SuperSum, by pass parity
 static const int kMaxSets = 3;   // of SuperMax: the loop's two, by pass parity, and
 static const int kGError = 2;    //   g_error, as the last error pass left it
 
@@ -122,10 +123,9 @@ struct DevGrid {
                            //   parent's box extents with the left child's at the split axis,
                            //   the right child's extent at the axis, the axis
     int4* part;            // [kChunkBlocks] per-workgroup (selected, split, samples held)
-    int2* part_off;        // [kChunkBlocks] exclusive prefix of the reconstruction's counts
     unsigned char* rcnt;   // [cap_l]      reconstruction tiles per leaf
     DevCounters* cnt;
-    SuperSum* ssum;        // [2][kSuper]
+    SuperSum* ssum;        // [kSumSets][kSuper]
     SuperMax* smax;        // [kMaxSets][kSuper]
     long long* lrows;      // rows offered to the learned collection so far (null: none)
     PassStat* pstats;
@@ -280,7 +280,6 @@ hipError_t launch_arm(Grid& g, bool errors, bool adaptive, hipStream_t st);
 hipError_t launch_compute_errors(Grid& g, hipStream_t st);
 hipError_t launch_adaptive(Grid& g, hipStream_t st);
 hipError_t launch_build_pts(Grid& g, int n_leaves, hipStream_t st);
-hipError_t launch_fill_i32(int* p, int v, long long n, hipStream_t st);
 hipError_t launch_fill_f32(float* p, float v, long long n, hipStream_t st);
 
 // Batched forms over a device array of n grids of dimension D, `blocks`

@@ -190,6 +190,9 @@ __device__ __forceinline__ bool loop_limit_reached(const DevCounters* c, int N, 
 __device__ __forceinline__ const TreeCounts& tree_counts(const DevCounters* c) { return c->slot[c->cur]; }
 __device__ __forceinline__ int leaf_total(const DevGrid& a) { return tree_counts(a.cnt).L; }
 
+// Chunks per super group, for `chunks` in all.
+__device__ __forceinline__ int super_size(int chunks) { return (chunks + kSuper - 1) / kSuper; }
+
 // Workgroup maximum of m (>= 0, float) into the super group of workgroup blk.
 __device__ __forceinline__ void super_max(SuperMax* smax, float m, int blk) {
     __shared__ float wmax[4];

@@ -180,6 +180,23 @@ def test_integrate_long_tiles(mdas, tile, b, e):
         assert np.array_equal(g.integrate_image(w, h).view(np.uint32), o.integrate(w, h).view(np.uint32))
 
 
+# The sort's digit widths (4 to 10 bits, one to three passes: the image's tiles)
+# against key counts from one to several tiles of 4096 keys per workgroup.
+@pytest.mark.parametrize("grid", [(1, 1, 1), (8, 8, 1), (16, 16, 4), (96, 64, 8)])
+@pytest.mark.parametrize("size", [(8, 8), (16, 8), (40, 24), (64, 64), (128, 64), (128, 128), (256, 128),
+                                  (256, 256), (300, 170), (513, 512), (1100, 600)])
+def test_recon_sort_widths(mdas, grid, size):
+    sw, sh, spp = grid
+    _say(f"sort grid={grid} size={size}")
+    g, o, sc, target = _make(mdas, 2, 4, 0, 1, sw, sh, spp, 0.25, 2)
+    g.Run(sc, target)
+    o.run(sc.params_bytes(), target)
+    tile = (8, 8) if max(size) < 512 else (4, 4)
+    g.set_recon_tile(*tile)
+    assert np.array_equal(g.integrate_image(*size).view(np.uint32), o.integrate(*size).view(np.uint32))
+    assert np.array_equal(g.recon_keys(), o.recon_keys(*size, *tile))
+
+
 def test_integrate_other_resolution(mdas):
     """Pixel grid finer and coarser than the sample space (scaleFactor != 1)."""
     g, o, sc, target = _make(mdas, 2, 4, 1, 2, 40, 30, 8, 0.25, 4)
