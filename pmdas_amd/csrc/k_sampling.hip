@@ -592,9 +592,10 @@ __device__ __forceinline__ void place_leaf(const DevGrid& a, int i, int k, int m
 // Where chunk blk's new samples and right children start (base: ranks among
 // all selected and split leaves), from the super groups and the partials of
 // its own group; every wave computes it for itself.  False if the pass would
-// exceed the capacity.  One thread writes the next slot, the pass's
-// statistics and the totals' zeros for the pass after (no kernel of this pass
-// reads those).
+// exceed the capacity.  One thread writes the next slot, a wave the totals' zeros
+// for the pass after (no kernel of this pass reads those) and the pass's
+// statistics, into the host's memory: the host knows before the placement
+// itself whether another pass follows.
 __device__ __forceinline__ bool pass_offsets(const DevGrid& a, int blk, int nblk, int par, int& L,
                                               int& N, int2& base) {
     DevCounters* cn = a.cnt;
@@ -607,7 +608,19 @@ __device__ __forceinline__ bool pass_offsets(const DevGrid& a, int blk, int nblk
     const int sel = wave_sum(t.sel), split = wave_sum(t.split);
     const bool fits = (long long)N + sel <= a.cap_s && (long long)L + split <= a.cap_l;
     if (blk == 0 && threadIdx.x < kSuper) {
-        const int held = wave_sum(t.held);
+        const int held = wave_sum(t.held), P = cn->passes;
+        // leaves whose errors were estimated since the last pass, and the
+        // values that took: the initial leaves, then the children
+        const int stale = P == 0 ? L : 2 * s.new_n, vals = P == 0 ? 4 * L : 5 * s.new_n;
+        if (lane < kPassWords) {
+            const int w[kPassWords] = {L, N, sel, split, held, stale, vals, fits ? 0 : MDAS_ERR_CAPACITY_DEV};
+            int v = 0;
+#pragma unroll
+            for (int q = 0; q < kPassWords; ++q) v = lane == q ? w[q] : v;
+            __hip_atomic_store(&a.hrun->row[P & (kHostRows - 1)][lane],
+                               ((unsigned long long)(a.htag + (unsigned)P) << 32) | (unsigned)v, __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_SYSTEM);
+        }
         if (fits) {
             SuperSum& z = a.ssum[(par ^ 1) * kSuper + lane];
             z.sel = z.split = z.held = 0;
@@ -618,11 +631,6 @@ __device__ __forceinline__ bool pass_offsets(const DevGrid& a, int blk, int nblk
                 cn->status = MDAS_ERR_CAPACITY_DEV;
                 cn->done = 1;
             } else {
-                const int P = cn->passes;
-                // leaves whose errors were estimated since the last pass, and
-                // the values that took: the initial leaves, then the children
-                const int stale = P == 0 ? L : 2 * s.new_n, vals = P == 0 ? 4 * L : 5 * s.new_n;
-                a.pstats[P & (kMaxPassStats - 1)] = PassStat{L, N, sel, split, held, stale, vals, 0};
                 cn->passes = P + 1;
                 cn->slot[par ^ 1] = TreeCounts{N + sel, L + split, N, L, sel, split};
                 cn->cur = par ^ 1;
@@ -793,12 +801,17 @@ __global__ void k_loop_status_b(const DevGrid* grids, int n, int* out) {
 
 // After the device-side loop: when it stopped at its limit, no error pass
 // followed the last placement, so its split children get the stale marker
-// (error -1, kdgrid.cu:466-469) the placement left out.  Raises `done`.
+// (error -1, kdgrid.cu:466-469) the placement left out.  Raises `done`, and
+// leaves the counters to the host.
 __device__ __forceinline__ void mark_last_children_body(const DevGrid& a, int blk, int nblk) {
     DevCounters* c = a.cnt;
     const TreeCounts s = tree_counts(c);
-    if (c->status != 0 || !loop_limit_reached(c, s.N, s.L)) return;
-    if (blk == 0 && threadIdx.x == 0) c->done = 1;
+    const bool stopped = c->status == 0 && loop_limit_reached(c, s.N, s.L);
+    if (blk == 0 && threadIdx.x == 0) {
+        if (stopped) c->done = 1;
+        a.hrun->cnt = *c;
+    }
+    if (!stopped) return;
     for (int t = blk * 256 + threadIdx.x; t < s.new_n; t += nblk * 256) {
         a.err[a.split_list[t]] = -1.0f;
         a.err[s.L_old + t] = -1.0f;

@@ -12,6 +12,7 @@
 #include <cmath>
 #include <fstream>
 #include <string>
+#include <thread>
 #include <vector>
 
 #include "mdas_handles.hpp"
@@ -57,17 +58,17 @@ void free_grid(Grid& g) {
     mdas::ReconBufs& rb = g.rb;
     void* ptrs[] = {d.coords,   d.values,  d.leaf,        d.err,        d.seed,     d.flags,
                     d.xpts,     d.split_list, d.sdat,     d.sext,       d.part,
-                    d.cnt,      d.ssum,    d.smax,        d.pstats,      rb.rrec,      rb.keys,    rb.keys_alt,
-                    rb.tile_start, rb.tile_end, rb.rs_hist, g.d_scalar, g.learn.feat, g.learn.perr,
+                    d.ssum,           rb.rrec,      rb.keys,    rb.keys_alt,
+                    rb.tile_start, rb.tile_end, rb.rs_hist, g.learn.feat, g.learn.perr,
                     g.learn.rows};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
+    if (d.hrun) (void)hipHostFree(d.hrun);
     for (hipEvent_t e : g.evpool) (void)hipEventDestroy(e);
     g.evpool.clear();
     d = mdas::DevGrid{};
     rb = mdas::ReconBufs{};
     g.keys_sorted = nullptr;
-    g.d_scalar = nullptr;
     g.learn = mdas::LearnDev{};
     g.learn_mode = 0;
 }
@@ -78,6 +79,50 @@ int sync_counters(Grid& g, hipStream_t st) {
     HIP_TRY(hipStreamSynchronize(st));
     g.host.name_counts();
     return MDAS_OK;
+}
+
+// The passes launched meanwhile are waited for by their tags (those of a run
+// that ends early are not used again either) and, in a loop, leave out the
+// stale markers.
+struct AwaitedPasses {
+    Grid& g;
+    int launched = 0;
+    AwaitedPasses(Grid& x, bool loop) : g(x) {
+        g.dev.in_loop = loop ? 1 : 0;
+        g.dev.htag = mdas::kRunTag | g.next_tag;
+    }
+    AwaitedPasses(const AwaitedPasses&) = delete;
+    AwaitedPasses& operator=(const AwaitedPasses&) = delete;
+    ~AwaitedPasses() {
+        g.dev.in_loop = 0;
+        g.next_tag = (g.next_tag + (unsigned)launched) & ~mdas::kRunTag;
+    }
+};
+
+// Waits for the row of pass p (every pass launched writes one unless the
+// stream fails).
+hipError_t wait_for_row(const Grid& g, int p, hipStream_t st, mdas::PassStat* out) {
+    const unsigned tag = g.dev.htag + (unsigned)p;
+    const unsigned long long* row = g.dev.hrun->row[p & (mdas::kHostRows - 1)];
+    int w[mdas::kPassWords];
+    auto whole = [&] {
+        for (int q = 0; q < mdas::kPassWords; ++q) {
+            const unsigned long long v = __atomic_load_n(&row[q], __ATOMIC_RELAXED);
+            if ((unsigned)(v >> 32) != tag) return false;
+            w[q] = (int)(unsigned)v;
+        }
+        memcpy(out, w, sizeof(w));
+        return true;
+    };
+    for (unsigned n = 1; !whole(); ++n) {
+        if (n % 4096 == 0) {  // the stream may have failed
+            const hipError_t e = hipStreamQuery(st);
+            if (e == hipSuccess) return whole() ? hipSuccess : hipErrorUnknown;
+            if (e != hipErrorNotReady) return e;
+        }
+        if (n % 64 == 0) std::this_thread::yield();
+    }
+    return hipSuccess;
 }
 
 // One "KEY\nvalue" pair as the reference writes it (kdgrid.cu:670-671,
@@ -166,18 +211,18 @@ namespace mdas {
 int set_error(int code, const std::string& msg) { return fail(code, msg); }
 void initial_extents(Grid& g) { set_initial_extents(g); }
 int sync_grid(Grid& g, hipStream_t st) { return sync_counters(g, st); }
-int drain_pass_stats(Grid& g, bool all) {
-    const int have = (int)g.pstats_host.size(), done = g.host.passes;
-    if (done <= have || (!all && done - have < kMaxPassStats / 2)) return MDAS_OK;
-    g.pstats_host.resize((size_t)done);
-    for (int p = have; p < done;) {  // contiguous stretches of the ring
-        const int r = p & (kMaxPassStats - 1);
-        const int n = std::min(done - p, kMaxPassStats - r);
-        HIP_TRY(hipMemcpy(&g.pstats_host[(size_t)p], g.dev.pstats + r, sizeof(PassStat) * (size_t)n,
-                          hipMemcpyDeviceToHost));
-        p += n;
+void take_counters(Grid& g) {
+    static_cast<mdas::DevCounters&>(g.host) = g.dev.hrun->cnt;
+    g.host.name_counts();
+}
+void take_pass_rows(Grid& g, int done) {
+    for (int p = (int)g.pstats_host.size(); p < done; ++p) {
+        int w[kPassWords];
+        for (int q = 0; q < kPassWords; ++q) w[q] = (int)(unsigned)g.dev.hrun->row[p & (kHostRows - 1)][q];
+        PassStat ps;
+        memcpy(&ps, w, sizeof(ps));
+        g.pstats_host.push_back(ps);
     }
-    return MDAS_OK;
 }
 }  // namespace mdas
 
@@ -235,19 +280,21 @@ int mdas_create(const mdas_config* cfg, mdas_handle* out) {
     if (e == hipSuccess) e = dalloc(&d.split_list, cl);
     if (e == hipSuccess) e = dalloc(&d.sdat, 2 * (cl / 2 + 1));  // splits per pass <= cap_l / 2
     if (e == hipSuccess) e = dalloc(&d.part, (size_t)mdas::kChunkBlocks);
-    if (e == hipSuccess) e = dalloc(&d.cnt, 1);
-    if (e == hipSuccess) e = dalloc(&d.ssum, (size_t)(mdas::kSumSets * mdas::kSuper));
-    if (e == hipSuccess) e = dalloc(&d.smax, (size_t)(mdas::kMaxSets * mdas::kSuper));
-    if (e == hipSuccess) e = dalloc(&d.pstats, (size_t)mdas::kMaxPassStats);
-    if (e == hipSuccess) e = dalloc(&g.d_scalar, 64);
+    mdas::DevTotals* totals = nullptr;
+    if (e == hipSuccess) e = dalloc(&totals, 1);
+    if (e == hipSuccess) e = hipHostMalloc((void**)&d.hrun, sizeof(mdas::HostRun), hipHostMallocCoherent);
+    if (totals) {
+        d.ssum = totals->ssum;  // the allocation's first bytes
+        d.smax = totals->smax;
+        d.cnt = &totals->cnt;
+    }
     if (e != hipSuccess) {
         free_grid(g);
         delete h;
         return fail(MDAS_ERR_HIP, std::string("device allocation failed: ") + hipGetErrorString(e));
     }
-    e = hipMemset(d.cnt, 0, sizeof(mdas::DevCounters));
-    if (e == hipSuccess) e = hipMemset(d.ssum, 0, sizeof(mdas::SuperSum) * mdas::kSumSets * mdas::kSuper);
-    if (e == hipSuccess) e = hipMemset(d.smax, 0, sizeof(mdas::SuperMax) * mdas::kMaxSets * mdas::kSuper);
+    memset(static_cast<void*>(d.hrun), 0, sizeof(mdas::HostRun));  // no row has a run's tag
+    e = hipMemset(totals, 0, sizeof(mdas::DevTotals));
     if (e == hipSuccess) e = hipMemset(d.values, 0, sizeof(float) * cs * 3);
     // overflow rows start as -1 slots (a stale slot is then -1 or an index
     // written before, never garbage)
@@ -337,9 +384,26 @@ static int adaptive_sampling(Grid& g, bool armed, hipStream_t st) {
         HIP_TRY(hipEventRecord(ev.e[0], st));
     }
     if (!armed) HIP_TRY(mdas::launch_arm(g, false, true, st));
-    HIP_TRY(mdas::launch_adaptive(g, st));
-    int rc = sync_counters(g, st);  // kdgrid.cu:753-759 reads the counters back
-    if (rc) return rc;
+    // kdgrid.cu:753-759 reads the counters back; here the pass has sent them
+    mdas::PassStat ps;
+    {
+        AwaitedPasses passes(g, false);
+        const int p = g.host.passes;  // its number in the tree, by which its row goes
+        passes.launched = p + 1;
+        HIP_TRY(mdas::launch_adaptive(g, st));
+        HIP_TRY(hipStreamSynchronize(st));
+        HIP_TRY(wait_for_row(g, p, st, &ps));
+    }
+    if (ps.status == 0) {
+        g.host.cur ^= 1;
+        g.host.slot[g.host.cur] = mdas::TreeCounts{ps.N + ps.sel, ps.L + ps.split, ps.N, ps.L, ps.sel, ps.split};
+        g.host.passes++;
+        g.host.done = g.host.status = 0;
+        g.host.name_counts();
+    } else {
+        int rc = sync_counters(g, st);
+        if (rc) return rc;
+    }
     if (g.host.status != 0) {
         int s = g.host.status;
         // clear the device error so that the grid stays usable
@@ -777,7 +841,7 @@ int mdas_run(mdas_handle h, mdas_scene_handle s, long long target, void* stream)
     hipStream_t st = S(stream);
     const int L0 = 1 << (g.b * g.D + 2 * g.e);
     const long long limit = std::min<long long>(target, g.max_samples);
-    const int B = std::max(2, g.passes_per_sync & ~1);  // even: the fused passes alternate
+    const int B = g.passes_per_check;
     // the log needs per-pass times: logging times the run like mdas_set_timing
     const bool logging = g.logging();
     const bool timing_was = g.timing;
@@ -800,67 +864,74 @@ int mdas_run(mdas_handle h, mdas_scene_handle s, long long target, void* stream)
     mdas::kbeg(g, st, "k_eval");
     HIP_TRY(mdas::launch_eval(g, s->dev, 0, 4 * L0, false, st));
     mdas::kend(g, st);
-    long long last_n = -1;  // samples after the last block of passes
+    long long last_n = -1;  // samples at the last test for progress
     // every timed launch in order (name, ms); folded after each block, so the
     // event pool holds one block's events however many passes the run takes
     std::vector<std::pair<std::string, double>> seq;
-    struct LoopMode {  // the pass kernels of this loop skip the stale markers
-        mdas::DevGrid& d;
-        explicit LoopMode(mdas::DevGrid& x) : d(x) { d.in_loop = 1; }
-        ~LoopMode() { d.in_loop = 0; }
-    } loop_mode{g.dev};
+    AwaitedPasses passes(g, true);
     // The placement takes the integrand along and, for the plain method, the
     // children's errors (the learned error pass is a kernel of its own);
     // timing and logs want the phases apart.  The results are the same.
     const int mode = g.timing ? mdas::PLACE_ONLY : (g.learn_mode ? mdas::PLACE_EVAL : mdas::PLACE_ERRORS);
-    bool errors_taken = false;  // by the placement before
-    for (;;) {
-        for (int b = 0; b < B; ++b) {
-            const int par = b & 1;
-            if (!errors_taken) {
-                mdas::kbeg(g, st, "k_errors");
-                HIP_TRY(g.learn_mode ? mdas::launch_errors_learned(g, par, st) : mdas::launch_errors(g, par, st));
-                mdas::kend(g, st);
-                errors_taken = mode == mdas::PLACE_ERRORS;
-            }
-            mdas::kbeg(g, st, "k_select");
-            HIP_TRY(mdas::launch_select(g, par, st));
+    // The counts after a pass are known, and with its row here, when its
+    // placement begins; the next pass is launched behind the placement, without
+    // a wait for it and only if there is to be one.  (Four passes and a
+    // synchronising copy of the counters in turn left the card idle for 20 us
+    // each time, and ran up to three passes that found the limit reached: 64x48
+    // in 12 passes 409 -> 307 us, 3D 256x256 in 32 695 -> 600, 1080p 5D 14.20 ->
+    // 14.12 ms.)
+    long long N = 4LL * L0, L = L0;
+    const long long guard = limit >= g.cap_s ? g.cap_s : 0;
+    int status = MDAS_OK;
+    for (int p = 0; N < limit && (guard == 0 || N + L <= guard); ++p) {
+        const int par = p & 1;
+        if (p == 0 || mode != mdas::PLACE_ERRORS) {  // else the placement before took them
+            mdas::kbeg(g, st, "k_errors");
+            HIP_TRY(g.learn_mode ? mdas::launch_errors_learned(g, par, st) : mdas::launch_errors(g, par, st));
             mdas::kend(g, st);
-            mdas::kbeg(g, st, "k_place");
-            HIP_TRY(mdas::launch_place(g, par, mode, s->dev, s->host.n_obj, st));
-            mdas::kend(g, st);
-            if (mode == mdas::PLACE_ONLY) {
-                mdas::kbeg(g, st, "k_eval");
-                HIP_TRY(mdas::launch_eval(g, s->dev, 0, 0, true, st));
-                mdas::kend(g, st);
-            }
         }
-        int rc = sync_counters(g, st);
-        if (rc == MDAS_OK) rc = mdas::drain_pass_stats(g, false);
-        if (rc) return rc;
-        if (g.timing) collect_kernel_times(g, logging ? &seq : nullptr);
-        // the stopping rule, as the next pass's kernels would find it
-        if (g.host.done || g.host.status || g.host.n_samples >= g.host.limit ||
-            (g.host.guard_cap != 0 && (long long)g.host.n_samples + g.host.n_leaves > (long long)g.host.guard_cap))
-            break;
+        mdas::kbeg(g, st, "k_select");
+        HIP_TRY(mdas::launch_select(g, par, st));
+        mdas::kend(g, st);
+        passes.launched = p + 1;
+        mdas::kbeg(g, st, "k_place");
+        HIP_TRY(mdas::launch_place(g, par, mode, s->dev, s->host.n_obj, st));
+        mdas::kend(g, st);
+        if (mode == mdas::PLACE_ONLY) {
+            mdas::kbeg(g, st, "k_eval");
+            HIP_TRY(mdas::launch_eval(g, s->dev, 0, 0, true, st));
+            mdas::kend(g, st);
+        }
+        mdas::PassStat ps;
+        HIP_TRY(wait_for_row(g, p, st, &ps));
+        status = ps.status;
+        if (status) break;
+        g.pstats_host.push_back(ps);
+        N = (long long)ps.N + ps.sel;
+        L = (long long)ps.L + ps.split;
+        if ((p + 1) % B) continue;
+        if (g.timing) {
+            HIP_TRY(hipStreamSynchronize(st));
+            collect_kernel_times(g, logging ? &seq : nullptr);
+        }
         // every pass selects the leaf of maximum error (its ratio is 1), so
-        // each block adds samples and the loop ends at the limit; a block that
-        // adds none means no leaf passed the selection test: the maximum error
+        // the passes add samples and the loop ends at the limit; passes that
+        // add none mean no leaf passed the selection test: the maximum error
         // is not finite (e.g. a NaN integrand) or zero (scores that underflow)
-        if (g.host.n_samples == last_n)
-            return fail(MDAS_ERR_STATE, "a block of passes added no sample (no leaf selected: "
-                                        "non-finite or zero maximum error)");
-        last_n = g.host.n_samples;
+        if (N == last_n) break;
+        last_n = N;
     }
+    const bool stuck = status == MDAS_OK && N < limit && (guard == 0 || N + L <= guard);
     mdas::kbeg(g, st, "k_mark_last");
     HIP_TRY(mdas::launch_mark_last_children(g, st));
     mdas::kend(g, st);
+    HIP_TRY(hipStreamSynchronize(st));
+    mdas::take_counters(g);
+    if (stuck)
+        return fail(MDAS_ERR_STATE, "a block of passes added no sample (no leaf selected: "
+                                    "non-finite or zero maximum error)");
     g.passes = g.host.passes;
     collect_kernel_times(g, logging ? &seq : nullptr);
-    {
-        int rc = mdas::drain_pass_stats(g, true);
-        if (rc) return rc;
-    }
     if (logging && seq.size() >= 2) {
         // the app's and the library's keys in the order they write them
         // (kdgrid.cu:670-671, 713, 769-770; optixMotionBlur.cpp:774, 788):

@@ -24,7 +24,7 @@ struct Group {
     mdas::DevGrid* d_grids = nullptr;    // device copies of the descriptors
     const void** d_params = nullptr;     // device array of scene parameter blocks
     int* d_limits = nullptr;
-    int* d_status = nullptr;             // (done, status, samples, passes) per member
+    int* status = nullptr;               // pinned: (done, status, samples, passes) per member
     mdas::LearnDev* d_learn = nullptr;   // per member, when any member is in learned mode
     int blocks = 0;
     int max_chunks = 1;                  // chunks the largest member's capacity fills
@@ -104,6 +104,15 @@ hipError_t leave_stream(mdas_batch* b, hipStream_t st) {
     return e;
 }
 
+// The host's mirror of every image's counters, where a run ends in an error.
+int sync_all(mdas_batch* b, hipStream_t st) {
+    for (mdas_handle h : b->grids) {
+        const int rc = mdas::sync_grid(h->g, st);
+        if (rc) return rc;
+    }
+    return MDAS_OK;
+}
+
 void drop_recon_graph(mdas_batch* b) {
     if (b->recon_exec) (void)hipGraphExecDestroy(b->recon_exec);
     if (b->recon_graph) (void)hipGraphDestroy(b->recon_graph);
@@ -149,6 +158,7 @@ int mdas_batch_create(mdas_handle* grids, mdas_scene_handle* scenes, int n, mdas
         for (int k = 0; k < m; ++k) {
             dg[k] = grids[gr.members[k]]->g.dev;
             dg[k].in_loop = 1;  // batches only run the device-side loop
+            dg[k].htag = 0;
             dp[k] = scenes[gr.members[k]]->dev;
             dl[k] = grids[gr.members[k]]->g.learn;  // feat == null: plain error for this member
             learned = learned || grids[gr.members[k]]->g.learn_mode != 0;
@@ -156,7 +166,7 @@ int mdas_batch_create(mdas_handle* grids, mdas_scene_handle* scenes, int n, mdas
         hipError_t e = hipMalloc(&gr.d_grids, sizeof(mdas::DevGrid) * m);
         if (e == hipSuccess) e = hipMalloc((void**)&gr.d_params, sizeof(void*) * m);
         if (e == hipSuccess) e = hipMalloc(&gr.d_limits, sizeof(int) * m);
-        if (e == hipSuccess) e = hipMalloc(&gr.d_status, sizeof(int) * 4 * m);
+        if (e == hipSuccess) e = hipHostMalloc((void**)&gr.status, sizeof(int) * 4 * m, hipHostMallocCoherent);
         if (e == hipSuccess) e = hipMemcpy(gr.d_grids, dg.data(), sizeof(mdas::DevGrid) * m, hipMemcpyHostToDevice);
         if (e == hipSuccess) e = hipMemcpy(gr.d_params, dp.data(), sizeof(void*) * m, hipMemcpyHostToDevice);
         if (e == hipSuccess && learned) e = hipMalloc(&gr.d_learn, sizeof(mdas::LearnDev) * m);
@@ -181,7 +191,7 @@ int mdas_batch_destroy(mdas_batch_handle b) {
         if (g.d_grids) (void)hipFree(g.d_grids);
         if (g.d_params) (void)hipFree((void*)g.d_params);
         if (g.d_limits) (void)hipFree(g.d_limits);
-        if (g.d_status) (void)hipFree(g.d_status);
+        if (g.status) (void)hipHostFree(g.status);
         if (g.d_learn) (void)hipFree(g.d_learn);
     }
     drop_recon_graph(b);
@@ -246,7 +256,7 @@ int mdas_batch_run(mdas_batch_handle b, const long long* targets, void* stream, 
             } else {
                 for (int p = 0; p < B; ++p) B_TRY(g.pass(p, st));
             }
-            B_TRY(mdas::launch_loop_status_b(g.d_grids, m, g.d_status, st));
+            B_TRY(mdas::launch_loop_status_b(g.d_grids, m, g.status, st));
         }
         ++blocks_run;
         B_TRY(hipStreamSynchronize(st));
@@ -255,29 +265,29 @@ int mdas_batch_run(mdas_batch_handle b, const long long* targets, void* stream, 
             if (finished[gi]) continue;
             Group& g = b->groups[gi];
             const int m = (int)g.members.size();
-            std::vector<int> s(4 * m);
-            B_TRY(hipMemcpy(s.data(), g.d_status, sizeof(int) * 4 * m, hipMemcpyDeviceToHost));
+            const int* s = g.status;
             bool done = true;
             for (int k = 0; k < m; ++k) {
                 if (s[4 * k + 1] != 0) {
-                    finished[gi] = 1;
+                    const int rc = sync_all(b, st);
+                    if (rc) return rc;
                     return mdas::set_error(s[4 * k + 1], "image " + std::to_string(g.members[k]) +
                                                              ": adaptive pass would exceed max_samples");
                 }
                 // every pass selects the leaf of maximum error, so a block of
                 // passes that adds no sample means the errors are not finite
                 int& prev = last_n[g.members[k]];
-                if (s[4 * k] == 0 && s[4 * k + 2] == prev)
+                if (s[4 * k] == 0 && s[4 * k + 2] == prev) {
+                    const int rc = sync_all(b, st);
+                    if (rc) return rc;
                     return mdas::set_error(MDAS_ERR_STATE, "image " + std::to_string(g.members[k]) +
                                                                ": a block of passes added no sample "
                                                                "(no leaf selected: non-finite or zero "
                                                                "maximum error)");
+                }
                 prev = s[4 * k + 2];
                 done = done && s[4 * k] != 0;
-                mdas::Grid& gk = b->grids[g.members[k]]->g;  // rows before the ring wraps
-                gk.host.passes = s[4 * k + 3];
-                const int rc = mdas::drain_pass_stats(gk, false);
-                if (rc) return rc;
+                mdas::take_pass_rows(b->grids[g.members[k]]->g, s[4 * k + 3]);
             }
             finished[gi] = done ? 1 : 0;
             all = all && done;
@@ -286,13 +296,11 @@ int mdas_batch_run(mdas_batch_handle b, const long long* targets, void* stream, 
     }
     for (Group& g : b->groups)
         B_TRY(mdas::launch_mark_last_children_b(g.d_grids, (int)g.members.size(), st));
+    B_TRY(hipStreamSynchronize(st));
     for (int i = 0; i < n; ++i) {
         mdas::Grid& gg = b->grids[i]->g;
-        int rc = mdas::sync_grid(gg, st);
-        if (rc) return rc;
+        mdas::take_counters(gg);
         gg.passes = gg.host.passes;
-        rc = mdas::drain_pass_stats(gg, true);
-        if (rc) return rc;
     }
     B_TRY(leave_stream(b, st));
     b->last_ms = std::chrono::duration<double, std::milli>(std::chrono::steady_clock::now() - t0).count();

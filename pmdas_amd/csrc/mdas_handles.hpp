@@ -22,8 +22,9 @@ int set_error(int code, const std::string& msg);
 int sync_grid(Grid& g, hipStream_t st);
 // The largest leaf extents of a fresh initial grid (after initial sampling).
 void initial_extents(Grid& g);
-// Appends the per-pass rows written since the last drain (g.host.passes must
-// be current) to g.pstats_host; unless `all`, only once half the device ring
-// is pending, so that a short run copies its rows once, at its end.
-int drain_pass_stats(Grid& g, bool all);
+// What a run's last kernel left of the counters, once it has finished.
+void take_counters(Grid& g);
+// Appends the rows of the passes before `done`, which have finished, to
+// g.pstats_host (at most kHostRows of them since the last call).
+void take_pass_rows(Grid& g, int done);
 }  // namespace mdas

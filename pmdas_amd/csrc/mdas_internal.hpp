@@ -64,8 +64,28 @@ static const int kGError = 2;    //   g_error, as the last error pass left it
 // held by the selected leaves, the stale leaves whose error was recomputed
 // and the sample values those read.
 struct PassStat {
-    int L, N, sel, split, selcnt, stale, stale_vals, pad;
+    int L, N, sel, split, selcnt, stale, stale_vals, status;
 };
+
+// A grid's counters and totals, one allocation.
+struct DevTotals {
+    SuperSum ssum[kSumSets * kSuper];
+    SuperMax smax[kMaxSets * kSuper];
+    DevCounters cnt;
+};
+
+// What the host reads of a grid without a copy: pinned memory that the kernels
+// write.  A pass's row is the words of its PassStat (the last one its status),
+// each with the pass's tag in its upper half, so that a row is whole once every
+// word has the tag, in whatever order they arrive.
+static const int kPassWords = sizeof(PassStat) / sizeof(int);
+static const int kHostRows = 256;  // rows in turn; the host takes them before they wrap
+struct HostRun {
+    unsigned long long row[kHostRows][kPassWords];
+    DevCounters cnt;  // as the last kernel of a run leaves them
+};
+static const unsigned kRunTag = 0x80000000u;  // set in the tags that a host waits for: those of a
+                                              // batch's passes, which nothing waits for, stay below
 
 // One timed kernel launch (HIP events on the launching stream).
 struct KRec {
@@ -75,8 +95,6 @@ struct KRec {
 
 static const int kChunkBlocks = 32768;  // max workgroups of the chunked leaf kernels
 static const int kErrBlocks = 8192;     // max workgroups of the error kernels
-static const int kMaxPassStats = 4096;  // device ring of per-pass rows (a power of two); the
-                                        // host drains it before it wraps
 
 // Leaf lines.  Each leaf owns one aligned 128-byte line (kLineFloats floats):
 // its sample slots, the box (mn[0..D-1], mx[0..D-1]) and the points of its
@@ -123,12 +141,12 @@ struct DevGrid {
                            //   parent's box extents with the left child's at the split axis,
                            //   the right child's extent at the axis, the axis
     int4* part;            // [kChunkBlocks] per-workgroup (selected, split, samples held)
-    unsigned char* rcnt;   // [cap_l]      reconstruction tiles per leaf
     DevCounters* cnt;
     SuperSum* ssum;        // [kSumSets][kSuper]
     SuperMax* smax;        // [kMaxSets][kSuper]
     long long* lrows;      // rows offered to the learned collection so far (null: none)
-    PassStat* pstats;
+    HostRun* hrun;         // pinned
+    unsigned htag;         // tag of the run's first pass
     int D;
     int cap_s, cap_l;
     int cand;
@@ -193,6 +211,7 @@ struct Grid {
     bool initialized = false;
     DevGrid dev{};
     HostCounters host{};  // mirror after the last synchronising call
+    unsigned next_tag = 0;    // of the next pass that the host waits for: no two share one
     std::string log_path;
     // log sink (mdas_set_log_sink): each "KEY", value pair the reference
     // writes to its std::ofstream; is_count marks integral values
@@ -207,7 +226,6 @@ struct Grid {
     // largest leaf extent along x and y (sample-space units): the initial cell's,
     // which splits only shrink, or the largest of an uploaded state's boxes
     double ext_x = 0.0, ext_y = 0.0;
-    int* d_scalar = nullptr;      // small device scratch
     // timing: per-kernel events when enabled
     bool timing = false;
     std::vector<KRec> krecs;
@@ -221,7 +239,7 @@ struct Grid {
     std::vector<KStat> kstats;
     double t_initial = 0, t_errors = 0, t_adaptive = 0, t_integrand = 0, t_recon = 0, t_sort = 0;
     int passes = 0;
-    int passes_per_sync = 4;
+    int passes_per_check = 4;  // passes of mdas_run between its tests for progress
     std::vector<PassStat> pstats_host;
     long long recon_pixels = 0;
     int recon_sort_passes = 0;

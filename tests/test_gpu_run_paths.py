@@ -2,7 +2,8 @@
 apart (no timing, no log, no learned mode) and through one kernel per phase
 otherwise.  Both leave the same tree, counters and statistics, also where a
 pass is refused for capacity, where the initial grid already meets the
-target, and for the single calls that follow a run."""
+target, and for the single calls that follow a run.  The passes' statistics
+come in rows that the kernels write to the host, in turn."""
 import numpy as np
 import pytest
 
@@ -83,3 +84,31 @@ def test_both_paths_agree(mdas, case):
     assert np.array_equal(out[0][2], out[1][2])
     for i, when in enumerate(("run", "after")):
         _equal(out[0][0][i], out[1][0][i], when)
+
+
+@pytest.mark.parametrize("target", [4, 5, 1000, 4000])
+def test_rows_of_runs_batches_and_single_passes(mdas, target):
+    """From no pass at all to more passes than there are rows (256), on one
+    grid by turns: a batch leaves the rows a run leaves, and single passes and
+    another run after either see their own."""
+    args = (3, 8000, 4, 0, 0, 1.0, 1.0, 1.0)
+    sc = mdas.Scene(1, 3, 3, 1.0, 1.0)
+    a, b = mdas.KDGrid(*args), mdas.KDGrid(*args)
+    batch = mdas.Batch([b], [sc])
+    for turn in range(3):
+        passes = a.Run(sc, target)
+        batch.run([target])
+        rows = a.pass_stats(max_rows=passes + 1)
+        assert rows.shape[0] == passes and (passes > 256 or target < 4000)
+        assert np.array_equal(rows, b.pass_stats(max_rows=passes + 1))
+        assert np.array_equal(rows[1:, 1], rows[:-1, 1] + rows[:-1, 2])
+        assert a.GetNumberOfSamples() == (rows[-1, 1] + rows[-1, 2] if passes else 4)
+        for _ in range(turn):
+            for g in (a, b):
+                g.SamplingPass()
+                g.EvalNewSamples(sc)
+            assert a.GetNewSamples() == b.GetNewSamples() > 0
+        _equal(a.download_state(), b.download_state(), (target, turn))
+    batch.close()
+    for x in (a, b, sc):
+        x.close()
