@@ -8,8 +8,7 @@
 // group tests over all spheres: the 5D 1080p run's 41 launches 7.53 -> 2.79 ms,
 // a launch for the ~500 samples of a thumbnail's pass 38 -> 10 us, the FP64
 // ground truth at 240x135, 64 samples per pixel 2.28 -> 0.49 ms.
-#include "mdas_device.hpp"
-#include "mdas_internal.hpp"
+#include "mdas_leaf.hpp"
 #include "scenes.hpp"
 
 #pragma clang fp contract(off)
@@ -65,10 +64,11 @@ __global__ __launch_bounds__(256) void k_eval(const float* __restrict__ coords,
     eval_body(coords, values, dim, B, first, count, cnt, dev_range, blockIdx.x, gridDim.x);
 }
 
-__global__ __launch_bounds__(256) void k_eval_b(const DevGrid* grids, const void* const* params) {
-    const DevGrid& a = grids[blockIdx.y];
-    eval_body(a.coords, a.values, a.D, (const mscene::SceneBlock*)params[blockIdx.y], 0, 0, a.cnt,
-              1, blockIdx.x, gridDim.x);
+__global__ __launch_bounds__(256) void k_eval_b(const DevGrid* __restrict__ grids,
+                                                const void* const* __restrict__ params) {
+    const DevGrid a = batch_grid(grids);
+    eval_body(a.coords, a.values, a.D, in_constant((const mscene::SceneBlock*)params[blockIdx.y]), 0, 0,
+              a.cnt, 1, blockIdx.x, gridDim.x);
 }
 
 // The words of a scene's cells (scenes.hpp), once per scene: a wave per word,

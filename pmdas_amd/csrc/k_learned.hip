@@ -291,7 +291,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) voi
 template <int D>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4, 4))) void k_errors_learned_b(
     const DevGrid* grids, const LearnDev* ls, int par) {
-    errors_learned_body<D>(grids[blockIdx.y], ls[blockIdx.y], blockIdx.x, gridDim.x, par);
+    errors_learned_body<D>(batch_grid(grids), *in_constant(ls + blockIdx.y), blockIdx.x, gridDim.x, par);
 }
 
 hipError_t launch_errors_learned(Grid& g, int parity, hipStream_t st) {

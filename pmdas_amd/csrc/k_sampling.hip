@@ -90,8 +90,8 @@ __global__ __launch_bounds__(256) void k_initial(DevGrid a, int L0) {
 // Batched form: image blockIdx.y of the set, initial leaf count from its
 // configuration.
 template <int D>
-__global__ __launch_bounds__(256) void k_initial_b(const DevGrid* grids) {
-    const DevGrid a = grids[blockIdx.y];
+__global__ __launch_bounds__(256) void k_initial_b(const DevGrid* __restrict__ grids) {
+    const DevGrid a = batch_grid(grids);
     initial_body<D>(a, 1 << (a.b * D + 2 * a.e), blockIdx.x, gridDim.x);
 }
 
@@ -206,8 +206,8 @@ __global__ __launch_bounds__(256) void k_errors(DevGrid a, int par) {
     errors_body<D>(a, blockIdx.x, gridDim.x, par);
 }
 template <int D>
-__global__ __launch_bounds__(256) void k_errors_b(const DevGrid* grids, int par) {
-    const DevGrid a = grids[blockIdx.y];  // by value: scalar registers
+__global__ __launch_bounds__(256) void k_errors_b(const DevGrid* __restrict__ grids, int par) {
+    const DevGrid a = batch_grid(grids);
     errors_body<D>(a, blockIdx.x, gridDim.x, par);
 }
 
@@ -325,8 +325,8 @@ __device__ __forceinline__ void select_body(const DevGrid& a, int blk, int n, in
 __global__ __launch_bounds__(256) void k_select(DevGrid a, int n, int cpw, int par, int loop) {
     select_body(a, blockIdx.x, n, cpw, par, loop);
 }
-__global__ __launch_bounds__(256) void k_select_b(const DevGrid* grids, int n, int cpw, int par) {
-    const DevGrid a = grids[blockIdx.y];  // by value: scalar registers
+__global__ __launch_bounds__(256) void k_select_b(const DevGrid* __restrict__ grids, int n, int cpw, int par) {
+    const DevGrid a = batch_grid(grids);
     select_body(a, blockIdx.x, n, cpw, par, 1);
 }
 
@@ -546,9 +546,19 @@ __device__ __forceinline__ void place_leaf(const DevGrid& a, int i, int k, int m
     // the leaf's own state (already jumped) and count were written by the
     // selection and compaction kernels
     if constexpr (MODE != PLACE_ONLY) {
-        // the line's stores are out and its registers free; the values of a
-        // split's other samples load while the new one is evaluated
+        // the line's stores are out and its registers free; a split's other
+        // samples' values come after the new one (held meanwhile, their registers
+        // cost a wave per SIMD)
         const bool split = MODE == PLACE_ERRORS && cnt == 4u;
+        float xe[6];
+#pragma unroll
+        for (int d = 0; d < 6; ++d) xe[d] = d < D ? best[d] : 0.0f;
+        const mscene::V3<float> val =
+            mscene::eval<float>(B->p, obj, xe, &B->accel, &B->cells, reinterpret_cast<const uint64_t*>(B + 1));
+        float* vo = a.values + (size_t)k * 3;
+        vo[0] = val.x;
+        vo[1] = val.y;
+        vo[2] = val.z;
         LeafSamples ch[2];
         if (split) {
 #pragma unroll
@@ -561,15 +571,6 @@ __device__ __forceinline__ void place_leaf(const DevGrid& a, int i, int k, int m
                 c.vz[q] = o[2];
             }
         }
-        float xe[6];
-#pragma unroll
-        for (int d = 0; d < 6; ++d) xe[d] = d < D ? best[d] : 0.0f;
-        const mscene::V3<float> val =
-            mscene::eval<float>(B->p, obj, xe, &B->accel, &B->cells, reinterpret_cast<const uint64_t*>(B + 1));
-        float* vo = a.values + (size_t)k * 3;
-        vo[0] = val.x;
-        vo[1] = val.y;
-        vo[2] = val.z;
         if (split) {
 #pragma unroll
             for (int j = 0; j < 5; ++j) {
@@ -596,19 +597,23 @@ __device__ __forceinline__ void place_leaf(const DevGrid& a, int i, int k, int m
 // for the pass after (no kernel of this pass reads those) and the pass's
 // statistics, into the host's memory: the host knows before the placement
 // itself whether another pass follows.
-__device__ __forceinline__ bool pass_offsets(const DevGrid& a, int blk, int nblk, int par, int& L,
-                                              int& N, int2& base) {
+// s, P and t (the lane's super group) are loaded by the caller, together.
+__device__ __forceinline__ bool pass_offsets(const DevGrid& a, int blk, int nblk, int par, const TreeCounts& s,
+                                             int P, const int3& t, int2& base) {
     DevCounters* cn = a.cnt;
-    const TreeCounts s = cn->slot[par];
-    L = s.L;
-    N = s.N;
+    const int L = s.L, N = s.N;
     const int lane = threadIdx.x & 63;
     const int per = super_size(nblk), g = blk / per;
-    const SuperSum t = a.ssum[par * kSuper + lane];
-    const int sel = wave_sum(t.sel), split = wave_sum(t.split);
+    int2 own = make_int2(0, 0);
+    for (int c = g * per + lane; c < blk; c += 64) {
+        const int4 p = a.part[c];
+        own.x += p.x;
+        own.y += p.y;
+    }
+    const int sel = wave_sum(t.x), split = wave_sum(t.y);
     const bool fits = (long long)N + sel <= a.cap_s && (long long)L + split <= a.cap_l;
     if (blk == 0 && threadIdx.x < kSuper) {
-        const int held = wave_sum(t.held), P = cn->passes;
+        const int held = wave_sum(t.z);
         // leaves whose errors were estimated since the last pass, and the
         // values that took: the initial leaves, then the children
         const int stale = P == 0 ? L : 2 * s.new_n, vals = P == 0 ? 4 * L : 5 * s.new_n;
@@ -638,14 +643,8 @@ __device__ __forceinline__ bool pass_offsets(const DevGrid& a, int blk, int nblk
         }
     }
     if (!fits) return false;
-    int2 own = make_int2(0, 0);
-    for (int c = g * per + lane; c < blk; c += 64) {
-        const int4 p = a.part[c];
-        own.x += p.x;
-        own.y += p.y;
-    }
-    base.x = wave_sum(own.x + (lane < g ? t.sel : 0));
-    base.y = wave_sum(own.y + (lane < g ? t.split : 0));
+    base.x = wave_sum(own.x + (lane < g ? t.x : 0));
+    base.y = wave_sum(own.y + (lane < g ? t.y : 0));
     return true;
 }
 
@@ -658,14 +657,21 @@ __device__ __forceinline__ bool pass_offsets(const DevGrid& a, int blk, int nblk
 // they start from queue up in LDS and are placed a round of 256 at a time,
 // one per thread.  Every leaf's count and LCG state are rewritten in the
 // same sweep, as they stand after the placement, in full coalesced lines.
-// What bounds it at 1080p is the traffic of its scattered leaf lines; a small
-// tree's pass is the chain of its launches and of one leaf's work.  FUSED (the
-// new sample's integrand and the children's errors taken here) leaves the
-// traffic of a large pass as it was less the split entries, and two launches
-// of six: 5D 1080p (1.5 M leaves a pass) 15.6 -> 14.7 ms a run, 64x48 (12
-// passes of 2000) 617 -> 458 us, 3D 256x256 1240 -> 850 us.  One chunk per wave
-// in place of one per workgroup (fewer barriers, 4x the chunks) was slower at
-// 1080p (12.0 -> 12.9 ms a run at its best count) and no faster below.
+// What bounds it at 1080p is both the chains of its loads (520 MB a pass of
+// 238 us, most of it scattered lines) and the vector units, half the time busy
+// with some 3000 instructions per 64 new samples, a third of them the
+// integrand's; a small tree's pass is the chain of its launches and of one
+// leaf's work.  So the loads before the first leaf go out in two rounds, what
+// the kernel does not write it reads through the scalar cache (the scene's
+// 105 uniform loads in the integrand were vector loads, each waited for; a batch
+// read its pointers as flat ones and spilled 20 registers), and registers are
+// held to five waves: 4D 1080p 8.85 -> 7.95 ms a run, 5D 14.76 -> 14.26, batch of
+// eight 12.70 -> 10.82, 333x517 874 -> 829 us.  Taking the integrand and the
+// children's errors along saves two launches of four and the split entries: 5D
+// 1080p (1.5 M leaves a pass) 15.6 -> 14.7 ms a run, 64x48 (12 passes of 2000)
+// 617 -> 458 us, 3D 256x256 1240 -> 850 us.  One chunk per wave in place of one
+// per workgroup (fewer barriers, 4x the chunks) was slower at 1080p (12.0 ->
+// 12.9 ms a run at its best count) and no faster below.
 // MODE: see place_leaf.  The offsets come from the super groups' totals and
 // the partials of the chunk's own group; every workgroup finds the same
 // totals, so a pass beyond the capacity writes nothing.
@@ -677,19 +683,37 @@ __device__ __forceinline__ void compact_place_body(const DevGrid& a, int blk, in
     __shared__ int lds[8];
     __shared__ int2 qe[QCAP];
     __shared__ unsigned qs[QCAP];
-    if (a.cnt->done) return;
-    nblk = live_chunks(a.cnt->slot[par].L, nblk);
+    // two rounds of loads before the first leaf's line: the counts and totals,
+    // then the partials, the scene's objects and the first flags and states
+    const int done = a.cnt->done, P = a.cnt->passes;
+    const TreeCounts s = a.cnt->slot[par];
+    const int lane = threadIdx.x & 63;
+    const SuperSum& ts_ = a.ssum[par * kSuper + lane];
+    const int3 t = make_int3(ts_.sel, ts_.split, ts_.held);
+    int n_obj = 0;
+    if constexpr (MODE != PLACE_ONLY) n_obj = B->p.n_obj;
+    if (done) return;
+    nblk = live_chunks(s.L, nblk);
     if (blk >= nblk) return;
-    int L, N0;
-    int2 base;
-    if (!pass_offsets(a, blk, nblk, par, L, N0, base)) return;
-    if constexpr (MODE != PLACE_ONLY) {
-        for (int q = threadIdx.x; q < B->p.n_obj * mscene::OBJ_STRIDE; q += 256) obj[q] = B->p.obj[q];
-        __syncthreads();
-    }
-    float emax = 0.0f;
+    const int L = s.L, N0 = s.N;
     int beg, end;
     chunk_range(L, nblk, blk, beg, end);
+    unsigned fv[U], sv[U];
+    auto load_tiles = [&](int t00) {
+#pragma unroll
+        for (int r = 0; r < U; ++r) {
+            const int i = t00 + r * 256 + threadIdx.x;
+            fv[r] = i < end ? a.flags[i] : 0u;
+            sv[r] = i < end ? a.seed[i] : 0u;
+        }
+    };
+    load_tiles(beg);
+    if constexpr (MODE != PLACE_ONLY) {
+        for (int q = threadIdx.x; q < n_obj * mscene::OBJ_STRIDE; q += 256) obj[q] = B->p.obj[q];
+    }
+    int2 base;
+    if (!pass_offsets(a, blk, nblk, par, s, P, t, base)) return;
+    float emax = 0.0f;
     int jq = base.x;  // global rank of the entry at the front of the queue
     int qn = 0;       // queued entries
     auto place_round = [&](int p0, int count) {
@@ -701,13 +725,7 @@ __device__ __forceinline__ void compact_place_body(const DevGrid& a, int blk, in
         }
     };
     for (int t00 = beg; t00 < end; t00 += U * 256) {
-        unsigned fv[U], sv[U];
-#pragma unroll
-        for (int r = 0; r < U; ++r) {
-            const int i = t00 + r * 256 + threadIdx.x;
-            fv[r] = i < end ? a.flags[i] : 0u;
-            sv[r] = i < end ? a.seed[i] : 0u;
-        }
+        if (t00 > beg) load_tiles(t00);
 #pragma unroll
         for (int r = 0; r < U; ++r) {
             const int t0 = t00 + r * 256;
@@ -760,30 +778,28 @@ __device__ __forceinline__ void compact_place_body(const DevGrid& a, int blk, in
     place_round(0, qn);
     if constexpr (MODE == PLACE_ERRORS) {
         emax = wave_max(emax);
-        __syncthreads();
-        if ((threadIdx.x & 63) == 0) lds[threadIdx.x >> 6] = (int)__float_as_uint(emax);
-        __syncthreads();
-        if (threadIdx.x == 0) {
-            const unsigned m = max(max((unsigned)lds[0], (unsigned)lds[1]), max((unsigned)lds[2], (unsigned)lds[3]));
-            if (m != 0u) atomicMax(&a.smax[(par ^ 1) * kSuper + blk / super_size(nblk)].err, m);
-        }
+        if (lane == 0 && emax != 0.0f)
+            atomicMax(&a.smax[(par ^ 1) * kSuper + blk / super_size(nblk)].err, __float_as_uint(emax));
     }
 }
 
-// The scene's objects in dynamic LDS (48 bytes each).  Four waves per SIMD
-// without spills where the integrand is taken along.
+// The scene's objects in dynamic LDS (48 bytes each).  The registers are held to
+// five waves per SIMD, which nothing spills for (4D 1080p, 57 passes: four
+// waves 8.46 ms a run, five 7.95, six with spills 8.60); a 6D leaf needs the
+// registers of four.
 template <int D, int MODE>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_compact_place(
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 6 ? 4 : 5))) void k_compact_place(
     DevGrid a, const mscene::SceneBlock* B, int par) {
     extern __shared__ float obj[];
-    compact_place_body<D, MODE>(a, blockIdx.x, gridDim.x, par, B, obj);
+    compact_place_body<D, MODE>(a, blockIdx.x, gridDim.x, par, in_constant(B), obj);
 }
 template <int D, int MODE>
-__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(4))) void k_compact_place_b(
-    const DevGrid* grids, const void* const* params, int par) {
+__global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 6 ? 4 : 5))) void k_compact_place_b(
+    const DevGrid* __restrict__ grids, const void* const* __restrict__ params, int par) {
     extern __shared__ float obj[];
-    const DevGrid a = grids[blockIdx.y];  // by value: scalar registers
-    compact_place_body<D, MODE>(a, blockIdx.x, gridDim.x, par, (const mscene::SceneBlock*)params[blockIdx.y], obj);
+    const DevGrid a = batch_grid(grids);
+    compact_place_body<D, MODE>(a, blockIdx.x, gridDim.x, par,
+                                in_constant((const mscene::SceneBlock*)params[blockIdx.y]), obj);
 }
 
 // The loop's state per image: finished once `done` or at the limit, so that the
@@ -821,7 +837,7 @@ __global__ __launch_bounds__(256) void k_mark_last_children(DevGrid a) {
     mark_last_children_body(a, blockIdx.x, gridDim.x);
 }
 __global__ __launch_bounds__(256) void k_mark_last_children_b(const DevGrid* grids) {
-    mark_last_children_body(grids[blockIdx.y], blockIdx.x, gridDim.x);
+    mark_last_children_body(batch_grid(grids), blockIdx.x, gridDim.x);
 }
 
 // The leaves' points in their lines and overflow rows from the sample

@@ -155,16 +155,47 @@ __device__ __forceinline__ int lanes_below(unsigned long long mask) {
                                      __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0u));
 }
 
+// Reductions of a whole wave (every lane active) by data-parallel moves: six
+// steps of a few cycles each, where exchanges through the LDS take some fifty.
+// A step's moves that have no source leave `none`.
+template <int CTRL, int ROWS>
+__device__ __forceinline__ int dpp_from(int none, int v) {
+    return __builtin_amdgcn_update_dpp(none, v, CTRL, ROWS, 0xf, false);
+}
 __device__ __forceinline__ int wave_sum(int v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o, 64);
-    return v;
+    v += dpp_from<0x111, 0xf>(0, v);  // one, two, four, eight lanes up in the rows of 16
+    v += dpp_from<0x112, 0xf>(0, v);
+    v += dpp_from<0x114, 0xf>(0, v);
+    v += dpp_from<0x118, 0xf>(0, v);
+    v += dpp_from<0x142, 0xa>(0, v);  // a row's last lane to the next row
+    v += dpp_from<0x143, 0xc>(0, v);  // lane 31 to the upper half
+    return __builtin_amdgcn_readlane(v, 63);
 }
 
 __device__ __forceinline__ float wave_max(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-    return v;
+    auto step = [&](auto from) { v = fmaxf(v, __int_as_float(from(__float_as_int(v)))); };
+    step([](int x) { return dpp_from<0x111, 0xf>(x, x); });
+    step([](int x) { return dpp_from<0x112, 0xf>(x, x); });
+    step([](int x) { return dpp_from<0x114, 0xf>(x, x); });
+    step([](int x) { return dpp_from<0x118, 0xf>(x, x); });
+    step([](int x) { return dpp_from<0x142, 0xa>(x, x); });
+    step([](int x) { return dpp_from<0x143, 0xc>(x, x); });
+    return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), 63));
+}
+
+// p, to memory that nothing writes while the kernel reads it: a uniform load
+// then goes through the scalar cache and may move past stores (an ordinary
+// pointer's is a vector load, waited for where it is used).  By way of an
+// integer, since a cast there and back is dropped.
+template <typename T>
+__device__ __forceinline__ const T* in_constant(const T* p) {
+    return (const T*)(const __attribute__((address_space(4))) T*)(uintptr_t)p;
+}
+// p, to global memory: a pointer read from memory might be of any address space,
+// and the accesses to an unknown one wait for each other and for the LDS.
+template <typename T>
+__device__ __forceinline__ T* in_global(T* p) {
+    return (T*)(__attribute__((address_space(1))) T*)(uintptr_t)p;
 }
 
 // Exclusive scan of two 0/1 predicates over a 256-thread workgroup in thread

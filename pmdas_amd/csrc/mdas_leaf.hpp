@@ -11,6 +11,28 @@
 
 namespace mdas {
 
+// Image blockIdx.y's grid of a batch, in scalar registers.
+__device__ __forceinline__ DevGrid batch_grid(const DevGrid* __restrict__ grids) {
+    DevGrid a = *in_constant(grids + blockIdx.y);
+    a.coords = in_global(a.coords);
+    a.values = in_global(a.values);
+    a.leaf = in_global(a.leaf);
+    a.xpts = in_global(a.xpts);
+    a.err = in_global(a.err);
+    a.seed = in_global(a.seed);
+    a.flags = in_global(a.flags);
+    a.split_list = in_global(a.split_list);
+    a.sdat = in_global(a.sdat);
+    a.sext = in_global(a.sext);
+    a.part = in_global(a.part);
+    a.cnt = in_global(a.cnt);
+    a.ssum = in_global(a.ssum);
+    a.smax = in_global(a.smax);
+    a.lrows = in_global(a.lrows);
+    a.hrun = in_global(a.hrun);
+    return a;
+}
+
 // The whole line of leaf i (8 float4 loads of one 128-byte line).
 __device__ __forceinline__ void load_line(const DevGrid& a, int i, float* f) {
     const float4* p = a.leaf + (size_t)i * (kLineFloats / 4);

@@ -393,6 +393,38 @@ MDAS_HD bool group_may_hit(const float* g, V3<real> o, V3<real> d, real e, real 
     return l2 - p * p - k * l2 <= W * W && p + W >= tmin && p - W <= tmax;
 }
 
+// The lowest sphere of a set, taken out of it.
+MDAS_HD int first_of(uint64_t& m) {
+    const int k = __builtin_ctzll(m);
+    m &= m - 1;
+    return k;
+}
+
+// The same as hit_sphere() for the sphere at s, moved to time t, without an
+// upper end and without branches: the loops over a cell's set take two spheres
+// at a time, so that one's chain of operations fills the other's (a pass's
+// placement at 64x48 17.1 -> 16.2 us, 1080p 5D 14.38 -> 14.26 ms a run; in FP64,
+// bound by the operations themselves, the second would cost 2 %: there it is
+// the first again, and falls away).
+template <typename real>
+constexpr bool kPairs = sizeof(real) == sizeof(float);
+template <typename real>
+MDAS_HD bool meet_sphere(const float* s, V3<real> o, V3<real> d, real t, real tmin, real* hit) {
+    const real cx = (real)s[0] + (real)s[4] * t;
+    const real cy = (real)s[1] + (real)s[5] * t;
+    const real cz = (real)s[2] + (real)s[6] * t;
+    const real r = (real)s[3];
+    const V3<real> oc = v3(o.x - cx, o.y - cy, o.z - cz);
+    const real b = dot3(oc, d);
+    const real c = dot3(oc, oc) - r * r;
+    const real disc = b * b - c;
+    const real sq = r_sqrt(disc < (real)0 ? (real)0 : disc);
+    const real near = -b - sq, far = -b + sq;
+    const real th = near <= tmin ? far : near;
+    *hit = th;
+    return !(disc < (real)0) && th > tmin;
+}
+
 // Closest hit among spheres (centres moved to time t) and the ground plane.
 // Returns the hit distance (tmax on a miss); *id = sphere index, -1 plane, -2 miss.
 // With a cell's set (of `words` words) only its spheres are tested; else with
@@ -409,14 +441,12 @@ MDAS_HD real trace(const Params& P, const float* obj, V3<real> o, V3<real> d, re
         for (int w = 0; w < words; ++w) {
             uint64_t m = cell[w];
             while (m != 0) {
-                const int k = 64 * w + __builtin_ctzll(m);
-                m &= m - 1;
-                const float* s = obj + k * OBJ_STRIDE;
-                real cx = (real)s[0] + (real)s[4] * t;
-                real cy = (real)s[1] + (real)s[5] * t;
-                real cz = (real)s[2] + (real)s[6] * t;
-                real th = hit_sphere(o, d, cx, cy, cz, (real)s[3], tmin, best);
-                if (th < best) { best = th; *id = k; }
+                const int k0 = first_of(m), k1 = kPairs<real> && m != 0 ? first_of(m) : k0;
+                real t0, t1;
+                const bool h0 = meet_sphere(obj + (64 * w + k0) * OBJ_STRIDE, o, d, t, tmin, &t0);
+                const bool h1 = meet_sphere(obj + (64 * w + k1) * OBJ_STRIDE, o, d, t, tmin, &t1);
+                if (h0 && t0 < best) { best = t0; *id = 64 * w + k0; }
+                if (h1 && t1 < best) { best = t1; *id = 64 * w + k1; }
             }
         }
     } else if (A != nullptr && A->n_grp > 0) {
@@ -491,12 +521,11 @@ MDAS_HD bool occluded_by_set(const float* obj, V3<real> o, V3<real> d, real t, r
     for (int w = 0; w < words; ++w) {
         uint64_t m = cell[w];
         while (m != 0) {
-            const float* s = obj + (64 * w + __builtin_ctzll(m)) * OBJ_STRIDE;
-            m &= m - 1;
-            real cx = (real)s[0] + (real)s[4] * t;
-            real cy = (real)s[1] + (real)s[5] * t;
-            real cz = (real)s[2] + (real)s[6] * t;
-            if (hit_sphere(o, d, cx, cy, cz, (real)s[3], tmin, tmax) < tmax) return true;
+            const int k0 = first_of(m), k1 = kPairs<real> && m != 0 ? first_of(m) : k0;
+            real t0, t1;
+            const bool h0 = meet_sphere(obj + (64 * w + k0) * OBJ_STRIDE, o, d, t, tmin, &t0);
+            const bool h1 = meet_sphere(obj + (64 * w + k1) * OBJ_STRIDE, o, d, t, tmin, &t1);
+            if ((h0 && t0 < tmax) || (h1 && t1 < tmax)) return true;
         }
     }
     return false;
