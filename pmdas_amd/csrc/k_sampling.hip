@@ -430,7 +430,7 @@ __device__ __forceinline__ void place_leaf(const DevGrid& a, int i, int k, int m
     }
     float* out = a.coords + (size_t)k * D;
 #pragma unroll
-    for (int d = 0; d < D; ++d) out[d] = best[d];
+    for (int d = 0; d < D; ++d) __builtin_nontemporal_store(best[d], out + d);
     int kid[5] = {k, k, k, k, k};     // PLACE_ERRORS: a split's samples in sorted order,
     float vol_l = 0.0f, vol_r = 0.0f;  // its children's volumes
     if (cnt < 4u) {
@@ -671,7 +671,10 @@ __device__ __forceinline__ bool pass_offsets(const DevGrid& a, int blk, int nblk
 // 1080p (1.5 M leaves a pass) 15.6 -> 14.7 ms a run, 64x48 (12 passes of 2000)
 // 617 -> 458 us, 3D 256x256 1240 -> 850 us.  One chunk per wave in place of one
 // per workgroup (fewer barriers, 4x the chunks) was slower at 1080p (12.0 ->
-// 12.9 ms a run at its best count) and no faster below.
+// 12.9 ms a run at its best count) and no faster below.  What streams through
+// once, the flags and states of the sweep and the new coordinates, goes past
+// the caches (5D 14.27 -> 13.86 ms, 333x517 829 -> 820 us); a line's float4s,
+// several accesses each, must not (loads 17.6 ms, stores 15.2).
 // MODE: see place_leaf.  The offsets come from the super groups' totals and
 // the partials of the chunk's own group; every workgroup finds the same
 // totals, so a pass beyond the capacity writes nothing.
@@ -703,8 +706,8 @@ __device__ __forceinline__ void compact_place_body(const DevGrid& a, int blk, in
 #pragma unroll
         for (int r = 0; r < U; ++r) {
             const int i = t00 + r * 256 + threadIdx.x;
-            fv[r] = i < end ? a.flags[i] : 0u;
-            sv[r] = i < end ? a.seed[i] : 0u;
+            fv[r] = i < end ? __builtin_nontemporal_load(a.flags + i) : 0u;
+            sv[r] = i < end ? __builtin_nontemporal_load(a.seed + i) : 0u;
         }
     };
     load_tiles(beg);
@@ -748,8 +751,8 @@ __device__ __forceinline__ void compact_place_body(const DevGrid& a, int blk, in
                 qs[qn + rs] = s1;
             }
             if (i < end) {
-                a.flags[i] = (unsigned char)(split ? 2u : (sel ? cnt + 1u : cnt));
-                a.seed[i] = sel ? a.jmul * s1 + a.jadd : s1;
+                __builtin_nontemporal_store((unsigned char)(split ? 2u : (sel ? cnt + 1u : cnt)), a.flags + i);
+                __builtin_nontemporal_store(sel ? a.jmul * s1 + a.jadd : s1, a.seed + i);
             }
             qn += ts;
             base.y += tl;
