@@ -39,6 +39,7 @@ struct ReconGeo {
     float stepX, stepY;   // scale / width (kdgrid.cu:501-503)
     float invPixArea;     // 1 / ((sX*sY) / float(W*H)) (kdgrid.cu:532, vec_math.h:483-487)
     int TW, TH, tilesX, tilesY;
+    int lw, lh;           // TW = 2^lw, TH = 2^lh (a tile holds 16 or 64 pixels)
     int tbits;            // Morton bits per tile axis
 };
 
@@ -65,7 +66,7 @@ __device__ __forceinline__ void record_span(const float4& q0, const ReconGeo& G,
 
 __device__ __forceinline__ int tiles_of(int x0, int x1, int y0, int y1, const ReconGeo& G) {
     if (x0 >= x1 || y0 >= y1) return 0;
-    return ((x1 - 1) / G.TW - x0 / G.TW + 1) * ((y1 - 1) / G.TH - y0 / G.TH + 1);
+    return (((x1 - 1) >> G.lw) - (x0 >> G.lw) + 1) * (((y1 - 1) >> G.lh) - (y0 >> G.lh) + 1);
 }
 
 // Keys counted by each of the reconstruction's chunks (the passes' partials are
@@ -178,8 +179,8 @@ __global__ __launch_bounds__(256) void k_recon_emit(DevGrid a, ReconGeo G, const
         }
         int off = base + block_exscan(c, lds, total);
         if (c > 0) {
-            for (int ty = y0 / G.TH; ty <= (y1 - 1) / G.TH; ++ty)
-                for (int tx = x0 / G.TW; tx <= (x1 - 1) / G.TW; ++tx)
+            for (int ty = y0 >> G.lh; ty <= (y1 - 1) >> G.lh; ++ty)
+                for (int tx = x0 >> G.lw; tx <= (x1 - 1) >> G.lw; ++tx)
                     keys[off++] = ((unsigned long long)morton2(tx, ty) << 32) | (unsigned)i;
         }
         base += total;
@@ -436,10 +437,14 @@ __global__ __launch_bounds__(256) void k_tile_ranges(const unsigned long long* k
 // and the overlap with each of its columns and rows, kept in LDS (a pixel's
 // lane did both for itself, per record: 920 us at 1080p for 26 M records, now
 // 525; 640x360 48 -> 25 us), and the lanes of the
-// pixels it overlaps get its bit with LDS atomics (one ballot per pixel where
-// a record overlaps more than kOrPixels).  A pixel then adds its records'
+// pixels it overlaps get its bit with LDS atomics.  Where a record overlaps more
+// than kOrPixels (7) the atomics of the busiest lane cost more than a ballot
+// for each column and each row: a pixel's records are its column's that are
+// also its row's (up to kBallots columns and rows: 640x360 27 -> 22.7 us, 6D
+// 960x540 181 -> 169; ballots everywhere made 3D 256x256 27 -> 34 us, and 64x1
+// tiles 540 -> 690).  A pixel then adds its records'
 // contributions in index order: two overlaps, a product and a quotient each.
-static const int kOrPixels = 20;
+static const int kOrPixels = 7, kBallots = 24;
 // Dynamic LDS of one wave: means and volumes, coverage words, xy areas, and
 // the overlaps, TW + TH per record (an odd stride spreads them over the banks).
 __host__ __device__ constexpr int gather_stride(int TW, int TH) { return (TW + TH) | 1; }
@@ -483,7 +488,7 @@ __global__ __launch_bounds__(256) void k_gather(ReconGeo G, const float4* __rest
     const int ntiles = G.tilesX * G.tilesY;
     const bool live = tile < ntiles;
     const int tx = live ? tile % G.tilesX : 0, ty = live ? tile / G.tilesX : 0;
-    const int pc = gl % G.TW, pr = gl / G.TW;       // this lane's pixel in the tile
+    const int pc = gl & (G.TW - 1), pr = gl >> G.lw;       // this lane's pixel in the tile
     const int ox = tx * G.TW, oy = ty * G.TH;
     int s0 = 0, s1 = 0;
     if (live) {
@@ -508,22 +513,17 @@ __global__ __launch_bounds__(256) void k_gather(ReconGeo G, const float4* __rest
     }
     unsigned long long knext = gl < nrec_of(1) ? keys[s0 + GS + gl] : 0ull;
     for (int rd = 0; rd < rounds; ++rd) {
-        covers[lane] = 0ull;
-        unsigned long long own = 0ull;  // the tile's pixels this lane's record overlaps
+        unsigned long long cols = 0ull, rows = 0ull;  // of the tile that this lane's record overlaps
         if (gl < nrec_of(rd)) {
             int x0, x1, y0, y1;
             record_span(c0, G, x0, x1, y0, y1);
             float* o = ov + lane * stride;
-            const unsigned long long cols = axis_overlaps(c0.x, c0.y, x0, (float)x0 * G.sX / G.fW, G.stepX,
-                                                          max(x0, ox), min(x1, ox + G.TW), ox, o);
-            unsigned long long rows = axis_overlaps(c0.z, c0.w, y0, (float)y0 * G.sY / G.fH, G.stepY,
-                                                    max(y0, oy), min(y1, oy + G.TH), oy, o + G.TW);
+            cols = axis_overlaps(c0.x, c0.y, x0, (float)x0 * G.sX / G.fW, G.stepX, max(x0, ox),
+                                 min(x1, ox + G.TW), ox, o);
+            rows = axis_overlaps(c0.z, c0.w, y0, (float)y0 * G.sY / G.fH, G.stepY, max(y0, oy),
+                                 min(y1, oy + G.TH), oy, o + G.TW);
             mean[lane] = c1;
             area[lane] = (c0.y - c0.x) * (c0.w - c0.z);
-            while (rows != 0ull) {
-                own |= cols << (G.TW * __builtin_ctzll(rows));
-                rows &= rows - 1ull;
-            }
         }
         wave_sync_lds();
         if (gl < nrec_of(rd + 1)) {
@@ -535,14 +535,27 @@ __global__ __launch_bounds__(256) void k_gather(ReconGeo G, const float4* __rest
         // the round's records that overlap this lane's pixel, bit j for the
         // tile's record j
         unsigned long long cov = 0ull;
-        if (GS > 32 && __any(__popcll(own) > kOrPixels)) {
-            // one tile per wave, record j in lane j: the wave's coverage
-            // matrix transposed by ballots, column p delivered to lane p
-            for (int p = 0; p < 64; ++p) {
-                const unsigned long long b = __ballot(((own >> p) & 1ull) != 0ull);
-                cov = lane == p ? b : cov;
+        if (G.TW + G.TH <= kBallots && __any(__popcll(cols) * __popcll(rows) > kOrPixels)) {
+            // the records of the pixel's column and those of its row
+            unsigned long long rcov = 0ull;
+            for (int c = 0; c < G.TW; ++c) {
+                const unsigned long long b = __ballot((cols >> c) & 1ull);
+                cov = pc == c ? b : cov;
             }
+            for (int r = 0; r < G.TH; ++r) {
+                const unsigned long long b = __ballot((rows >> r) & 1ull);
+                rcov = pr == r ? b : rcov;
+            }
+            cov &= rcov;
+            if (GS < 64) cov = (cov >> gbase) & ((1ull << (GS & 63)) - 1ull);
         } else {
+            unsigned long long own = 0ull;  // the tile's pixels this lane's record overlaps
+            while (rows != 0ull) {
+                own |= cols << (__builtin_ctzll(rows) << G.lw);
+                rows &= rows - 1ull;
+            }
+            covers[lane] = 0ull;
+            wave_sync_lds();
             while (own != 0ull) {
                 atomicOr(&covers[gbase + __builtin_ctzll(own)], 1ull << gl);
                 own &= own - 1ull;
@@ -664,6 +677,8 @@ static ReconGeo make_geo(const Grid& g, int W, int H) {
     G.invPixArea = 1.0f / pixArea;
     G.TW = g.tile_w;
     G.TH = g.tile_h;
+    G.lw = __builtin_ctz(G.TW);
+    G.lh = __builtin_ctz(G.TH);
     G.tilesX = (W + G.TW - 1) / G.TW;
     G.tilesY = (H + G.TH - 1) / G.TH;
     int m = G.tilesX > G.tilesY ? G.tilesX : G.tilesY;
