@@ -657,10 +657,10 @@ __device__ __forceinline__ bool pass_offsets(const DevGrid& a, int blk, int nblk
 // they start from queue up in LDS and are placed a round of 256 at a time,
 // one per thread.  Every leaf's count and LCG state are rewritten in the
 // same sweep, as they stand after the placement, in full coalesced lines.
-// What bounds it at 1080p is both the chains of its loads (520 MB a pass of
-// 238 us, most of it scattered lines) and the vector units, half the time busy
-// with some 3000 instructions per 64 new samples, a third of them the
-// integrand's; a small tree's pass is the chain of its launches and of one
+// What bounds it at 1080p is the traffic of its scattered lines (5D: 800 MB a
+// pass of 238 us, 3/4 of a copy's rate) and, beside it, the vector units, half
+// the time busy with some 3000 instructions per 64 new samples, a third of them
+// the integrand's; a small tree's pass is the chain of its launches and of one
 // leaf's work.  So the loads before the first leaf go out in two rounds, what
 // the kernel does not write it reads through the scalar cache (the scene's
 // 105 uniform loads in the integrand were vector loads, each waited for; a batch
