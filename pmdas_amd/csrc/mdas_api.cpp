@@ -95,7 +95,7 @@ struct AwaitedPasses {
     AwaitedPasses& operator=(const AwaitedPasses&) = delete;
     ~AwaitedPasses() {
         g.dev.in_loop = 0;
-        g.next_tag = (g.next_tag + (unsigned)launched) & ~mdas::kRunTag;
+        g.next_tag = (g.next_tag + (unsigned)launched) & (mdas::kRunTag / 2 - 1);  // no carry into kRunTag
     }
 };
 
