@@ -13,6 +13,7 @@
 #include <limits>
 #include <vector>
 
+#include "recon_geo.hpp"  // the product's tile counts, held by tests
 #include "scenes.hpp"  // analytic integrands (input generator shared with the GPU path)
 
 namespace {
@@ -767,6 +768,20 @@ int orc_eval_scene_cells(const void* params, const void* coords, int dim, long l
         }
     }
     return C.words > 0 ? C.n_cells : 0;
+}
+
+// The product's tables of the tiles' key ranges: their entries, and of those
+// that thread `tid` of `threads` clears the first, the last and the number.
+long long orc_tile_entries(int w, int hgt, int tw, int th) {
+    return mdas::tile_entries(mdas::recon_geo(w, hgt, (float)w, (float)hgt, tw, th));
+}
+void orc_entries_of_thread(long long n, long long tid, long long threads, long long* out) {
+    out[0] = out[1] = -1;
+    out[2] = 0;
+    mdas::each_entry(n, tid, threads, [&](long long t) {
+        if (out[2]++ == 0) out[0] = t;
+        out[1] = t;
+    });
 }
 
 float orc_halton(int dim, int i) { return halton<float>(dim, i); }

@@ -64,6 +64,9 @@ void orc_eval_scene_grouped(const void* scene_params, const void* coords, int di
 long long orc_div_by_mismatches(const double* x, long long count);
 int orc_eval_scene_cells(const void* scene_params, const void* coords, int dim, long long count,
                          int fp64, void* values);
+/* Counts of the product's reconstruction (recon_geo.hpp). */
+long long orc_tile_entries(int w, int h, int tw, int th);
+void orc_entries_of_thread(long long n, long long tid, long long threads, long long* first_last_count);
 /* The plain QMC sampler's image (cuda/sampler.h:4-28, random.h:74-89,
  * whitted.cu:59-69): float4 pixels (fp64 = 0) or double4 (fp64 = 1). */
 void orc_qmc_image(const void* scene_params, int w, int h, int spp, int first_sample,

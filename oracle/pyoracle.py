@@ -38,6 +38,8 @@ _SIGS = {
     "orc_eval_scene_grouped": (None, [_P, _P, _I, _LL, _I, _P]),
     "orc_div_by_mismatches": (_LL, [_P, _LL]),
     "orc_eval_scene_cells": (_I, [_P, _P, _I, _LL, _I, _P]),
+    "orc_tile_entries": (_LL, [_I, _I, _I, _I]),
+    "orc_entries_of_thread": (None, [_LL, _LL, _LL, _P]),
     "orc_qmc_image": (None, [_P, _I, _I, _I, _I, _U, _I, _P]),
     "orc_halton": (_F, [_I, _I]),
     "orc_eval_range": (None, [_P, _P, _LL, _LL]),
@@ -249,6 +251,18 @@ def eval_scene_cells(params, coords, dim, fp64=False):
 def div_by_mismatches(x):
     x = np.ascontiguousarray(x, np.float64)
     return load().orc_div_by_mismatches(vp(x), len(x))
+
+
+def tile_entries(w, h, tw, th):
+    """Entries of the product's tables of tile ranges."""
+    return load().orc_tile_entries(w, h, tw, th)
+
+
+def entries_of_thread(n, tid, threads):
+    """(first, last, count) of the n entries that a thread clears."""
+    out = np.empty(3, np.int64)
+    load().orc_entries_of_thread(n, tid, threads, vp(out))
+    return tuple(int(v) for v in out)
 
 
 def qmc_image(params, w, h, spp, first_sample=0, frame=0, fp64=False):

@@ -21,6 +21,7 @@
 #include <cmath>
 
 #include "mdas_leaf.hpp"
+#include "recon_geo.hpp"
 
 #pragma clang fp contract(off)
 
@@ -31,17 +32,6 @@ static int recon_chunks(const Grid& g) { return std::min(g.chunks(), kReconChunk
 static const int kSortBlocks = 1024;
 static const int kSortMaxBits = 10;  // digit width limit (histograms of 1024 bins)
 static const int kSortKeysPerThread = 16;  // scatter tile: 4096 keys staged in LDS (8192: slower)
-
-struct ReconGeo {
-    int W, H;
-    float fW, fH;
-    float sX, sY;
-    float stepX, stepY;   // scale / width (kdgrid.cu:501-503)
-    float invPixArea;     // 1 / ((sX*sY) / float(W*H)) (kdgrid.cu:532, vec_math.h:483-487)
-    int TW, TH, tilesX, tilesY;
-    int lw, lh;           // TW = 2^lw, TH = 2^lh (a tile holds 16 or 64 pixels)
-    int tbits;            // Morton bits per tile axis
-};
 
 // kdgrid.cu:524-529: pixel span [x0, x1) x [y0, y1) of a leaf box
 __device__ __forceinline__ void pixel_span(float mn0, float mx0, float mn1, float mx1,
@@ -148,13 +138,13 @@ __global__ __launch_bounds__(256) void k_count_keys(DevGrid a, int chunks) {
 
 // Every workgroup sums the chunks' counts for itself (at most kReconChunks, 16
 // coalesced loads a thread: about 1 us in place of a scan kernel of 7 and its
-// launch).  Also clears the tiles' ranges (n_tiles entries each) for
-// k_tile_ranges.
+// launch).  Also clears the tiles' ranges for k_tile_ranges.
 __global__ __launch_bounds__(256) void k_recon_emit(DevGrid a, ReconGeo G, const float4* rrec,
                                                     unsigned long long* keys, long long cap_keys,
-                                                    int* tstart, int* tend, int n_tiles) {
+                                                    int* tstart, int* tend) {
     __shared__ int lds[4];
-    for (int t = blockIdx.x * 256 + threadIdx.x; t < n_tiles; t += gridDim.x * 256) tstart[t] = tend[t] = 0;
+    each_entry(tile_entries(G), blockIdx.x * 256ll + threadIdx.x, gridDim.x * 256ll,
+               [&](long long t) { tstart[t] = tend[t] = 0; });
     const int L = leaf_total(a);
     int beg, end, base, first_end;
     chunk_range(L, gridDim.x, blockIdx.x, beg, end);
@@ -664,28 +654,7 @@ __global__ __launch_bounds__(256) void k_bytes(const float4* px, uchar4* out, lo
 
 // ------------------------------------------------------------ launchers --
 static ReconGeo make_geo(const Grid& g, int W, int H) {
-    ReconGeo G;
-    G.W = W;
-    G.H = H;
-    G.fW = (float)W;
-    G.fH = (float)H;
-    G.sX = g.sX;
-    G.sY = g.sY;
-    G.stepX = g.sX / (float)W;
-    G.stepY = g.sY / (float)H;
-    const float pixArea = (g.sX * g.sY) / (float)(W * H);
-    G.invPixArea = 1.0f / pixArea;
-    G.TW = g.tile_w;
-    G.TH = g.tile_h;
-    G.lw = __builtin_ctz(G.TW);
-    G.lh = __builtin_ctz(G.TH);
-    G.tilesX = (W + G.TW - 1) / G.TW;
-    G.tilesY = (H + G.TH - 1) / G.TH;
-    int m = G.tilesX > G.tilesY ? G.tilesX : G.tilesY;
-    int bits = 0;
-    while ((1 << bits) < m) ++bits;
-    G.tbits = bits;
-    return G;
+    return recon_geo(W, H, g.sX, g.sY, g.tile_w, g.tile_h);
 }
 
 #define MDAS_DISPATCH_D(D_, STMT)                      \
@@ -736,14 +705,14 @@ static const long long kKeyBoundBytes = 8ll << 30;
 static long long align256(long long b) { return (b + 255) / 256 * 256; }
 
 long long recon_key_bound(const Grid& g, int W, int H) { return key_bound(g, make_geo(g, W, H)); }
-long long recon_tiles_cap(const Grid& g, int W, int H) { return 1ll << (2 * make_geo(g, W, H).tbits); }
+long long recon_tiles_cap(const Grid& g, int W, int H) { return tile_entries(make_geo(g, W, H)); }
 
 long long recon_bytes_needed(const Grid& g, int W, int H) {
     const ReconGeo G = make_geo(g, W, H);
     const long long kb = key_bound(g, G);
     if (kb > 0x7fffffffLL) return -1;
     const long long L = std::max<long long>(g.host.n_leaves, 1);
-    return align256(sizeof(unsigned) * kSortHistWords) + 2 * align256(sizeof(int) << (2 * G.tbits)) +
+    return align256(sizeof(unsigned) * kSortHistWords) + 2 * align256(sizeof(int) * tile_entries(G)) +
            align256(sizeof(float4) * 2 * L) + 2 * align256(sizeof(unsigned long long) * kb);
 }
 
@@ -770,7 +739,7 @@ hipError_t recon_reserve(Grid& g, int W, int H) {
         hipError_t e = grow_keys(rb, kb);
         if (e != hipSuccess) return e;
     }
-    const long long tiles = 1ll << (2 * G.tbits);
+    const long long tiles = tile_entries(G);
     if (tiles > rb.tiles_cap) {
         if (rb.tile_start) (void)hipFree(rb.tile_start);
         if (rb.tile_end) (void)hipFree(rb.tile_end);
@@ -819,10 +788,9 @@ hipError_t recon_prepare(Grid& g, int W, int H, hipStream_t st) {
 static hipError_t recon_finish(Grid& g, ReconBufs& rb, float* pixels, int W, int H, hipStream_t st,
                                hipEvent_t ev_sort0, hipEvent_t ev_sort1) {
     ReconGeo G = make_geo(g, W, H);
-    const long long tiles = 1ll << (2 * G.tbits);
     kbeg(g, st, "k_recon_emit");
     hipLaunchKernelGGL(k_recon_emit, dim3(recon_chunks(g)), dim3(256), 0, st, g.dev, G, rb.rrec, rb.keys, rb.keys_cap,
-                       rb.tile_start, rb.tile_end, (int)tiles);
+                       rb.tile_start, rb.tile_end);
     kend(g, st);
     // keys there can be: the bound, or the buffers where they were sized from
     // the count
