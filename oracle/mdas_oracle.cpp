@@ -775,6 +775,24 @@ int orc_eval_scene_cells(const void* params, const void* coords, int dim, long l
 long long orc_tile_entries(int w, int hgt, int tw, int th) {
     return mdas::tile_entries(mdas::recon_geo(w, hgt, (float)w, (float)hgt, tw, th));
 }
+// The product's tiles of count boxes (mn0, mx0, mn1, mx1) in a sample space of
+// sx by sy: out[4 k ..] the first and last tile along x, then along y of box k,
+// -1 where it touches none; returns the tiles of them all.
+long long orc_box_tiles(int w, int hgt, float sx, float sy, int tw, int th, const float* box, long long count,
+                        int* out) {
+    const mdas::ReconGeo G = mdas::recon_geo(w, hgt, sx, sy, tw, th);
+    long long n = 0;
+    for (long long k = 0; k < count; ++k) {
+        const float* b = box + 4 * k;
+        int x0, x1, y0, y1;
+        mdas::pixel_span(b[0], b[1], b[2], b[3], G, x0, x1, y0, y1);
+        const int c = mdas::tiles_of(x0, x1, y0, y1, G);
+        const int t[4] = {x0 >> G.lw, (x1 - 1) >> G.lw, y0 >> G.lh, (y1 - 1) >> G.lh};
+        for (int q = 0; q < 4; ++q) out[4 * k + q] = c > 0 ? t[q] : -1;
+        n += c;
+    }
+    return n;
+}
 void orc_entries_of_thread(long long n, long long tid, long long threads, long long* out) {
     out[0] = out[1] = -1;
     out[2] = 0;

@@ -39,6 +39,7 @@ _SIGS = {
     "orc_div_by_mismatches": (_LL, [_P, _LL]),
     "orc_eval_scene_cells": (_I, [_P, _P, _I, _LL, _I, _P]),
     "orc_tile_entries": (_LL, [_I, _I, _I, _I]),
+    "orc_box_tiles": (_LL, [_I, _I, _F, _F, _I, _I, _P, _LL, _P]),
     "orc_entries_of_thread": (None, [_LL, _LL, _LL, _P]),
     "orc_qmc_image": (None, [_P, _I, _I, _I, _I, _U, _I, _P]),
     "orc_halton": (_F, [_I, _I]),
@@ -256,6 +257,14 @@ def div_by_mismatches(x):
 def tile_entries(w, h, tw, th):
     """Entries of the product's tables of tile ranges."""
     return load().orc_tile_entries(w, h, tw, th)
+
+
+def box_tiles(w, h, sx, sy, tw, th, boxes):
+    """(rows of first x, last x, first y, last y tile of each box (mn0, mx0,
+    mn1, mx1), or -1; tiles in all) by the product's span."""
+    b = np.ascontiguousarray(boxes, np.float32).reshape(-1, 4)
+    out = np.empty((len(b), 4), np.int32)
+    return out, load().orc_box_tiles(w, h, sx, sy, tw, th, vp(b), len(b), vp(out))
 
 
 def entries_of_thread(n, tid, threads):

@@ -33,30 +33,9 @@ static const int kSortBlocks = 1024;
 static const int kSortMaxBits = 10;  // digit width limit (histograms of 1024 bins)
 static const int kSortKeysPerThread = 16;  // scatter tile: 4096 keys staged in LDS (8192: slower)
 
-// kdgrid.cu:524-529: pixel span [x0, x1) x [y0, y1) of a leaf box
-__device__ __forceinline__ void pixel_span(float mn0, float mx0, float mn1, float mx1,
-                                           const ReconGeo& G, int& x0, int& x1, int& y0,
-                                           int& y1) {
-    x0 = (int)(mn0 * G.fW / G.sX);
-    int xx = (int)(mx0 * G.fW / G.sX);
-    y0 = (int)(mn1 * G.fH / G.sY);
-    int yy = (int)(mx1 * G.fH / G.sY);
-    x1 = min(xx + 1, G.W);
-    y1 = min(yy + 1, G.H);
-}
-
-// The span with the start clamped to the image (a span starting past the
-// image is empty), from a record's xy box.
 __device__ __forceinline__ void record_span(const float4& q0, const ReconGeo& G, int& x0, int& x1,
                                             int& y0, int& y1) {
     pixel_span(q0.x, q0.y, q0.z, q0.w, G, x0, x1, y0, y1);
-    x0 = min(x0, G.W);
-    y0 = min(y0, G.H);
-}
-
-__device__ __forceinline__ int tiles_of(int x0, int x1, int y0, int y1, const ReconGeo& G) {
-    if (x0 >= x1 || y0 >= y1) return 0;
-    return (((x1 - 1) >> G.lw) - (x0 >> G.lw) + 1) * (((y1 - 1) >> G.lh) - (y0 >> G.lh) + 1);
 }
 
 // Keys counted by each of the reconstruction's chunks (the passes' partials are

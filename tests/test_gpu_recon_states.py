@@ -51,3 +51,43 @@ def test_tiles_without_a_leaf(mdas, size, tile):
         assert (keep.sum() > 0) == bool(want.any())
     g.close()
     o.close()
+
+
+def _overlaps_64(st, dim, W, H, sx, sy):
+    """The image of kdgrid.cu:483-582 in 64 bits (sx, sy: the sample space)."""
+    px = np.zeros((H, W, 3))
+    val = np.where(st["idx"][..., None] >= 0, st["values"][np.maximum(st["idx"], 0)].astype(np.float64), 0.0)
+    mean = val.sum(1) / (st["idx"] >= 0).sum(1)[:, None]
+    box = st["box"].astype(np.float64)
+    ext = box[:, dim:] - box[:, :dim]
+    depth = ext[:, 2:].prod(1)  # volume over xy area
+    ex, ey = (np.arange(n + 1) * s / n for n, s in ((W, sx), (H, sy)))
+    for i in range(len(box)):
+        ox = np.clip(np.minimum(ex[1:], box[i, dim]) - np.maximum(ex[:-1], box[i, 0]), 0, None)
+        oy = np.clip(np.minimum(ey[1:], box[i, dim + 1]) - np.maximum(ey[:-1], box[i, 1]), 0, None)
+        px += np.multiply.outer(np.multiply.outer(oy, ox) * depth[i], mean[i])
+    return px * (W * H / (sx * sy))
+
+
+@pytest.mark.parametrize("tile", [(8, 8), (4, 4), (64, 1), (1, 16)])
+@pytest.mark.parametrize("off", [(-3.5, 0.0), (-6.25, -9.75), (-40.0, 2.5), (20.0, -11.0)])
+def test_boxes_outside_the_image(mdas, tile, off):
+    """Boxes moved off the image by some pixels, by both reconstructions."""
+    W, H = 75, 50
+    _say(f"boxes outside {tile} {off}")
+    args, o, st = _tree(3, W, H, 2000)
+    o.close()
+    st["box"][:, 0::3] += np.float32(off[0])
+    st["box"][:, 1::3] += np.float32(off[1])
+    st["coords"][:, :2] += np.float32(off)
+    g = mdas.KDGrid(*args)
+    g.set_recon_tile(*tile)
+    _upload(g, st)
+    want = _overlaps_64(st, 3, W, H, W, H)
+    # a pixel bound is a sum of at most 75 steps, each rounded below 75: within
+    # 3.4e-4 pixels, an overlap within twice that; the depths of the leaves over
+    # a point sum to 1 and a pixel has a few leaves side by side: 7 of them
+    for scatter in (False, True):
+        got = g.integrate_image(W, H, scatter=scatter)[..., :3]
+        assert np.abs(got - want).max() < 5e-3 and want.max() > 0.1
+    g.close()

@@ -1,6 +1,7 @@
 """Counts of the reconstruction's geometry (recon_geo.hpp) on the CPU, where
 their tables need not exist: tiles of one pixel along an axis of up to 65535
 make tables of 2^32 entries, every one of which has to be cleared."""
+import numpy as np
 import pytest
 
 
@@ -19,3 +20,34 @@ def test_every_tile_range_is_cleared(orc, size, tile):
             if want:
                 assert (first, last) == (tid, tid + (want - 1) * threads)
         assert orc.entries_of_thread(n, (n - 1) % threads, threads)[1] == n - 1
+
+
+@pytest.mark.parametrize("size,tile,scale", [((75, 50), (8, 8), (75.0, 50.0)), ((201, 33), (4, 16), (1.0, 1.0)),
+                                             ((64, 300), (64, 1), (64.0, 300.0)), ((17, 16), (1, 16), (2.0, 1.0))])
+def test_a_box_touches_the_images_tiles_only(orc, size, tile, scale):
+    """Boxes that begin or end outside the image (an uploaded state's may)."""
+    (W, H), (TW, TH), (sx, sy) = size, tile, scale
+    r = np.random.default_rng(W)
+    n = 20000
+    step = np.float32([sx / W, sy / H])
+    lo = np.float32([-0.1, -0.1]) * (sx, sy) - 9 * TW * step * (r.random((n, 1)) < 0.3) * r.random((n, 2))
+    mn = np.float32(lo + r.random((n, 2)) * 1.3 * (sx, sy))
+    mx = np.float32(mn + r.random((n, 2)) ** 4 * (sx, sy))
+    out, total = orc.box_tiles(W, H, sx, sy, TW, TH, np.stack([mn[:, 0], mx[:, 0], mn[:, 1], mx[:, 1]], 1))
+    hit = out[:, 0] >= 0
+    assert np.array_equal(hit, np.all(out >= 0, 1))
+    assert total == ((out[:, 1] - out[:, 0] + 1) * (out[:, 3] - out[:, 2] + 1))[hit].sum()
+    assert np.all(out[hit][:, [0, 2]] <= out[hit][:, [1, 3]])
+    assert np.all(out[hit][:, 1] < -(-W // TW)) and np.all(out[hit][:, 3] < -(-H // TH))
+    # in 64 bits, a thousandth of a pixel apart: the tiles that the box's part
+    # of the image meets
+    px = np.float64([W / sx, H / sy])
+    a, b = mn * px, mx * px
+    inside = np.all((b > 1e-3) & (a < np.float64([W, H]) - 1e-3), 1)
+    assert np.all(hit[inside]) and not np.any(hit[np.any((b < -1 - 1e-3) | (a > np.float64([W, H]) + 1e-3), 1)])
+    first = np.maximum(a[inside] - 1e-3, 0) // (TW, TH)
+    last = np.minimum(b[inside] + 1e-3, np.float64([W, H]) - 1e-3) // (TW, TH)
+    assert np.all(out[inside][:, [0, 2]] >= first) and np.all(out[inside][:, [1, 3]] <= last)
+    first = np.maximum(a[inside] + 1e-3, 0) // (TW, TH)
+    last = np.clip(b[inside] - 1e-3, 0, np.float64([W, H]) - 1e-3) // (TW, TH)
+    assert np.all(out[inside][:, [0, 2]] <= first) and np.all(out[inside][:, [1, 3]] >= last)
