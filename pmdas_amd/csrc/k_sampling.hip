@@ -218,8 +218,10 @@ __global__ __launch_bounds__(256) void k_errors_b(const DevGrid* __restrict__ gr
 // fill their waves.  Runs without reconstruction, against 256 leaves up to 4096
 // chunks: 333x517 884 -> 773 us, 3D 256x256 809 -> 740 us, 1080p the same; at
 // least 1024 leaves (795 us) or 512 chunks (880 us) were slower at 333x517.
+// One for a tree without leaves (an uploaded state): its pass adds nothing, and
+// is reported like any other.
 __device__ __forceinline__ int live_chunks(int L, int n) {
-    return min(n, max(min((L + 255) / 256, 1024), L / 512));
+    return min(n, max(max(min((L + 255) / 256, 1024), L / 512), 1));
 }
 
 // kdgrid.cu:316-326.  Per leaf: the seed (tea4(i,0) when unset), one draw u,
