@@ -258,7 +258,7 @@ __device__ __forceinline__ void select_chunk(const DevGrid& a, int L, float gmax
                 fv[r] = a.flags[i];
             }
         }
-        const float gmax = wave_max(gmax_part);  // no NaN among them: each is a maximum from 0
+        const float gmax = wave_max(gmax_part);  // each a maximum from 0, or all an uploaded g_error
 #pragma unroll
         for (int r = 0; r < U; ++r) {
             const int i = i0 + r * 256;

@@ -631,9 +631,10 @@ int mdas_upload_state(mdas_handle h, int n, int l, const float* coords, const fl
         HIP_TRY(mdas::launch_build_pts(g, l, 0));
         HIP_TRY(hipDeviceSynchronize());
     }
-    // g_error in one of its groups, the others and the loop's sets zero
+    // g_error in all of its groups (what is not a maximum of errors, a NaN or
+    // below 0, must not give way to a group's 0), the loop's sets zero
     std::vector<mdas::SuperMax> sm((size_t)(mdas::kMaxSets * mdas::kSuper), mdas::SuperMax{});
-    memcpy(&sm[(size_t)(mdas::kGError * mdas::kSuper)].err, &max_error, 4);
+    for (int k = 0; k < mdas::kSuper; ++k) memcpy(&sm[(size_t)(mdas::kGError * mdas::kSuper + k)].err, &max_error, 4);
     HIP_TRY(hipMemcpy(g.dev.smax, sm.data(), sizeof(mdas::SuperMax) * sm.size(), hipMemcpyHostToDevice));
     HIP_TRY(hipMemset(g.dev.ssum, 0, sizeof(mdas::SuperSum) * mdas::kSumSets * mdas::kSuper));
     mdas::HostCounters c{};

@@ -42,3 +42,31 @@ def test_passes_over_no_leaf(mdas, dim, samples):
         assert g.GetNewSamples() > 0
     g.close()
     sc.close()
+
+
+@pytest.mark.parametrize("dim,kind", [(3, 1), (5, 3)])
+@pytest.mark.parametrize("g_error", [np.nan, -np.nan, -1.0, -0.0, 0.0, 1e-45, 1e-3, np.inf])
+def test_selection_against_an_uploaded_g_error(mdas, dim, kind, g_error):
+    """AdaptiveSampling takes g_error as uploaded, whatever it is: against a
+    NaN or a negative one no leaf is selected, against 0 every leaf."""
+    _say(f"g_error {g_error} dim={dim}")
+    args = (dim, 20000, 4, 0, 2, 0.25, 48.0, 32.0)
+    o = pyoracle.OracleGrid(*args)
+    o.run(pyoracle.make_scene(kind, 5, dim, 48.0, 32.0), 3000)
+    o.compute_errors()
+    st = o.state()
+    o.set_state(st, g_error)
+    o.adaptive_sampling()
+    g = mdas.KDGrid(*args)
+    g.upload_state(*[st[k] for k in ("coords", "values", "idx", "box", "err", "seed")], g_error)
+    assert np.float32(g.GetMaxError()).tobytes() == np.float32(g_error).tobytes()
+    g.AdaptiveSampling()
+    added = o.n_samples - len(st["coords"])
+    assert added == {"nan": 0, "-1.0": 0, "-0.0": 0, "0.0": len(st["idx"]), "inf": added}.get(str(g_error), added)
+    assert (g.GetNumberOfSamples(), g.GetNumberOfNodes()) == (o.n_samples, o.n_leaves)
+    a, b = g.download_state(), o.state()
+    for k in b:
+        n = len(st["values"]) if k == "values" else None  # the new ones are not evaluated
+        assert np.array_equal(a[k][:n].view(np.uint32), b[k][:n].view(np.uint32)), k
+    g.close()
+    o.close()
