@@ -124,15 +124,23 @@ __global__ __launch_bounds__(kMaxSets* kSuper) void k_initial_counters_b(const D
 
 // Before a single call: the pass kernels run again after a loop or a refused
 // pass, without the loop's limit, from zero totals; before ComputeErrors
-// (kdgrid.cu:684-685) g_error = 0.
-__global__ __launch_bounds__(kSuper) void k_arm(DevGrid a, int errors, int adaptive) {
+// (kdgrid.cu:684-685) g_error = 0.  The tree's counts move to the slot that the
+// host launches the pass with, if they are in the other one (a graph of the
+// caller's may have set the grid up since the host last saw it).
+__global__ __launch_bounds__(kSuper) void k_arm(DevGrid a, int errors, int adaptive, int par) {
     DevCounters* c = a.cnt;
-    SuperSum& t = a.ssum[c->cur * kSuper + threadIdx.x];
+    SuperSum& t = a.ssum[par * kSuper + threadIdx.x];
     if (adaptive) t.sel = t.split = t.held = 0;
     if (errors) a.smax[kGError * kSuper + threadIdx.x].err = 0u;
     if (threadIdx.x != 0) return;
     c->done = 0;
-    if (adaptive) c->status = 0;
+    if (adaptive) {
+        c->status = 0;
+        if (c->cur != par) {
+            c->slot[par] = c->slot[par ^ 1];
+            c->cur = par;
+        }
+    }
     if (errors) {
         c->limit = 0x7fffffff;
         c->guard_cap = 0;
@@ -601,9 +609,9 @@ __device__ __forceinline__ void place_leaf(const DevGrid& a, int i, int k, int m
 // all selected and split leaves), from the super groups and the partials of
 // its own group; every wave computes it for itself.  False if the pass would
 // exceed the capacity.  One thread writes the next slot, a wave the totals' zeros
-// for the pass after (no kernel of this pass reads those) and the pass's
-// statistics, into the host's memory: the host knows before the placement
-// itself whether another pass follows.
+// for the pass after (no kernel of this pass reads those) and, into the host's
+// memory, the pass's statistics in a loop, which knows before the placement
+// itself whether another pass follows, or a single call's counters.
 // s, P and t (the lane's super group) are loaded by the caller, together.
 __device__ __forceinline__ bool pass_offsets(const DevGrid& a, int blk, int nblk, int par, const TreeCounts& s,
                                              int P, const int3& t, int2& base) {
@@ -624,7 +632,7 @@ __device__ __forceinline__ bool pass_offsets(const DevGrid& a, int blk, int nblk
         // leaves whose errors were estimated since the last pass, and the
         // values that took: the initial leaves, then the children
         const int stale = P == 0 ? L : 2 * s.new_n, vals = P == 0 ? 4 * L : 5 * s.new_n;
-        if (lane < kPassWords) {
+        if (a.in_loop && lane < kPassWords) {
             const int w[kPassWords] = {L, N, sel, split, held, stale, vals, fits ? 0 : MDAS_ERR_CAPACITY_DEV};
             int v = 0;
 #pragma unroll
@@ -647,6 +655,7 @@ __device__ __forceinline__ bool pass_offsets(const DevGrid& a, int blk, int nblk
                 cn->slot[par ^ 1] = TreeCounts{N + sel, L + split, N, L, sel, split};
                 cn->cur = par ^ 1;
             }
+            if (!a.in_loop) a.hrun->cnt = *cn;
         }
     }
     if (!fits) return false;
@@ -898,7 +907,7 @@ hipError_t launch_initial(Grid& g, int L0, int limit, hipStream_t st) {
 }
 
 hipError_t launch_arm(Grid& g, bool errors, bool adaptive, hipStream_t st) {
-    hipLaunchKernelGGL(k_arm, dim3(1), dim3(kSuper), 0, st, g.dev, errors ? 1 : 0, adaptive ? 1 : 0);
+    hipLaunchKernelGGL(k_arm, dim3(1), dim3(kSuper), 0, st, g.dev, errors ? 1 : 0, adaptive ? 1 : 0, g.host.cur);
     return hipGetLastError();
 }
 
@@ -934,7 +943,7 @@ hipError_t launch_place(Grid& g, int parity, int mode, const void* dparams, int 
 }
 
 hipError_t launch_adaptive(Grid& g, hipStream_t st) {
-    const int parity = g.host.cur;  // the host is current after every call that changes the tree
+    const int parity = g.host.cur;  // where launch_arm has put the counts
     hipError_t e = select_chunks(g, parity, 0, st);
     if (e == hipSuccess) e = launch_place(g, parity, PLACE_ONLY, nullptr, 0, st);
     return e;

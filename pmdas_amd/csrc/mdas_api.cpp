@@ -81,14 +81,14 @@ int sync_counters(Grid& g, hipStream_t st) {
     return MDAS_OK;
 }
 
-// The passes launched meanwhile are waited for by their tags (those of a run
-// that ends early are not used again either) and, in a loop, leave out the
-// stale markers.
+// The passes of a run launched meanwhile are waited for by their tags (those of
+// a run that ends early are not used again either) and leave out the stale
+// markers.
 struct AwaitedPasses {
     Grid& g;
     int launched = 0;
-    AwaitedPasses(Grid& x, bool loop) : g(x) {
-        g.dev.in_loop = loop ? 1 : 0;
+    explicit AwaitedPasses(Grid& x) : g(x) {
+        g.dev.in_loop = 1;
         g.dev.htag = mdas::kRunTag | g.next_tag;
     }
     AwaitedPasses(const AwaitedPasses&) = delete;
@@ -384,26 +384,9 @@ static int adaptive_sampling(Grid& g, bool armed, hipStream_t st) {
         HIP_TRY(hipEventRecord(ev.e[0], st));
     }
     if (!armed) HIP_TRY(mdas::launch_arm(g, false, true, st));
-    // kdgrid.cu:753-759 reads the counters back; here the pass has sent them
-    mdas::PassStat ps;
-    {
-        AwaitedPasses passes(g, false);
-        const int p = g.host.passes;  // its number in the tree, by which its row goes
-        passes.launched = p + 1;
-        HIP_TRY(mdas::launch_adaptive(g, st));
-        HIP_TRY(hipStreamSynchronize(st));
-        HIP_TRY(wait_for_row(g, p, st, &ps));
-    }
-    if (ps.status == 0) {
-        g.host.cur ^= 1;
-        g.host.slot[g.host.cur] = mdas::TreeCounts{ps.N + ps.sel, ps.L + ps.split, ps.N, ps.L, ps.sel, ps.split};
-        g.host.passes++;
-        g.host.done = g.host.status = 0;
-        g.host.name_counts();
-    } else {
-        int rc = sync_counters(g, st);
-        if (rc) return rc;
-    }
+    HIP_TRY(mdas::launch_adaptive(g, st));
+    HIP_TRY(hipStreamSynchronize(st));
+    mdas::take_counters(g);  // kdgrid.cu:753-759 reads them back; here the pass has sent them
     if (g.host.status != 0) {
         int s = g.host.status;
         // clear the device error so that the grid stays usable
@@ -869,7 +852,7 @@ int mdas_run(mdas_handle h, mdas_scene_handle s, long long target, void* stream)
     // every timed launch in order (name, ms); folded after each block, so the
     // event pool holds one block's events however many passes the run takes
     std::vector<std::pair<std::string, double>> seq;
-    AwaitedPasses passes(g, true);
+    AwaitedPasses passes(g);
     // The placement takes the integrand along and, for the plain method, the
     // children's errors (the learned error pass is a kernel of its own);
     // timing and logs want the phases apart.  The results are the same.

@@ -82,7 +82,7 @@ static const int kPassWords = sizeof(PassStat) / sizeof(int);
 static const int kHostRows = 256;  // rows in turn; the host takes them before they wrap
 struct HostRun {
     unsigned long long row[kHostRows][kPassWords];
-    DevCounters cnt;  // as the last kernel of a run leaves them
+    DevCounters cnt;  // as a run's last kernel or a single pass leaves them
 };
 static const unsigned kRunTag = 0x80000000u;  // set in the tags that a host waits for: those of a
                                               // batch's passes, which nothing waits for, stay below
@@ -152,7 +152,8 @@ struct DevGrid {
     int cand;
     unsigned jmul, jadd;  // LCG jump over candidatesNum * D draws
     int in_loop;                // 1 inside the device-side loop: the placement leaves the
-                                //   children's stale markers to the next error pass
+                                //   children's stale markers to the next error pass, and
+                                //   reports the pass in a row
     int b, e;
     float alpha, sX, sY;
 };
@@ -292,8 +293,8 @@ hipError_t launch_select(Grid& g, int parity, hipStream_t st);
 hipError_t launch_place(Grid& g, int parity, int mode, const void* dparams, int n_obj, hipStream_t st);
 hipError_t launch_mark_last_children(Grid& g, hipStream_t st);
 // Single calls: ComputeErrors over every leaf (g_error starts from 0), and
-// AdaptiveSampling against g_error on the host's slot; arm resets what an
-// earlier loop or a refused pass left.
+// AdaptiveSampling against g_error; arm resets what an earlier loop or a
+// refused pass left, and puts the counts into the slot the host names.
 hipError_t launch_arm(Grid& g, bool errors, bool adaptive, hipStream_t st);
 hipError_t launch_compute_errors(Grid& g, hipStream_t st);
 hipError_t launch_adaptive(Grid& g, hipStream_t st);

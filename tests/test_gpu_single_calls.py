@@ -70,3 +70,56 @@ def test_selection_against_an_uploaded_g_error(mdas, dim, kind, g_error):
         assert np.array_equal(a[k][:n].view(np.uint32), b[k][:n].view(np.uint32)), k
     g.close()
     o.close()
+
+
+def _check(g, o, what):
+    a, b = g.download_state(), o.state()
+    for k in b:
+        assert np.array_equal(a[k].view(np.uint32), b[k].view(np.uint32)), (what, k)
+
+
+@pytest.mark.parametrize("kind,dim", [(1, 3), (3, 5)])
+def test_single_calls_after_a_captured_setup(mdas, kind, dim):
+    """A caller's graph that sets the grid up (InitialSampling, its integrand,
+    ComputeErrors) is replayed after any number of passes: the host has not
+    seen the tree start over, and the next single calls find it as it is."""
+    from pmdas_amd import hip
+    W, H = 48.0, 32.0
+    args = (dim, 30000, 4, 0, 2, 0.25, W, H)
+    g, sc = mdas.KDGrid(*args), mdas.Scene(kind, 5, dim, W, H)
+    params = sc.params_bytes()
+    st = hip.Stream()
+    g.stream = st
+    graph = hip.Graph(st)
+    graph.begin()
+    g.InitialSampling()
+    g.EvalNewSamples(sc)
+    g.ComputeErrors()
+    graph.end()
+    for turn in range(5):
+        _say(f"captured setup {kind} replay {turn}")
+        graph.launch()
+        st.synchronize()
+        o = pyoracle.OracleGrid(*args)
+        o.initial_sampling()
+        o.eval_scene(params, 0, o.n_samples)
+        o.compute_errors()
+        for p in range(1 + turn):  # odd and even numbers of passes
+            if p == 0:
+                g.AdaptiveSampling()
+                o.adaptive_sampling()
+            else:
+                g.SamplingPass()
+                o.sampling_pass()
+            assert (g.GetNewSamples(), g.GetNewNodes()) == (o.new_samples, o.new_nodes)
+            assert (g.GetNumberOfSamples(), g.GetNumberOfNodes()) == (o.n_samples, o.n_leaves)
+            g.EvalNewSamples(sc)
+            st.synchronize()
+            o.eval_scene(params, o.n_samples - o.new_samples, o.new_samples)
+            _check(g, o, (turn, p))
+        o.close()
+    g.stream = None
+    graph.destroy()
+    st.destroy()
+    g.close()
+    sc.close()
