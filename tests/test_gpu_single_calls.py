@@ -123,3 +123,30 @@ def test_single_calls_after_a_captured_setup(mdas, kind, dim):
     st.destroy()
     g.close()
     sc.close()
+
+
+def test_max_error_brings_the_counts(mdas):
+    """GetMaxError reads the grid's counters back, after which the host's
+    counts are the tree's: also of one that a graph has started over."""
+    from pmdas_amd import hip
+    g, sc = mdas.KDGrid(3, 30000, 4, 0, 2, 0.25, 48.0, 32.0), mdas.Scene(1, 5, 3, 48.0, 32.0)
+    st = hip.Stream()
+    g.stream = st
+    graph = hip.Graph(st)
+    graph.begin()
+    g.InitialSampling()
+    graph.end()
+    g.Run(sc, 3000)
+    assert g.GetNumberOfSamples() >= 3000
+    graph.launch()
+    st.synchronize()
+    assert g.GetMaxError() == 0.0
+    assert (g.GetNumberOfSamples(), g.GetNumberOfNodes()) == (64, 16)
+    assert (g.GetNewSamples(), g.GetNewNodes()) == (64, 0)
+    g.Run(sc, 3000)
+    n, e = g.GetNumberOfSamples(), g.GetMaxError()
+    assert n == g.GetNumberOfSamples() >= 3000 and e > 0
+    graph.destroy()
+    st.destroy()
+    g.close()
+    sc.close()
