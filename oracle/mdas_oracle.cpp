@@ -793,6 +793,17 @@ long long orc_box_tiles(int w, int hgt, float sx, float sy, int tw, int th, cons
     }
     return n;
 }
+// The product's guess of a reconstruction's keys, for a tree of `leaves` leaves
+// grown from 2^(b dim + 2 e) cells, and the sort's workgroups for it.
+int orc_expected_keys(int w, int hgt, float sx, float sy, int tw, int th, int dim, int b, int e, long long leaves,
+                      double* keys) {
+    double ext[6];
+    for (int d = 0; d < dim; ++d)
+        ext[d] = (d == 0 ? sx : (d == 1 ? sy : 1.0)) / (double)(1 << (d < 2 ? b + e : b));
+    const mdas::ReconGeo G = mdas::recon_geo(w, hgt, sx, sy, tw, th);
+    *keys = mdas::expected_keys(G, (double)leaves, (double)(1ll << (b * dim + 2 * e)), dim, ext);
+    return mdas::sort_blocks(*keys, mdas::sort_digit(2 * G.tbits));
+}
 void orc_entries_of_thread(long long n, long long tid, long long threads, long long* out) {
     out[0] = out[1] = -1;
     out[2] = 0;

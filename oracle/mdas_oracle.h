@@ -68,6 +68,8 @@ int orc_eval_scene_cells(const void* scene_params, const void* coords, int dim, 
 long long orc_tile_entries(int w, int h, int tw, int th);
 long long orc_box_tiles(int w, int h, float sx, float sy, int tw, int th, const float* box, long long count,
                         int* out);
+int orc_expected_keys(int w, int h, float sx, float sy, int tw, int th, int dim, int b, int e, long long leaves,
+                      double* keys);
 void orc_entries_of_thread(long long n, long long tid, long long threads, long long* first_last_count);
 /* The plain QMC sampler's image (cuda/sampler.h:4-28, random.h:74-89,
  * whitted.cu:59-69): float4 pixels (fp64 = 0) or double4 (fp64 = 1). */

@@ -40,6 +40,7 @@ _SIGS = {
     "orc_eval_scene_cells": (_I, [_P, _P, _I, _LL, _I, _P]),
     "orc_tile_entries": (_LL, [_I, _I, _I, _I]),
     "orc_box_tiles": (_LL, [_I, _I, _F, _F, _I, _I, _P, _LL, _P]),
+    "orc_expected_keys": (_I, [_I, _I, _F, _F, _I, _I, _I, _I, _I, _LL, ctypes.POINTER(ctypes.c_double)]),
     "orc_entries_of_thread": (None, [_LL, _LL, _LL, _P]),
     "orc_qmc_image": (None, [_P, _I, _I, _I, _I, _U, _I, _P]),
     "orc_halton": (_F, [_I, _I]),
@@ -265,6 +266,13 @@ def box_tiles(w, h, sx, sy, tw, th, boxes):
     b = np.ascontiguousarray(boxes, np.float32).reshape(-1, 4)
     out = np.empty((len(b), 4), np.int32)
     return out, load().orc_box_tiles(w, h, sx, sy, tw, th, vp(b), len(b), vp(out))
+
+
+def expected_keys(w, h, sx, sy, tw, th, dim, b, e, leaves):
+    """(keys, workgroups of their sort) that the product expects of a tree."""
+    k = ctypes.c_double(0.0)
+    n = load().orc_expected_keys(w, h, sx, sy, tw, th, dim, b, e, int(leaves), ctypes.byref(k))
+    return k.value, n
 
 
 def entries_of_thread(n, tid, threads):

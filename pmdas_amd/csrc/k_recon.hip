@@ -29,8 +29,6 @@ namespace mdas {
 
 static const int kReconChunks = 4096;  // most leaf chunks of the record and key kernels
 static int recon_chunks(const Grid& g) { return std::min(g.chunks(), kReconChunks); }
-static const int kSortBlocks = 1024;
-static const int kSortMaxBits = 10;  // digit width limit (histograms of 1024 bins)
 static const int kSortKeysPerThread = 16;  // scatter tile: 4096 keys staged in LDS (8192: slower)
 
 __device__ __forceinline__ void record_span(const float4& q0, const ReconGeo& G, int& x0, int& x1,
@@ -326,13 +324,6 @@ __global__ __launch_bounds__(256) void k_rs_scatter(const unsigned long long* in
     }
 }
 
-// Workgroups of the sort: half a tile of the expected keys each (a leaf is in
-// 1.1 to 1.5 tiles), at most kSortBlocks; the kernels take any number of keys.
-static int sort_blocks(long long leaves, long long bound) {
-    const long long keys = std::min(leaves + leaves / 2, bound);
-    return (int)std::max<long long>(1, std::min<long long>(kSortBlocks, (keys + 2047) / 2048));
-}
-
 static void scan_u32(unsigned* data, int n, unsigned* sums, hipStream_t st) {
     const int nb = (n + 1023) / 1024;
     hipLaunchKernelGGL(k_scan_reduce, dim3(nb), dim3(1024), 0, st, data, n, sums);
@@ -358,16 +349,14 @@ static void sort_pass(Grid& g, unsigned* rs_hist, const unsigned long long* a, u
 
 // Sorts keys[0, n) by bits [lo, hi) in ceil((hi - lo) / 10) passes of equal
 // digit width; returns the buffer holding the result.
-static unsigned long long* radix_sort_keys(Grid& g, ReconBufs& rb, int lo, int hi, long long bound,
+static unsigned long long* radix_sort_keys(Grid& g, ReconBufs& rb, int lo, int hi, double expected,
                                            hipStream_t st) {
     unsigned long long* a = rb.keys;
     unsigned long long* b = rb.keys_alt;
     g.recon_sort_passes = 0;
     const int total = hi - lo;
     if (total <= 0) return a;
-    const int passes = (total + kSortMaxBits - 1) / kSortMaxBits;
-    const int bits = max(4, (total + passes - 1) / passes);
-    const int blocks = sort_blocks(g.host.n_leaves, bound);
+    const int bits = sort_digit(total), blocks = sort_blocks(expected, bits);
     for (int sh = lo; sh < hi; sh += bits) {
         switch (bits) {
         case 4: sort_pass<4>(g, rb.rs_hist, a, b, sh, blocks, st); break;
@@ -762,6 +751,14 @@ hipError_t recon_prepare(Grid& g, int W, int H, hipStream_t st) {
     return hipGetLastError();
 }
 
+// Keys that a tree of that many leaves is expected to give.
+static double recon_expected_keys(const Grid& g, long long leaves, int W, int H) {
+    const ReconGeo G = make_geo(g, W, H);
+    double e[6] = {g.ext_x, g.ext_y};
+    for (int d = 2; d < g.D; ++d) e[d] = 1.0 / (double)(1 << g.b);
+    return expected_keys(G, (double)leaves, (double)(1ll << (g.b * g.D + 2 * g.e)), g.D, e);
+}
+
 // Keys in leaf order, their sort, the tiles' key ranges and the gather, on
 // the buffers of rb (records already written by k_recon_prep).
 static hipError_t recon_finish(Grid& g, ReconBufs& rb, float* pixels, int W, int H, hipStream_t st,
@@ -777,7 +774,8 @@ static hipError_t recon_finish(Grid& g, ReconBufs& rb, float* pixels, int W, int
     if (ev_sort0) (void)hipEventRecord(ev_sort0, st);
     // the sorted keys end in keys or keys_alt by the parity of the pass
     // count; the buffers keep their roles, so a captured graph stays valid
-    unsigned long long* sorted = radix_sort_keys(g, rb, 32, 32 + 2 * G.tbits, bound, st);
+    const double expected = recon_expected_keys(g, g.host.n_leaves, W, H);
+    unsigned long long* sorted = radix_sort_keys(g, rb, 32, 32 + 2 * G.tbits, expected, st);
     g.keys_sorted = sorted;
     if (ev_sort1) (void)hipEventRecord(ev_sort1, st);
     kbeg(g, st, "k_tile_ranges");

@@ -72,6 +72,48 @@ MDAS_GEO int tiles_of(int x0, int x1, int y0, int y1, const ReconGeo& G) {
     return (((x1 - 1) >> G.lw) - (x0 >> G.lw) + 1) * (((y1 - 1) >> G.lh) - (y0 >> G.lh) + 1);
 }
 
+// Keys (leaves, once for each tile they touch) that a tree of `leaves` leaves
+// gives, from what the host knows: the initial cells' extents and number.  A
+// leaf is split along its longest axis, so one of a tree grown by 2^s has s
+// halvings behind it, taken in that order; one of p by q pixels touches
+// (1 + p / TW) (1 + q / TH) tiles on average.  Over 3 to 6 dimensions, sample
+// spaces of the unit square and of pixels, 1 .. 8192 initial cells and 100 to
+// 70000 leaves the count was 0.4 to 2.0 of this.  The keys per leaf run from 1.1
+// to thousands, since at a unit square x and y are halved no sooner than time
+// and lens: 354 leaves with 1.1 M keys at 1920x1080 took 7.05 ms with the sort
+// launched for 1.5 keys per leaf (one workgroup), 4.75 with 1024 workgroups
+// always and 0.90 with this; a 640x360 image of 314 thousand leaves is the same
+// in 8 x 8 and 4 x 4 tiles.
+inline double expected_keys(const ReconGeo& G, double leaves, double initial, int D, const double* extent) {
+    double e[8];
+    for (int d = 0; d < D; ++d) e[d] = extent[d];
+    for (double n = 2.0 * initial; n <= leaves; n *= 2.0) {
+        int k = 0;
+        for (int d = 1; d < D; ++d)
+            if (e[d] > e[k]) k = d;
+        e[k] *= 0.5;
+    }
+    const double x = 1.0 + e[0] * G.W / G.sX / G.TW, y = 1.0 + e[1] * G.H / G.sY / G.TH;
+    return leaves * (x < G.tilesX ? x : G.tilesX) * (y < G.tilesY ? y : G.tilesY);
+}
+
+// The sort's digits: ceil(bits / 10) passes of equal width, at least 4 bits.
+static const int kSortMaxBits = 10;  // histograms of 1024 bins
+inline int sort_digit(int bits) {
+    const int passes = (bits + kSortMaxBits - 1) / kSortMaxBits, d = (bits + passes - 1) / passes;
+    return d > 4 ? d : 4;
+}
+// Its workgroups for that many keys, at most 1024 (its kernels take any number
+// of keys): half a tile of 4096 each, a whole one for 10-bit digits, since each
+// brings counters for all its digits' values (a 640x360 image in 1 x 64 tiles,
+// 925 thousand keys: 561 workgroups 180 us, 281 166 us).
+static const int kSortBlocks = 1024;
+inline int sort_blocks(double keys, int digit) {
+    const int each = (4 << digit) > 2048 ? 4 << digit : 2048;
+    const double n = keys / each;
+    return n >= kSortBlocks ? kSortBlocks : (n <= 1.0 ? 1 : (int)n + 1);
+}
+
 // f(t) for the entries t of a table of n that thread `tid` of `threads` takes.
 template <typename F>
 MDAS_GEO void each_entry(long long n, long long tid, long long threads, F f) {

@@ -51,3 +51,23 @@ def test_a_box_touches_the_images_tiles_only(orc, size, tile, scale):
     first = np.maximum(a[inside] + 1e-3, 0) // (TW, TH)
     last = np.clip(b[inside] - 1e-3, 0, np.float64([W, H]) - 1e-3) // (TW, TH)
     assert np.all(out[inside][:, [0, 2]] <= first) and np.all(out[inside][:, [1, 3]] >= last)
+
+
+# dim, scene, b, e, sample space (None: the image's pixels)
+@pytest.mark.parametrize("dim,kind,b,e,scale", [(3, 1, 0, 0, 1.0), (5, 3, 0, 0, 1.0), (6, 4, 1, 0, 1.0), (4, 2, 0, 2, 1.0),
+                                                (5, 3, 0, 0, None), (5, 3, 1, 3, None), (3, 1, 0, 5, None)])
+def test_expected_keys(orc, dim, kind, b, e, scale):
+    """The sort is launched for the keys that the host expects of a tree: of
+    the order of its keys, from a leaf on the whole image to a leaf per tile."""
+    sx, sy = (scale, scale) if scale else (320.0, 180.0)
+    params = orc.make_scene(kind, 3, dim, sx, sy)
+    for n in (300, 3000, 30000):
+        o = orc.OracleGrid(dim, 4 * n + (8 << (b * dim + 2 * e)), 4, b, e, 0.25, sx, sy)
+        o.run(params, n)
+        for size, tile in (((320, 180), (8, 8)), ((1920, 1080), (8, 8)), ((80, 45), (4, 4)), ((320, 180), (64, 1))):
+            keys = len(o.recon_keys(*size, *tile))
+            want, blocks = orc.expected_keys(*size, sx, sy, *tile, dim, b, e, o.n_leaves)
+            assert want / 4 < keys < want * 4, (n, size, tile, o.n_leaves)
+            # no workgroup has more than 8 tiles of 4096 keys, unless all 1024 are at work
+            assert 1 <= blocks <= 1024 and (blocks == 1024 or keys <= blocks * 8 * 4096)
+        o.close()
