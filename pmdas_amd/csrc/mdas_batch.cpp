@@ -313,7 +313,8 @@ int mdas_batch_run(mdas_batch_handle b, const long long* targets, void* stream, 
 // into a hipGraph and replayed while every image's size, gather tile, output
 // and reconstruction buffers stay the same; the buffers are sized before the
 // capture from each image's leaf count, so nothing in the graph allocates or
-// waits for the host.  Stream-ordered: the caller synchronises.
+// waits for the host, and its launches are sized for the most leaves that they
+// hold.  Stream-ordered: the caller synchronises.
 int mdas_batch_integrate(mdas_batch_handle b, float* const* pixels, const int* widths,
                          const int* heights, void* stream, int use_graph) {
     if (!b || !pixels || !widths || !heights) return mdas::set_error(MDAS_ERR_INVALID, "null argument");
@@ -348,6 +349,7 @@ int mdas_batch_integrate(mdas_batch_handle b, float* const* pixels, const int* w
             (unsigned long long)(uintptr_t)pixels[i], (unsigned long long)widths[i],
             (unsigned long long)heights[i], (unsigned long long)g.tile_w, (unsigned long long)g.tile_h,
             (unsigned long long)g.chunk_blocks, (unsigned long long)(uintptr_t)g.rb.rrec,
+            (unsigned long long)mdas::recon_expected_keys(g, g.rb.rrec_cap, widths[i], heights[i]),
             (unsigned long long)(uintptr_t)g.rb.keys, (unsigned long long)(uintptr_t)g.rb.keys_alt,
             (unsigned long long)g.rb.keys_cap, (unsigned long long)(uintptr_t)g.rb.tile_start,
             (unsigned long long)(uintptr_t)g.rb.tile_end, (unsigned long long)(uintptr_t)g.rb.rs_hist};

@@ -338,6 +338,8 @@ long long recon_bytes_needed(const Grid& g, int W, int H);
 // Its parts: the key bound and the tile-range entries.
 long long recon_key_bound(const Grid& g, int W, int H);
 long long recon_tiles_cap(const Grid& g, int W, int H);
+// Keys that a tree of that many leaves is expected to give.
+double recon_expected_keys(const Grid& g, long long leaves, int W, int H);
 hipError_t launch_integrate_scatter(Grid& g, float* pixels, int W, int H, hipStream_t st);
 hipError_t launch_bytes(const float* pixels, unsigned char* out, long long n, hipStream_t st);
 

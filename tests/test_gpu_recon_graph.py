@@ -136,3 +136,72 @@ def test_batch_graph_keeps_null_stream_order(mdas):
     b.close()
     for x in bufs + grids + scenes:
         x.close() if hasattr(x, "close") else x.free()
+
+
+def _grids_of(graph):
+    """Workgroups of the captured graph's kernels, in node order."""
+    from pmdas_amd import hip
+
+    class Dim3(ctypes.Structure):
+        _fields_ = [(a, ctypes.c_uint32) for a in "xyz"]
+
+    class Kernel(ctypes.Structure):  # hipKernelNodeParams
+        _fields_ = [("block", Dim3), ("extra", ctypes.c_void_p), ("func", ctypes.c_void_p), ("grid", Dim3),
+                    ("params", ctypes.c_void_p), ("lds", ctypes.c_uint)]
+
+    lib = hip.lib()
+    n = ctypes.c_size_t(0)
+    assert lib.hipGraphGetNodes(ctypes.c_void_p(graph.graph), None, ctypes.byref(n)) == 0 and n.value > 0
+    nodes = (ctypes.c_void_p * n.value)()
+    assert lib.hipGraphGetNodes(ctypes.c_void_p(graph.graph), nodes, ctypes.byref(n)) == 0
+    out = []
+    for v in nodes:
+        kind = ctypes.c_int(-1)
+        assert lib.hipGraphNodeGetType(ctypes.c_void_p(v), ctypes.byref(kind)) == 0
+        assert kind.value == 0  # kernels only
+        k = Kernel()
+        assert lib.hipGraphKernelNodeGetParams(ctypes.c_void_p(v), ctypes.byref(k)) == 0
+        out.append(k.grid.x)
+    return out
+
+
+def test_graph_of_a_small_tree_suits_a_large_one(mdas):
+    """A reconstruction captured while the tree is small is replayed for the
+    trees that its buffers hold: its launches are theirs, and its pixels."""
+    from pmdas_amd import hip
+    W, H = 256, 192
+    g, sc, target = _grid(mdas, 5, W, H, 16, 3, 4, e=4)
+    g.Run(sc, target)
+    want = g.integrate_image(W, H)  # buffers for the large tree
+    st = hip.Stream()
+    buf = hip.DeviceBuffer(W * H * 16)
+    graphs = []
+    for size in ("small", "large"):
+        if size == "small":
+            g.InitialSampling()
+            g.EvalNewSamples(sc)
+        else:
+            g.Run(sc, target)
+        hip.synchronize()
+        g.stream = st
+        graph = hip.Graph(st)
+        graph.begin()
+        g.Integrate(buf.ptr, W, H)
+        graph.end()
+        g.stream = None
+        graphs.append(graph)
+    assert _grids_of(graphs[0]) == _grids_of(graphs[1])
+    for r in range(3):
+        for graph in graphs:
+            buf.upload(np.full(W * H * 4, np.nan, np.float32))
+            graph.launch()
+            st.synchronize()
+            got = buf.download(np.float32, W * H * 4).reshape(H, W, 4)
+            assert np.array_equal(got.view(np.uint32), want.view(np.uint32)), r
+        assert np.array_equal(g.integrate_image(W, H).view(np.uint32), want.view(np.uint32))
+    for graph in graphs:
+        graph.destroy()
+    st.destroy()
+    buf.free()
+    g.close()
+    sc.close()
