@@ -10,7 +10,6 @@
 #include <cfloat>
 #include <chrono>
 #include <cmath>
-#include <cstddef>
 #include <fstream>
 #include <string>
 #include <thread>
@@ -719,23 +718,11 @@ float mdas_get_scale_x(mdas_handle h) { return h ? h->g.sX : 0.0f; }
 float mdas_get_scale_y(mdas_handle h) { return h ? h->g.sY : 0.0f; }
 float mdas_get_max_error(mdas_handle h) {
     if (!h) return 0.0f;
-    // g_error's groups and the counters, which lie behind them
-    struct {
-        mdas::SuperMax g_error[mdas::kSuper];
-        mdas::DevCounters cnt;
-    } t;
-    static_assert(offsetof(mdas::DevTotals, cnt) ==
-                      offsetof(mdas::DevTotals, smax) + sizeof(mdas::SuperMax) * (mdas::kGError + 1) * mdas::kSuper,
-                  "the counters behind g_error's groups");
     Grid& g = h->g;
-    if (hipMemcpy(&t, g.dev.smax + mdas::kGError * mdas::kSuper, sizeof(t), hipMemcpyDeviceToHost) != hipSuccess)
-        return 0.0f;
-    static_cast<mdas::DevCounters&>(g.host) = t.cnt;
-    g.host.name_counts();
-    unsigned bits = 0u;
-    for (const auto& m : t.g_error) bits = std::max(bits, m.err);
+    if (mdas::launch_report(g, nullptr) != hipSuccess || hipStreamSynchronize(nullptr) != hipSuccess) return 0.0f;
+    mdas::take_counters(g);
     float e;
-    memcpy(&e, &bits, 4);
+    memcpy(&e, &g.dev.hrun->g_error, 4);
     return e;
 }
 int mdas_get_passes(mdas_handle h) { return h ? h->g.passes : 0; }

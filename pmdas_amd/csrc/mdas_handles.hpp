@@ -22,8 +22,8 @@ int set_error(int code, const std::string& msg);
 int sync_grid(Grid& g, hipStream_t st);
 // The largest leaf extents of a fresh initial grid (after initial sampling).
 void initial_extents(Grid& g);
-// What a run's last kernel or a single pass left of the counters, once it has
-// finished.
+// What a run's last kernel, a single pass or a report left of the counters,
+// once it has finished.
 void take_counters(Grid& g);
 // Appends the rows of the passes before `done`, which have finished, to
 // g.pstats_host (at most kHostRows of them since the last call).

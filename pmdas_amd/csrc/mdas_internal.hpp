@@ -82,7 +82,8 @@ static const int kPassWords = sizeof(PassStat) / sizeof(int);
 static const int kHostRows = 256;  // rows in turn; the host takes them before they wrap
 struct HostRun {
     unsigned long long row[kHostRows][kPassWords];
-    DevCounters cnt;  // as a run's last kernel or a single pass leaves them
+    DevCounters cnt;  // as a run's last kernel, a single pass or a report leaves them
+    unsigned g_error;  // float bits, as a report leaves them
 };
 static const unsigned kRunTag = 0x80000000u;  // set in the tags that a host waits for: those of a
                                               // batch's passes, which nothing waits for, stay below
@@ -298,6 +299,8 @@ hipError_t launch_mark_last_children(Grid& g, hipStream_t st);
 hipError_t launch_arm(Grid& g, bool errors, bool adaptive, hipStream_t st);
 hipError_t launch_compute_errors(Grid& g, hipStream_t st);
 hipError_t launch_adaptive(Grid& g, hipStream_t st);
+// g_error and the counters as they stand, into the host's memory.
+hipError_t launch_report(Grid& g, hipStream_t st);
 hipError_t launch_build_pts(Grid& g, int n_leaves, hipStream_t st);
 hipError_t launch_fill_f32(float* p, float v, long long n, hipStream_t st);
 
