@@ -134,6 +134,37 @@ def test_mlp_gradient_row_counts(mdas, n):
     m.close()
 
 
+# The last rows decide: those before `first` have the network's own output for a
+# target (up to its rounding), the others are 8 off, the very last 24.  The row
+# counts end in a tile's, a workgroup's and the largest grid's last rows and
+# first ones.
+@pytest.mark.parametrize("n,first", [(15, 14), (16, 15), (17, 16), (64, 63), (65, 64), (1024, 1023), (1025, 1024),
+                                     (32768, 32752), (32768 + 1, 32768), (32768 + 17, 32768),
+                                     (65536, 65520), (65536 + 65, 65536)])
+def test_mlp_gradient_of_the_last_rows(mdas, n, first):
+    _say(f"mlp gradient n={n} from {first}")
+    p = _params(6)
+    r = np.random.default_rng(n)
+    X = r.standard_normal((n, 16)).astype(np.float32)
+    T = mo.forward(p, X).astype(np.float32)
+    T[first:] -= 8.0
+    T[-1] -= 16.0
+    gw, lw = mo.grad(p, X, T)
+    # 1 % as for the rows of the test above (an activation at a bf16 tie), of
+    # which the first rows have next to nothing to add; without the last rows,
+    # without the last one or with it alone the oracle is far off
+    for rows in {(0, first), (0, n - 1)} | ({(n - 1, n)} if first < n - 1 else set()):
+        part, lp = mo.grad(p, X[slice(*rows)], T[slice(*rows)])
+        k = (rows[1] - rows[0]) / n
+        assert np.linalg.norm(part * k - gw) > 0.05 * np.linalg.norm(gw) and abs(lp * k - lw) > 0.05 * lw
+    m = mdas.Mlp(0)
+    m.set_params(p)
+    g, loss = m.grad(X, T)
+    assert abs(loss - lw) < 1e-2 * lw
+    assert np.linalg.norm(g - gw) < 1e-2 * np.linalg.norm(gw)
+    m.close()
+
+
 def test_adam_step_matches_oracle(mdas):
     _say("adam step")
     from pmdas_amd import hip
