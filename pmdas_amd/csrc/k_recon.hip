@@ -357,6 +357,7 @@ static unsigned long long* radix_sort_keys(Grid& g, ReconBufs& rb, int lo, int h
     const int total = hi - lo;
     if (total <= 0) return a;
     const int bits = sort_digit(total), blocks = sort_blocks(expected, bits);
+    g.recon_sort_blocks = blocks;
     for (int sh = lo; sh < hi; sh += bits) {
         switch (bits) {
         case 4: sort_pass<4>(g, rb.rs_hist, a, b, sh, blocks, st); break;

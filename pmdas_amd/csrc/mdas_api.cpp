@@ -988,7 +988,8 @@ static double kernel_bytes(const Grid& g, const std::string& k) {
     if (k == "k_recon_prep") return L * (SB + 32.0) + 12.0 * N;
     if (k == "k_recon_emit") return L * 16.0 + K * 8.0;
     if (k == "k_rs_hist") return K * 8.0 * g.recon_sort_passes;
-    if (k == "k_rs_scan") return 3.0 * 4.0 * (1 << g.recon_sort_bits) * 1024 * g.recon_sort_passes;
+    if (k == "k_rs_scan")  // a workgroup's counters read, read again and written
+        return 3.0 * 4.0 * (1 << g.recon_sort_bits) * g.recon_sort_blocks * g.recon_sort_passes;
     if (k == "k_rs_scatter") return K * 16.0 * g.recon_sort_passes;
     if (k == "k_tile_ranges") return K * 8.0;
     if (k == "k_gather") return K * (8.0 + 32.0) + 16.0 * (double)g.recon_pixels;

@@ -246,6 +246,7 @@ struct Grid {
     long long recon_pixels = 0;
     int recon_sort_passes = 0;
     int recon_sort_bits = 8;  // digit width of the last reconstruction sort
+    int recon_sort_blocks = 0;  // its workgroups
     // launch shape of the per-pass kernels (mdas_set_launch_shape)
     int chunk_blocks = 4096;   // leaf chunks of selection / compaction / reconstruction
     int err_blocks = 1024;     // workgroups of the error pass

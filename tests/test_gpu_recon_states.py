@@ -91,3 +91,22 @@ def test_boxes_outside_the_image(mdas, tile, off):
         got = g.integrate_image(W, H, scatter=scatter)[..., :3]
         assert np.abs(got - want).max() < 5e-3 and want.max() > 0.1
     g.close()
+
+
+@pytest.mark.parametrize("size", [(48, 32), (640, 360)])
+def test_the_sorts_bytes(mdas, size):
+    """The byte model of the sort's scan holds the counters that it had, those
+    of the workgroups launched for the tree."""
+    W, H = size
+    g, sc = mdas.KDGrid(5, 40000, 4, 0, 2, 0.25, float(W), float(H)), mdas.Scene(3, 3, 5, float(W), float(H))
+    g.set_timing(True)
+    g.Run(sc, 20000)
+    g.integrate_image(W, H)
+    tiles = max(-(-W // 8), -(-H // 8))
+    bits = 2 * (tiles - 1).bit_length()
+    passes = -(-bits // 10)
+    digit = max(4, -(-bits // passes))
+    blocks = pyoracle.expected_keys(W, H, W, H, 8, 8, 5, 0, 2, g.GetNumberOfNodes())[1]
+    assert g.kernel_stats()["k_rs_scan"][2] == 12.0 * 2 ** digit * blocks * passes
+    g.close()
+    sc.close()
