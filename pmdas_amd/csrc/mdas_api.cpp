@@ -345,7 +345,7 @@ int mdas_initial_sampling(mdas_handle h, void* stream) {
     HIP_TRY(mdas::launch_initial(g, L0, 0x7fffffff, st));
     g.initialized = true;
     set_initial_extents(g);
-    g.host = mdas::HostCounters{};
+    g.host.cur = g.host.passes = 0;  // the last reconstruction's key count stays
     g.host.slot[0] = mdas::TreeCounts{4 * L0, L0, 0, 0, 4 * L0, 0};
     g.host.name_counts();
     if (logging) {

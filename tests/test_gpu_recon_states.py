@@ -110,3 +110,18 @@ def test_the_sorts_bytes(mdas, size):
     assert g.kernel_stats()["k_rs_scan"][2] == 12.0 * 2 ** digit * blocks * passes
     g.close()
     sc.close()
+
+
+def test_bytes_of_a_reconstruction_outlive_its_tree(mdas):
+    """kernel_stats is of the last reconstruction, also once the grid has
+    started over."""
+    g, sc = mdas.KDGrid(3, 40000, 4, 0, 2, 0.25, 48.0, 32.0), mdas.Scene(1, 3, 3, 48.0, 32.0)
+    g.set_timing(True)
+    g.Run(sc, 20000)
+    g.integrate_image(48, 32)
+    before = g.kernel_stats()
+    assert before["k_rs_hist"][2] == 8.0 * len(g.recon_keys()) * before["k_rs_hist"][0]
+    g.InitialSampling()
+    assert g.kernel_stats()["k_rs_hist"] == before["k_rs_hist"]
+    g.close()
+    sc.close()
