@@ -612,7 +612,9 @@ __device__ __forceinline__ void place_leaf(const DevGrid& a, int i, int k, int m
 // for the pass after (no kernel of this pass reads those) and, into the host's
 // memory, the pass's statistics in a loop, which knows before the placement
 // itself whether another pass follows, or a single call's counters.
-// s, P and t (the lane's super group) are loaded by the caller, together.
+// s, P and t (the lane's super group) are loaded by the caller, together.  Only
+// PLACE_ONLY runs outside a loop too.
+template <int MODE>
 __device__ __forceinline__ bool pass_offsets(const DevGrid& a, int blk, int nblk, int par, const TreeCounts& s,
                                              int P, const int3& t, int2& base) {
     DevCounters* cn = a.cnt;
@@ -632,7 +634,8 @@ __device__ __forceinline__ bool pass_offsets(const DevGrid& a, int blk, int nblk
         // leaves whose errors were estimated since the last pass, and the
         // values that took: the initial leaves, then the children
         const int stale = P == 0 ? L : 2 * s.new_n, vals = P == 0 ? 4 * L : 5 * s.new_n;
-        if (a.in_loop && lane < kPassWords) {
+        const bool in_loop = MODE != PLACE_ONLY || a.in_loop != 0;
+        if (in_loop && lane < kPassWords) {
             const int w[kPassWords] = {L, N, sel, split, held, stale, vals, fits ? 0 : MDAS_ERR_CAPACITY_DEV};
             int v = 0;
 #pragma unroll
@@ -655,7 +658,7 @@ __device__ __forceinline__ bool pass_offsets(const DevGrid& a, int blk, int nblk
                 cn->slot[par ^ 1] = TreeCounts{N + sel, L + split, N, L, sel, split};
                 cn->cur = par ^ 1;
             }
-            if (!a.in_loop) a.hrun->cnt = *cn;
+            if (!in_loop) a.hrun->cnt = *cn;
         }
     }
     if (!fits) return false;
@@ -731,7 +734,7 @@ __device__ __forceinline__ void compact_place_body(const DevGrid& a, int blk, in
         for (int q = threadIdx.x; q < n_obj * mscene::OBJ_STRIDE; q += 256) obj[q] = B->p.obj[q];
     }
     int2 base;
-    if (!pass_offsets(a, blk, nblk, par, s, P, t, base)) return;
+    if (!pass_offsets<MODE>(a, blk, nblk, par, s, P, t, base)) return;
     float emax = 0.0f;
     int jq = base.x;  // global rank of the entry at the front of the queue
     int qn = 0;       // queued entries
