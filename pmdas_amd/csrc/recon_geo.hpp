@@ -104,13 +104,14 @@ inline int sort_digit(int bits) {
     return d > 4 ? d : 4;
 }
 // Its workgroups for that many keys, at most 1024 (its kernels take any number
-// of keys): half a tile of 4096 each, a whole one for 10-bit digits, since each
-// brings counters for all its digits' values (a 640x360 image in 1 x 64 tiles,
-// 925 thousand keys: 561 workgroups 180 us, 281 166 us).
+// of keys): half a tile of 4096 each, up to a whole one for 10-bit digits where
+// every CU has one, since each brings counters for all its digits' values (a
+// 640x360 image in 1 x 64 tiles, 925 thousand keys: 561 workgroups 180 us, 281
+// 166 us).
 static const int kSortBlocks = 1024;
 inline int sort_blocks(double keys, int digit) {
-    const int each = (4 << digit) > 2048 ? 4 << digit : 2048;
-    const double n = keys / each;
+    double n = keys / 2048.0;
+    if (digit > 9 && n > 256.0) n = n > 512.0 ? 0.5 * n : 256.0;
     return n >= kSortBlocks ? kSortBlocks : (n <= 1.0 ? 1 : (int)n + 1);
 }
 
