@@ -20,8 +20,8 @@
  *    (SDK/cuda/whitted.h:76-81).
  *  - a pass that would exceed max_samples returns MDAS_ERR_CAPACITY and leaves
  *    samples and tree unchanged (the reference writes out of bounds).
- *  - indices are allocated in leaf order by a device-wide scan, so results are
- *    deterministic (the reference's warp atomics are one of many orders).
+ *  - indices are allocated in leaf order (from the chunks' counts), so results
+ *    are deterministic (the reference's warp atomics are one of many orders).
  */
 #ifndef MDAS_H
 #define MDAS_H

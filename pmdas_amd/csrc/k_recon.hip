@@ -726,7 +726,7 @@ hipError_t recon_reserve(Grid& g, int W, int H) {
     return hipSuccess;
 }
 
-// Per-leaf records, tile counts and their scan.  Stream-ordered when the key
+// Per-leaf records and tile counts.  Stream-ordered when the key
 // buffers hold the bound; otherwise the key count is read back (a
 // synchronisation) and the buffers grown to it.
 hipError_t recon_prepare(Grid& g, int W, int H, hipStream_t st) {

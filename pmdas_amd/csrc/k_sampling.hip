@@ -1,6 +1,6 @@
 // Sampling kernels of the MDAS grid: initial Morton grid, per-leaf error with
 // the global max, and the adaptive pass (selection, best-candidate placement,
-// median split) with indices allocated by a deterministic device-wide scan.
+// median split) with indices allocated in leaf order.
 //
 // Layout (HBM): sample coordinates AoS float[D] and values float3 (the
 // integrand contract); one 128-byte line per leaf (slots, box and its first
@@ -676,19 +676,20 @@ __device__ __forceinline__ bool pass_offsets(const DevGrid& a, int blk, int nblk
 // they start from queue up in LDS and are placed a round of 256 at a time,
 // one per thread.  Every leaf's count and LCG state are rewritten in the
 // same sweep, as they stand after the placement, in full coalesced lines.
-// What bounds it at 1080p is the traffic of its scattered lines (5D: 800 MB a
-// pass of 238 us, 3/4 of a copy's rate) and, beside it, the vector units, half
+// What bounds it at 1080p is the traffic of its scattered lines (5D, 39
+// passes: 800 MB a pass of 238 us, 3/4 of a copy's rate) and, beside it, the vector units, half
 // the time busy with some 3000 instructions per 64 new samples, a third of them
 // the integrand's; a small tree's pass is the chain of its launches and of one
 // leaf's work.  So the loads before the first leaf go out in two rounds, what
 // the kernel does not write it reads through the scalar cache (the scene's
 // 105 uniform loads in the integrand were vector loads, each waited for; a batch
 // read its pointers as flat ones and spilled 20 registers), and registers are
-// held to five waves: 4D 1080p 8.85 -> 7.95 ms a run, 5D 14.76 -> 14.26, batch of
-// eight 12.70 -> 10.82, 333x517 874 -> 829 us.  Taking the integrand and the
+// held to five waves: 4D 1080p 8.26 -> 7.50 ms a run, 5D 13.78 -> 13.65, batch of
+// eight 12.48 -> 10.73, 333x517 840 -> 796 us (both timed in turn on one card,
+// reconstruction included).  Taking the integrand and the
 // children's errors along saves two launches of four and the split entries: 5D
-// 1080p (1.5 M leaves a pass) 15.6 -> 14.7 ms a run, 64x48 (12 passes of 2000)
-// 617 -> 458 us, 3D 256x256 1240 -> 850 us.  One chunk per wave in place of one
+// 1080p (1.5 M leaves a pass) 15.6 -> 14.6 ms a run, 64x48 (12 passes of 2000)
+// 617 -> 457 us, 3D 256x256 1240 -> 861 us.  One chunk per wave in place of one
 // per workgroup (fewer barriers, 4x the chunks) was slower at 1080p (12.0 ->
 // 12.9 ms a run at its best count) and no faster below.  What streams through
 // once, the flags and states of the sweep and the new coordinates, goes past
@@ -806,8 +807,8 @@ __device__ __forceinline__ void compact_place_body(const DevGrid& a, int blk, in
 }
 
 // The scene's objects in dynamic LDS (48 bytes each).  The registers are held to
-// five waves per SIMD, which nothing spills for (4D 1080p, 57 passes: four
-// waves 8.46 ms a run, five 7.95, six with spills 8.60); a 6D leaf needs the
+// five waves per SIMD, which nothing spills for (4D 1080p, 57 passes: a run takes
+// 6 % more with four, 8 % more with six, which spill); a 6D leaf needs the
 // registers of four.
 template <int D, int MODE>
 __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(D == 6 ? 4 : 5))) void k_compact_place(

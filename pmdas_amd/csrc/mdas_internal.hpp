@@ -141,7 +141,8 @@ struct DevGrid {
     int4* sext;            // [cap_l/2+1][2] learned mode only (else null): per split the
                            //   parent's box extents with the left child's at the split axis,
                            //   the right child's extent at the axis, the axis
-    int4* part;            // [kChunkBlocks] per-workgroup (selected, split, samples held)
+    int4* part;            // [kChunkBlocks] per chunk (selected, split, samples held); between
+                           //   passes a reconstruction's key counts
     DevCounters* cnt;
     SuperSum* ssum;        // [kSumSets][kSuper]
     SuperMax* smax;        // [kMaxSets][kSuper]

@@ -366,7 +366,7 @@ MDAS_HD uint64_t cell_word(const Params& P, const Cells& C, int c, int w) {
 
 // A cell's set: its words, and the first of them, which is loaded where the cell
 // is known, ahead of its use (a load is some 600 ns away: a pass's placement at
-// 64x48 15.6 -> 14.0 us, 4D 1080p 7.93 -> 7.62 ms a run).
+// 64x48 15.6 -> 14.0 us, 4D 1080p 7.28 -> 6.99 ms a run).
 struct CellSet {
     const uint64_t* words;
     uint64_t first;
